@@ -175,10 +175,16 @@ std::atomic<unsigned int> g_team_calls{0};
 // clock: one second unless mi355x_rownorm_set_team_wait_us() says otherwise.
 std::atomic<unsigned long long> g_team_wait_ticks{100000000ull};
 
-// The slot and id of a new call on the current device, or null when the team
-// kernel is not to be used: the address is not known, or the stream is being
-// captured (a replay would run with the id of the capture).
-void* team_slot_for_call(hipStream_t stream, unsigned int* id) {
+// The same for the strided softmax, whose workgroups pass numbers for every column.
+static __device__ __align__(256) __attribute__((used)) TeamColumns team_columns[kTeamSlots];
+std::atomic<void*> g_team_columns_ptr[kMaxDevices];
+
+// The slot and id of a new call on the current device out of the kTeamSlots slots of `slot_bytes`
+// at `symbol` (its per-device addresses: `table`), or null when the team kernel is not to be
+// used: the address is not known, or the stream is being captured (a replay would run with the
+// id of the capture).
+void* team_memory_for_call(std::atomic<void*>* table, const void* symbol, size_t slot_bytes,
+                           hipStream_t stream, unsigned int* id) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &st) != hipSuccess) {
     (void)hipGetLastError();
@@ -187,18 +193,26 @@ void* team_slot_for_call(hipStream_t stream, unsigned int* id) {
   if (st != hipStreamCaptureStatusNone) return nullptr;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
-  void* p = g_team_ptr[dev].load(std::memory_order_acquire);
+  void* p = table[dev].load(std::memory_order_acquire);
   if (p == nullptr) {
-    if (hipGetSymbolAddress(&p, HIP_SYMBOL(team_slots)) != hipSuccess || p == nullptr) {
+    if (hipGetSymbolAddress(&p, symbol) != hipSuccess || p == nullptr) {
       (void)hipGetLastError();
       return nullptr;
     }
-    g_team_ptr[dev].store(p, std::memory_order_release);
+    table[dev].store(p, std::memory_order_release);
   }
   unsigned int n = g_team_calls.fetch_add(1, std::memory_order_relaxed) + 1;
   if (n == 0) n = g_team_calls.fetch_add(1, std::memory_order_relaxed) + 1;  // 0 tags nothing
   *id = n;
-  return (char*)p + (size_t)(n % kTeamSlots) * sizeof(TeamSlot);
+  return (char*)p + (size_t)(n % kTeamSlots) * slot_bytes;
+}
+
+void* team_slot_for_call(hipStream_t stream, unsigned int* id) {
+  return team_memory_for_call(g_team_ptr, HIP_SYMBOL(team_slots), sizeof(TeamSlot), stream, id);
+}
+void* team_columns_for_call(hipStream_t stream, unsigned int* id) {
+  return team_memory_for_call(g_team_columns_ptr, HIP_SYMBOL(team_columns), sizeof(TeamColumns),
+                              stream, id);
 }
 
 int esize_of(int dt) {
@@ -874,6 +888,13 @@ int mi355x_softmax_strided_fwd(const void* x, void* y, int64_t outer, int64_t di
     return e;
   SoftmaxStridedFwdArgs a{x, y, outer, (int)dim_size, (int)inner, flags};
   hipStream_t s = (hipStream_t)stream;
+  // (a workgroup whose team does not come together reads the whole strip again; a team of one
+  // has nobody to wait for)
+  const int64_t n = outer * dim_size * inner;
+  if (plan.team > 1 && regions_disjoint(y, n * esize_of(od), x, n * esize_of(id))) {
+    a.team_slot = team_columns_for_call(s, &a.team_id);
+    a.team_wait_ticks = g_team_wait_ticks.load(std::memory_order_relaxed);
+  }
   if (id == ROWNORM_F32) return launch_softmax_strided_fwd<float, float>(plan, a, s);
   if (id == ROWNORM_BF16) return launch_softmax_strided_fwd<bf16, bf16>(plan, a, s);
   return od == ROWNORM_F32 ? launch_softmax_strided_fwd<f16, float>(plan, a, s)
@@ -899,6 +920,12 @@ int mi355x_softmax_strided_bwd(const void* grad, const void* y, void* gi, int64_
     return e;
   SoftmaxStridedBwdArgs a{grad, y, gi, outer, (int)dim_size, (int)inner, flags};
   hipStream_t s = (hipStream_t)stream;
+  const int64_t n = outer * dim_size * inner;
+  if (plan.team > 1 && regions_disjoint(gi, n * esize_of(od), grad, n * esize_of(gd)) &&
+      regions_disjoint(gi, n * esize_of(od), y, n * esize_of(gd))) {
+    a.team_slot = team_columns_for_call(s, &a.team_id);
+    a.team_wait_ticks = g_team_wait_ticks.load(std::memory_order_relaxed);
+  }
   if (gd == ROWNORM_BF16) return launch_softmax_strided_bwd<bf16, bf16>(plan, a, s);
   if (gd == ROWNORM_F16) return launch_softmax_strided_bwd<f16, f16>(plan, a, s);
   return od == ROWNORM_F16 ? launch_softmax_strided_bwd<float, f16>(plan, a, s)

@@ -95,6 +95,11 @@ struct SoftmaxStridedFwdArgs {
   int64_t outer;
   int D, inner;
   int flags;
+  // strips held by teams of workgroups (softmax_strided_team.hpp): the call's exchange memory
+  // (null: not for this call), its id and the bound of a wait
+  void* team_slot = nullptr;
+  unsigned int team_id = 0;
+  unsigned long long team_wait_ticks = 0;
 };
 
 struct SoftmaxStridedBwdArgs {
@@ -104,6 +109,11 @@ struct SoftmaxStridedBwdArgs {
   int64_t outer;
   int D, inner;
   int flags;
+  // strips held by teams of workgroups (softmax_strided_team.hpp): the call's exchange memory
+  // (null: not for this call), its id and the bound of a wait
+  void* team_slot = nullptr;
+  unsigned int team_id = 0;
+  unsigned long long team_wait_ticks = 0;
 };
 
 // GroupNorm on [N, C, HxW] with C = groups * D: rows = N * groups rows of L = D * HxW.

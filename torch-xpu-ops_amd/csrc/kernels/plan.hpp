@@ -119,6 +119,15 @@ struct TeamSlot {
   unsigned int pad[3];
 };
 
+// Columns (elements of `inner`) a strip of the strided team kernels has at most, and one call's
+// exchange memory there: [round parity][workgroup][number][column] words (softmax_strided_team.hpp).
+constexpr int kTeamColumns = 256;
+struct TeamColumns {
+  unsigned long long word[2][kTeamMaxWorkgroups][2 * kTeamColumns];
+  unsigned int gave_up;  // as in TeamSlot
+  unsigned int pad[3];
+};
+
 // softmax_fwd_team_kernel / softmax_bwd_team_kernel: rows of at least this many packs (64 KiB),
 // and the packs a lane the backward holds of each of its two tensors at most.
 constexpr int64_t kSoftmaxTeamMinPacks = 4096;
@@ -1067,7 +1076,8 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
 // as a row of `inner` has packs, capped so that a group is one wavefront where
 // that leaves at least 8 lanes (128-byte segments) per row, and 256 threads
 // otherwise.  A group of one wavefront reduces with shuffles alone.  D beyond
-// 64 rows x 8 packs x 4 lanes takes the multi-pass kernel.
+// 64 rows x 8 packs x 4 lanes takes the multi-pass kernel; from D = 257 strips of whole packs are
+// held by teams of workgroups where the call allows it.
 struct StridedPlan {
   bool resident = true;
   bool fast = true;  // inner % E == 0
@@ -1076,7 +1086,22 @@ struct StridedPlan {
   // multi-pass kernels with too few tiles for the machine: the D rows are cut into
   // `chunks` chunks of `chunk_rows` rows, one workgroup each (0 or 1: not split)
   int chunks = 0, chunk_rows = 0;
+  // strips held by teams of workgroups (softmax_strided_team.hpp); team 0: not this call.
+  // team_grid = teams * team workgroups, team_tx_log2 = log2 of the packs a strip is wide,
+  // team_v = packs a lane
+  int team = 0, team_v = 0, team_tx_log2 = 0;
+  int64_t team_grid = 0;
 };
+
+// The packs a lane the strided team kernels are built for: the forward holds one tensor, the
+// backward two.
+constexpr int kStridedTeamV[2][10] = {{1, 2, 3, 4, 6, 8, 10, 12, 14, 16}, {1, 2, 3, 4, 5, 6, 7, 8}};
+constexpr int strided_team_max_v(bool backward) { return backward ? 8 : 16; }
+// Lanes along `inner` at most: 256-byte row segments, or 512-byte ones.
+constexpr int kStridedTeamTx = 16;
+constexpr int kStridedTeamWideTx = 32;
+constexpr int64_t kStridedTeamMinD = 256;
+constexpr int64_t kStridedTeamWideMaxD = 4096;
 
 constexpr int kStridedSplitUnroll = 4;  // rows a lane of the split kernels requests at a time
 
@@ -1173,6 +1198,44 @@ inline int make_strided_plan(bool backward, int64_t outer, int64_t D, int64_t in
       // workgroups per compute unit
       while (TX > 4 && outer * ((packs + TX - 1) / TX) < 2 * (int64_t)num_cus) TX >>= 1;
       TY = kStridedBlock / TX;
+    }
+  }
+  // Strips held by teams of workgroups: as few workgroups a strip as hold its D rows, as many
+  // teams as strips and compute units allow, evened out over the rounds; then a strip is spread
+  // over the workgroups its team can have.  From D = 257, where the one-workgroup tile above is
+  // down to 64-byte row segments (bf16 forward / backward, tile -> team: [4, 512, 8192] 29.3 / 39.0
+  // -> 17.7 / 20.4 us, [64, 300, 800] 24.7 / 30.4 -> 17.5 / 26.4; at D = 200 the tile is ahead:
+  // [20, 200, 4096] 20.5 / 22.5 against 23.2 / 25.5).  Strips of 16 packs where a team holds them
+  // all at once or D needs large teams (the exchange grows with the columns), of 32 otherwise
+  // ([35, 1000, 1904]: 16 packs 95 / 111 us, 32 packs 79 / 97; [1, 8192, 8192]: 73 / 104, 79 / 103).
+  if (D > kStridedTeamMinD && p.fast && ov.G == 0 && ov.V == 0 && ov.bpc == 0) {
+    const int vmax = strided_team_max_v(backward);
+    const int64_t wgs = num_cus * kTeamPerCu < kTeamMaxWorkgroups ? num_cus * kTeamPerCu : kTeamMaxWorkgroups;
+    for (int wide = 0; wide < 2; ++wide) {
+      const int most_tx = wide ? kStridedTeamWideTx : kStridedTeamTx;
+      const int tx = px < most_tx ? px : most_tx;
+      const int64_t ty = kTeamBlock / tx;
+      const int64_t need = (D + ty * vmax - 1) / (ty * vmax);
+      const int64_t strips = outer * ((packs + tx - 1) / tx);
+      // (byte offsets of a lane inside a workgroup's rows are 32 bits wide)
+      if (need > wgs || ty * vmax * inner * 4 >= (int64_t(1) << 31)) break;
+      int64_t teams = wgs / need < strips ? wgs / need : strips;
+      const int64_t rounds = (strips + teams - 1) / teams;
+      teams = (strips + rounds - 1) / rounds;
+      const int64_t most = (D + ty - 1) / ty;
+      int64_t team = wgs / teams < most ? wgs / teams : most;
+      int64_t v = (D + ty * team - 1) / (ty * team);
+      for (int c : kStridedTeamV[backward ? 1 : 0])
+        if (c >= v) {
+          v = c;
+          break;
+        }
+      team = (D + ty * v - 1) / (ty * v);
+      p.team = (int)team;
+      p.team_v = (int)v;
+      p.team_tx_log2 = log2_of_pow2(tx);
+      p.team_grid = teams * team;
+      if (rounds == 1 || D > kStridedTeamWideMaxD || px <= kStridedTeamTx) break;
     }
   }
   p.resident = !stream;

@@ -2,8 +2,28 @@
 #pragma once
 #include "launch.hpp"
 #include "softmax_strided_kernels.hpp"
+#include "softmax_strided_team.hpp"
 
 namespace rownorm {
+
+template <int E>
+StridedTeamShape strided_team_shape(const StridedPlan& p, int64_t outer, int D, int inner) {
+  const int64_t packs = inner / E;
+  const int64_t xtiles = (packs + (1 << p.team_tx_log2) - 1) >> p.team_tx_log2;
+  return StridedTeamShape{outer * xtiles, xtiles, D, inner, p.team_tx_log2, p.team};
+}
+
+// Launches the instance whose packs a lane the plan names; false if there is none.
+template <bool BACKWARD, size_t I = 0, class Go>
+bool launch_strided_team(int v, Go go) {
+  constexpr int V = kStridedTeamV[BACKWARD ? 1 : 0][I];
+  if (v == V) {
+    go(std::integral_constant<int, V>{});
+    return true;
+  }
+  if constexpr (V < strided_team_max_v(BACKWARD)) return launch_strided_team<BACKWARD, I + 1>(v, go);
+  return false;
+}
 
 template <class TI, class TO, int V, bool FAST>
 void launch_strided_fwd_v(const StridedPlan& p, const SoftmaxStridedFwdArgs& a, hipStream_t s) {
@@ -30,7 +50,17 @@ bool launch_strided_fwd_f(const StridedPlan& p, const SoftmaxStridedFwdArgs& a, 
 template <class TI, class TO>
 int launch_softmax_strided_fwd(const StridedPlan& p, const SoftmaxStridedFwdArgs& a,
                                hipStream_t s) {
-  if (p.resident) {
+  if (p.team == 1 || (p.team > 1 && a.team_slot != nullptr)) {
+    const StridedTeamShape sh =
+        strided_team_shape<elems_per_pack<TI>::value>(p, a.outer, a.D, a.inner);
+    const bool ok = launch_strided_team<false>(p.team_v, [&](auto v) {
+      hipLaunchKernelGGL((softmax_strided_team_fwd_kernel<TI, TO, decltype(v)::value>),
+                         dim3((unsigned)p.team_grid), dim3(kTeamBlock), 0, s, (const TI*)a.x,
+                         (TO*)a.y, sh, a.flags, (TeamColumns*)a.team_slot, a.team_id,
+                         a.team_wait_ticks);
+    });
+    if (!ok) return (int)hipErrorInvalidConfiguration;
+  } else if (p.resident) {
     const bool ok = p.fast ? launch_strided_fwd_f<TI, TO, true>(p, a, s)
                            : launch_strided_fwd_f<TI, TO, false>(p, a, s);
     if (!ok) return (int)hipErrorInvalidConfiguration;
@@ -86,7 +116,17 @@ bool launch_strided_bwd_f(const StridedPlan& p, const SoftmaxStridedBwdArgs& a, 
 template <class TG, class TO>
 int launch_softmax_strided_bwd(const StridedPlan& p, const SoftmaxStridedBwdArgs& a,
                                hipStream_t s) {
-  if (p.resident) {
+  if (p.team == 1 || (p.team > 1 && a.team_slot != nullptr)) {
+    const StridedTeamShape sh =
+        strided_team_shape<elems_per_pack<TG>::value>(p, a.outer, a.D, a.inner);
+    const bool ok = launch_strided_team<true>(p.team_v, [&](auto v) {
+      hipLaunchKernelGGL((softmax_strided_team_bwd_kernel<TG, TO, decltype(v)::value>),
+                         dim3((unsigned)p.team_grid), dim3(kTeamBlock), 0, s, (const TG*)a.grad,
+                         (const TG*)a.y, (TO*)a.gi, sh, a.flags, (TeamColumns*)a.team_slot,
+                         a.team_id, a.team_wait_ticks);
+    });
+    if (!ok) return (int)hipErrorInvalidConfiguration;
+  } else if (p.resident) {
     const bool ok = p.fast ? launch_strided_bwd_f<TG, TO, true>(p, a, s)
                            : launch_strided_bwd_f<TG, TO, false>(p, a, s);
     if (!ok) return (int)hipErrorInvalidConfiguration;

@@ -1,0 +1,561 @@
+// softmax / log_softmax over a dimension that is not innermost, D beyond the one-workgroup tile of
+// softmax_strided_kernels.hpp: every element crosses the memory interface once.
+//
+// The tensor is [outer, D, inner]; a strip is TX consecutive 16-byte packs of `inner` (256 or 512
+// bytes) and all D rows under them.  A team of `team` workgroups of 512 threads holds a strip in
+// registers: workgroup c the rows [c * TY * V, (c + 1) * TY * V), thread (ty, tx) the V packs
+// of rows ty, ty + TY, ... of pack column tx.  A workgroup reduces its rows per column (each
+// lane over its packs, a wavefront by shuffles, the eight wavefronts through LDS), publishes the
+// C = TX * E columns' numbers -- running maximum and sum of exp(x - maximum), or the sum the
+// backward needs --, gathers its team's, merges them in a fixed order and writes its rows out of
+// its registers.  A team of one exchanges nothing.  Teams walk the strips in rounds.
+//
+// What bounds it.  The split over launches that served these shapes reads the inputs twice and
+// pays three launches; the multi-pass kernel reads them three times.  Here it is HBM plus what
+// does not run under it: the forward's two exponentials an element (31 us of vector ALU time a
+// [8192, 8192] call) and the exchange, about 5 us a round, since a tensor twice the size of what
+// 512 workgroups hold makes two (forward) or four rounds in step (without the exchange the same
+// kernel takes 63 / 92 us there).  bf16 forward / backward us, before -> with teams:
+// [8192, 8192] over dim 0 78.5 / 114 -> 72 / 104; [4000, 16384] 76.7 / 113 -> 63 / 82;
+// [8192, 64] 18.1 / 13.3 -> 10.9 / 8.1; [8, 1000, 1024] 23.4 / 18.5 -> 12.4 / 13.1;
+// [35, 1000, 1904] 151 / 176 -> 79 / 97; [100, 2000, 128] 39.0 / 46.4 -> 24.7 / 33.8.
+// Requesting the next strip ahead of the exchange (half the packs a lane, twice the rounds)
+// measured slower (84-90 us on [8192, 8192]), as did rows dealt out in bands over the team.
+//
+// The exchange.  A column's number travels as a self-validating 64-bit word {float32, tag} in
+// library-owned memory (TeamColumns; tags, the bounded wait, the lost tag and the hint word as
+// described in device/team.hpp): the writer orders nothing, a reader accepts a word whose tag is
+// the round's.  The first wavefront polls one word a member (all threads polling their own words
+// would be 16 MB of memory traffic a poll); once they are there every thread gathers: thread
+// (q, column) reads members q, q + Q, ... of its team, Q = 512 / C.  Two buffers suffice: a
+// workgroup publishes round r + 2 only after it has gathered round r + 1, which every mate
+// published after it had gathered round r.
+// A workgroup whose wait runs out walks all D rows of the strip itself (the output must not
+// overlap an input) and publishes the lost tag from then on.
+#pragma once
+#include "device/team.hpp"
+#include "softmax_strided_kernels.hpp"
+
+namespace rownorm {
+
+struct StridedTeamShape {
+  int64_t strips, xtiles;  // outer * xtiles strips, xtiles of them side by side along inner
+  int D, inner, tx_log2, team;
+};
+
+// A thread's place in a strip: pack column tx, rows ty, ty + TY, ...; the element of `inner` its
+// packs start at (0 where the strip is wider than what is left of `inner`: loaded, never stored).
+template <int E>
+struct StridedTeamPlace {
+  int tx, ty, TY, e0;
+  bool in;
+  __device__ __forceinline__ StridedTeamPlace(const StridedTeamShape& s, int tid, int64_t strip) {
+    tx = tid & ((1 << s.tx_log2) - 1);
+    ty = tid >> s.tx_log2;
+    TY = kTeamBlock >> s.tx_log2;
+    const int64_t e = (((strip % s.xtiles) << s.tx_log2) + tx) * E;
+    in = e < s.inner;
+    e0 = in ? (int)e : 0;
+  }
+};
+
+// A pointer into global memory, byte offset added per lane (an address made from an integer is
+// otherwise a generic one, whose accesses wait for everything outstanding).
+template <class P>
+__device__ __forceinline__ P* global_at(P* p, uint32_t off) {
+  typedef __attribute__((address_space(1))) P* GlobalPtr;
+  return (P*)reinterpret_cast<GlobalPtr>(reinterpret_cast<uintptr_t>(p) + off);
+}
+
+// A wavefront-uniform pointer the compiler cannot trace back: the V row pointers of a chunk are
+// formed one after the other, not held in registers all at once.
+template <class P>
+__device__ __forceinline__ P* scalar_again(P* p) {
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
+// The V packs of this thread: rows r0 + ty + k * TY, pack column e0 (an element index inside the
+// row).  One straight line for every workgroup (two versions of it would each want the packs in
+// registers of their own): rows past D - 1 read row D - 1 and are replaced by `fill`.
+template <class T, int E, int V>
+__device__ __forceinline__ void strided_team_load(Pack<T, E> (&p)[V], const T* strip, int r0,
+                                                  int ty, int TY, int e0, int D, int inner,
+                                                  float fill) {
+  const T* base = strip + (int64_t)r0 * inner;
+  const int last = D - 1 - r0;
+  ty = lane_again(ty);  // (offsets and bounds of the packs are formed here, not ahead of the strips)
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const int row = ty + k * TY;
+    const int rc = row < last ? row : last;
+    p[k] = Pack<T, E>::load_stream(
+        global_at(base, ((uint32_t)rc * (uint32_t)inner + (uint32_t)e0) * (uint32_t)sizeof(T)));
+  }
+  const Pack<T, E> f = Pack<T, E>::splat(fill);
+#pragma unroll
+  for (int k = 0; k < V; ++k)
+    if (ty + k * TY > last) p[k] = f;
+}
+
+// NF words a column: publishes v[0..NF) of the C columns (threads below C hold them).
+template <int NF>
+__device__ __forceinline__ void columns_publish(unsigned long long* mine, int C, bool lost,
+                                                unsigned int call_id, unsigned int round,
+                                                const float (&v)[NF]) {
+  if ((int)threadIdx.x < C) {
+    const unsigned long long tag =
+        (unsigned long long)(lost ? team_lost_tag(call_id) : team_word_tag(call_id, round)) << 32;
+#pragma unroll
+    for (int k = 0; k < NF; ++k)
+      team_store(&mine[k * kTeamColumns + (int)threadIdx.x],
+                 tag | (unsigned long long)__builtin_bit_cast(unsigned int, v[k]));
+  }
+}
+
+constexpr int kGatherWords = 8;  // words a thread requests before it looks at the first
+
+// Merges N (maximum, sum) pairs into (m, s): one maximum, then N + 1 independent exponentials
+// (pair by pair each merge would wait for the one before).
+template <bool PRECISE, int N>
+__device__ __forceinline__ void merge_pairs(float& m, float& s, const float (&vm)[N],
+                                            const float (&vs)[N]) {
+  float nm = m;
+#pragma unroll
+  for (int b = 0; b < N; ++b) nm = fmaxf(nm, vm[b]);
+  // (nothing finite: the sums are 0, or NaN if an operand carries one, whatever they are scaled by)
+  const float ref = nm == -INFINITY ? 0.0f : nm;
+  s *= row_exp<PRECISE>(m - ref);
+#pragma unroll
+  for (int b = 0; b < N; ++b) s = fmaf(vs[b], row_exp<PRECISE>(vm[b] - ref), s);
+  m = nm;
+}
+
+// Gathers this thread's share of the team: merge(v) is called with v[number][member] for members
+// q, q + Q, ..., B at a time, after reset(); -inf / 0 stand for members past the team's end.  Every thread of the workgroup calls it; the result is uniform: true when
+// all words of the round were there, false when the wait ran out or the call is lost.
+template <int NF, class Reset, class Merge>
+__device__ __forceinline__ bool columns_gather(TeamColumns* slot, const unsigned long long* mates,
+                                               int C, int team,
+                                               unsigned int call_id, unsigned int round,
+                                               unsigned long long wait_ticks,
+                                               int (&votes)[2][kTeamBlock / 64 + 1], Reset reset,
+                                               Merge merge) {
+  constexpr int B = kGatherWords / NF;
+  const int col = (int)threadIdx.x & (C - 1), q = (int)threadIdx.x / C, Q = kTeamBlock / C;
+  const unsigned int expect = team_word_tag(call_id, round);
+  const unsigned long long t0 = wall_clock64();
+  for (unsigned int polls = 0;; ++polls) {
+    int status = 0;  // 1, a word is missing; 2, a lost tag, a hint or the end of the wait
+    if (threadIdx.x < 64) {
+      // one word of every member, until they are all there
+      for (unsigned int n = 0;; ++n) {
+        bool ok = true;
+        status = 0;
+        for (int j = (int)threadIdx.x; j < team; j += 64) {
+          const unsigned int tag =
+              (unsigned int)(team_load(&mates[(int64_t)j * (2 * kTeamColumns) + C - 1]) >> 32);
+          ok = ok && tag == expect;
+          if (team_tag_is_lost(tag, call_id)) status = 2;
+        }
+        const bool late = wall_clock64() - t0 > wait_ticks;
+        if (__ballot(ok) == __ballot(true) && !(polls > 0 && late)) break;
+        // (the hint word is one address for the whole grid: looked at every 16th time)
+        if ((n & 15u) == 0 && __hip_atomic_load(&slot->gave_up, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT) == call_id)
+          status = 2;
+        if (late) status = 2;
+        if (__ballot(status != 0) != 0) break;
+        __builtin_amdgcn_s_sleep(8);
+      }
+    }
+    int (&vote)[kTeamBlock / 64 + 1] = votes[polls & 1u];
+    if (threadIdx.x < 64) {
+      const bool stop = __ballot(status != 0) != 0;
+      if (threadIdx.x == 0) vote[kTeamBlock / 64] = stop ? 2 : 0;
+    }
+    __syncthreads();
+    if (vote[kTeamBlock / 64] != 0) break;
+    reset();
+    status = 0;
+    for (int j0 = q; j0 < team; j0 += B * Q) {
+      unsigned long long w[B][NF];
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        const int j = j0 + b * Q;
+#pragma unroll
+        for (int k = 0; k < NF; ++k) w[b][k] = 0;
+        if (j < team) {
+#pragma unroll
+          for (int k = 0; k < NF; ++k)
+            w[b][k] = team_load(&mates[((int64_t)j * 2 + k) * kTeamColumns + col]);
+        }
+      }
+      float v[NF][B];
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+#pragma unroll
+        for (int k = 0; k < NF; ++k) v[k][b] = NF == 2 && k == 0 ? -INFINITY : 0.0f;
+        if (j0 + b * Q < team) {
+#pragma unroll
+          for (int k = 0; k < NF; ++k) {
+            if ((unsigned int)(w[b][k] >> 32) != expect) status = 1;
+            v[k][b] = __builtin_bit_cast(float, (unsigned int)(w[b][k] & 0xffffffffull));
+          }
+        }
+      }
+      merge(v);
+    }
+    const bool missing = __ballot(status != 0) != 0;
+    if ((threadIdx.x & 63) == 0) vote[threadIdx.x >> 6] = missing ? 1 : 0;
+    __syncthreads();
+    int all = 0;
+#pragma unroll
+    for (int w = 0; w < kTeamBlock / 64; ++w) all |= vote[w];
+    if (all == 0) return true;
+    // (the words that were missing are on their way, or the wait ends above)
+  }
+  if (threadIdx.x == 0)
+    __hip_atomic_store(&slot->gave_up, call_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return false;
+}
+
+// A wavefront's (m, s) per column, in every lane, from the lanes' own pairs.
+template <int E, bool PRECISE>
+__device__ __forceinline__ void wave_columns_merge(float (&m)[E], float (&s)[E], int TX) {
+  float own[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) own[i] = m[i];
+  for (int off = TX; off < 64; off <<= 1)
+#pragma unroll
+    for (int i = 0; i < E; ++i) m[i] = fmaxf(m[i], __shfl_xor(m[i], off, 64));
+#pragma unroll
+  for (int i = 0; i < E; ++i) s[i] = m[i] == -INFINITY ? s[i] : s[i] * row_exp<PRECISE>(own[i] - m[i]);
+  for (int off = TX; off < 64; off <<= 1)
+#pragma unroll
+    for (int i = 0; i < E; ++i) s[i] += __shfl_xor(s[i], off, 64);
+}
+
+constexpr int kStridedTeamGroup = 4;
+
+template <class TI, class TO, int V>
+__global__ void __launch_bounds__(kTeamBlock, kTeamPerCu * kTeamBlock / 256)
+softmax_strided_team_fwd_kernel(const TI* __restrict__ x, TO* __restrict__ y, StridedTeamShape sh,
+                                int flags, TeamColumns* slot, unsigned int call_id,
+                                unsigned long long wait_ticks) {
+  constexpr int E = elems_per_pack<TI>::value;
+  constexpr bool PRECISE = sizeof(TO) == 4;
+  constexpr int NW = kTeamBlock / 64;
+  __shared__ float wm[NW * kTeamColumns], ws[NW * kTeamColumns];  // the wavefronts' pairs
+  __shared__ int votes[2][kTeamBlock / 64 + 1];
+  __shared__ float gm[kTeamBlock], gs[kTeamBlock];                // the gathering threads' pairs
+  __shared__ __align__(16) float fm[kTeamColumns], fk[kTeamColumns];  // maximum, 1/sum or log(sum)
+  const bool is_log = (flags & kSoftmaxLog) != 0;
+  const bool is_safe = (flags & kSoftmaxSafe) != 0;
+  const int D = sh.D, inner = sh.inner, team = sh.team;
+  const int TX = 1 << sh.tx_log2, C = TX * E;
+  const int tm = (int)blockIdx.x / team;
+  const int teams = (int)gridDim.x / team;
+  const int r0 = ((int)blockIdx.x - tm * team) * (kTeamBlock >> sh.tx_log2) * V;
+  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+  bool lost = false;
+  unsigned int round = 0;
+  for (int64_t strip = tm; strip < sh.strips; strip += teams, ++round) {
+    Pack<TI, E> xp[V];
+    {
+      const StridedTeamPlace<E> t(sh, lane_again((int)threadIdx.x), strip);
+      strided_team_load<TI, E, V>(xp, x + (strip / sh.xtiles) * (int64_t)D * inner, r0, t.ty, t.TY,
+                                  t.e0, D, inner, -INFINITY);
+    }
+    // The lane's running maxima and sums, kGroup packs at a time: the exponentials of one group are
+    // formed while the next ones are still on their way.
+    float m[E], s[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      m[i] = -INFINITY;
+      s[i] = 0.0f;
+    }
+#pragma unroll
+    for (int k0 = 0; k0 < V; k0 += kStridedTeamGroup) {
+      const int kn = k0 + kStridedTeamGroup < V ? k0 + kStridedTeamGroup : V;
+      float ref[E];
+#pragma unroll
+      for (int i = 0; i < E; ++i) ref[i] = m[i];
+#pragma unroll
+      for (int k = k0; k < kn; ++k) {
+#pragma unroll
+        for (int i = 0; i < E; ++i) ref[i] = fmaxf(ref[i], xp[k].get(i));
+        keep_packed(xp[k]);
+      }
+      // (nothing finite so far: against 0, -inf elements add 0 and NaN still poisons)
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+        const float own = m[i];
+        m[i] = ref[i];
+        ref[i] = ref[i] == -INFINITY ? 0.0f : ref[i];
+        if (k0 > 0) s[i] *= row_exp<PRECISE>(own - ref[i]);
+      }
+#pragma unroll
+      for (int k = k0; k < kn; ++k) {
+#pragma unroll
+        for (int i = 0; i < E; ++i) s[i] += row_exp<PRECISE>(xp[k].get(i) - ref[i]);
+        keep_packed(xp[k]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    // (formed here: moved behind the reduction of the maxima it would need a copy of the packs)
+#pragma unroll
+    for (int i = 0; i < E; ++i) asm volatile("" : "+v"(s[i]));
+    // the pair of column threadIdx.x < C: the workgroup's, then the strip's
+    float pm = -INFINITY, ps = 0.0f;
+    auto merge_workgroup = [&]() {
+      wave_columns_merge<E, PRECISE>(m, s, TX);
+      if (lane < TX) {
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+          wm[wave * kTeamColumns + lane * E + i] = m[i];
+          ws[wave * kTeamColumns + lane * E + i] = s[i];
+        }
+      }
+      __syncthreads();
+      if ((int)threadIdx.x < C) {
+        float vm[NW], vs[NW];
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+          vm[w] = wm[w * kTeamColumns + threadIdx.x];
+          vs[w] = ws[w * kTeamColumns + threadIdx.x];
+        }
+        pm = -INFINITY;
+        ps = 0.0f;
+        merge_pairs<PRECISE>(pm, ps, vm, vs);
+      }
+    };
+    merge_workgroup();
+    unsigned long long* words = &slot->word[round & 1u][0][0];
+    if (team > 1)
+      columns_publish<2>(words + (int64_t)blockIdx.x * (2 * kTeamColumns), C, lost, call_id, round,
+                         {pm, ps});
+    if (team > 1) {
+      float am = -INFINITY, as = 0.0f;
+      if (!lost)
+        lost = !columns_gather<2>(
+            slot, words + (int64_t)tm * team * (2 * kTeamColumns), C, team, call_id, round,
+            wait_ticks, votes,
+            [&]() {
+              am = -INFINITY;
+              as = 0.0f;
+            },
+            [&](const auto& v) { merge_pairs<PRECISE>(am, as, v[0], v[1]); });
+      if (!lost) {
+        gm[threadIdx.x] = am;
+        gs[threadIdx.x] = as;
+        __syncthreads();
+        if ((int)threadIdx.x < C) {
+          pm = gm[threadIdx.x];
+          ps = gs[threadIdx.x];
+          const int n = kTeamBlock / C < team ? kTeamBlock / C : team;
+          for (int g = 1; g < n; ++g)
+            online_merge<PRECISE>(pm, ps, gm[g * C + threadIdx.x], gs[g * C + threadIdx.x]);
+        }
+      } else {
+        // the team did not come together: all rows of the strip, then this workgroup's again
+        const StridedTeamPlace<E> t(sh, (int)threadIdx.x, strip);
+        const TI* xs = x + (strip / sh.xtiles) * (int64_t)D * inner + t.e0;
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+          m[i] = -INFINITY;
+          s[i] = 0.0f;
+        }
+        for (int d = t.ty; d < D; d += t.TY) {
+          const Pack<TI, E> p = Pack<TI, E>::load(xs + (int64_t)d * inner);
+#pragma unroll
+          for (int i = 0; i < E; ++i) {
+            const float nm = fmaxf(m[i], p.get(i));
+            const float rf = nm == -INFINITY ? 0.0f : nm;
+            s[i] = s[i] * row_exp<PRECISE>(m[i] - rf) + row_exp<PRECISE>(p.get(i) - rf);
+            m[i] = nm;
+          }
+        }
+        __syncthreads();  // (wm / ws have been read)
+        merge_workgroup();
+      }
+    }
+    if ((int)threadIdx.x < C) {
+      fm[threadIdx.x] = pm;
+      fk[threadIdx.x] = is_log ? logf(ps) : 1.0f / ps;
+    }
+    __syncthreads();
+    // (the lane's place again, after the exchange: offsets and bounds of its rows are not
+    // carried through it)
+    const StridedTeamPlace<E> t(sh, lane_again((int)threadIdx.x), strip);
+    float kf[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      m[i] = fm[t.tx * E + i];
+      kf[i] = fk[t.tx * E + i];
+    }
+    TO* yb = y + ((strip / sh.xtiles) * (int64_t)D + r0) * inner;
+    const bool full = r0 + t.TY * V <= D;
+    auto store_rows = [&](auto value) {
+      const uint32_t off = ((uint32_t)t.ty * (uint32_t)inner + (uint32_t)t.e0) * (uint32_t)sizeof(TO);
+      const int64_t step = (int64_t)t.TY * inner;
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        Pack<TO, E> out;
+#pragma unroll
+        for (int i = 0; i < E; ++i) out.set(i, value(xp[k].get(i), i));
+        if (full || r0 + t.ty + k * t.TY < D) out.store_stream(global_at(yb, off));
+        yb = scalar_again(yb + step);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    if (t.in) {
+      if (is_log) {
+        ROWNORM_UNIFORM_ARM("log_softmax, a strip held by a team");
+        store_rows([&](float v, int i) { return (v - m[i]) - kf[i]; });
+      } else {
+        ROWNORM_UNIFORM_ARM("softmax, a strip held by a team");
+        if (is_safe) {
+#pragma unroll
+          for (int i = 0; i < E; ++i)
+            if (m[i] == -INFINITY) m[i] = kf[i] = 0.0f;  // exp(-inf - 0) * 0
+        }
+        store_rows([&](float v, int i) { return row_exp<PRECISE>(v - m[i]) * kf[i]; });
+      }
+    }
+  }
+}
+
+// Backward: V packs a lane of grad and of y; the columns' sums of y * grad (log_softmax: of grad)
+// cross the team.
+template <class TG, class TO, int V>
+__global__ void __launch_bounds__(kTeamBlock, kTeamPerCu * kTeamBlock / 256)
+softmax_strided_team_bwd_kernel(const TG* __restrict__ grad, const TG* __restrict__ y,
+                                TO* __restrict__ gi, StridedTeamShape sh, int flags,
+                                TeamColumns* slot, unsigned int call_id,
+                                unsigned long long wait_ticks) {
+  constexpr int E = elems_per_pack<TG>::value;
+  constexpr bool PRECISE = sizeof(TO) == 4 && sizeof(TG) == 4;
+  constexpr int NW = kTeamBlock / 64;
+  __shared__ float ws[NW * kTeamColumns];
+  __shared__ int votes[2][kTeamBlock / 64 + 1];
+  __shared__ float gs[kTeamBlock];
+  __shared__ __align__(16) float fs[kTeamColumns];
+  const bool is_log = (flags & kSoftmaxLog) != 0;
+  const int D = sh.D, inner = sh.inner, team = sh.team;
+  const int TX = 1 << sh.tx_log2, C = TX * E;
+  const int tm = (int)blockIdx.x / team;
+  const int teams = (int)gridDim.x / team;
+  const int r0 = ((int)blockIdx.x - tm * team) * (kTeamBlock >> sh.tx_log2) * V;
+  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+  bool lost = false;
+  unsigned int round = 0;
+  for (int64_t strip = tm; strip < sh.strips; strip += teams, ++round) {
+    Pack<TG, E> gp[V], yp[V];
+    {
+      const StridedTeamPlace<E> t(sh, lane_again((int)threadIdx.x), strip);
+      const int64_t slab = (strip / sh.xtiles) * (int64_t)D * inner;
+      strided_team_load<TG, E, V>(gp, grad + slab, r0, t.ty, t.TY, t.e0, D, inner, 0.0f);
+      strided_team_load<TG, E, V>(yp, y + slab, r0, t.ty, t.TY, t.e0, D, inner, 0.0f);
+    }
+    float s[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) s[i] = 0.0f;
+    // (no branch on the variant: two arms would each want the packs in registers of their own)
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+#pragma unroll
+      for (int i = 0; i < E; ++i) s[i] = fmaf(is_log ? 1.0f : yp[k].get(i), gp[k].get(i), s[i]);
+      keep_packed(gp[k]);
+      keep_packed(yp[k]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int i = 0; i < E; ++i) asm volatile("" : "+v"(s[i]));
+    float ps = 0.0f;  // the sum of column threadIdx.x < C: the workgroup's, then the strip's
+    auto merge_workgroup = [&]() {
+      for (int off = TX; off < 64; off <<= 1)
+#pragma unroll
+        for (int i = 0; i < E; ++i) s[i] += __shfl_xor(s[i], off, 64);
+      if (lane < TX) {
+#pragma unroll
+        for (int i = 0; i < E; ++i) ws[wave * kTeamColumns + lane * E + i] = s[i];
+      }
+      __syncthreads();
+      if ((int)threadIdx.x < C) {
+        ps = ws[threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) ps += ws[w * kTeamColumns + threadIdx.x];
+      }
+    };
+    merge_workgroup();
+    unsigned long long* words = &slot->word[round & 1u][0][0];
+    if (team > 1)
+      columns_publish<1>(words + (int64_t)blockIdx.x * (2 * kTeamColumns), C, lost, call_id, round,
+                         {ps});
+    if (team > 1) {
+      float as = 0.0f;
+      if (!lost)
+        lost = !columns_gather<1>(
+            slot, words + (int64_t)tm * team * (2 * kTeamColumns), C, team, call_id, round,
+            wait_ticks, votes, [&]() { as = 0.0f; }, [&](const auto& v) {
+#pragma unroll
+              for (float f : v[0]) as += f;
+            });
+      if (!lost) {
+        gs[threadIdx.x] = as;
+        __syncthreads();
+        if ((int)threadIdx.x < C) {
+          ps = gs[threadIdx.x];
+          const int n = kTeamBlock / C < team ? kTeamBlock / C : team;
+          for (int g = 1; g < n; ++g) ps += gs[g * C + threadIdx.x];
+        }
+      } else {
+        // the team did not come together: all rows of the strip, then this workgroup's again
+        const StridedTeamPlace<E> t(sh, (int)threadIdx.x, strip);
+        const int64_t at = (strip / sh.xtiles) * (int64_t)D * inner + t.e0;
+#pragma unroll
+        for (int i = 0; i < E; ++i) s[i] = 0.0f;
+        for (int d = t.ty; d < D; d += t.TY) {
+          const Pack<TG, E> pg = Pack<TG, E>::load(grad + at + (int64_t)d * inner);
+          const Pack<TG, E> py = Pack<TG, E>::load(y + at + (int64_t)d * inner);
+#pragma unroll
+          for (int i = 0; i < E; ++i) s[i] += is_log ? pg.get(i) : py.get(i) * pg.get(i);
+        }
+        __syncthreads();  // (ws has been read)
+        merge_workgroup();
+      }
+    }
+    if ((int)threadIdx.x < C) fs[threadIdx.x] = ps;
+    __syncthreads();
+    const StridedTeamPlace<E> t(sh, lane_again((int)threadIdx.x), strip);
+#pragma unroll
+    for (int i = 0; i < E; ++i) s[i] = fs[t.tx * E + i];
+    TO* ob = gi + ((strip / sh.xtiles) * (int64_t)D + r0) * inner;
+    const bool full = r0 + t.TY * V <= D;
+    auto store_rows = [&](auto value) {
+      const uint32_t off = ((uint32_t)t.ty * (uint32_t)inner + (uint32_t)t.e0) * (uint32_t)sizeof(TO);
+      const int64_t step = (int64_t)t.TY * inner;
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        Pack<TO, E> out;
+#pragma unroll
+        for (int i = 0; i < E; ++i) out.set(i, value(gp[k].get(i), yp[k].get(i), s[i]));
+        if (full || r0 + t.ty + k * t.TY < D) out.store_stream(global_at(ob, off));
+        ob = scalar_again(ob + step);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    if (t.in) {
+      if (is_log) {
+        ROWNORM_UNIFORM_ARM("log_softmax backward, a strip held by a team");
+        store_rows([](float g, float v, float sum) { return g - row_exp<PRECISE>(v) * sum; });
+      } else {
+        ROWNORM_UNIFORM_ARM("softmax backward, a strip held by a team");
+        store_rows([](float g, float v, float sum) { return v * (g - sum); });
+      }
+    }
+  }
+}
+
+}  // namespace rownorm
