@@ -1,0 +1,68 @@
+"""Norm backward of ragged rows (N not a whole number of packs) off a 16-byte boundary: a row's last
+pack is read as the last whole pack inside the row and moved into place.  Every remainder, rows just
+above a pack, rows shorter than one (a forced layout included), NaN on both sides of every input,
+against the float64 oracle (the reference's unaligned path: can_vectorize() false,
+src/ATen/native/xpu/sycl/LayerNormKernels.cpp:1121-1163)."""
+import pytest
+import torch
+
+from helpers import assert_close, gen, to_np32
+
+pytestmark = pytest.mark.gpu
+
+
+def _inside(t, off, gpu):
+    buf = torch.full((t.numel() + 64,), float("nan"), dtype=t.dtype, device=gpu)
+    v = buf[16 + off:16 + off + t.numel()].view(t.shape)
+    v.copy_(t)
+    return v
+
+
+def _check(cabi, oracle, gpu, M, N, dtype, offs):
+    print("case ragged norm backward", dtype, (M, N), offs, flush=True)
+    g = gen(2500 + N + offs[0])
+    x = (0.5 + torch.randn(M, N, generator=g)).to(dtype)
+    dy = torch.randn(M, N, generator=g).to(dtype)
+    gamma = (1 + 0.1 * torch.randn(N, generator=g)).to(dtype)
+    xg, dyg = _inside(x, offs[0], gpu), _inside(dy, offs[1], gpu)
+    gg = _inside(gamma, 1, gpu)
+    what = "[%d, %d] %s offsets %s" % (M, N, dtype, offs)
+    _, mean, rstd = cabi.layer_norm_fwd(xg, gg, None, 1e-5)
+    xhat = (x.float() - mean.float().cpu()[:, None]) * rstd.float().cpu()[:, None]
+    # float32 sums over the rows, in another order: a few ulps of the magnitudes' sum
+    slack_g = (dy.float() * xhat).abs().sum(dim=0) * 2.0 ** -21
+    slack_b = dy.float().abs().sum(dim=0) * 2.0 ** -21
+    odx, odg, odb = oracle.layer_norm_bwd(to_np32(dy), to_np32(x), (N,), to_np32(mean),
+                                          to_np32(rstd), to_np32(gamma))
+    over = _inside(dy, offs[1], gpu)
+    for dx_out, dyt in ((None, dyg), (over, over)):
+        dx, dg, db = cabi.layer_norm_bwd(dyt, xg, mean, rstd, gg, dx=dx_out)
+        assert_close(dx, odx, dtype, "layer_norm dx " + what)
+        assert_close(dg, odg, dtype, "layer_norm dgamma " + what, slack=slack_g)
+        assert_close(db, odb, dtype, "layer_norm dbeta " + what, slack=slack_b)
+    _, rr = cabi.rms_norm_fwd(xg, gg, 1e-6)
+    slack_g = (dy.float() * x.float() * rr.float().cpu()[:, None]).abs().sum(dim=0) * 2.0 ** -21
+    rdx, rdg = cabi.rms_norm_bwd(dyg, xg, rr, gg)
+    ordx, ordg = oracle.rms_norm_bwd(to_np32(dy), to_np32(x), (N,), to_np32(rr), to_np32(gamma))
+    assert_close(rdx, ordx, dtype, "rms_norm dx " + what)
+    assert_close(rdg, ordg, dtype, "rms_norm dgamma " + what, slack=slack_g)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("offs", [(2, 2), (1, 7), (5, 0)], ids=str)
+def test_ragged_rows_off_a_boundary(cabi, oracle, gpu, dtype, offs):
+    widths = [3, 9, 129, 130, 131, 132, 133, 134, 135, 257, 1001, 1027, 2050, 2801, 4097, 8195]
+    for N in widths:
+        _check(cabi, oracle, gpu, 7 if N % 2 else 1100, N, dtype, offs)
+
+
+@pytest.mark.parametrize("N,dtype", [(5, torch.float16), (7, torch.bfloat16), (3, torch.float32)],
+                         ids=str)
+def test_rows_shorter_than_a_pack_on_a_forced_layout(cabi, oracle, gpu, N, dtype):
+    packs = 4 if dtype == torch.float32 else 2
+    try:
+        for op in (cabi.OP_LAYER_NORM_BWD, cabi.OP_RMS_NORM_BWD):
+            cabi.set_override(op, 32, packs, 0, 0)
+        _check(cabi, oracle, gpu, 300, N, dtype, (1, 3))
+    finally:
+        cabi.clear_overrides()

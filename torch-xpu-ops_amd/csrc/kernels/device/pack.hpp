@@ -205,6 +205,33 @@ __device__ __forceinline__ void trim_window_pack(Pack<T, E>& r, int e0, int n, f
   }
 }
 
+// The pack at element e0 of a row of n >= E elements in two steps, the row's own alignment: a
+// pack that would end past the row is read E elements before the row's end instead -- one
+// unconditional 128-bit load inside the row, so a lane's loads are straight-line code -- and
+// settle_clamped_pack, run over the packs after all of them have been requested, moves its
+// elements into place.  What lies outside the row becomes zero.
+template <class T, int E>
+__device__ __forceinline__ Pack<T, E> load_clamped_pack(const T* row, int e0, int n) {
+  return Pack<T, E>::load_stream(row + (e0 + E <= n ? e0 : n - E));
+}
+template <class T, int E>
+__device__ __forceinline__ void settle_clamped_pack(Pack<T, E>& p, int e0, int n, bool ok) {
+  static_assert(sizeof(T) == 2 || sizeof(T) == 4, "elements of half a word or a word");
+  if (ok && e0 + E <= n) return;
+  asm volatile("" : "+v"(e0));  // as in load_row_pack
+  typedef uint32_t raw_t __attribute__((ext_vector_type(4)));
+  raw_t w = __builtin_bit_cast(raw_t, p.v);
+  // the elements to drop from the front, in half words (8: none is left)
+  int h = (e0 + E - n) * (int)(sizeof(T) / 2);
+  if (!ok || h > 8) h = 8;
+  if (h & 8) w = raw_t{0u, 0u, 0u, 0u};
+  if (h & 4) w = raw_t{w[2], w[3], 0u, 0u};
+  if (h & 2) w = raw_t{w[1], w[2], w[3], 0u};
+  if (sizeof(T) == 2 && (h & 1))
+    w = raw_t{w[0] >> 16 | w[1] << 16, w[1] >> 16 | w[2] << 16, w[2] >> 16 | w[3] << 16, w[3] >> 16};
+  p.v = __builtin_bit_cast(typename Pack<T, E>::vec_t, w);
+}
+
 template <class T, int E, bool STREAM>
 __device__ __forceinline__ void store_row_pack(T* row, int e0, int n, bool row_ok,
                                                const Pack<T, E>& p, int lo = 0) {

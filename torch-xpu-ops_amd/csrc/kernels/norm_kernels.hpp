@@ -1812,6 +1812,15 @@ norm_bwd_resident_kernel(const T* __restrict__ dy, const T* __restrict__ x, cons
     }
   };
 
+  // CLAMP (norm_bwd_clamps()): ragged rows of at least one pack are read with whole packs,
+  // nothing conditional between the requests.  With the element loads of a row's last pack in a
+  // branch of their own the wavefront that holds it waited for X, then for dY, and the whole
+  // workgroup for it: fp16 LayerNorm backward of 16384 rows 2 elements into their buffers, us:
+  // N = 1401 47.9 -> 39.2, 2801 81.6 -> 67.0, 4097 116.6 -> 109.3, 6143 164.7 -> 151.3; of 2048
+  // rows: 2049 22.3 -> 19.5, 2801 26.2 -> 22.0.  (Three packs a lane in workgroups of 256 threads,
+  // three of those a compute unit, lose to two packs on all the lanes: 2048 rows of 2801 26.1, of
+  // 6143 37.9 against 34.4.)
+  constexpr bool CLAMP = norm_bwd_clamps(G, FAST);
   const int64_t nrb = (M + RPI - 1) / RPI;
   // A row slot past the end of the tensor gets all-zero x and dy, so it adds
   // nothing to the column sums; its dx is not stored.
@@ -1830,11 +1839,25 @@ norm_bwd_resident_kernel(const T* __restrict__ dy, const T* __restrict__ x, cons
       const int64_t rowc = fok[r] ? frow0 + r : 0;
       fmu[r] = RMS ? 0.0f : mean[rowc];
       frs[r] = rstd[rowc];
+      if constexpr (!CLAMP) {
 #pragma unroll
-      for (int c = 0; c < V; ++c) {
-        const int e0 = (c * G + lane) * E;
-        fx[r][c] = row_load<T, E, true, FAST>(x + rowc * (int64_t)N, e0, N, fok[r], 0.0f);
-        fd[r][c] = row_load<T, E, true, FAST>(dy + rowc * (int64_t)N, e0, N, fok[r], 0.0f);
+        for (int c = 0; c < V; ++c) {
+          const int e0 = (c * G + lane) * E;
+          fx[r][c] = row_load<T, E, true, FAST>(x + rowc * (int64_t)N, e0, N, fok[r], 0.0f);
+          fd[r][c] = row_load<T, E, true, FAST>(dy + rowc * (int64_t)N, e0, N, fok[r], 0.0f);
+        }
+      } else {
+#pragma unroll
+        for (int c = 0; c < V; ++c) {
+          const int e0 = (c * G + lane) * E;
+          fx[r][c] = load_clamped_pack<T, E>(x + rowc * (int64_t)N, e0, N);
+          fd[r][c] = load_clamped_pack<T, E>(dy + rowc * (int64_t)N, e0, N);
+        }
+#pragma unroll
+        for (int c = 0; c < V; ++c) {
+          settle_clamped_pack<T, E>(fx[r][c], (c * G + lane) * E, N, fok[r]);
+          settle_clamped_pack<T, E>(fd[r][c], (c * G + lane) * E, N, fok[r]);
+        }
       }
     }
   };

@@ -422,6 +422,12 @@ constexpr bool block_built(OpClass oc, int G, int block) {
   return block == block_threads(oc, G);
 }
 
+// Whether the resident norm backward reads the last pack of a ragged row as the row's last whole
+// pack (load_clamped_pack), which takes rows of a pack or more.  Shorter rows (N < 8 or 4
+// elements) run on kMinG lanes, whose kernels keep the element loads; make_plan() sees to it
+// that a forced layout does the same.
+constexpr bool norm_bwd_clamps(int G, bool fast) { return !fast && G > kMinG; }
+
 // Workgroups per compute unit of the grid-stride launch.  The norm kernels keep
 // gamma/beta (and the backward column sums) in registers across the rows of a
 // workgroup.  Forward: four times as many workgroups as fit on the machine at
@@ -770,7 +776,12 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
       p.G = G;
       p.V = V;
       p.block = block;
-      p.rpb = p.block / G;
+      if (oc == OC_NORM_BWD && N < E && norm_bwd_clamps(G, p.fast)) {
+        p.G = kMinG;
+        p.V = v_pref(oc, esize);
+        p.block = block_threads(oc, kMinG);
+      }
+      p.rpb = p.block / p.G;
       // 16-bit forward rows likewise (plain calls: no residual add, no output cast)
       if (oc == OC_NORM_FWD && p.fast && !fused_add && !p.forced && ov.bpc == 0) {
         const int xi = norm_fwd_exact_index(esize, packs, M, num_cus);
