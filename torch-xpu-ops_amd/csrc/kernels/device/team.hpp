@@ -215,6 +215,61 @@ __device__ __forceinline__ bool team_gather_tagged(TeamSlot* slot, const TeamEnt
   return complete;
 }
 
+// The same with the team's numbers left one by one in part[j][0..K) (LDS): the kernel adds them
+// up by a rule of its own.  (The lanes of a wavefront see one another's LDS stores in program
+// order.)
+template <int K>
+__device__ __forceinline__ bool team_gather_each(TeamSlot* slot, const TeamEntry* mates, int team,
+                                                 unsigned int call_id, unsigned int round,
+                                                 unsigned long long wait_ticks, float (*part)[K]) {
+  constexpr int B = kTeamGatherBatch;
+  const int lane = (int)threadIdx.x;
+  const unsigned int expect = team_word_tag(call_id, round);
+  const unsigned long long t0 = wall_clock64();
+  bool complete = false;
+  unsigned int polls = 0;
+  for (;;) {
+    bool ok = true, lost_seen = false;
+    for (int j0 = lane; j0 < team; j0 += 64 * B) {
+      unsigned long long w[B][K];
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        const int j = j0 + 64 * b;
+        const unsigned long long* words = &mates[j < team ? j : j0].pad[0];
+#pragma unroll
+        for (int k = 0; k < K; ++k) w[b][k] = team_load(&words[k]);
+      }
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        const int j = j0 + 64 * b;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          ok = ok && (unsigned int)(w[b][k] >> 32) == expect;
+          lost_seen = lost_seen || team_tag_is_lost((unsigned int)(w[b][k] >> 32), call_id);
+          if (j < team)
+            part[j][k] = __builtin_bit_cast(float, (unsigned int)(w[b][k] & 0xffffffffull));
+        }
+      }
+    }
+    if (__ballot(lost_seen) != 0) break;
+    if (__ballot(ok) == __ballot(true)) {
+      complete = true;
+      break;
+    }
+    // (the hint word is one address for the whole grid: looked at every 16th time)
+    if ((polls++ & 15u) == 0) {
+      const unsigned int hint =
+          __hip_atomic_load(&slot->gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (hint == call_id) break;
+    }
+    if (wall_clock64() - t0 > wait_ticks) break;
+    __builtin_amdgcn_s_sleep(8);
+  }
+  if (!complete && lane == 0)
+    __hip_atomic_store(&slot->gave_up, call_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return complete;
+}
+
 // The same two halves for K float64 values a workgroup (K <= 6), each cut into two words
 // {32 bits, tag} of pad[] as in team_publish_and_gather, summed over the team in the fixed
 // order of team_gather_tagged.

@@ -1174,4 +1174,205 @@ gn_bwd_team_kernel(const T* __restrict__ dy, const T* __restrict__ x,
   }
 }
 
+// The same for a team that works through several slabs: four packs of each tensor a lane, twice.
+// While one slab is exchanged and written, the next one the team takes is on its way or already
+// summed and published, so neither the loads nor the exchange are waited for with nothing else to
+// do (the kernel above loads, exchanges and stores one after the other, in step on the whole
+// machine).  The exchange is that of norm_bwd_team_kernel, words that carry their own tag: one
+// round trip.  Whole backward in 32 groups, us (the kernel above -> this one), bf16:
+// [16, 512, 128, 128] 182 -> 153 (4.4 -> 5.3 TB/s), [4, 256, 128, 128] 26.7 -> 24.1,
+// [1, 512, 512, 512] 178 -> 167, [2, 128, 1024, 1024] 360 -> 343; fp32 [4, 256, 256, 256]
+// 154 -> 146.
+template <class T, class WT>
+__global__ void __launch_bounds__(kTeamBlock, kTeamPerCu * kTeamBlock / 256)
+gn_bwd_team_ahead_kernel(const T* __restrict__ dy, const T* __restrict__ x,
+                         const WT* __restrict__ mean, const WT* __restrict__ rstd,
+                         const WT* __restrict__ gamma, T* __restrict__ dx,
+                         float* __restrict__ part_dg, float* __restrict__ part_db, int64_t rows,
+                         GroupShape s, int team, int wpc, TeamSlot* slot, unsigned int call_id,
+                         unsigned long long wait_ticks) {
+  constexpr int E = elems_per_pack<T>::value;
+  constexpr int BLOCK = kTeamBlock;
+  constexpr int V = kGnTeamAheadPacks;
+  __shared__ float red[reduce_lds_floats<BLOCK, BLOCK, 4>::value];
+  __shared__ float tpart[kTeamMaxWorkgroups][2];
+  __shared__ float stat[3];  // s1, s2, whether the team failed
+  int phase = 0;
+  bool lost = false;  // (first wavefront) the workgroup has stopped waiting for its team
+  const int tm = (int)blockIdx.x / team;
+  const int c = (int)blockIdx.x - tm * team;
+  const int teams = (int)gridDim.x / team;
+  const int ch = c / wpc;          // the channel of the group this workgroup works on
+  const int piece = c - ch * wpc;  // and its piece of the channel
+  const int cp = s.HxW / E;        // packs a channel
+  const int pk0 = piece * (V * BLOCK) + (int)threadIdx.x;
+  const float fL = (float)s.L;
+  const uint32_t loff = (uint32_t)(pk0 < cp ? pk0 : 0) * 16u;
+  auto at = [](auto* p, uint32_t off) {
+    using Elem = std::remove_pointer_t<decltype(p)>;
+    typedef __attribute__((address_space(1))) Elem* GlobalPtr;
+    return (Elem*)reinterpret_cast<GlobalPtr>(reinterpret_cast<uintptr_t>(p) + off);
+  };
+  auto load_pack_pair = [&](int64_t row, int k, Pack<T, E>& pd, Pack<T, E>& px) {
+    pd = Pack<T, E>::zero();
+    px = Pack<T, E>::zero();
+    if (pk0 + k * BLOCK < cp && row < rows) {
+      const int64_t base = row * (int64_t)s.L + (int64_t)ch * s.HxW + k * BLOCK * E;
+      pd = Pack<T, E>::load_stream(at(dy + base, loff));
+      px = Pack<T, E>::load_stream(at(x + base, loff));
+    }
+  };
+  auto load_slab = [&](int64_t row, Pack<T, E> (&pd)[V], Pack<T, E> (&px)[V]) {
+#pragma unroll
+    for (int k = 0; k < V; ++k) load_pack_pair(row, k, pd[k], px[k]);
+  };
+  // The piece's sums of the slab held in pd / px, published as round `round`.
+  auto sums_and_publish = [&](int64_t row, unsigned int round, Pack<T, E> (&pd)[V],
+                              Pack<T, E> (&px)[V]) {
+    const float mu = (float)mean[row], rs = (float)rstd[row];
+    float acc[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      if (pk0 + k * BLOCK < cp) {
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+          const float gy = pd[k].get(i);
+          acc[1] += gy;
+          acc[0] = fmaf(gy, px[k].get(i) - mu, acc[0]);
+        }
+      }
+      keep_packed(pd[k]);
+      keep_packed(px[k]);
+      __builtin_amdgcn_sched_barrier(0);  // (one pack widened at a time: registers)
+    }
+    group_allreduce<BLOCK, BLOCK, 2, SumOp>(acc, red, phase);
+    acc[0] *= rs;
+    if (threadIdx.x == 0)
+      team_publish_tagged<2>(&slot->entry[round & 3u][blockIdx.x], call_id, round, acc, lost);
+  };
+  // The sums of slab `row` (published as round `round`) across the team and its dX; each pack's
+  // registers go to the same pack of slab `next` as soon as its dX has been stored.  (other, po*:
+  // the slab in the other register set, loaded again after the rare pass over the whole slab)
+  auto finish = [&](int64_t row, unsigned int round, Pack<T, E> (&pd)[V], Pack<T, E> (&px)[V],
+                    int64_t next, int64_t other, Pack<T, E> (&pod)[V], Pack<T, E> (&pox)[V]) {
+    const int g = (int)((uint32_t)row % (uint32_t)s.groups);
+    const int64_t out0 = row * (int64_t)s.D;  // the slab's channels in the [N, C] partial buffers
+    const float mu = (float)mean[row], rs = (float)rstd[row];
+    // (every thread has read the stat[] of the slab before)
+    __syncthreads();
+    if (threadIdx.x < 64) {
+      const int lane = (int)threadIdx.x;
+      const bool complete =
+          team_gather_each<2>(slot, slot->entry[round & 3u] + tm * team, team, call_id, round,
+                              wait_ticks, tpart);
+      lost = lost || !complete;
+      float s1 = 0.0f, s2 = 0.0f;
+      if (complete) {
+        for (int d = lane; d < s.D; d += 64) {
+          float dg = 0.0f, db = 0.0f;
+          for (int q = 0; q < wpc; ++q) {
+            dg += tpart[d * wpc + q][0];
+            db += tpart[d * wpc + q][1];
+          }
+          const float ga = gn_weight(gamma, g * s.D + d, 1.0f);
+          s1 = fmaf(db, ga, s1);
+          s2 = fmaf(dg, ga, s2);
+          if (d == ch && piece == 0 && part_dg != nullptr) {
+            part_dg[out0 + d] = dg;
+            if (part_db != nullptr) part_db[out0 + d] = db;
+          }
+        }
+        s1 = wave_group_allreduce<64, SumOp>(s1);
+        s2 = wave_group_allreduce<64, SumOp>(s2);
+      }
+      if (lane == 0) {
+        stat[0] = s1;
+        stat[1] = s2;
+        stat[2] = complete ? 0.0f : 1.0f;
+      }
+    }
+    __syncthreads();
+    if (stat[2] != 0.0f) {  // (uniform over the workgroup)
+      // The team did not come together: the slab's sums in a pass over the whole slab, then the
+      // packs again, as in the kernel above.
+      const T* gr = dy + row * (int64_t)s.L;
+      const T* xr = x + row * (int64_t)s.L;
+      float w[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // s1, s2 / rstd, own channel's dg / rstd and db
+      for (int pk = (int)threadIdx.x; pk < s.D * cp; pk += BLOCK) {
+        const int d = pk / cp;
+        const Pack<T, E> qd = Pack<T, E>::load(gr + (int64_t)pk * E);
+        const Pack<T, E> qx = Pack<T, E>::load(xr + (int64_t)pk * E);
+        const float ga = gn_weight(gamma, g * s.D + d, 1.0f);
+        float a = 0.0f, b = 0.0f;
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+          const float gy = qd.get(i);
+          b += gy;
+          a = fmaf(gy, qx.get(i) - mu, a);
+        }
+        w[0] = fmaf(b, ga, w[0]);
+        w[1] = fmaf(a, ga, w[1]);
+        if (d == ch) {
+          w[2] += a;
+          w[3] += b;
+        }
+      }
+      group_allreduce<BLOCK, BLOCK, 4, SumOp>(w, red, phase);
+      if (threadIdx.x == 0) {
+        stat[0] = w[0];
+        stat[1] = w[1] * rs;
+        if (piece == 0 && part_dg != nullptr) {
+          part_dg[out0 + ch] = w[2] * rs;
+          if (part_db != nullptr) part_db[out0 + ch] = w[3];
+        }
+      }
+      __syncthreads();
+      load_slab(row, pd, px);
+      load_slab(other, pod, pox);  // (a slab beyond the tensor: zeros)
+    }
+    const float s1 = stat[0], s2 = stat[1], term1 = rs / fL;
+    const float ga = gn_weight(gamma, g * s.D + ch, 1.0f);
+    T* ob = dx + row * (int64_t)s.L + (int64_t)ch * s.HxW;
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      if (pk0 + k * BLOCK < cp) {
+        Pack<T, E> o;
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+          float f = fL * (pd[k].get(i) * ga);
+          f -= ((px[k].get(i) - mu) * rs) * s2;
+          f -= s1;
+          o.set(i, f * term1);
+        }
+        o.store_stream(at(ob + k * BLOCK * E, loff));
+      }
+      load_pack_pair(next, k, pd[k], px[k]);
+      // (pack k + 1 is widened after pack k has been stored, not before: registers)
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  // Slab j of the team (tm + j * teams) lives in register set j % 2.  The words of a round are
+  // overwritten four rounds later, when every workgroup of the team has gathered them: none
+  // publishes round j + 1 before it has gathered round j - 1.
+  Pack<T, E> ad[V], ax[V], bd[V], bx[V];
+  int64_t row = tm;
+  unsigned int round = 0;
+  if (row < rows) {
+    load_slab(row, ad, ax);
+    load_slab(row + teams, bd, bx);
+    sums_and_publish(row, 0, ad, ax);
+  }
+  while (row < rows) {
+    const int64_t r1 = row + teams, r2 = r1 + teams, r3 = r2 + teams;
+    if (r1 < rows) sums_and_publish(r1, round + 1, bd, bx);
+    finish(row, round, ad, ax, r2, r1, bd, bx);
+    if (r1 >= rows) break;
+    if (r2 < rows) sums_and_publish(r2, round + 2, ad, ax);
+    finish(r1, round + 1, bd, bx, r3, r2, ad, ax);
+    row = r2;
+    round += 2;
+  }
+}
+
 }  // namespace rownorm

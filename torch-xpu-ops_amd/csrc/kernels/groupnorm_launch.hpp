@@ -209,17 +209,16 @@ int launch_group_norm_bwd(const Plan& plan, const GroupNormBwdArgs& a, hipStream
     // slabs beyond the registers, dY and X read once: teams of workgroups
     GroupNormBwdArgs k = a;
     if (!want_cols) k.part_dg = k.part_db = nullptr;
-    auto go = [&](auto v) {
-      constexpr int V = decltype(v)::value;
-      hipLaunchKernelGGL((gn_bwd_team_kernel<T, WT, V>), dim3((unsigned)a.team_grid),
-                         dim3(kTeamBlock), 0, stream, (const T*)a.dy, (const T*)a.x,
-                         (const WT*)a.mean, (const WT*)a.rstd, (const WT*)a.gamma, (T*)a.dx,
-                         k.part_dg, k.part_db, a.rows, shape, a.team, a.team_wpc,
-                         (TeamSlot*)a.team_slot, a.team_id, a.team_wait_ticks);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)a.team_grid), dim3(kTeamBlock), 0, stream,
+                         (const T*)a.dy, (const T*)a.x, (const WT*)a.mean, (const WT*)a.rstd,
+                         (const WT*)a.gamma, (T*)a.dx, k.part_dg, k.part_db, a.rows, shape, a.team,
+                         a.team_wpc, (TeamSlot*)a.team_slot, a.team_id, a.team_wait_ticks);
     };
-    switch (a.team_v) {
-      case 4: go(std::integral_constant<int, 4>{}); break;
-      case 8: go(std::integral_constant<int, 8>{}); break;
+    switch (a.team_ahead ? 0 : a.team_v) {
+      case 0: go(gn_bwd_team_ahead_kernel<T, WT>); break;
+      case 4: go(gn_bwd_team_kernel<T, WT, 4>); break;
+      case 8: go(gn_bwd_team_kernel<T, WT, 8>); break;
       default: return (int)hipErrorInvalidConfiguration;
     }
   } else if (need_sums && !fused_cols) {

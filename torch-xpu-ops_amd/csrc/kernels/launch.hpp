@@ -151,6 +151,7 @@ struct GroupNormBwdArgs {
   // bookkeeping memory, its id and the bound of a wait, as in GroupNormFwdArgs; team == 0 or
   // a null slot: not for this call
   int team = 0, team_wpc = 0, team_v = 0;
+  bool team_ahead = false;  // gn_bwd_team_ahead_kernel (team_v is its kGnTeamAheadPacks)
   int64_t team_grid = 0;
   void* team_slot = nullptr;
   unsigned int team_id = 0;

@@ -93,6 +93,8 @@ constexpr int kTeamGroup = 2;  // packs whose weights are requested together
 constexpr int kTeamMaxWorkgroups = 512;
 constexpr int kTeamSlots = 16;
 constexpr int kTeamMinTeams = 8;
+// gn_bwd_team_ahead_kernel: packs a lane holds of each tensor and slab (two slabs at a time).
+constexpr int kGnTeamAheadPacks = 4;
 // norm_bwd_team_kernel: rows a team holds at a time, packs of a row a lane holds of each
 // tensor, workgroups a compute unit
 constexpr int kTeamBwdRows = 4;
