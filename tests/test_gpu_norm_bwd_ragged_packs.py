@@ -56,6 +56,16 @@ def test_ragged_rows_off_a_boundary(cabi, oracle, gpu, dtype, offs):
         _check(cabi, oracle, gpu, 7 if N % 2 else 1100, N, dtype, offs)
 
 
+@pytest.mark.parametrize("M,N,dtype", [(1, 8193, torch.float16), (300, 10005, torch.bfloat16),
+                                       (300, 12295, torch.float16), (270, 13311, torch.bfloat16),
+                                       (270, 16383, torch.float16), (270, 12289, torch.float32),
+                                       (8150, 6145, torch.float32)], ids=str)
+def test_both_ways_of_reading_a_ragged_row(cabi, oracle, gpu, M, N, dtype):
+    """Rows on 1024 lanes on both sides of the line between whole packs and element loads, and a
+    float32 tensor of more than 50 million elements, whose long rows keep the element loads."""
+    _check(cabi, oracle, gpu, M, N, dtype, (1, 3))
+
+
 @pytest.mark.parametrize("N,dtype", [(5, torch.float16), (7, torch.bfloat16), (3, torch.float32)],
                          ids=str)
 def test_rows_shorter_than_a_pack_on_a_forced_layout(cabi, oracle, gpu, N, dtype):

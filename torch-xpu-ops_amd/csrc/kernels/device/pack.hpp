@@ -214,17 +214,18 @@ template <class T, int E>
 __device__ __forceinline__ Pack<T, E> load_clamped_pack(const T* row, int e0, int n) {
   return Pack<T, E>::load_stream(row + (e0 + E <= n ? e0 : n - E));
 }
-template <class T, int E>
+// (only the wavefront that holds the row's end has anything to move; CLEAR: lanes wholly past the
+// row hold a pack of it and are cleared, otherwise they hold zeros already)
+template <class T, int E, bool CLEAR>
 __device__ __forceinline__ void settle_clamped_pack(Pack<T, E>& p, int e0, int n, bool ok) {
   static_assert(sizeof(T) == 2 || sizeof(T) == 4, "elements of half a word or a word");
-  if (ok && e0 + E <= n) return;
+  if (!ok || (CLEAR && e0 >= n)) p = Pack<T, E>::zero();
+  if (e0 + E <= n || e0 >= n) return;
   asm volatile("" : "+v"(e0));  // as in load_row_pack
   typedef uint32_t raw_t __attribute__((ext_vector_type(4)));
   raw_t w = __builtin_bit_cast(raw_t, p.v);
-  // the elements to drop from the front, in half words (8: none is left)
-  int h = (e0 + E - n) * (int)(sizeof(T) / 2);
-  if (!ok || h > 8) h = 8;
-  if (h & 8) w = raw_t{0u, 0u, 0u, 0u};
+  // the elements to drop from the front, in half words (1 to 7)
+  const int h = (e0 + E - n) * (int)(sizeof(T) / 2);
   if (h & 4) w = raw_t{w[2], w[3], 0u, 0u};
   if (h & 2) w = raw_t{w[1], w[2], w[3], 0u};
   if (sizeof(T) == 2 && (h & 1))

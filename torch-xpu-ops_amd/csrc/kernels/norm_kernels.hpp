@@ -1740,7 +1740,7 @@ __device__ __forceinline__ void fold_row_slots(const float (&sums)[V][E], float*
 // before the arithmetic, the reduction and the stores of the current one, and
 // wait in registers of their own.
 template <class T, class WT, int G, int V, int BLOCK, int R, bool RMS, bool FAST,
-          bool ADD = false>
+          bool ADD = false, NormBwdRead READ = norm_bwd_read((int)sizeof(T), G, FAST, RMS)>
 __global__ void __launch_bounds__(BLOCK)
 norm_bwd_resident_kernel(const T* __restrict__ dy, const T* __restrict__ x, const T* dres,
                          const float* __restrict__ mean, const float* __restrict__ rstd,
@@ -1812,15 +1812,13 @@ norm_bwd_resident_kernel(const T* __restrict__ dy, const T* __restrict__ x, cons
     }
   };
 
-  // CLAMP (norm_bwd_clamps()): ragged rows of at least one pack are read with whole packs,
-  // nothing conditional between the requests.  With the element loads of a row's last pack in a
-  // branch of their own the wavefront that holds it waited for X, then for dY, and the whole
-  // workgroup for it: fp16 LayerNorm backward of 16384 rows 2 elements into their buffers, us:
-  // N = 1401 47.9 -> 39.2, 2801 81.6 -> 67.0, 4097 116.6 -> 109.3, 6143 164.7 -> 151.3; of 2048
-  // rows: 2049 22.3 -> 19.5, 2801 26.2 -> 22.0.  (Three packs a lane in workgroups of 256 threads,
-  // three of those a compute unit, lose to two packs on all the lanes: 2048 rows of 2801 26.1, of
-  // 6143 37.9 against 34.4.)
-  constexpr bool CLAMP = norm_bwd_clamps(G, FAST);
+  // READ (NormBwdRead): ragged rows of at least one pack are read with whole packs, nothing
+  // conditional between the requests of one lane.  With the element loads of a row's last pack in
+  // a branch of their own the wavefront that holds it waited for X, then for dY, and the whole
+  // workgroup for it: fp16 LayerNorm backward of 16384 rows, us, element loads -> whole packs:
+  // N = 1401 47.4 -> 37.5, 3001 82.9 -> 66.9, 4097 116.3 -> 99.2, 6143 163.6 -> 142.8.  Where the
+  // element loads stay: norm_bwd_reads_elements().
+  constexpr bool CLAMP = READ != kReadElements;
   const int64_t nrb = (M + RPI - 1) / RPI;
   // A row slot past the end of the tensor gets all-zero x and dy, so it adds
   // nothing to the column sums; its dx is not stored.
@@ -1850,13 +1848,19 @@ norm_bwd_resident_kernel(const T* __restrict__ dy, const T* __restrict__ x, cons
 #pragma unroll
         for (int c = 0; c < V; ++c) {
           const int e0 = (c * G + lane) * E;
-          fx[r][c] = load_clamped_pack<T, E>(x + rowc * (int64_t)N, e0, N);
-          fd[r][c] = load_clamped_pack<T, E>(dy + rowc * (int64_t)N, e0, N);
+          if constexpr (READ == kReadClampedInside) {
+            fx[r][c] = Pack<T, E>::zero();
+            fd[r][c] = Pack<T, E>::zero();
+          }
+          if (READ == kReadClamped || e0 < N) {
+            fx[r][c] = load_clamped_pack<T, E>(x + rowc * (int64_t)N, e0, N);
+            fd[r][c] = load_clamped_pack<T, E>(dy + rowc * (int64_t)N, e0, N);
+          }
         }
 #pragma unroll
         for (int c = 0; c < V; ++c) {
-          settle_clamped_pack<T, E>(fx[r][c], (c * G + lane) * E, N, fok[r]);
-          settle_clamped_pack<T, E>(fd[r][c], (c * G + lane) * E, N, fok[r]);
+          settle_clamped_pack<T, E, READ == kReadClamped>(fx[r][c], (c * G + lane) * E, N, fok[r]);
+          settle_clamped_pack<T, E, READ == kReadClamped>(fd[r][c], (c * G + lane) * E, N, fok[r]);
         }
       }
     }

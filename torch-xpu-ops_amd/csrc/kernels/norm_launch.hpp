@@ -203,11 +203,19 @@ struct NormBwdLauncher {
                     block_built(OC_NORM_BWD, G, BLOCK) &&
                     (!FAST || norm_bwd_instance_ok(sizeof(T), sizeof(WT), G, V, RMS, ADD))) {
         if (c.plan.G == G && c.plan.V == V && c.plan.block == BLOCK) {
-          hipLaunchKernelGGL((norm_bwd_resident_kernel<T, WT, G, V, BLOCK, 1, RMS, FAST, ADD>),
-                             dim3((unsigned)c.plan.grid), dim3(BLOCK), 0, c.stream,
-                             (const T*)c.a.dy, (const T*)c.a.x, (const T*)c.a.dres, c.a.mean,
-                             c.a.rstd, (const WT*)c.a.gamma, (T*)c.a.dx, c.a.part_dg,
-                             c.a.part_db, c.a.M, c.a.N);
+          auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)c.plan.grid), dim3(BLOCK), 0, c.stream,
+                               (const T*)c.a.dy, (const T*)c.a.x, (const T*)c.a.dres, c.a.mean,
+                               c.a.rstd, (const WT*)c.a.gamma, (T*)c.a.dx, c.a.part_dg,
+                               c.a.part_db, c.a.M, c.a.N);
+          };
+          if constexpr (!FAST && norm_bwd_reads_elements_built(sizeof(T), G, V, RMS)) {
+            if (norm_bwd_reads_elements(sizeof(T), sizeof(WT), G, V, RMS, c.a.M, c.a.N)) {
+              go(norm_bwd_resident_kernel<T, WT, G, V, BLOCK, 1, RMS, FAST, ADD, kReadElements>);
+              return true;
+            }
+          }
+          go(norm_bwd_resident_kernel<T, WT, G, V, BLOCK, 1, RMS, FAST, ADD>);
           return true;
         }
       }

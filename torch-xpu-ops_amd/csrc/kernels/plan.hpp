@@ -424,11 +424,46 @@ constexpr bool block_built(OpClass oc, int G, int block) {
   return block == block_threads(oc, G);
 }
 
-// Whether the resident norm backward reads the last pack of a ragged row as the row's last whole
-// pack (load_clamped_pack), which takes rows of a pack or more.  Shorter rows (N < 8 or 4
-// elements) run on kMinG lanes, whose kernels keep the element loads; make_plan() sees to it
-// that a forced layout does the same.
+// How the resident norm backward reads a ragged row.
+//   kReadElements: a row's last pack element by element, in a branch of its own.
+//   kReadClamped: every lane reads a whole pack, the row's last one where its own would end past
+//     the row (load_clamped_pack); takes rows of a pack or more.
+//   kReadClampedInside: the same, but lanes wholly past the row read nothing.
+// Rows shorter than a pack (N < 8 or 4 elements) run on kMinG lanes, whose kernels keep the element
+// loads; make_plan() sees to it that a forced layout does the same.
+enum NormBwdRead { kReadElements = 0, kReadClamped = 1, kReadClampedInside = 2 };
 constexpr bool norm_bwd_clamps(int G, bool fast) { return !fast && G > kMinG; }
+// The clamped form an instance is built for: lanes past the row stay out of it -- their requests
+// and the moving of their packs cost up to 8 % of the row loop (fp32 LayerNorm [16384, 4097] 163.5
+// -> 148.7 us, fp16 120.8 -> 108.6 at N = 5001) -- except where the branches make the kernel spill
+// (the 16-bit LayerNorm on 1024 lanes, which spills without them already: fp16 [8192, 16383] 209 us
+// against 226).
+constexpr NormBwdRead norm_bwd_read(int esize, int G, bool fast, bool rms) {
+  if (!norm_bwd_clamps(G, fast)) return kReadElements;
+  return esize == 2 && G >= kMaxG && !rms ? kReadClamped : kReadClampedInside;
+}
+// The instances that exist with element loads as well, and the calls those serve because they
+// measured faster (us, element loads / whole packs):
+//   16-bit LayerNorm rows that leave much of 1024 lanes idle -- a wavefront wholly past the row has
+//   next to nothing to do there, while the clamped form clears its packs: 16384 fp16 rows of 8193
+//   241 / 276, 12289 324 / 339, 13001 369 / 354; with fp32 weights 4096 rows of 8193 79.2 / 81.0,
+//   9001 89.3 / 84.0.  In 32nds of the pack slots.
+//   Tensors far beyond the caches, rows that fill most of their lanes -- memory-bound, and the
+//   requests of the next rows keep the memory busy while one wavefront waits for its elements: fp32
+//   LayerNorm [32768, 6143] 456 / 490, RMSNorm 450 / 484, LayerNorm [8192, 6143] 122.2 / 123.9 but
+//   [4096, 6143] 70.4 / 68.2 and [16384, 4097], half the slots idle, 157 / 149; fp16 RMSNorm on 512
+//   lanes x 3 packs [16384, 8193] 183 / 191, [4096, 8193] 57.0 / 56.6.
+constexpr bool norm_bwd_reads_elements_built(int esize, int G, int V, bool rms) {
+  if (esize == 4) return G == 256 || G == 512;
+  return rms ? G == 512 && V == 3 : G >= kMaxG;
+}
+inline bool norm_bwd_reads_elements(int esize, int wsize, int G, int V, bool rms, int64_t M,
+                                    int64_t N) {
+  if (!norm_bwd_reads_elements_built(esize, G, V, rms)) return false;
+  const int64_t packs = (N * esize + 15) / 16, slots = (int64_t)G * V;
+  if (esize == 4) return packs * 16 > slots * 9 && M * N > 50000000;
+  return rms ? M * N > 100000000 : packs * 32 <= slots * (wsize > 2 ? 17 : 25);
+}
 
 // Workgroups per compute unit of the grid-stride launch.  The norm kernels keep
 // gamma/beta (and the backward column sums) in registers across the rows of a
