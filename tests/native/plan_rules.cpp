@@ -10,4 +10,11 @@ int rule_norm_bwd_reads_elements(int esize, int wsize, int G, int V, int rms, in
   return norm_bwd_reads_elements(esize, wsize, G, V, rms != 0, M, N) ? 1 : 0;
 }
 
+// out: workgroups a team, workgroups a channel, packs a lane, whether the next slab is on its way,
+// workgroups launched
+void rule_gn_bwd_team(int64_t rows, int64_t D, int64_t cp, int esize, int64_t out[5]) {
+  const GnBwdTeam t = gn_bwd_team(rows, D, cp, esize, 256);
+  out[0] = t.team, out[1] = t.wpc, out[2] = t.v, out[3] = t.ahead, out[4] = t.grid;
+}
+
 }  // extern "C"

@@ -13,10 +13,13 @@ pytestmark = pytest.mark.gpu
 # (N, C, packs a channel, groups, dtype), of 512 workgroups: teams of 8, 140 slabs on 64 of them
 # (three rounds, the last for 12 teams), channels one pack short of their workgroup's; 80 slabs
 # (two rounds); 4 teams of 128, 32 slabs (eight rounds); one team of 440 and seven slabs, the last
-# workgroup of a channel half full; one slab a team; one team of 264 with eight packs a lane
+# workgroup of a channel half full; one slab a team; one team of 264 with eight packs a lane; 224
+# slabs on 42 teams of 12, eight packs a lane (six rounds), and 96 on 10 of 48 (ten), where the
+# layout that looks ahead would fill its workgroups less well
 SHAPES = [(70, 16, 2047, 2, torch.bfloat16), (40, 16, 1100, 2, torch.float16),
           (4, 128, 16384, 8, torch.float32), (7, 8, 55 * 2048 - 1000, 1, torch.float32),
-          (2, 16, 1025, 2, torch.float32), (1, 16, 65 * 2048 - 10, 2, torch.float32)]
+          (2, 16, 1025, 2, torch.float32), (1, 16, 65 * 2048 - 10, 2, torch.float32),
+          (28, 96, 2704, 8, torch.float32), (3, 512, 11552, 32, torch.bfloat16)]
 
 
 @pytest.mark.parametrize("N,C,packs,groups,dtype", SHAPES, ids=str)

@@ -42,3 +42,49 @@ def test_how_a_ragged_row_of_the_norm_backward_is_read(cabi, rules):
             for N in (5, 1401, 3001, 4097, 6143, 7777, 8193, 16383):
                 assert not reads_elements(cabi.F32, cabi.F32, rms, M, N)
         assert [reads_elements(cabi.F32, cabi.F32, rms, 32768, N) for N in (1401, 2049, 3001, 4097, 5001, 7777)] == [0, 0, 1, 0, 1, 1]
+
+
+def _gn_team(rules, N, C, side, esize, groups=32):
+    out = (ctypes.c_int64 * 5)()
+    hw, E = side * side, 16 // esize
+    assert hw % E == 0
+    rules.rule_gn_bwd_team(ctypes.c_int64(N * groups), ctypes.c_int64(C // groups), ctypes.c_int64(hw // E),
+                           esize, out)
+    return dict(zip(("team", "wpc", "v", "ahead", "grid"), out))
+
+
+def test_group_norm_backward_teams(rules):
+    """Every plan holds its channels and fits the machine, and the next slab is on its way only where
+    that neither idles workgroups nor runs clearly more rounds of packs."""
+    for esize in (2, 4):
+        for C in (32, 128, 256, 512, 1024):
+            for side in range(16, 520, 8):
+                cp = side * side * esize // 16
+                for N in (1, 2, 3, 5, 8, 64):
+                    t = _gn_team(rules, N, C, side, esize)
+                    if t["team"] == 0:  # (short channels, or one slab beyond the machine)
+                        continue
+                    D, slots = C // 32, t["wpc"] * t["v"] * 512
+                    assert t["v"] in (4, 8) and t["team"] == D * t["wpc"] >= 2
+                    assert slots >= cp and 2 * cp >= slots, "a channel is held, its workgroups half full at least"
+                    assert t["grid"] % t["team"] == 0 and t["team"] <= t["grid"] <= 512
+                    if t["ahead"]:
+                        assert t["v"] == 4 and N * 32 > t["grid"] // t["team"]
+                        # against eight packs a lane: no fewer workgroups at work, pack-rounds within an eighth
+                        wpc8 = -(-cp // 4096)
+                        if cp > 2048 and D * wpc8 <= 512:
+                            teams8 = min(512 // (D * wpc8), N * 32)
+                            rounds8 = -(-N * 32 // teams8)
+                            rounds = -(-N * 32 // (t["grid"] // t["team"]))
+                            assert t["grid"] >= 480 and 4 * rounds <= 9 * rounds8, (N, C, side, t)
+    # where the look-ahead kernel measured slower ...
+    for N, C, sides, esize in ((1, 512, range(320, 345, 8), 2), (1, 512, range(368, 393, 8), 2),
+                               (1, 512, range(408, 473, 8), 2), (1, 256, range(448, 481, 8), 2),
+                               (3, 512, (232,), 2), (4, 512, (152,), 2), (7, 128, (248,), 2), (1, 512, (296, 312), 4), (7, 384, (104,), 4)):
+        for side in sides:
+            assert not _gn_team(rules, N, C, side, esize)["ahead"], (N, C, side)
+    # ... and where faster
+    for N, C, side, esize in ((1, 512, 480, 2), (1, 512, 496, 2), (1, 512, 512, 2), (16, 512, 128, 2), (4, 256, 128, 2),
+                              (2, 512, 200, 2), (5, 256, 184, 2), (8, 128, 512, 2), (4, 256, 256, 4), (1, 512, 256, 4),
+                              (4, 128, 200, 4), (8, 128, 136, 4), (1, 512, 248, 4), (1, 384, 232, 4)):
+        assert _gn_team(rules, N, C, side, esize)["ahead"], (N, C, side)

@@ -800,51 +800,20 @@ int mi355x_group_norm_bwd(const void* dy, const void* x, const void* mean, const
   hipStream_t s = (hipStream_t)stream;
   // slabs beyond the registers whose channels are whole packs, 16-byte aligned tensors, dX
   // apart from dY and X (a workgroup whose team does not come together reads the whole slab
-  // of both while others write theirs): teams of workgroups, dY and X read once.  As few
-  // packs a lane (4 or 8 of each tensor) as hold a channel on one workgroup, else 8 and
-  // several workgroups a channel, the last of them at least half full.
+  // of both while others write theirs): teams of workgroups, dY and X read once.
   const int64_t E = 16 / esize_of(xd);
   if (!plan.resident && dx && HxW % E == 0 &&
       ((((uintptr_t)dy) | ((uintptr_t)x) | ((uintptr_t)dx)) & 15u) == 0) {
     const size_t nbytes = (size_t)d.rows * (size_t)d.L * (size_t)esize_of(xd);
     const char *ob = (const char*)dx, *gb = (const char*)dy, *xb = (const char*)x;
-    const int64_t cp = HxW / E;
-    constexpr int64_t kAheadChunk = (int64_t)kGnTeamAheadPacks * kTeamBlock;
-    int v = 8;
-    for (int t = 1; t < 8; t *= 2)
-      if ((int64_t)t * kTeamBlock >= cp) {
-        v = t;
-        break;
-      }
-    const int64_t cus = current_num_cus() * kTeamPerCu < kTeamMaxWorkgroups
-                            ? current_num_cus() * kTeamPerCu
-                            : kTeamMaxWorkgroups;
-    // A team that works through several slabs has the next one on its way meanwhile
-    // (gn_bwd_team_ahead_kernel): from two slabs a team where four packs a lane hold a channel
-    // (bf16 [4, 256, 128, 128] in 32 groups, two slabs a team: 26.7 -> 24.1 us), from more than
-    // three where that halves the eight packs a lane held (fp32 [4, 256, 256, 256], eight slabs a
-    // team: 154 -> 146 us; with two, bf16 [1, 256, 320, 320], it loses: 40.4 -> 47.3 us).
-    const int64_t per = d.D * ((cp + (int64_t)v * kTeamBlock - 1) / ((int64_t)v * kTeamBlock));
-    const int64_t ahead = d.D * ((cp + kAheadChunk - 1) / kAheadChunk);
-    if (v >= kGnTeamAheadPacks && per <= cus && ahead <= cus &&
-        d.rows > (v == kGnTeamAheadPacks ? 1 : 3) * (cus / per)) {
-      v = kGnTeamAheadPacks;
-      a.team_ahead = true;
-    }
-    const int64_t chunk = (int64_t)v * kTeamBlock;
-    const int64_t wpc = (cp + chunk - 1) / chunk;
-    const int64_t team = d.D * wpc;
     const bool apart = !(ob < gb + nbytes && gb < ob + nbytes) && !(ob < xb + nbytes && xb < ob + nbytes);
-    // (channels of at most 1024 packs -- one or two packs a lane -- move too little between
-    // two exchanges: bf16 [2, 2048, 64, 64] in 32 groups, 8 rounds of 8 KB a workgroup and
-    // tensor, 56.6 us against 35.0 us for the two launches)
-    if (apart && v >= 4 && team >= 2 && team <= cus && 2 * cp >= wpc * chunk) {
-      int64_t teams = cus / team;
-      if (teams > d.rows) teams = d.rows;
-      a.team = (int)team;
-      a.team_wpc = (int)wpc;
-      a.team_v = v;
-      a.team_grid = teams * team;
+    const GnBwdTeam t = gn_bwd_team(d.rows, d.D, HxW / E, esize_of(xd), current_num_cus());
+    if (apart && t.team > 0) {
+      a.team = t.team;
+      a.team_wpc = t.wpc;
+      a.team_v = t.v;
+      a.team_ahead = t.ahead;
+      a.team_grid = t.grid;
       a.team_slot = team_slot_for_call(s, &a.team_id);
       a.team_wait_ticks = g_team_wait_ticks.load(std::memory_order_relaxed);
     }

@@ -1115,6 +1115,71 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
   return 0;
 }
 
+// GroupNorm backward of slabs beyond the registers held by teams of workgroups, one workgroup or
+// several (`wpc`) a channel: gn_bwd_team_kernel (v packs a lane and tensor), or the one that has a
+// team's next slab on its way meanwhile, gn_bwd_team_ahead_kernel (ahead; v = kGnTeamAheadPacks).
+// team 0: not this shape.
+struct GnBwdTeam {
+  int team = 0, wpc = 0, v = 0;
+  bool ahead = false;
+  int64_t grid = 0;
+};
+
+// rows slabs of D channels of cp packs each.  As few packs a lane (4 or 8 of each tensor) as hold a
+// channel on one workgroup, else 8 and several workgroups a channel.
+inline GnBwdTeam gn_bwd_team(int64_t rows, int64_t D, int64_t cp, int esize, int num_cus) {
+  if (num_cus <= 0) num_cus = 256;
+  const int64_t wgs = (int64_t)num_cus * kTeamPerCu < kTeamMaxWorkgroups
+                          ? (int64_t)num_cus * kTeamPerCu
+                          : (int64_t)kTeamMaxWorkgroups;
+  GnBwdTeam none, t;
+  // (channels of at most 1024 packs -- one or two packs a lane -- move too little between two
+  // exchanges: bf16 [2, 2048, 64, 64] in 32 groups, 8 rounds of 8 KB a workgroup and tensor, 56.6
+  // us against 35.0 us for the two launches)
+  if (rows < 1 || D < 1 || cp <= 2 * kTeamBlock) return none;
+  auto layout = [&](int v) {
+    const int64_t chunk = (int64_t)v * kTeamBlock;
+    const int64_t wpc = (cp + chunk - 1) / chunk, team = D * wpc;
+    GnBwdTeam l;
+    if (team < 2 || team > wgs) return l;
+    const int64_t teams = wgs / team < rows ? wgs / team : rows;
+    l.team = (int)team;
+    l.wpc = (int)wpc;
+    l.v = v;
+    l.grid = teams * team;
+    return l;
+  };
+  t = layout(cp <= 4 * kTeamBlock ? 4 : 8);
+  if (t.team == 0) return none;
+  // A team that works through several slabs with the next one on its way.  Where four packs a lane
+  // hold a channel that costs nothing, and any second slab gains (bf16, 32 groups, us, without /
+  // with: [4, 256, 128, 128], two slabs a team, 26.8 / 24.5; [7, 512, 120, 120] 77.3 / 67.6).
+  // Where eight did, half as many slabs are held at a time and there are twice as many exchanges:
+  // from four slabs a team, on a grid that leaves no more than a sixteenth of the machine idle
+  // ([1, 512, 416, 416], 352 workgroups, 122 / 150; [1, 256, 448, 448], 416, 75.6 / 81.1), and only
+  // if a channel fits four packs a lane clearly better ([2, 512, 200, 200], three workgroups a
+  // channel for two, 69.6 / 63.4; fp32 [8, 128, 136, 136] 62.0 / 55.0; [4, 512, 152, 152], four
+  // for two, 65.3 / 75.5), or fills its workgroups (fp32 [4, 256, 256, 256] 154.6 / 144.3, bf16
+  // [1, 256, 512, 512] 87.6 / 86.9; [7, 128, 248, 248], 94 % filled, 67.6 / 71.4), or nearly does
+  // over eight slabs a team ([1, 512, 496, 496] 173.9 / 166.6; four: [1, 256, 496, 496] 85.4 / 87.2).
+  // fp32, half the arithmetic a pack, gains from four slabs if it nearly does ([1, 512, 248, 248]
+  // 80.4 / 76.3, [1, 384, 232, 232] 60.3 / 55.0; [7, 384, 104, 104], two thirds filled, 75.9 / 84.9).
+  const int64_t teams = t.grid / t.team;
+  if (t.v == kGnTeamAheadPacks) {
+    t.ahead = rows > teams;
+    return t;
+  }
+  const GnBwdTeam h = layout(kGnTeamAheadPacks);
+  if (h.team == 0 || rows <= 3 * teams || h.grid * 16 < wgs * 15) return t;
+  const int64_t slots = (int64_t)h.wpc * kGnTeamAheadPacks * kTeamBlock;
+  if (3 * h.wpc <= 5 * t.wpc || cp * 100 >= slots * 98 ||
+      (cp * 16 >= slots * 15 && (esize == 4 || rows > 7 * teams))) {
+    t = h;
+    t.ahead = true;
+  }
+  return t;
+}
+
 // ---- softmax over a non-innermost dimension: [outer, D, inner] ----------------
 //
 // A group of TX * TY threads owns one tile: TX lanes along `inner` (one 16-byte
