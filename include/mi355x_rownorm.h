@@ -387,7 +387,7 @@ int mi355x_rownorm_plan_at(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_
  * never a mix.  Production callers never use it: with no override set (the
  * state a process starts in) every entry point is re-entrant, and the only
  * mutable global state any of them touches is the call counter and the
- * bookkeeping slots of the team forward described at
+ * bookkeeping slots of the team launches described at
  * mi355x_rownorm_set_team_wait_us.  A call whose shape the forced variant cannot hold
  * fails with ROWNORM_ERR_OVERRIDE instead of silently choosing another, and so
  * does a field outside 0..65535. */
@@ -404,12 +404,11 @@ int mi355x_rownorm_set_override(rownorm_op op, int lanes_per_row, int packs_per_
  * microseconds; 0xffffffff
  * restores the default, one second.  0 makes every wait give up at once, which is
  * how the tests exercise that path without making any kernel hang.  Process-global.
- * Such calls draw an id and one of 16 bookkeeping slots in library-owned device
- * memory from process-wide counters; results do not depend on which slot a call
- * gets, and two calls that share a slot while both run (more than 16 such calls in
- * flight across streams) each detect it, their workgroups summing their rows
- * themselves.  On a stream under capture these rows take the multi-launch kernels
- * instead. */
+ * Such calls draw an id from a process-wide counter and use the bookkeeping slot of their
+ * stream, in library-owned device memory (48 MiB a GPU); results do not depend on the slot.
+ * A stream takes a slot with its first such call and keeps it; streams beyond the 64 slots
+ * take the multi-launch kernels, which exchange nothing, and so do these rows on a stream
+ * under capture. */
 int mi355x_rownorm_set_team_wait_us(unsigned int microseconds);
 
 /* Measurement aid, no counterpart in the reference: a plain streaming kernel over

@@ -1,6 +1,7 @@
 // The host-side rules that choose a kernel (plan.hpp has no HIP types in it) behind plain C functions,
 // for tests/test_plan_rules.py, which compiles this file with g++ and loads it.
 #include "../../torch-xpu-ops_amd/csrc/kernels/plan.hpp"
+#include "../../torch-xpu-ops_amd/csrc/kernels/team_slots.hpp"
 
 using namespace rownorm;
 
@@ -16,5 +17,11 @@ void rule_gn_bwd_team(int64_t rows, int64_t D, int64_t cp, int esize, int64_t ou
   const GnBwdTeam t = gn_bwd_team(rows, D, cp, esize, 256);
   out[0] = t.team, out[1] = t.wpc, out[2] = t.v, out[3] = t.ahead, out[4] = t.grid;
 }
+
+// one table of slots for streams, as the library keeps one per device
+int rule_team_slots() { return kTeamSlots; }
+void* rule_slots_new() { return new StreamSlots<kTeamSlots>(); }
+void rule_slots_delete(void* t) { delete (StreamSlots<kTeamSlots>*)t; }
+int rule_slot_of(void* t, uintptr_t key) { return ((StreamSlots<kTeamSlots>*)t)->of(key); }
 
 }  // extern "C"

@@ -2,7 +2,9 @@
 header behind C functions) is compiled with g++ and called through ctypes."""
 import ctypes
 import os
+import random
 import subprocess
+import threading
 
 import pytest
 
@@ -88,3 +90,34 @@ def test_group_norm_backward_teams(rules):
                               (2, 512, 200, 2), (5, 256, 184, 2), (8, 128, 512, 2), (4, 256, 256, 4), (1, 512, 256, 4),
                               (4, 128, 200, 4), (8, 128, 136, 4), (1, 512, 248, 4), (1, 384, 232, 4)):
         assert _gn_team(rules, N, C, side, esize)["ahead"], (N, C, side)
+
+
+def test_every_stream_has_its_own_exchange_memory(rules):
+    """Slots are handed out by stream, whatever the order and the number of calls: one stream always gets
+    the same, two never share one, a stream beyond the last slot gets none; also from several threads."""
+    rules.rule_slots_new.restype = ctypes.c_void_p
+    n = rules.rule_team_slots()
+    table = ctypes.c_void_p(rules.rule_slots_new())
+    of = lambda key: rules.rule_slot_of(table, ctypes.c_size_t(key))  # noqa: E731
+    try:
+        keys = [1] + [0x7f0000001000 + 64 * i for i in range(n - 1)]
+        got, start = [{} for _ in range(8)], threading.Barrier(8)
+
+        def calls(mine, seed):
+            order = keys * 20
+            random.Random(seed).shuffle(order)
+            start.wait()
+            for k in order:
+                s = of(k)
+                assert mine.setdefault(k, s) == s, "a stream's slot changed"
+
+        threads = [threading.Thread(target=calls, args=(got[i], i)) for i in range(8)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert all(g == got[0] for g in got) and sorted(got[0].values()) == list(range(n))
+        assert of(0x7f1000000000) == -1 and of(0x7f1000000040) == -1
+        assert all(of(k) == got[0][k] for k in keys)
+    finally:
+        rules.rule_slots_delete(table)

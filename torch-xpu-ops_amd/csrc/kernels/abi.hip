@@ -5,6 +5,7 @@
 
 #include <atomic>
 #include "launch.hpp"
+#include "team_slots.hpp"
 
 namespace rownorm {
 // defined in the per-dtype translation units
@@ -165,25 +166,39 @@ int static_scratch(void** out) {
   return 0;
 }
 
-// Bookkeeping memory of norm_fwd_team_kernel (the workgroups' partial sums), one slot
-// a call, slots handed out round-robin; per device, like `scratch`.  Zero at load and
-// never cleared: every word a call reads is tagged with the call's id.
+// Exchange memory of the team launches (the workgroups' partial sums), one slot a stream
+// (StreamSlots); per device, like `scratch`.  Zero at load and never cleared: every word a call
+// reads is tagged with the call's id.  16 MiB, and 32 MiB for the strided softmax, whose
+// workgroups pass numbers for every column.
 static __device__ __align__(256) __attribute__((used)) TeamSlot team_slots[kTeamSlots];
-std::atomic<void*> g_team_ptr[kMaxDevices];
+static __device__ __align__(256) __attribute__((used)) TeamColumns team_columns[kTeamColumnSlots];
+
+template <int N>
+struct TeamMemory {
+  std::atomic<void*> address[kMaxDevices];
+  StreamSlots<N> slots[kMaxDevices];
+};
+TeamMemory<kTeamSlots> g_team_slots;
+TeamMemory<kTeamColumnSlots> g_team_columns;
 std::atomic<unsigned int> g_team_calls{0};
 // Bound of a workgroup's wait for its team, in ticks of the 100 MHz constant-rate
 // clock: one second unless mi355x_rownorm_set_team_wait_us() says otherwise.
 std::atomic<unsigned long long> g_team_wait_ticks{100000000ull};
 
-// The same for the strided softmax, whose workgroups pass numbers for every column.
-static __device__ __align__(256) __attribute__((used)) TeamColumns team_columns[kTeamSlots];
-std::atomic<void*> g_team_columns_ptr[kMaxDevices];
+// What tells streams apart.  The null stream has two names; hipStreamPerThread is another stream
+// in every thread, so there it is something of the thread's own.
+uintptr_t stream_key(hipStream_t stream) {
+  static thread_local char own;
+  if (stream == nullptr || stream == hipStreamLegacy) return (uintptr_t)1;
+  if (stream == hipStreamPerThread) return (uintptr_t)&own;
+  return (uintptr_t)stream;
+}
 
-// The slot and id of a new call on the current device out of the kTeamSlots slots of `slot_bytes`
-// at `symbol` (its per-device addresses: `table`), or null when the team kernel is not to be
-// used: the address is not known, or the stream is being captured (a replay would run with the
-// id of the capture).
-void* team_memory_for_call(std::atomic<void*>* table, const void* symbol, size_t slot_bytes,
+// The slot and id of a new call on the current device out of the N slots of `slot_bytes` at
+// `symbol`, or null when the team kernel is not to be used: the address is not known, the stream is
+// being captured (a replay would run with the id of the capture), or other streams have all slots.
+template <int N>
+void* team_memory_for_call(TeamMemory<N>& memory, const void* symbol, size_t slot_bytes,
                            hipStream_t stream, unsigned int* id) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &st) != hipSuccess) {
@@ -193,25 +208,27 @@ void* team_memory_for_call(std::atomic<void*>* table, const void* symbol, size_t
   if (st != hipStreamCaptureStatusNone) return nullptr;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
-  void* p = table[dev].load(std::memory_order_acquire);
+  void* p = memory.address[dev].load(std::memory_order_acquire);
   if (p == nullptr) {
     if (hipGetSymbolAddress(&p, symbol) != hipSuccess || p == nullptr) {
       (void)hipGetLastError();
       return nullptr;
     }
-    table[dev].store(p, std::memory_order_release);
+    memory.address[dev].store(p, std::memory_order_release);
   }
+  const int slot = memory.slots[dev].of(stream_key(stream));
+  if (slot < 0) return nullptr;
   unsigned int n = g_team_calls.fetch_add(1, std::memory_order_relaxed) + 1;
   if (n == 0) n = g_team_calls.fetch_add(1, std::memory_order_relaxed) + 1;  // 0 tags nothing
   *id = n;
-  return (char*)p + (size_t)(n % kTeamSlots) * slot_bytes;
+  return (char*)p + (size_t)slot * slot_bytes;
 }
 
 void* team_slot_for_call(hipStream_t stream, unsigned int* id) {
-  return team_memory_for_call(g_team_ptr, HIP_SYMBOL(team_slots), sizeof(TeamSlot), stream, id);
+  return team_memory_for_call(g_team_slots, HIP_SYMBOL(team_slots), sizeof(TeamSlot), stream, id);
 }
 void* team_columns_for_call(hipStream_t stream, unsigned int* id) {
-  return team_memory_for_call(g_team_columns_ptr, HIP_SYMBOL(team_columns), sizeof(TeamColumns),
+  return team_memory_for_call(g_team_columns, HIP_SYMBOL(team_columns), sizeof(TeamColumns),
                               stream, id);
 }
 

@@ -17,9 +17,10 @@
 // reader needs one round trip (see team_publish_tagged).  Every access is a device-scope
 // atomic store or load, which goes to memory: no read-modify-write (256 workgroups
 // counting on one word took hundreds of microseconds), and no release or acquire fence
-// (each writes back or invalidates a whole L2).  Two calls that were handed the same slot
-// while both run -- possible only with more such calls in flight than slots -- overwrite
-// each other's tags and therefore never accept each other's numbers.
+// (each writes back or invalidates a whole L2).  The memory is the stream's own
+// (team_slots.hpp); should two calls use it at once all the same (a stream destroyed with
+// work outstanding whose handle a new one was given), they overwrite each other's tags and
+// never accept each other's numbers.
 //
 // The wait is bounded, and no workgroup depends on another to finish.  A workgroup
 // stops waiting when its team is complete, when any workgroup of the call has given

@@ -85,13 +85,16 @@ struct Plan {
 };
 
 // norm_fwd_team_kernel: threads a workgroup, packs a lane at most, workgroups of
-// the grid at most (one a compute unit), slots of bookkeeping memory.
+// the grid at most.
 constexpr int kTeamBlock = 512;
 constexpr int kTeamPerCu = 2;  // workgroups of a team launch a compute unit holds
 constexpr int kTeamMaxV = 16;
 constexpr int kTeamGroup = 2;  // packs whose weights are requested together
 constexpr int kTeamMaxWorkgroups = 512;
-constexpr int kTeamSlots = 16;
+// streams with a slot of exchange memory of their own (team_slots.hpp): more than the default
+// stream and the 32 of a framework's pool; for the strided softmax, whose slots are 4 MiB, eight
+constexpr int kTeamSlots = 64;
+constexpr int kTeamColumnSlots = 8;
 constexpr int kTeamMinTeams = 8;
 // gn_bwd_team_ahead_kernel: packs a lane holds of each tensor and slab (two slabs at a time).
 constexpr int kGnTeamAheadPacks = 4;
