@@ -18,6 +18,16 @@ void rule_gn_bwd_team(int64_t rows, int64_t D, int64_t cp, int esize, int64_t ou
   out[0] = t.team, out[1] = t.wpc, out[2] = t.v, out[3] = t.ahead, out[4] = t.grid;
 }
 
+// out: workgroups a team, packs a lane, lanes along inner, workgroups launched; then whether the tile
+// kernel holds D, its lanes along inner and along D, rows a lane and workgroups, chunks
+void rule_strided_plan(int backward, int64_t outer, int64_t D, int64_t inner, int esize, int64_t out[10]) {
+  StridedPlan p;
+  make_strided_plan(backward != 0, outer, D, inner, esize, 256, Override{}, &p);
+  out[0] = p.team, out[1] = p.team_v, out[2] = 1 << p.team_tx_log2, out[3] = p.team_grid;
+  out[4] = p.resident, out[5] = 1 << p.tx_log2, out[6] = 1 << p.ty_log2, out[7] = p.V, out[8] = p.grid;
+  out[9] = p.chunks;
+}
+
 // one table of slots for streams, as the library keeps one per device
 int rule_team_slots() { return kTeamSlots; }
 void* rule_slots_new() { return new StreamSlots<kTeamSlots>(); }

@@ -1,0 +1,74 @@
+"""Team launches on several streams at once: every stream has exchange memory of its own and no team
+is larger than an eighth of the machine, so calls that share the machine finish without waiting for
+one another's end, with the results they have alone; a stream beyond the slots takes the launches that
+exchange nothing.  (The reference's kernels share nothing between calls: SpatialSoftmaxForward,
+src/ATen/native/xpu/sycl/SoftMaxKernels.cpp:725-950, LayerNormKernels.cpp:360-470.)"""
+import time
+
+import pytest
+import torch
+
+from helpers import assert_close, gen
+
+pytestmark = pytest.mark.gpu
+
+
+def _calls(cabi, gpu, seed):
+    """Thunks of one stream: strips on 64 workgroups, on a few, forward and backward, and rows of the
+    norm and softmax kernels held by teams."""
+    g = gen(seed)
+    x = torch.randn(1, 32000, 64, generator=g).bfloat16().to(gpu)
+    w = torch.randn(4, 1025, 1024, generator=g).bfloat16().to(gpu)
+    y = torch.softmax(w.float(), 1).bfloat16()
+    r = torch.randn(16, 140000, generator=g).bfloat16().to(gpu)
+    gamma = torch.ones(140000, dtype=torch.bfloat16, device=gpu)
+    return [lambda: cabi.softmax_strided_fwd(x, 1), lambda: cabi.softmax_strided_fwd(w, 1, cabi.LOG_SOFTMAX),
+            lambda: cabi.softmax_strided_bwd(w, y, 1),
+            lambda: cabi.layer_norm_fwd(r, gamma, None, 1e-5)[0], lambda: cabi.softmax_fwd(r)]
+
+
+def test_calls_on_three_streams_do_not_wait_for_one_another(cabi, gpu):
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    calls = [_calls(cabi, gpu, 2600 + i) for i in range(3)]
+    alone = [[f() for f in fs] for fs in calls]
+    got = [[None] * len(fs) for fs in calls]
+    for i, s in enumerate(streams):  # (the streams' slots, the allocator's blocks)
+        s.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            got[i] = [f() for f in calls[i]]
+    torch.cuda.synchronize()
+    print("case three streams, 40 rounds of five calls each", flush=True)
+    t0 = time.perf_counter()
+    for k in range(40):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                for j, f in enumerate(calls[i]):
+                    # (every stream meets the others' calls at another place)
+                    j = (j + k * (i + 1)) % len(calls[i])
+                    got[i][j] = calls[i][j]()
+    torch.cuda.synchronize()
+    # (one wait that runs out is a second)
+    assert time.perf_counter() - t0 < 0.9
+    for i in range(3):
+        for j in range(len(calls[i])):
+            assert torch.equal(got[i][j].view(torch.uint8), alone[i][j].view(torch.uint8)), (i, j)
+
+
+def test_more_streams_than_slots(cabi, gpu):
+    """Twelve streams, eight of them with a slot of the strided softmax: the others' results come from
+    the launches that exchange nothing."""
+    g = gen(2650)
+    x = (3 * torch.randn(2, 1500, 256, generator=g)).to(gpu)
+    grad = torch.randn(2, 1500, 256, generator=g).to(gpu)
+    want = torch.softmax(x.double(), 1)
+    wgrad = want * (grad.double() - (want * grad.double()).sum(1, keepdim=True))
+    torch.cuda.synchronize()
+    outs = []
+    for s in [torch.cuda.Stream() for _ in range(12)]:
+        with torch.cuda.stream(s):
+            y = cabi.softmax_strided_fwd(x, 1)
+            outs.append((y, cabi.softmax_strided_bwd(grad, y, 1)))
+    torch.cuda.synchronize()
+    for k, (y, gi) in enumerate(outs):
+        assert_close(y, want.float().cpu().numpy(), torch.float32, "y of stream %d" % k)
+        assert_close(gi, wgrad.float().cpu().numpy(), torch.float32, "gi of stream %d" % k)

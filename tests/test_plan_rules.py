@@ -121,3 +121,37 @@ def test_every_stream_has_its_own_exchange_memory(rules):
         assert all(of(k) == got[0][k] for k in keys)
     finally:
         rules.rule_slots_delete(table)
+
+
+def _strided(rules, backward, outer, D, inner, esize):
+    out = (ctypes.c_int64 * 10)()
+    i64 = ctypes.c_int64
+    rules.rule_strided_plan(backward, i64(outer), i64(D), i64(inner), esize, out)
+    return dict(zip(("team", "v", "tx", "grid", "resident", "tile_tx", "tile_ty", "tile_v", "tile_grid",
+                     "chunks"), out))
+
+
+def test_strided_softmax_teams(rules):
+    """Every row of a strip is held, on instances that exist, by teams of at most an eighth of the
+    machine: launches on several streams always hold whole teams, which finish."""
+    built = {0: (1, 2, 3, 4, 6, 8, 10, 12, 14, 16), 1: (1, 2, 3, 4, 5, 6, 7, 8)}
+    rng = random.Random(31)
+    shapes = [(o, D, px) for o in (1, 8, 200, 2000) for D in (257, 700, 2048, 8192, 60000, 262144, 1 << 20)
+              for px in (1, 2, 3, 8, 17, 33, 40, 238, 1024)]
+    shapes += [(rng.randint(1, 300), int(2 ** rng.uniform(8, 20)), int(2 ** rng.uniform(0, 14))) for _ in range(3000)]
+    teams = 0
+    for outer, D, px in shapes:
+        for esize in (2, 4):
+            for backward in (0, 1):
+                p = _strided(rules, backward, outer, D, px * 16 // esize, esize)
+                if p["team"] == 0:
+                    continue
+                teams += 1
+                ty = 512 // p["tx"]
+                assert p["tx"] in (1, 2, 4, 8, 16, 32) and p["v"] in built[backward]
+                assert p["team"] * ty * p["v"] >= D > (p["team"] - 1) * ty * p["v"], "held, no workgroup without a row"
+                assert p["team"] <= 64, (outer, D, px, esize, backward, p)
+                assert p["grid"] % p["team"] == 0 and p["team"] <= p["grid"] <= 512
+                assert p["grid"] // p["team"] <= outer * -(-px // p["tx"])
+                assert ty * p["v"] * px * 16 < 2 ** 31
+    assert teams > 3000

@@ -1327,6 +1327,12 @@ inline int make_strided_plan(bool backward, int64_t outer, int64_t D, int64_t in
   if (D > kStridedTeamMinD && p.fast && ov.G == 0 && ov.V == 0 && ov.bpc == 0) {
     const int vmax = strided_team_max_v(backward);
     const int64_t wgs = num_cus * kTeamPerCu < kTeamMaxWorkgroups ? num_cus * kTeamPerCu : kTeamMaxWorkgroups;
+    // A team is an eighth of the machine at most.  Workgroups start in order, so a launch that shares
+    // the machine with others holds whole teams as soon as it holds that much of it, and those
+    // finish and make room: calls on several streams cannot keep one another's teams apart until
+    // the waits end.  (Larger teams gain nothing either, their exchange takes longer: bf16 [1, 8192,
+    // 136] forward on 64 workgroups 11.8 us, on 256 27.9; fp32 [8, 8192, 16] 64 at most.)
+    const int64_t most_wgs = wgs / kTeamMinTeams > 0 ? wgs / kTeamMinTeams : 1;
     for (int wide = 0; wide < 2; ++wide) {
       const int most_tx = wide ? kStridedTeamWideTx : kStridedTeamTx;
       const int tx = px < most_tx ? px : most_tx;
@@ -1334,12 +1340,13 @@ inline int make_strided_plan(bool backward, int64_t outer, int64_t D, int64_t in
       const int64_t need = (D + ty * vmax - 1) / (ty * vmax);
       const int64_t strips = outer * ((packs + tx - 1) / tx);
       // (byte offsets of a lane inside a workgroup's rows are 32 bits wide)
-      if (need > wgs || ty * vmax * inner * 4 >= (int64_t(1) << 31)) break;
+      if (need > most_wgs || ty * vmax * inner * 4 >= (int64_t(1) << 31)) break;
       int64_t teams = wgs / need < strips ? wgs / need : strips;
       const int64_t rounds = (strips + teams - 1) / teams;
       teams = (strips + rounds - 1) / rounds;
       const int64_t most = (D + ty - 1) / ty;
       int64_t team = wgs / teams < most ? wgs / teams : most;
+      if (team > most_wgs) team = most_wgs;
       int64_t v = (D + ty * team - 1) / (ty * team);
       for (int c : kStridedTeamV[backward ? 1 : 0])
         if (c >= v) {
