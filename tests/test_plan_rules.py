@@ -155,3 +155,29 @@ def test_strided_softmax_teams(rules):
                 assert p["grid"] // p["team"] <= outer * -(-px // p["tx"])
                 assert ty * p["v"] * px * 16 < 2 ** 31
     assert teams > 3000
+
+
+def test_strided_softmax_tile_or_teams(rules):
+    """Teams where they measured faster than the one-workgroup tile, and strips of the width that measured
+    faster: [outer, D, packs of inner], in 16 bits unless stated."""
+    for outer, D, px in ((2000, 257, 1), (200, 512, 1), (2000, 300, 2), (200, 1025, 1), (2000, 512, 4),  # the tile spans the row
+                         (8, 257, 8), (1, 257, 64), (200, 256, 238), (8, 450, 72), (8, 512, 100)):
+        for esize in (2, 4):
+            for backward in (0, 1):
+                p = _strided(rules, backward, outer, D, px * 16 // esize, esize)
+                assert p["team"] == 0 and p["resident"], (outer, D, px, esize, backward, p)
+                assert p["tile_ty"] * p["tile_v"] >= D
+    for outer, D, px, esize in ((200, 257, 40, 2), (40, 257, 72, 2), (40, 384, 72, 4), (1, 512, 1024, 4)):
+        assert _strided(rules, 0, outer, D, px * 16 // esize, esize)["team"] == 0
+    for outer, D, px in ((4, 512, 1024), (64, 300, 100), (200, 512, 17), (40, 512, 238), (1, 700, 4), (8, 2048, 2),
+                         (1, 8192, 1024), (1, 30000, 8), (35, 1000, 238)):
+        for esize in (2, 4):
+            for backward in (0, 1):
+                assert _strided(rules, backward, outer, D, px * 16 // esize, esize)["team"] >= 1, (outer, D, px)
+    width = lambda *a: _strided(rules, *a)["tx"]  # noqa: E731
+    assert width(0, 35, 1000, 1904, 2) == width(1, 35, 1000, 1904, 2) == 32
+    assert width(0, 200, 700, 320, 2) == 16 and width(0, 200, 257, 800, 2) == 16  # a last strip mostly past the row
+    assert width(1, 200, 700, 264, 2) == 32
+    assert width(0, 1, 8192, 8192, 2) == width(1, 1, 8192, 8192, 2) == 16
+    assert width(0, 1, 8192, 136, 2) == 8 and width(1, 1, 30000, 136, 2) == 8
+    assert _strided(rules, 0, 8, 8192, 16, 4)["team"] == 16

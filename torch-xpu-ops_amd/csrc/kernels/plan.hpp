@@ -1192,8 +1192,8 @@ inline GnBwdTeam gn_bwd_team(int64_t rows, int64_t D, int64_t cp, int esize, int
 // as a row of `inner` has packs, capped so that a group is one wavefront where
 // that leaves at least 8 lanes (128-byte segments) per row, and 256 threads
 // otherwise.  A group of one wavefront reduces with shuffles alone.  D beyond
-// 64 rows x 8 packs x 4 lanes takes the multi-pass kernel; from D = 257 strips of whole packs are
-// held by teams of workgroups where the call allows it.
+// 64 rows x 8 packs x 4 lanes takes the multi-pass kernel.  Strips of whole packs are
+// held by teams of workgroups instead where the call allows it and they are faster.
 struct StridedPlan {
   bool resident = true;
   bool fast = true;  // inner % E == 0
@@ -1228,6 +1228,131 @@ inline int log2_of_pow2(int v) {
   int l = 0;
   while ((1 << l) < v) ++l;
   return l;
+}
+
+// Strips of tx packs held by teams: as few workgroups a strip as hold its D rows, as many teams as
+// strips and compute units allow, evened out over the rounds; then a strip is spread over the
+// workgroups its team can have.
+struct StridedTeam {
+  int team = 0, v = 0, tx = 0;
+  bool capped = false;  // there were workgroups for a larger team
+  int64_t rounds = 0, grid = 0;
+};
+inline StridedTeam strided_team_of(bool backward, int64_t outer, int64_t D, int64_t packs, int esize, int tx,
+                                   int num_cus) {
+  const int64_t wgs = (int64_t)num_cus * kTeamPerCu < kTeamMaxWorkgroups ? (int64_t)num_cus * kTeamPerCu
+                                                                        : (int64_t)kTeamMaxWorkgroups;
+  // A team is an eighth of the machine at most.  Workgroups start in order, so a launch that shares
+  // the machine with others holds whole teams as soon as it holds that much of it, and those
+  // finish and make room: calls on several streams cannot keep one another's teams apart until
+  // the waits end.  (Larger teams gain nothing either, their exchange takes longer: bf16 [1, 8192,
+  // 136] forward on 64 workgroups 11.8 us, on 256 27.5.)
+  const int64_t most_wgs = wgs / kTeamMinTeams > 0 ? wgs / kTeamMinTeams : 1;
+  const int64_t ty = kTeamBlock / tx, vmax = strided_team_max_v(backward);
+  const int64_t need = (D + ty * vmax - 1) / (ty * vmax);
+  const int64_t strips = outer * ((packs + tx - 1) / tx);
+  StridedTeam t;
+  // (byte offsets of a lane inside a workgroup's rows are 32 bits wide; a float32 output of a 16-bit
+  // tensor has twice the bytes)
+  if (need > most_wgs || ty * vmax * packs * 32 >= (int64_t(1) << 31)) return t;
+  int64_t teams = wgs / need < strips ? wgs / need : strips;
+  t.rounds = (strips + teams - 1) / teams;
+  teams = (strips + t.rounds - 1) / t.rounds;
+  const int64_t most = (D + ty - 1) / ty;
+  int64_t team = wgs / teams < most ? wgs / teams : most;
+  t.capped = team > most_wgs;
+  if (t.capped) team = most_wgs;
+  // (one pack a lane on most of the machine: half as many workgroups with two exchange sooner --
+  // bf16 [8, 8192, 32] 12.2 -> 10.2 us)
+  if (team > most_wgs / 2 && ty * team >= D && 2 * teams * team > wgs) team = (team + 1) / 2;
+  // (a float32 forward of at most 16 columns: a column's thread merges its team's pairs one after the
+  // other, two exponentials each -- [8, 8192, 16] on 64 workgroups a team 15.2 us, 32 13.1, 16 11.4;
+  // not where that makes it more than eight packs a lane: [1, 30000, 16] 14.2, on 16 19.2)
+  if (!backward && esize == 4 && tx <= 4 && team > 16 && D <= ty * 16 * 8) team = 16;
+  int64_t v = (D + ty * team - 1) / (ty * team);
+  for (int c : kStridedTeamV[backward ? 1 : 0])
+    if (c >= v) {
+      v = c;
+      break;
+    }
+  team = (D + ty * v - 1) / (ty * v);
+  t.team = (int)team;
+  t.v = (int)v;
+  t.tx = tx;
+  t.grid = teams * team;
+  return t;
+}
+
+// The strip's width: 16 packs (256-byte segments), fewer where D needs more workgroups than a team
+// may have, or where one round of such teams leaves workgroups over (bf16 [1, 8192, 136] 11.8 us
+// with 16 packs, 10.4 with 8; backward of [1, 16384, 136] 11.7, 10.1).
+// Or 32 packs, half as many strips to exchange ([35, 1000, 1904] forward / backward 77 / 96 us, 16
+// packs 95 / 111), but not
+//   where a team holds the strips all at once or D needs large teams, whose exchange grows with the
+//   columns ([1, 8192, 8192] 77 / 106, 16 packs 71 / 104);
+//   where the last strip, mostly past the row, makes more rounds of packs of it ([200, 700, 320],
+//   5/8 of two strips: 62 us, 16 packs 54; [200, 257, 800] 62, 41).  Rows that are not whole
+//   128-byte lines share a line with either neighbour, which narrow strips read twice as often: there
+//   only if the rounds are a third more (backward: over a third; [200, 700, 264] 64 / 70, 16 packs
+//   64 / 76; fp32 [200, 1025, 132] backward 98, 103);
+//   where 16 packs take one workgroup a strip, nothing to exchange, and no more rounds ([200, 257,
+//   512] 35, 16 packs 27; off the lines only short strips: [200, 512, 264] 47, 54).
+// One round of workgroups that each hold a strip alone and are too few to fill two thirds of the
+// machine ([40, 257, 800] 14.5 us) take 32 packs too (12.4).
+inline StridedTeam strided_team(bool backward, int64_t outer, int64_t D, int64_t packs, int esize, int num_cus) {
+  const int px = packs >= 64 ? 64 : pow2_ceil(packs);
+  int tx = px < kStridedTeamTx ? px : kStridedTeamTx;
+  StridedTeam n = strided_team_of(backward, outer, D, packs, esize, tx, num_cus);
+  while (tx > 4 && n.team == 0) {
+    n = strided_team_of(backward, outer, D, packs, esize, tx /= 2, num_cus);
+    // (narrow segments in many rounds lose to the launches without teams: bf16 backward of [1, 30000,
+    // 1904], four rounds, 152 us against 124; [8, 30000, 136], three, 91 against 98)
+    if (n.rounds > 3) return StridedTeam{};
+  }
+  if (n.capped && tx > 8 && n.rounds == 1) {
+    const StridedTeam h = strided_team_of(backward, outer, D, packs, esize, tx / 2, num_cus);
+    if (h.team > 0 && h.rounds == 1) return h;
+  }
+  if (n.team == 0 || tx < kStridedTeamTx || px <= kStridedTeamTx || D > kStridedTeamWideMaxD) return n;
+  if (n.rounds == 1 && !(n.team == 1 && n.grid > kTeamMaxWorkgroups / 2 && 3 * n.grid < 2 * kTeamMaxWorkgroups)) return n;
+  const StridedTeam w = strided_team_of(backward, outer, D, packs, esize, kStridedTeamWideTx, num_cus);
+  if (w.team == 0) return n;
+  const int64_t nc = n.rounds * n.v, wc = w.rounds * w.v;
+  const bool lines = packs % 8 == 0;
+  if (n.team == 1 && wc >= nc && (lines || n.v <= 10)) return n;
+  return (lines ? 8 * wc > 9 * nc : backward ? 3 * wc > 4 * nc : 3 * wc >= 4 * nc) ? n : w;
+}
+
+// Whether teams serve a shape that the one-workgroup tile (TX lanes along `inner`) holds.  D <= 256
+// is the tile's (at D = 200 [20, 200, 4096] 20.5 / 22.5 us, teams 23.2 / 25.5), and so is a tile
+// that spans the row or eight lanes of it: one pass, no exchange (bf16 [2000, 512, 16] 14.1 us, teams
+// 26.3).  Beyond, the tile's segments are 64 bytes: teams where bandwidth counts, from about 7 MB
+// (bf16 forward / backward, tile -> teams: [4, 512, 8192] 28.6 / 38.1 -> 16.2 / 19.0 us, [64, 300,
+// 800] 23.5 / 29.9 -> 15.8 / 25.8; below, [8, 257, 512] 8.0 / 6.8 against 9.0 / 7.5); later for a
+// forward whose rows those segments divide (bf16 [200, 320, 64], 8.2 MB, 9.7 against 10.1) and for a
+// float32 forward, whose arithmetic the tile hides better ([200, 257, 68], 14 MB, 16.5 against
+// 14.9); and a forward of such rows never where teams would leave half of their packs empty, a
+// quarter in float32, a little more where nothing is exchanged (bf16 [200, 257, 320] 24.4 against 26.6, [40, 257, 576] 11.6 against 12.4, but
+// [200, 257, 192], one workgroup a strip, 18.6 against 14.5; fp32 [40, 384, 288] 11.0 against 12.9,
+// [40, 384, 256] 13.9 against 11.5, [2000, 257, 32], one workgroup a strip, 37.8 against 34.9).  Smaller calls on more than eight packs go by the length of the
+// tile's serial part, if they are few tiles or their rows are not divided by the segments (bf16 [8,
+// 384, 136] 9.9 -> 8.4 forward, [1, 512, 512] 8.3 -> 6.6 backward, but [8, 512, 576] 9.4 against
+// 9.9; fp32 [1, 512, 132] 7.2 -> 6.5 backward, [8, 512, 256] 8.7 -> 7.8, [8, 512, 160] 6.8 against
+// 7.5).
+inline bool strided_team_beats_tile(bool backward, int64_t outer, int64_t D, int64_t packs, int esize, int TX,
+                                    const StridedTeam& t) {
+  if (D <= kStridedTeamMinD || TX >= 8 || TX >= packs) return false;
+  const int64_t bytes = outer * D * packs * 16, tiles = outer * ((packs + TX - 1) / TX);
+  const bool divided = packs % TX == 0, few = tiles <= 64;
+  // packs of the teams' rounds that hold an element, in 64ths
+  const int64_t held = outer * D * packs * 64 / (t.rounds * t.v * kTeamMaxWorkgroups * kTeamBlock);
+  if (!backward && divided && !few && held < (esize == 4 ? (t.team > 1 ? 48 : 40) : t.team > 1 ? 32 : 29))
+    return false;
+  if (bytes >= (backward ? 7000000 : esize == 4 ? 13500000 : divided ? 10000000 : 7000000)) return true;
+  if (packs <= 8 || (esize == 4 && !backward)) return false;
+  const bool even = tiles <= 128 && packs % 16 == 0;
+  if (backward) return divided ? D >= 448 && (even || (few && esize == 2)) : D >= (esize == 4 ? 448 : 320);
+  return divided ? D >= 384 && few : D >= 320;
 }
 
 // Override: G = lanes along inner (power of two 1..64; -1 forces the multi-pass
@@ -1316,49 +1441,15 @@ inline int make_strided_plan(bool backward, int64_t outer, int64_t D, int64_t in
       TY = kStridedBlock / TX;
     }
   }
-  // Strips held by teams of workgroups: as few workgroups a strip as hold its D rows, as many
-  // teams as strips and compute units allow, evened out over the rounds; then a strip is spread
-  // over the workgroups its team can have.  From D = 257, where the one-workgroup tile above is
-  // down to 64-byte row segments (bf16 forward / backward, tile -> team: [4, 512, 8192] 29.3 / 39.0
-  // -> 17.7 / 20.4 us, [64, 300, 800] 24.7 / 30.4 -> 17.5 / 26.4; at D = 200 the tile is ahead:
-  // [20, 200, 4096] 20.5 / 22.5 against 23.2 / 25.5).  Strips of 16 packs where a team holds them
-  // all at once or D needs large teams (the exchange grows with the columns), of 32 otherwise
-  // ([35, 1000, 1904]: 16 packs 95 / 111 us, 32 packs 79 / 97; [1, 8192, 8192]: 73 / 104, 79 / 103).
-  if (D > kStridedTeamMinD && p.fast && ov.G == 0 && ov.V == 0 && ov.bpc == 0) {
-    const int vmax = strided_team_max_v(backward);
-    const int64_t wgs = num_cus * kTeamPerCu < kTeamMaxWorkgroups ? num_cus * kTeamPerCu : kTeamMaxWorkgroups;
-    // A team is an eighth of the machine at most.  Workgroups start in order, so a launch that shares
-    // the machine with others holds whole teams as soon as it holds that much of it, and those
-    // finish and make room: calls on several streams cannot keep one another's teams apart until
-    // the waits end.  (Larger teams gain nothing either, their exchange takes longer: bf16 [1, 8192,
-    // 136] forward on 64 workgroups 11.8 us, on 256 27.9; fp32 [8, 8192, 16] 64 at most.)
-    const int64_t most_wgs = wgs / kTeamMinTeams > 0 ? wgs / kTeamMinTeams : 1;
-    for (int wide = 0; wide < 2; ++wide) {
-      const int most_tx = wide ? kStridedTeamWideTx : kStridedTeamTx;
-      const int tx = px < most_tx ? px : most_tx;
-      const int64_t ty = kTeamBlock / tx;
-      const int64_t need = (D + ty * vmax - 1) / (ty * vmax);
-      const int64_t strips = outer * ((packs + tx - 1) / tx);
-      // (byte offsets of a lane inside a workgroup's rows are 32 bits wide)
-      if (need > most_wgs || ty * vmax * inner * 4 >= (int64_t(1) << 31)) break;
-      int64_t teams = wgs / need < strips ? wgs / need : strips;
-      const int64_t rounds = (strips + teams - 1) / teams;
-      teams = (strips + rounds - 1) / rounds;
-      const int64_t most = (D + ty - 1) / ty;
-      int64_t team = wgs / teams < most ? wgs / teams : most;
-      if (team > most_wgs) team = most_wgs;
-      int64_t v = (D + ty * team - 1) / (ty * team);
-      for (int c : kStridedTeamV[backward ? 1 : 0])
-        if (c >= v) {
-          v = c;
-          break;
-        }
-      team = (D + ty * v - 1) / (ty * v);
-      p.team = (int)team;
-      p.team_v = (int)v;
-      p.team_tx_log2 = log2_of_pow2(tx);
-      p.team_grid = teams * team;
-      if (rounds == 1 || D > kStridedTeamWideMaxD || px <= kStridedTeamTx) break;
+  // Strips held by teams of workgroups, where D is beyond the one-workgroup tile or teams are faster
+  // than that.
+  if (p.fast && ov.G == 0 && ov.V == 0 && ov.bpc == 0) {
+    const StridedTeam t = strided_team(backward, outer, D, packs, esize, num_cus);
+    if (t.team > 0 && (stream || strided_team_beats_tile(backward, outer, D, packs, esize, TX, t))) {
+      p.team = t.team;
+      p.team_v = t.v;
+      p.team_tx_log2 = log2_of_pow2(t.tx);
+      p.team_grid = t.grid;
     }
   }
   p.resident = !stream;

@@ -1,8 +1,10 @@
-// softmax / log_softmax over a dimension that is not innermost, D beyond the one-workgroup tile of
-// softmax_strided_kernels.hpp: every element crosses the memory interface once.
+// softmax / log_softmax over a dimension that is not innermost, where D is beyond the one-workgroup
+// tile of softmax_strided_kernels.hpp or teams are faster than that (strided_team_beats_tile()): every
+// element crosses the memory interface once.
 //
-// The tensor is [outer, D, inner]; a strip is TX consecutive 16-byte packs of `inner` (256 or 512
-// bytes) and all D rows under them.  A team of `team` workgroups of 512 threads holds a strip in
+// The tensor is [outer, D, inner], inner a whole number of 16-byte packs (any alignment); a strip is
+// TX consecutive packs of `inner` (up to 32: 512 bytes) and all D rows under them.  A team of `team`
+// workgroups of 512 threads holds a strip in
 // registers: workgroup c the rows [c * TY * V, (c + 1) * TY * V), thread (ty, tx) the V packs
 // of rows ty, ty + TY, ... of pack column tx.  A workgroup reduces its rows per column (each
 // lane over its packs, a wavefront by shuffles, the eight wavefronts through LDS), publishes the
@@ -13,12 +15,12 @@
 // What bounds it.  The split over launches that served these shapes reads the inputs twice and
 // pays three launches; the multi-pass kernel reads them three times.  Here it is HBM plus what
 // does not run under it: the forward's two exponentials an element (31 us of vector ALU time a
-// [8192, 8192] call) and the exchange, about 5 us a round, since a tensor twice the size of what
-// 512 workgroups hold makes two (forward) or four rounds in step (without the exchange the same
-// kernel takes 63 / 92 us there).  bf16 forward / backward us, before -> with teams:
-// [8192, 8192] over dim 0 78.5 / 114 -> 72 / 104; [4000, 16384] 76.7 / 113 -> 63 / 82;
-// [8192, 64] 18.1 / 13.3 -> 10.9 / 8.1; [8, 1000, 1024] 23.4 / 18.5 -> 12.4 / 13.1;
-// [35, 1000, 1904] 151 / 176 -> 79 / 97; [100, 2000, 128] 39.0 / 46.4 -> 24.7 / 33.8.
+// [8192, 8192] call) and the exchange, 4 us a round in the forward and 3 in the backward, since a
+// tensor twice the size of what 512 workgroups hold makes two (forward) or four rounds in step
+// (without the exchange the same kernel takes 63 / 92 us there).  bf16 forward / backward us,
+// without -> with teams: [8192, 8192] over dim 0 78.3 / 115 -> 71.0 / 103; [4000, 16384] 75.9 / 112
+// -> 64.6 / 83.6; [8192, 64] 17.6 / 12.1 -> 9.8 / 7.5; [8, 1000, 1024] 22.8 / 17.9 -> 12.0 / 12.3;
+// [35, 1000, 1904] 150 / 176 -> 76.6 / 95.7; [100, 2000, 128] 38.6 / 45.6 -> 22.8 / 32.0.
 // Requesting the next strip ahead of the exchange (half the packs a lane, twice the rounds)
 // measured slower (84-90 us on [8192, 8192]), as did rows dealt out in bands over the team.
 //
@@ -44,7 +46,8 @@ struct StridedTeamShape {
 };
 
 // A thread's place in a strip: pack column tx, rows ty, ty + TY, ...; the element of `inner` its
-// packs start at (0 where the strip is wider than what is left of `inner`: loaded, never stored).
+// packs start at (where the strip is wider than what is left of `inner`, the row's last pack, which
+// a neighbouring lane reads as well: loaded, never stored).
 template <int E>
 struct StridedTeamPlace {
   int tx, ty, TY, e0;
@@ -55,7 +58,7 @@ struct StridedTeamPlace {
     TY = kTeamBlock >> s.tx_log2;
     const int64_t e = (((strip % s.xtiles) << s.tx_log2) + tx) * E;
     in = e < s.inner;
-    e0 = in ? (int)e : 0;
+    e0 = in ? (int)e : s.inner - E;
   }
 };
 
