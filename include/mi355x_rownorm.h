@@ -340,7 +340,9 @@ int mi355x_softmax_strided_bwd(const void* grad, const void* y, void* gi, int64_
                                int64_t dim_size, int64_t inner, rownorm_dtype grad_dtype,
                                rownorm_dtype gi_dtype, int mode, void* stream);
 
-/* Launch layout of a strided softmax call (no launch).  In the result,
+/* Launch layout of a strided softmax call that shares nothing between workgroups running
+ * together (no launch): what runs where mi355x_softmax_strided_team_plan reports no team, and in
+ * place of teams of more than one workgroup wherever those are not possible (see there).  In the result,
  * lanes_per_row is the number of lanes along `inner` (one 16-byte pack each),
  * rows_per_block the number of threads along dim_size that share one such
  * lane position, packs_per_lane the dim_size rows each of those holds;
@@ -350,10 +352,25 @@ int mi355x_softmax_strided_bwd(const void* grad, const void* y, void* gi, int64_
 int mi355x_softmax_strided_plan(int backward, int64_t outer, int64_t dim_size, int64_t inner,
                                 rownorm_dtype dtype, rownorm_plan* out);
 
+/* The layout of such a call by teams of workgroups, which holds a strip of columns (lanes_per_row
+ * 16-byte packs of `inner`, all dim_size rows) in the registers of `reserved` workgroups of
+ * block_threads threads, packs_per_lane rows on each of the rows_per_block threads along
+ * dim_size; grid_blocks / reserved teams walk the strips.  `reserved` == 0: no teams, the rest is what
+ * mi355x_softmax_strided_plan reports.  Teams serve inner sizes of whole packs, any alignment, where
+ * they measured faster.  Teams of more than one workgroup pass the columns' partial results through
+ * the stream's bookkeeping slot, under the rules of mi355x_rownorm_set_team_wait_us (eight streams
+ * can hold a slot of this kind): a workgroup may wait for the others of its team for up to
+ * that bound, and reads the whole strip itself if it runs out.  They need an output that overlaps no
+ * input; such a call in place, on a stream under capture, or on a stream beyond the eight takes
+ * mi355x_softmax_strided_plan's layout.  A team of one waits for nobody and has none of these
+ * conditions. */
+int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_size, int64_t inner,
+                                     rownorm_dtype dtype, rownorm_plan* out);
+
 /* Reports the launch layout a call with these sizes would use on the current
  * device (no launch; needs no GPU when the device query fails: 256 compute
  * units are assumed).  x_dtype is the row dtype, w_dtype the weight dtype
- * (ignored by the softmax ops).  The strided softmax ops have their own query above.
+ * (ignored by the softmax ops).  The strided softmax ops have their own queries above.
  * The norm forwards and the softmax ops also look at their pointers: this reports the layout for
  * tensors that start on a 128-byte line; rows of at most 64 packs in tensors
  * that do not take one pack a lane (lanes_per_row = packs rounded up to a
@@ -398,16 +415,17 @@ int mi355x_rownorm_set_override(rownorm_op op, int lanes_per_row, int packs_per_
  * RMSNorm forward rows beyond 131072 16-bit or 65536 float32 elements, whole
  * 16-byte packs, no residual add, no cast, y not overlapping x; GroupNorm forward
  * slabs of that size; softmax / log_softmax forward and backward of few, very long
- * rows; LayerNorm / RMSNorm backward rows beyond one workgroup's registers in calls of
- * many rows; GroupNorm backward slabs of long whole-pack channels): how long a workgroup waits for the others of its team before it sums the
- * whole row itself (a second pass over the inputs, the same result to rounding), in
- * microseconds; 0xffffffff
+ * rows, and over a dimension that is not innermost (mi355x_softmax_strided_team_plan);
+ * LayerNorm / RMSNorm backward rows beyond one workgroup's registers in calls of
+ * many rows; GroupNorm backward slabs of long whole-pack channels): how long a workgroup
+ * waits for the others of its team before it sums the whole row (strip) itself (a second
+ * pass over the inputs, the same result to rounding), in microseconds; 0xffffffff
  * restores the default, one second.  0 makes every wait give up at once, which is
  * how the tests exercise that path without making any kernel hang.  Process-global.
  * Such calls draw an id from a process-wide counter and use the bookkeeping slot of their
  * stream, in library-owned device memory (48 MiB a GPU); results do not depend on the slot.
  * A stream takes a slot with its first such call and keeps it; streams beyond the 64 slots
- * take the multi-launch kernels, which exchange nothing, and so do these rows on a stream
+ * (8 of the strided softmax) take the multi-launch kernels, which exchange nothing, and so do these rows on a stream
  * under capture. */
 int mi355x_rownorm_set_team_wait_us(unsigned int microseconds);
 

@@ -438,6 +438,34 @@ def test_strided_softmax_validation_and_plans(cabi):
     cabi.clear_overrides()
 
 
+def test_strided_softmax_team_plans(cabi):
+    """The team query reports what a plain call runs: every row held by 512-thread workgroups, or no team
+    and the other query's layout."""
+    seen = set()
+    for dt, E in ((cabi.F32, 4), (cabi.BF16, 8)):
+        for outer, D, inner in ((1, 8192, 8192), (64, 300, 800), (600, 300, 64), (1, 30000, 64), (8, 257, 64),
+                                (4, 256, 4096), (2, 2500, 37), (35, 1000, 1904), (0, 8, 8)):
+            for bwd in (0, 1):
+                t, p = cabi.strided_team_plan(bwd, outer, D, inner, dt), cabi.strided_plan(bwd, outer, D, inner, dt)
+                if t["team"] == 0:
+                    assert {k: t[k] for k in p if k != "dim_chunks"} == {k: p[k] for k in p if k != "dim_chunks"}
+                    seen.add("none")
+                    continue
+                seen.add("one" if t["team"] == 1 else "several")
+                assert inner % E == 0 and t["resident"] == 1 and t["block_threads"] == 512
+                assert t["lanes_per_row"] * t["rows_per_block"] == 512
+                assert t["team"] * t["rows_per_block"] * t["packs_per_lane"] >= D
+                assert t["grid_blocks"] % t["team"] == 0 and t["grid_blocks"] <= 512
+    assert seen == {"none", "one", "several"}
+    for op in (cabi.OP_SOFTMAX_STRIDED_FWD, cabi.OP_SOFTMAX_STRIDED_BWD):
+        cabi.set_override(op, 0, 0, 0, 4)  # (forced layouts keep the kernels they name)
+    assert cabi.strided_team_plan(0, 1, 8192, 8192, cabi.BF16)["team"] == 0
+    cabi.clear_overrides()
+    p = cabi.Plan()
+    assert cabi.lib().mi355x_softmax_strided_team_plan(0, 1, -1, 8, cabi.F32, p) == -2
+    assert cabi.lib().mi355x_softmax_strided_team_plan(0, 1, 8, 8, 7, p) < 0
+
+
 def test_group_norm_validation_and_plans(cabi):
     L = cabi.lib()
     one, null = ctypes.c_void_p(256), None

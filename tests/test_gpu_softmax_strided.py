@@ -183,7 +183,9 @@ def test_many_rows_few_columns_are_split_over_workgroups(cabi, oracle, gpu, dtyp
             xg, gg = offset_view(x.to(gpu), 1), offset_view(grad.to(gpu), 3)
             for chunks in (0, 1, 2, 5):
                 for op in ops:
-                    cabi.set_override(op, -1 if chunks else 0, chunks)
+                    # (0: the planner's own split; a grid bound that binds nothing keeps teams out)
+                    cabi.set_override(op, -1 if chunks else 0, chunks, 0, 0 if chunks else 0xffff)
+                    assert cabi.strided_team_plan(op == ops[1], outer, D, inner, dt)["team"] == 0
                 p = cabi.strided_plan(False, outer, D, inner, dt)
                 assert p["resident"] == 0
                 if chunks:
@@ -236,6 +238,8 @@ def test_dim0_of_a_square_matrix_against_the_last_dim_kernels(cabi, gpu):
     g = gen(67)
     x = (2.0 * torch.randn(H, W, generator=g)).bfloat16().to(gpu)
     grad = torch.randn(H, W, generator=g).bfloat16().to(gpu)
+    for bwd in (False, True):  # held by teams; cut into chunks where teams are not possible
+        assert cabi.strided_team_plan(bwd, 1, H, W, cabi.BF16)["team"] > 1
     p = cabi.strided_plan(False, 1, H, W, cabi.BF16)
     assert p["resident"] == 0 and p["dim_chunks"] > 1, p
     y = cabi.softmax_strided_fwd(x, 0)

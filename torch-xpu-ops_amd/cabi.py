@@ -26,7 +26,7 @@ EXPORTED_SYMBOLS = (
     "mi355x_add_rms_norm_bwd", "mi355x_softmax_fwd",
     "mi355x_softmax_bwd", "mi355x_safe_softmax_fwd", "mi355x_masked_softmax_fwd",
     "mi355x_masked_softmax_bwd", "mi355x_softmax_strided_fwd", "mi355x_softmax_strided_bwd",
-    "mi355x_softmax_strided_plan", "mi355x_group_norm_fwd",
+    "mi355x_softmax_strided_plan", "mi355x_softmax_strided_team_plan", "mi355x_group_norm_fwd",
     "mi355x_group_norm_bwd_workspace_bytes", "mi355x_group_norm_bwd", "mi355x_group_norm_plan",
     "mi355x_rownorm_plan", "mi355x_rownorm_plan_at", "mi355x_rownorm_set_override",
     "mi355x_rownorm_stream_probe", "mi355x_rownorm_set_team_wait_us",
@@ -92,6 +92,9 @@ def lib():
                                                  _vp]
         L.mi355x_softmax_strided_plan.argtypes = [_int, _i64, _i64, _i64, _int,
                                                   ctypes.POINTER(Plan)]
+        L.mi355x_softmax_strided_team_plan.argtypes = [_int, _i64, _i64, _i64, _int,
+                                                       ctypes.POINTER(Plan)]
+        L.mi355x_softmax_strided_team_plan.restype = _int
         L.mi355x_group_norm_fwd.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _f,
                                             _int, _int, _vp]
         L.mi355x_group_norm_bwd_workspace_bytes.restype = ctypes.c_size_t
@@ -164,6 +167,16 @@ def strided_plan(backward, outer, dim_size, inner, dtype=F32):
                                              ctypes.byref(p)), "strided_plan")
     d = p.as_dict()
     d["dim_chunks"] = p.reserved  # workgroups the dim_size rows of a tile are split over (0: not split)
+    return d
+
+
+def strided_team_plan(backward, outer, dim_size, inner, dtype=F32):
+    """The layout by teams of workgroups; "team" 0: no teams, the rest is strided_plan()'s."""
+    p = Plan()
+    _check(lib().mi355x_softmax_strided_team_plan(int(backward), outer, dim_size, inner, dtype,
+                                                  ctypes.byref(p)), "strided_team_plan")
+    d = p.as_dict()
+    d["team"] = p.reserved
     return d
 
 

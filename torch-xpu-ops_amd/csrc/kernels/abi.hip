@@ -952,6 +952,25 @@ int mi355x_softmax_strided_plan(int backward, int64_t outer, int64_t dim_size, i
   return 0;
 }
 
+int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_size, int64_t inner,
+                                     rownorm_dtype dtype, rownorm_plan* out) {
+  if (int e = mi355x_softmax_strided_plan(backward, outer, dim_size, inner, dtype, out)) return e;
+  StridedPlan plan;
+  const int op = backward ? ROWNORM_OP_SOFTMAX_STRIDED_BWD : ROWNORM_OP_SOFTMAX_STRIDED_FWD;
+  if (int e = make_strided_plan(backward != 0, outer, dim_size, inner, esize_of((int)dtype),
+                                current_num_cus(), g_override[op], &plan))
+    return e;
+  out->reserved = plan.team;
+  if (plan.team == 0) return 0;
+  out->resident = 1;
+  out->lanes_per_row = 1 << plan.team_tx_log2;
+  out->packs_per_lane = plan.team_v;
+  out->block_threads = kTeamBlock;
+  out->rows_per_block = kTeamBlock >> plan.team_tx_log2;
+  out->grid_blocks = plan.team_grid;
+  return 0;
+}
+
 int mi355x_rownorm_plan_at(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_dtype,
                            rownorm_dtype w_dtype, int off_line, rownorm_plan* out) {
   if ((int)op < 0 || (int)op > ROWNORM_OP_SOFTMAX_BWD) return ROWNORM_ERR_SHAPE;
