@@ -76,3 +76,24 @@ def test_rows_shorter_than_a_pack_on_a_forced_layout(cabi, oracle, gpu, N, dtype
         _check(cabi, oracle, gpu, 300, N, dtype, (1, 3))
     finally:
         cabi.clear_overrides()
+
+
+@pytest.mark.parametrize("M,N,dtype", [(40, 8193, torch.float16), (40, 16383, torch.bfloat16),
+                                       (40, 5001, torch.float32), (8150, 6145, torch.float32)], ids=str)
+def test_the_residual_gradient_on_either_way_of_reading(cabi, gpu, M, N, dtype):
+    """The fused backward, dx + dh rounded once, on the same two ways: against the plain backward of the
+    same rows in float64 on the GPU."""
+    print("case ragged norm backward with the residual gradient", dtype, (M, N), flush=True)
+    g = torch.Generator(device=gpu).manual_seed(2560 + N)
+    h, dy, dh = (torch.empty(M, N, device=gpu).normal_(generator=g).to(dtype) for _ in range(3))
+    gamma = (1 + 0.1 * torch.empty(N, device=gpu).normal_(generator=g)).to(dtype)
+    _, mean, rstd = cabi.layer_norm_fwd(h, gamma, None, 1e-5)
+    dx, dg, db = cabi.add_layer_norm_bwd(dy, dh, h, mean, rstd, gamma)[:3]
+    xhat = (h.double() - mean.double().view(M, 1)) * rstd.double().view(M, 1)
+    gy = dy.double() * gamma.double()
+    want = (gy - gy.mean(1, keepdim=True) - xhat * (gy * xhat).mean(1, keepdim=True)) * rstd.double().view(M, 1) + dh.double()
+    assert_close(dx, to_np32(want.float()), dtype, "dx [%d, %d]" % (M, N))
+    # float32 sums over the rows: a few ulps of the magnitudes' sum
+    for got, terms, what in ((dg, dy.double() * xhat, "dgamma"), (db, dy.double(), "dbeta")):
+        assert_close(got, to_np32(terms.sum(0).float()), dtype, "%s [%d, %d]" % (what, M, N),
+                     slack=(terms.abs().sum(0) * 2.0 ** -21).float().cpu())

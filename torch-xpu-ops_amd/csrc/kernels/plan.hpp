@@ -106,7 +106,7 @@ constexpr int kTeamBwdPerCu = 1;
 // norm_fwd_rows_team_kernel: packs of a row a lane, and the rounds from which it is taken
 constexpr int kTeamFwdLongPacks = 10;
 constexpr int kTeamFwdMinRounds = 16;
-// One call's bookkeeping memory (see the kernel).
+// One stream's exchange memory (device/team.hpp, team_slots.hpp).
 struct TeamEntry {
   // the two-number exchange: (call id << 32) | (round + 1) once s1, s2 are in place, 0 while
   // they change; a workgroup's partial sums (float64 bit patterns)
@@ -124,7 +124,7 @@ struct TeamSlot {
   unsigned int pad[3];
 };
 
-// Columns (elements of `inner`) a strip of the strided team kernels has at most, and one call's
+// Columns (elements of `inner`) a strip of the strided team kernels has at most, and one stream's
 // exchange memory there: [round parity][workgroup][number][column] words (softmax_strided_team.hpp).
 constexpr int kTeamColumns = 256;
 struct TeamColumns {
