@@ -1329,16 +1329,17 @@ inline StridedTeam strided_team(bool backward, int64_t outer, int64_t D, int64_t
 // 26.3).  Beyond, the tile's segments are 64 bytes: teams where bandwidth counts, from about 7 MB
 // (bf16 forward / backward, tile -> teams: [4, 512, 8192] 28.6 / 38.1 -> 16.2 / 19.0 us, [64, 300,
 // 800] 23.5 / 29.9 -> 15.8 / 25.8; below, [8, 257, 512] 8.0 / 6.8 against 9.0 / 7.5); later for a
-// forward whose rows those segments divide (bf16 [200, 320, 64], 8.2 MB, 9.7 against 10.1) and for a
+// forward whose rows those segments divide (bf16 [200, 320, 64], 8.2 MB, 9.7 against 10.1; [40, 384,
+// 320], 9.8 MB, 11.3 against 10.4) and for a
 // float32 forward, whose arithmetic the tile hides better ([200, 257, 68], 14 MB, 16.5 against
 // 14.9); and a forward of such rows never where teams would leave half of their packs empty, a
 // quarter in float32, a little more where nothing is exchanged (bf16 [200, 257, 320] 24.4 against 26.6, [40, 257, 576] 11.6 against 12.4, but
 // [200, 257, 192], one workgroup a strip, 18.6 against 14.5; fp32 [40, 384, 288] 11.0 against 12.9,
-// [40, 384, 256] 13.9 against 11.5, [2000, 257, 32], one workgroup a strip, 37.8 against 34.9).  Smaller calls on more than eight packs go by the length of the
-// tile's serial part, if they are few tiles or their rows are not divided by the segments (bf16 [8,
-// 384, 136] 9.9 -> 8.4 forward, [1, 512, 512] 8.3 -> 6.6 backward, but [8, 512, 576] 9.4 against
-// 9.9; fp32 [1, 512, 132] 7.2 -> 6.5 backward, [8, 512, 256] 8.7 -> 7.8, [8, 512, 160] 6.8 against
-// 7.5).
+// [40, 384, 256] 13.9 against 11.5, [2000, 257, 32], one workgroup a strip, 37.8 against 34.9).
+// Smaller calls on more than eight packs go by the length of the tile's serial part, if they are few
+// tiles or their rows are not divided by the segments (bf16 [8, 384, 136] 9.9 -> 8.4 forward, [8, 384,
+// 64], eight packs, 8.5 -> 7.8, [1, 512, 512] 8.3 -> 6.6 backward, but [8, 512, 576] 9.4 against 9.9;
+// fp32 [1, 512, 132] 7.2 -> 6.5 backward, [8, 512, 256] 8.7 -> 7.8, [8, 512, 160] 6.8 against 7.5).
 inline bool strided_team_beats_tile(bool backward, int64_t outer, int64_t D, int64_t packs, int esize, int TX,
                                     const StridedTeam& t) {
   if (D <= kStridedTeamMinD || TX >= 8 || TX >= packs) return false;
@@ -1348,8 +1349,8 @@ inline bool strided_team_beats_tile(bool backward, int64_t outer, int64_t D, int
   const int64_t held = outer * D * packs * 64 / (t.rounds * t.v * kTeamMaxWorkgroups * kTeamBlock);
   if (!backward && divided && !few && held < (esize == 4 ? (t.team > 1 ? 48 : 40) : t.team > 1 ? 32 : 29))
     return false;
-  if (bytes >= (backward ? 7000000 : esize == 4 ? 13500000 : divided ? 10000000 : 7000000)) return true;
-  if (packs <= 8 || (esize == 4 && !backward)) return false;
+  if (bytes >= (backward ? 7000000 : esize == 4 ? 13500000 : divided ? 9000000 : 7000000)) return true;
+  if (packs < 8 || (packs == 8 && (backward || !few)) || (esize == 4 && !backward)) return false;
   const bool even = tiles <= 128 && packs % 16 == 0;
   if (backward) return divided ? D >= 448 && (even || (few && esize == 2)) : D >= (esize == 4 ? 448 : 320);
   return divided ? D >= 384 && few : D >= 320;
