@@ -1254,7 +1254,7 @@ inline StridedTeam strided_team_of(bool backward, int64_t outer, int64_t D, int6
   StridedTeam t;
   // (byte offsets of a lane inside a workgroup's rows are 32 bits wide; a float32 output of a 16-bit
   // tensor has twice the bytes)
-  if (need > most_wgs || ty * vmax * packs * 32 >= (int64_t(1) << 31)) return t;
+  if (need > most_wgs || ty * vmax * packs * (esize == 2 ? 32 : 16) >= (int64_t(1) << 31)) return t;
   int64_t teams = wgs / need < strips ? wgs / need : strips;
   t.rounds = (strips + teams - 1) / teams;
   teams = (strips + t.rounds - 1) / t.rounds;
@@ -1323,23 +1323,24 @@ inline StridedTeam strided_team(bool backward, int64_t outer, int64_t D, int64_t
   return (lines ? 8 * wc > 9 * nc : backward ? 3 * wc > 4 * nc : 3 * wc >= 4 * nc) ? n : w;
 }
 
-// Whether teams serve a shape that the one-workgroup tile (TX lanes along `inner`) holds.  D <= 256
-// is the tile's (at D = 200 [20, 200, 4096] 20.5 / 22.5 us, teams 23.2 / 25.5), and so is a tile
-// that spans the row or eight lanes of it: one pass, no exchange (bf16 [2000, 512, 16] 14.1 us, teams
-// 26.3).  Beyond, the tile's segments are 64 bytes: teams where bandwidth counts, from about 7 MB
-// (bf16 forward / backward, tile -> teams: [4, 512, 8192] 28.6 / 38.1 -> 16.2 / 19.0 us, [64, 300,
-// 800] 23.5 / 29.9 -> 15.8 / 25.8; below, [8, 257, 512] 8.0 / 6.8 against 9.0 / 7.5); later for a
-// forward whose rows those segments divide (bf16 [200, 320, 64], 8.2 MB, 9.7 against 10.1; [40, 384,
-// 320], 9.8 MB, 11.3 against 10.4) and for a
-// float32 forward, whose arithmetic the tile hides better ([200, 257, 68], 14 MB, 16.5 against
-// 14.9); and a forward of such rows never where teams would leave half of their packs empty, a
-// quarter in float32, a little more where nothing is exchanged (bf16 [200, 257, 320] 24.4 against 26.6, [40, 257, 576] 11.6 against 12.4, but
-// [200, 257, 192], one workgroup a strip, 18.6 against 14.5; fp32 [40, 384, 288] 11.0 against 12.9,
-// [40, 384, 256] 13.9 against 11.5, [2000, 257, 32], one workgroup a strip, 37.8 against 34.9).
-// Smaller calls on more than eight packs go by the length of the tile's serial part, if they are few
-// tiles or their rows are not divided by the segments (bf16 [8, 384, 136] 9.9 -> 8.4 forward, [8, 384,
-// 64], eight packs, 8.5 -> 7.8, [1, 512, 512] 8.3 -> 6.6 backward, but [8, 512, 576] 9.4 against 9.9;
-// fp32 [1, 512, 132] 7.2 -> 6.5 backward, [8, 512, 256] 8.7 -> 7.8, [8, 512, 160] 6.8 against 7.5).
+// Whether teams serve a shape that the one-workgroup tile (TX lanes along `inner`) holds.  D <=
+// 256 is the tile's (at D = 200 [20, 200, 4096] 20.5 / 22.5 us, teams 23.2 / 25.5), and so is a
+// tile that spans the row or eight lanes of it: one pass, no exchange (bf16 [2000, 512, 16] 14.1
+// us, teams 26.3).  Beyond, the tile's segments are 64 bytes: teams where bandwidth counts, from
+// about 7 MB (bf16 forward / backward, tile -> teams: [4, 512, 8192] 28.6 / 38.1 -> 16.2 / 19.0
+// us, [64, 300, 800] 23.5 / 29.9 -> 15.8 / 25.8; below, [8, 257, 512] 8.0 / 6.8 against 9.0 /
+// 7.5); later for a forward whose rows those segments divide (bf16 [200, 320, 64], 8.2 MB, 9.7
+// against 10.1; [40, 384, 320], 9.8 MB, 11.3 against 10.4) and for a float32 forward, whose
+// arithmetic the tile hides better ([200, 257, 68], 14 MB, 16.5 against 14.9); and a forward of
+// such rows never where teams would leave half of their packs empty, a quarter in float32, a
+// little more where nothing is exchanged (bf16 [200, 257, 320] 24.4 against 26.6, [40, 257, 576]
+// 11.6 against 12.4, but [200, 257, 192], one workgroup a strip, 18.6 against 14.5; fp32 [40,
+// 384, 288] 11.0 against 12.9, [40, 384, 256] 13.9 against 11.5, [2000, 257, 32], one workgroup
+// a strip, 37.8 against 34.9). Smaller calls on more than eight packs go by the length of the
+// tile's serial part, if they are few tiles or their rows are not divided by the segments (bf16
+// [8, 384, 136] 9.9 -> 8.4 forward, [8, 384, 64], eight packs, 8.5 -> 7.8, [1, 512, 512] 8.3 ->
+// 6.6 backward, but [8, 512, 576] 9.4 against 9.9; fp32 [1, 512, 132] 7.2 -> 6.5 backward, [8,
+// 512, 256] 8.7 -> 7.8, [8, 512, 160] 6.8 against 7.5).
 inline bool strided_team_beats_tile(bool backward, int64_t outer, int64_t D, int64_t packs, int esize, int TX,
                                     const StridedTeam& t) {
   if (D <= kStridedTeamMinD || TX >= 8 || TX >= packs) return false;
