@@ -1,0 +1,64 @@
+"""Strided softmax on workgroups that have a compute unit each: packs of a lane in registers and, beyond 48
+(backward 24 of each tensor), in LDS.  Every instance, full and with rows missing from the last workgroup,
+against the float64 oracle on some columns of every strip (float32 rtol = atol = 1e-5, 16-bit atol 1e-2, rtol
+1.6e-2), bit for bit from run to run, and against the path a workgroup takes when its wait gives up."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import assert_close, rowsum_slack, to_np32
+
+pytestmark = pytest.mark.gpu
+
+# (outer, D, packs of inner): packs a lane of the forward and the backward there (0: two workgroups a compute unit)
+SHAPES = {(1, 5000, 1024): (40, 20), (4, 4500, 230): (40, 0), (1, 12899, 484): (56, 28), (1, 8191, 1024): (64, 32),
+          (40, 4286, 28): (48, 24), (1, 8192, 1022): (64, 32), (6, 323, 1285): (0, 24)}
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("shape", list(SHAPES), ids=str)
+def test_large_teams_against_oracle_and_the_give_up_path(cabi, oracle, gpu, dtype, shape):
+    outer, D, packs = shape
+    E = 4 if dtype == torch.float32 else 8
+    inner = packs * E
+    print("case strided softmax, large teams", dtype, (outer, D, inner), flush=True)
+    plans = [cabi.strided_team_plan(b, outer, D, inner, cabi.dtype_code(dtype)) for b in (0, 1)]
+    for p, v, small in zip(plans, SHAPES[shape], (16, 8)):
+        assert p["packs_per_lane"] == v if v else p["packs_per_lane"] <= small, (plans, SHAPES[shape])
+    g = torch.Generator(device=gpu).manual_seed(D + packs)
+    x = torch.empty(outer, D, inner, device=gpu, dtype=dtype).normal_(0, 3.0, generator=g)
+    grad = torch.empty_like(x).normal_(0, 1.0, generator=g)
+    x[0, D // 3:, 0] = float("-inf")
+    x[0, :, 1] = float("-inf")
+    x[-1, D - 1, 2] = float("nan")
+    x[-1, :, 3] = torch.finfo(dtype).min
+    # two columns of every pack that begins or ends a 16-pack piece, and the last ones
+    cols = sorted({c for p in range(0, packs, 15) for c in (p * E, p * E + E - 1)} | {0, 1, 2, 3, inner - 1})[:97] + [inner - 1]
+    cols = sorted(set(cols))
+    pick = lambda t: t[:, :, cols].cpu()  # noqa: E731
+    last = lambda a: np.ascontiguousarray(np.moveaxis(to_np32(a), 1, -1))  # noqa: E731
+    back = lambda a: np.moveaxis(a, -1, 1)  # noqa: E731
+
+    def given_up(fn):
+        try:
+            cabi.set_team_wait_us(0)
+            return fn()
+        finally:
+            cabi.set_team_wait_us()
+
+    for mode, is_log in ((cabi.SOFTMAX, False), (cabi.LOG_SOFTMAX, True)):
+        what = "%s %s %s" % ("log_softmax" if is_log else "softmax", shape, dtype)
+        fwd = lambda: cabi.softmax_strided_fwd(x, 1, mode)  # noqa: E731
+        y = fwd()
+        oy = back(oracle.softmax_fwd(last(pick(x)), is_log))
+        assert_close(pick(y), oy, dtype, what)
+        assert torch.equal(y.view(torch.uint8), fwd().view(torch.uint8)), what + ": run to run"
+        assert_close(pick(given_up(fwd)), oy, dtype, what + ", every wait given up")
+        bwd = lambda: cabi.softmax_strided_bwd(grad, y, 1, mode)  # noqa: E731
+        gi = bwd()
+        ogi = back(oracle.softmax_bwd(last(pick(grad)), last(pick(y)), is_log))
+        yy, terms = pick(y).float().movedim(1, -1), pick(grad).float().movedim(1, -1)
+        sl = (rowsum_slack(terms, torch.exp(yy)) if is_log else rowsum_slack(yy * terms, yy)).movedim(-1, 1)
+        assert_close(pick(gi), ogi, dtype, what + " backward", slack=sl)
+        assert torch.equal(gi.view(torch.uint8), bwd().view(torch.uint8)), what + ": run to run"
+        assert_close(pick(given_up(bwd)), ogi, dtype, what + " backward, every wait given up", slack=sl)

@@ -1,0 +1,44 @@
+"""The rule that gives the strips of a strided softmax to workgroups with a compute unit each
+(strided_large_team() in plan.hpp), on the CPU."""
+import ctypes
+import random
+
+from test_plan_rules import _strided, rules  # noqa: F401
+
+i64 = ctypes.c_int64
+
+
+def _large(rules, backward, outer, D, inner, esize):  # noqa: F811
+    out = (i64 * 4)()
+    rules.rule_strided_large(backward, i64(outer), i64(D), i64(inner), esize, out)
+    return dict(zip(("team", "v", "tx", "grid"), list(out)))
+
+
+def test_large_teams(rules):  # noqa: F811
+    """Every row of a strip is held on instances that exist, on a grid that is resident at one workgroup a
+    compute unit, by teams of an eighth of the machine at most, in fewer rounds than two a compute unit."""
+    rng = random.Random(7)
+    built = {0: (40, 48, 56, 64), 1: (20, 24, 28, 32)}
+    shapes = [(1, 8192, 1024), (12, 9602, 25), (6, 323, 1285), (1, 65536, 16384), (92, 2206, 32)]
+    shapes += [(rng.randint(1, 300), int(2 ** rng.uniform(8, 17)), int(2 ** rng.uniform(1, 13))) for _ in range(4000)]
+    taken = 0
+    for outer, D, px in shapes:
+        for esize in (2, 4):
+            for backward in (0, 1):
+                a = (backward, outer, D, px * 16 // esize, esize)
+                p, l = _strided(rules, *a), _large(rules, *a)
+                if l["team"] == 0:
+                    continue
+                taken += 1
+                ty, strips = 512 // l["tx"], lambda t: outer * -(-px // t["tx"])
+                assert p["team"] > 0 and l["tx"] in (16, 32) and l["v"] in built[backward]
+                assert l["team"] * ty * l["v"] >= D > (l["team"] - 1) * ty * l["v"], "held, no workgroup without a row"
+                assert l["team"] <= 32 and l["grid"] % l["team"] == 0 and l["team"] <= l["grid"] <= 256
+                rounds = lambda t: -(-strips(t) // (t["grid"] // t["team"]))  # noqa: E731
+                assert rounds(l) < rounds(p) and ty * l["v"] * px * 16 * (2 if esize == 2 else 1) < 2 ** 31
+    assert taken > 300
+    assert _large(rules, 0, 1, 8192, 8192, 2) == dict(team=8, v=64, tx=32, grid=256)
+    assert _large(rules, 1, 1, 8192, 8192, 2) == dict(team=16, v=32, tx=32, grid=256)
+    # where two a compute unit measured faster
+    for a in ((0, 50, 954, 920, 2), (0, 6, 820, 10296, 2), (0, 4, 3419, 3912, 2), (1, 36, 2844, 384, 2), (0, 8, 2048, 2048, 2)):
+        assert _large(rules, *a)["team"] == 0, a

@@ -27,6 +27,15 @@ struct elems_per_pack {
   static constexpr int value = 16 / sizeof(T);
 };
 
+// f(integral_constant<int, I>) for I in [I0, I1): a loop whose index is a constant of the body.
+template <int I0, int I1, class F>
+__device__ __forceinline__ void static_for(F f) {
+  if constexpr (I0 < I1) {
+    f(std::integral_constant<int, I0>{});
+    static_for<I0 + 1, I1>(f);
+  }
+}
+
 // E consecutive elements of T held in registers in storage format.
 template <class T, int E>
 struct Pack {

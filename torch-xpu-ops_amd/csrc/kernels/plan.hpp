@@ -1202,17 +1202,31 @@ struct StridedPlan {
   // multi-pass kernels with too few tiles for the machine: the D rows are cut into
   // `chunks` chunks of `chunk_rows` rows, one workgroup each (0 or 1: not split)
   int chunks = 0, chunk_rows = 0;
-  // strips held by teams of workgroups (softmax_strided_team.hpp); team 0: not this call.
-  // team_grid = teams * team workgroups, team_tx_log2 = log2 of the packs a strip is wide,
-  // team_v = packs a lane
+  // strips held by teams of workgroups, two a compute unit (softmax_strided_team.hpp); team 0: not
+  // this call.  team_grid = teams * team workgroups, team_tx_log2 = log2 of the packs a strip is
+  // wide, team_v = packs a lane
   int team = 0, team_v = 0, team_tx_log2 = 0;
   int64_t team_grid = 0;
+  // the same strips by workgroups that have a compute unit to themselves (strided_large_team());
+  // large_team 0: two a compute unit
+  int large_team = 0, large_v = 0, large_tx_log2 = 0;
+  int64_t large_grid = 0;
 };
 
 // The packs a lane the strided team kernels are built for: the forward holds one tensor, the
 // backward two.
 constexpr int kStridedTeamV[2][10] = {{1, 2, 3, 4, 6, 8, 10, 12, 14, 16}, {1, 2, 3, 4, 5, 6, 7, 8}};
+constexpr int kStridedLargeV[2][4] = {{40, 48, 56, 64}, {20, 24, 28, 32}};
 constexpr int strided_team_max_v(bool backward) { return backward ? 8 : 16; }
+constexpr int strided_large_max_v(bool backward) { return backward ? 32 : 64; }
+// Workgroups of an instance a compute unit holds, and the packs a lane keeps in LDS: up to 48 packs
+// of a lane (the backward 24 of each tensor) fit 256 registers, the rest 16 bytes a thread each.
+constexpr int strided_team_per_cu(bool backward, int v) {
+  return v > strided_team_max_v(backward) ? 1 : kTeamPerCu;
+}
+constexpr int strided_team_parked(bool backward, int v) {
+  return v > (backward ? 24 : 48) ? v - (backward ? 24 : 48) : 0;
+}
 // Lanes along `inner` at most: 256-byte row segments, or 512-byte ones.
 constexpr int kStridedTeamTx = 16;
 constexpr int kStridedTeamWideTx = 32;
@@ -1230,7 +1244,7 @@ inline int log2_of_pow2(int v) {
   return l;
 }
 
-// Strips of tx packs held by teams: as few workgroups a strip as hold its D rows, as many teams as
+// Strips of tx packs held by teams (large: on workgroups that have a compute unit each): as few workgroups a strip as hold its D rows, as many teams as
 // strips and compute units allow, evened out over the rounds; then a strip is spread over the
 // workgroups its team can have.
 struct StridedTeam {
@@ -1239,16 +1253,16 @@ struct StridedTeam {
   int64_t rounds = 0, grid = 0;
 };
 inline StridedTeam strided_team_of(bool backward, int64_t outer, int64_t D, int64_t packs, int esize, int tx,
-                                   int num_cus) {
-  const int64_t wgs = (int64_t)num_cus * kTeamPerCu < kTeamMaxWorkgroups ? (int64_t)num_cus * kTeamPerCu
-                                                                        : (int64_t)kTeamMaxWorkgroups;
+                                   int num_cus, bool large = false) {
+  const int64_t per_cu = large ? 1 : kTeamPerCu, at_most = kTeamMaxWorkgroups / kTeamPerCu * per_cu;
+  const int64_t wgs = num_cus * per_cu < at_most ? num_cus * per_cu : at_most;
   // A team is an eighth of the machine at most.  Workgroups start in order, so a launch that shares
   // the machine with others holds whole teams as soon as it holds that much of it, and those
   // finish and make room: calls on several streams cannot keep one another's teams apart until
   // the waits end.  (Larger teams gain nothing either, their exchange takes longer: bf16 [1, 8192,
   // 136] forward on 64 workgroups 11.8 us, on 256 27.5.)
   const int64_t most_wgs = wgs / kTeamMinTeams > 0 ? wgs / kTeamMinTeams : 1;
-  const int64_t ty = kTeamBlock / tx, vmax = strided_team_max_v(backward);
+  const int64_t ty = kTeamBlock / tx, vmax = large ? strided_large_max_v(backward) : strided_team_max_v(backward);
   const int64_t need = (D + ty * vmax - 1) / (ty * vmax);
   const int64_t strips = outer * ((packs + tx - 1) / tx);
   StridedTeam t;
@@ -1270,11 +1284,12 @@ inline StridedTeam strided_team_of(bool backward, int64_t outer, int64_t D, int6
   // not where that makes it more than eight packs a lane: [1, 30000, 16] 14.2, on 16 19.2)
   if (!backward && esize == 4 && tx <= 4 && team > 16 && D <= ty * 16 * 8) team = 16;
   int64_t v = (D + ty * team - 1) / (ty * team);
-  for (int c : kStridedTeamV[backward ? 1 : 0])
-    if (c >= v) {
-      v = c;
-      break;
-    }
+  auto built = [&](const auto& list) {
+    for (int c : list)
+      if (c >= v) return c;
+    return 0;
+  };
+  v = large ? built(kStridedLargeV[backward ? 1 : 0]) : built(kStridedTeamV[backward ? 1 : 0]);
   team = (D + ty * v - 1) / (ty * v);
   t.team = (int)team;
   t.v = (int)v;
@@ -1321,6 +1336,28 @@ inline StridedTeam strided_team(bool backward, int64_t outer, int64_t D, int64_t
   const bool lines = packs % 8 == 0;
   if (n.team == 1 && wc >= nc && (lines || n.v <= 10)) return n;
   return (lines ? 8 * wc > 9 * nc : backward ? 3 * wc > 4 * nc : 3 * wc >= 4 * nc) ? n : w;
+}
+
+// The same strips held by workgroups that have a compute unit each: 48 packs a lane in registers and up
+// to 16 in LDS (the backward 24 and 8 of each tensor) hold twice what two workgroups hold in registers
+// alone, so there are half the rounds and a quarter of the members to a team.  Taken where that makes
+// fewer rounds of no more than a sixteenth more packs (a workgroup's packs come in coarser steps) and
+// the teams it replaces have twelve members or more; below, two workgroups a compute unit that run out
+// of step do as well as fewer rounds (us, two a compute unit / one: bf16 forward of [1, 8192, 8192]
+// 70.5 / 59.1, [1, 12899, 3872] 58.4 / 50.1, but [50, 954, 920], teams of 5, 50.5 / 59.4 and [6, 820,
+// 10296], of 4, 58.3 / 61.1; backward of [1, 8192, 8192] 103.7 / 82.9, [12, 9602, 200] 46.2 / 30.0,
+// [92, 2206, 256] 66.2 / 60.5, but [36, 2844, 384] with 4/3 of the packs 48.1 / 51.5).  Rows of an odd number of packs, whose 512-byte pieces start off 32 bytes, gain
+// from teams of 24 on (forward of [4, 3419, 3912], 16 members, 58.5 / 67.9, of [2, 13960, 1272], 44, 57.0
+// / 47.6).  A backward whose strips then need no exchange and make one round gains whatever the teams
+// were ([6, 323, 10280] 31.8 / 29.3, fp32 [4, 325, 7136] 24.7 / 18.4).
+inline StridedTeam strided_large_team(bool backward, int64_t outer, int64_t D, int64_t packs, int esize,
+                                      const StridedTeam& t, int num_cus) {
+  if (t.team == 0 || t.rounds < 2) return StridedTeam{};
+  const StridedTeam l = strided_team_of(backward, outer, D, packs, esize,
+                                        packs > kStridedTeamTx ? kStridedTeamWideTx : kStridedTeamTx, num_cus, true);
+  if (l.team == 0 || l.rounds >= t.rounds || 8 * l.rounds * l.v > 17 * t.rounds * t.v) return StridedTeam{};
+  if (l.team == 1) return backward && l.rounds == 1 ? l : StridedTeam{};
+  return t.team >= (packs % 2 == 0 ? 12 : 24) ? l : StridedTeam{};
 }
 
 // Whether teams serve a shape that the one-workgroup tile (TX lanes along `inner`) holds.  D <=
@@ -1452,6 +1489,11 @@ inline int make_strided_plan(bool backward, int64_t outer, int64_t D, int64_t in
       p.team_v = t.v;
       p.team_tx_log2 = log2_of_pow2(t.tx);
       p.team_grid = t.grid;
+      const StridedTeam l = strided_large_team(backward, outer, D, packs, esize, t, num_cus);
+      p.large_team = l.team;
+      p.large_v = l.v;
+      p.large_tx_log2 = log2_of_pow2(l.tx);
+      p.large_grid = l.grid;
     }
   }
   p.resident = !stream;

@@ -6,23 +6,32 @@
 
 namespace rownorm {
 
-template <int E>
-StridedTeamShape strided_team_shape(const StridedPlan& p, int64_t outer, int D, int inner) {
-  const int64_t packs = inner / E;
-  const int64_t xtiles = (packs + (1 << p.team_tx_log2) - 1) >> p.team_tx_log2;
-  return StridedTeamShape{outer * xtiles, xtiles, D, inner, p.team_tx_log2, p.team};
-}
-
-// Launches the instance whose packs a lane the plan names; false if there is none.
-template <bool BACKWARD, size_t I = 0, class Go>
-bool launch_strided_team(int v, Go go) {
-  constexpr int V = kStridedTeamV[BACKWARD ? 1 : 0][I];
-  if (v == V) {
-    go(std::integral_constant<int, V>{});
+// Launches the instance whose packs a lane the plan names: go(packs, shape, grid); false if there is
+// none.
+template <bool BACKWARD, bool LARGE, size_t I = 0, class Go>
+bool launch_strided_team_v(int v, Go go) {
+  constexpr auto& list = [] () -> auto& {
+    if constexpr (LARGE) return kStridedLargeV[BACKWARD ? 1 : 0];
+    else return kStridedTeamV[BACKWARD ? 1 : 0];
+  }();
+  if (v == list[I]) {
+    go(std::integral_constant<int, list[I]>{});
     return true;
   }
-  if constexpr (V < strided_team_max_v(BACKWARD)) return launch_strided_team<BACKWARD, I + 1>(v, go);
+  if constexpr (list[I] < (LARGE ? strided_large_max_v(BACKWARD) : strided_team_max_v(BACKWARD)))
+    return launch_strided_team_v<BACKWARD, LARGE, I + 1>(v, go);
   return false;
+}
+template <bool BACKWARD, int E, class Go>
+bool launch_strided_team(const StridedPlan& p, int64_t outer, int D, int inner, bool exchange, Go go) {
+  const bool large = p.large_team == 1 || (p.large_team > 1 && exchange);
+  const int tx_log2 = large ? p.large_tx_log2 : p.team_tx_log2;
+  const int64_t xtiles = (inner / E + (1 << tx_log2) - 1) >> tx_log2;
+  const StridedTeamShape sh{outer * xtiles, xtiles, D, inner, tx_log2, large ? p.large_team : p.team};
+  const dim3 grid((unsigned)(large ? p.large_grid : p.team_grid));
+  if (large)
+    return launch_strided_team_v<BACKWARD, true>(p.large_v, [&](auto v) { go(v, sh, grid); });
+  return launch_strided_team_v<BACKWARD, false>(p.team_v, [&](auto v) { go(v, sh, grid); });
 }
 
 template <class TI, class TO, int V, bool FAST>
@@ -51,14 +60,12 @@ template <class TI, class TO>
 int launch_softmax_strided_fwd(const StridedPlan& p, const SoftmaxStridedFwdArgs& a,
                                hipStream_t s) {
   if (p.team == 1 || (p.team > 1 && a.team_slot != nullptr)) {
-    const StridedTeamShape sh =
-        strided_team_shape<elems_per_pack<TI>::value>(p, a.outer, a.D, a.inner);
-    const bool ok = launch_strided_team<false>(p.team_v, [&](auto v) {
-      hipLaunchKernelGGL((softmax_strided_team_fwd_kernel<TI, TO, decltype(v)::value>),
-                         dim3((unsigned)p.team_grid), dim3(kTeamBlock), 0, s, (const TI*)a.x,
-                         (TO*)a.y, sh, a.flags, (TeamColumns*)a.team_slot, a.team_id,
-                         a.team_wait_ticks);
-    });
+    const bool ok = launch_strided_team<false, elems_per_pack<TI>::value>(
+        p, a.outer, a.D, a.inner, a.team_slot != nullptr, [&](auto v, const StridedTeamShape& sh, dim3 grid) {
+          hipLaunchKernelGGL((softmax_strided_team_fwd_kernel<TI, TO, decltype(v)::value>), grid,
+                             dim3(kTeamBlock), 0, s, (const TI*)a.x, (TO*)a.y, sh, a.flags,
+                             (TeamColumns*)a.team_slot, a.team_id, a.team_wait_ticks);
+        });
     if (!ok) return (int)hipErrorInvalidConfiguration;
   } else if (p.resident) {
     const bool ok = p.fast ? launch_strided_fwd_f<TI, TO, true>(p, a, s)
@@ -117,14 +124,12 @@ template <class TG, class TO>
 int launch_softmax_strided_bwd(const StridedPlan& p, const SoftmaxStridedBwdArgs& a,
                                hipStream_t s) {
   if (p.team == 1 || (p.team > 1 && a.team_slot != nullptr)) {
-    const StridedTeamShape sh =
-        strided_team_shape<elems_per_pack<TG>::value>(p, a.outer, a.D, a.inner);
-    const bool ok = launch_strided_team<true>(p.team_v, [&](auto v) {
-      hipLaunchKernelGGL((softmax_strided_team_bwd_kernel<TG, TO, decltype(v)::value>),
-                         dim3((unsigned)p.team_grid), dim3(kTeamBlock), 0, s, (const TG*)a.grad,
-                         (const TG*)a.y, (TO*)a.gi, sh, a.flags, (TeamColumns*)a.team_slot,
-                         a.team_id, a.team_wait_ticks);
-    });
+    const bool ok = launch_strided_team<true, elems_per_pack<TG>::value>(
+        p, a.outer, a.D, a.inner, a.team_slot != nullptr, [&](auto v, const StridedTeamShape& sh, dim3 grid) {
+          hipLaunchKernelGGL((softmax_strided_team_bwd_kernel<TG, TO, decltype(v)::value>), grid,
+                             dim3(kTeamBlock), 0, s, (const TG*)a.grad, (const TG*)a.y, (TO*)a.gi,
+                             sh, a.flags, (TeamColumns*)a.team_slot, a.team_id, a.team_wait_ticks);
+        });
     if (!ok) return (int)hipErrorInvalidConfiguration;
   } else if (p.resident) {
     const bool ok = p.fast ? launch_strided_bwd_f<TG, TO, true>(p, a, s)

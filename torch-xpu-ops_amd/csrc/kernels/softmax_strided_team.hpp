@@ -5,7 +5,7 @@
 // The tensor is [outer, D, inner], inner a whole number of 16-byte packs (any alignment); a strip is
 // TX consecutive packs of `inner` (up to 32: 512 bytes) and all D rows under them.  A team of `team`
 // workgroups of 512 threads holds a strip in
-// registers: workgroup c the rows [c * TY * V, (c + 1) * TY * V), thread (ty, tx) the V packs
+// registers (and, one workgroup a compute unit, in LDS: strided_large_team()): workgroup c the rows [c * TY * V, (c + 1) * TY * V), thread (ty, tx) the V packs
 // of rows ty, ty + TY, ... of pack column tx.  A workgroup reduces its rows per column (each
 // lane over its packs, a wavefront by shuffles, the eight wavefronts through LDS), publishes the
 // C = TX * E columns' numbers -- running maximum and sum of exp(x - maximum), or the sum the
@@ -15,11 +15,14 @@
 // What bounds it.  The split over launches that served these shapes reads the inputs twice and
 // pays three launches; the multi-pass kernel reads them three times.  Here it is HBM plus what
 // does not run under it: the forward's two exponentials an element (31 us of vector ALU time a
-// [8192, 8192] call) and the exchange, 4 us a round in the forward and 3 in the backward, since a
-// tensor twice the size of what 512 workgroups hold makes two (forward) or four rounds in step
-// (without the exchange the same kernel takes 63 / 92 us there).  bf16 forward / backward us,
-// without -> with teams: [8192, 8192] over dim 0 78.3 / 115 -> 71.0 / 103; [4000, 16384] 75.9 / 112
-// -> 64.6 / 83.6; [8192, 64] 17.6 / 12.1 -> 9.8 / 7.5; [8, 1000, 1024] 22.8 / 17.9 -> 12.0 / 12.3;
+// [8192, 8192] call) and the exchange, whose rounds run in step.  Two workgroups a compute unit hold
+// 64 MB in registers, so that call made two (forward) or four rounds; one workgroup of 256 registers a
+// lane with 16 packs a lane more in LDS holds 128 MB: one or two rounds of teams a quarter as large,
+// 70.5 / 103.7 -> 59.1 / 82.9 us (of the 59, reads 24, the exponentials 4 + 4 beside reads and writes,
+// the exchange 6).  The exponentials of a group of packs are formed while the next groups are on their
+// way: the rows past D are replaced group by group, not all at once, which waited for every load (71 ->
+// 68 us).  bf16 forward / backward us, without -> with teams of two workgroups a compute unit: [8192,
+// 8192] over dim 0 78.3 / 115 -> 67.8 / 102; [4000, 16384] 75.9 / 112 -> 64.6 / 83.6; [8192, 64] 17.6 / 12.1 -> 9.8 / 7.5; [8, 1000, 1024] 22.8 / 17.9 -> 12.0 / 12.3;
 // [35, 1000, 1904] 150 / 176 -> 76.6 / 95.7; [100, 2000, 128] 38.6 / 45.6 -> 22.8 / 32.0.
 // Requesting the next strip ahead of the exchange (half the packs a lane, twice the rounds)
 // measured slower (84-90 us on [8192, 8192]), as did rows dealt out in bands over the team.
@@ -78,27 +81,31 @@ __device__ __forceinline__ P* scalar_again(P* p) {
   return p;
 }
 
-// The V packs of this thread: rows r0 + ty + k * TY, pack column e0 (an element index inside the
-// row).  One straight line for every workgroup (two versions of it would each want the packs in
-// registers of their own): rows past D - 1 read row D - 1 and are replaced by `fill`.
-template <class T, int E, int V>
-__device__ __forceinline__ void strided_team_load(Pack<T, E> (&p)[V], const T* strip, int r0,
-                                                  int ty, int TY, int e0, int D, int inner,
-                                                  float fill) {
+// Packs [K0, K1) of this thread's V: rows r0 + ty + k * TY, pack column e0 (an element index inside
+// the row), into p[0 .. K1 - K0).  One straight line for every workgroup (two versions of it would
+// each want the packs in registers of their own): rows past D - 1 read row D - 1;
+// strided_team_fill replaces them by `fill`.
+template <class T, int E, int K0, int K1>
+__device__ __forceinline__ void strided_team_load(Pack<T, E>* p, const T* strip, int r0, int ty,
+                                                  int TY, int e0, int D, int inner) {
   const T* base = strip + (int64_t)r0 * inner;
   const int last = D - 1 - r0;
-  ty = lane_again(ty);  // (offsets and bounds of the packs are formed here, not ahead of the strips)
+  // (offsets and bounds of the packs are formed here, not ahead of the strips, and one after the other)
+  int row = lane_again(ty) + K0 * TY;
 #pragma unroll
-  for (int k = 0; k < V; ++k) {
-    const int row = ty + k * TY;
+  for (int k = K0; k < K1; ++k, row += TY) {
     const int rc = row < last ? row : last;
-    p[k] = Pack<T, E>::load_stream(
+    p[k - K0] = Pack<T, E>::load_stream(
         global_at(base, ((uint32_t)rc * (uint32_t)inner + (uint32_t)e0) * (uint32_t)sizeof(T)));
   }
+}
+template <class T, int E, int K0, int K1>
+__device__ __forceinline__ void strided_team_fill(Pack<T, E>* p, int last, int ty, int TY, float fill) {
   const Pack<T, E> f = Pack<T, E>::splat(fill);
+  int row = lane_again(ty) + K0 * TY;
 #pragma unroll
-  for (int k = 0; k < V; ++k)
-    if (ty + k * TY > last) p[k] = f;
+  for (int k = K0; k < K1; ++k, row += TY)
+    if (row > last) p[k - K0] = f;
 }
 
 // NF words a column: publishes v[0..NF) of the C columns (threads below C hold them).
@@ -241,18 +248,34 @@ __device__ __forceinline__ void wave_columns_merge(float (&m)[E], float (&s)[E],
 
 constexpr int kStridedTeamGroup = 4;
 
+// A lane's packs in LDS: a slot of 16 bytes a thread and pack, which only that thread uses.
+template <class T, int E, int L>
+struct StridedTeamPark {
+  typename Pack<T, E>::vec_t v[L > 0 ? L : 1][L > 0 ? kTeamBlock : 1];
+  __device__ __forceinline__ void put(int k, const Pack<T, E>& p) { v[k][threadIdx.x] = p.v; }
+  __device__ __forceinline__ Pack<T, E> get(int k) const {
+    Pack<T, E> p;
+    p.v = v[k][threadIdx.x];
+    return p;
+  }
+};
+
 template <class TI, class TO, int V>
-__global__ void __launch_bounds__(kTeamBlock, kTeamPerCu * kTeamBlock / 256)
+__global__ void __launch_bounds__(kTeamBlock, strided_team_per_cu(false, V) * kTeamBlock / 256)
 softmax_strided_team_fwd_kernel(const TI* __restrict__ x, TO* __restrict__ y, StridedTeamShape sh,
                                 int flags, TeamColumns* slot, unsigned int call_id,
                                 unsigned long long wait_ticks) {
   constexpr int E = elems_per_pack<TI>::value;
   constexpr bool PRECISE = sizeof(TO) == 4;
   constexpr int NW = kTeamBlock / 64;
+  constexpr int L = strided_team_parked(false, V), R = V - L;  // packs of a lane in LDS, in registers
+  constexpr int GR = kStridedTeamGroup;
+  static_assert(L % GR == 0 && L <= R, "parked packs pass through registers group by group");
   __shared__ float wm[NW * kTeamColumns], ws[NW * kTeamColumns];  // the wavefronts' pairs
   __shared__ int votes[2][kTeamBlock / 64 + 1];
   __shared__ float gm[kTeamBlock], gs[kTeamBlock];                // the gathering threads' pairs
   __shared__ __align__(16) float fm[kTeamColumns], fk[kTeamColumns];  // maximum, 1/sum or log(sum)
+  __shared__ StridedTeamPark<TI, E, L> park;
   const bool is_log = (flags & kSoftmaxLog) != 0;
   const bool is_safe = (flags & kSoftmaxSafe) != 0;
   const int D = sh.D, inner = sh.inner, team = sh.team;
@@ -264,12 +287,8 @@ softmax_strided_team_fwd_kernel(const TI* __restrict__ x, TO* __restrict__ y, St
   bool lost = false;
   unsigned int round = 0;
   for (int64_t strip = tm; strip < sh.strips; strip += teams, ++round) {
-    Pack<TI, E> xp[V];
-    {
-      const StridedTeamPlace<E> t(sh, lane_again((int)threadIdx.x), strip);
-      strided_team_load<TI, E, V>(xp, x + (strip / sh.xtiles) * (int64_t)D * inner, r0, t.ty, t.TY,
-                                  t.e0, D, inner, -INFINITY);
-    }
+    // packs 0 .. L - 1 go to LDS, packs L .. V - 1 to xp[0 .. R - 1]
+    Pack<TI, E> xp[R];
     // The lane's running maxima and sums, kGroup packs at a time: the exponentials of one group are
     // formed while the next ones are still on their way.
     float m[E], s[E];
@@ -278,17 +297,16 @@ softmax_strided_team_fwd_kernel(const TI* __restrict__ x, TO* __restrict__ y, St
       m[i] = -INFINITY;
       s[i] = 0.0f;
     }
-#pragma unroll
-    for (int k0 = 0; k0 < V; k0 += kStridedTeamGroup) {
-      const int kn = k0 + kStridedTeamGroup < V ? k0 + kStridedTeamGroup : V;
+    auto absorb = [&](Pack<TI, E>* p, auto k_first, auto n) {
+      constexpr int KN = decltype(n)::value;
       float ref[E];
 #pragma unroll
       for (int i = 0; i < E; ++i) ref[i] = m[i];
 #pragma unroll
-      for (int k = k0; k < kn; ++k) {
+      for (int k = 0; k < KN; ++k) {
 #pragma unroll
-        for (int i = 0; i < E; ++i) ref[i] = fmaxf(ref[i], xp[k].get(i));
-        keep_packed(xp[k]);
+        for (int i = 0; i < E; ++i) ref[i] = fmaxf(ref[i], p[k].get(i));
+        keep_packed(p[k]);
       }
       // (nothing finite so far: against 0, -inf elements add 0 and NaN still poisons)
 #pragma unroll
@@ -296,15 +314,40 @@ softmax_strided_team_fwd_kernel(const TI* __restrict__ x, TO* __restrict__ y, St
         const float own = m[i];
         m[i] = ref[i];
         ref[i] = ref[i] == -INFINITY ? 0.0f : ref[i];
-        if (k0 > 0) s[i] *= row_exp<PRECISE>(own - ref[i]);
+        if constexpr (decltype(k_first)::value > 0) s[i] *= row_exp<PRECISE>(own - ref[i]);
       }
 #pragma unroll
-      for (int k = k0; k < kn; ++k) {
+      for (int k = 0; k < KN; ++k) {
 #pragma unroll
-        for (int i = 0; i < E; ++i) s[i] += row_exp<PRECISE>(xp[k].get(i) - ref[i]);
-        keep_packed(xp[k]);
+        for (int i = 0; i < E; ++i) s[i] += row_exp<PRECISE>(p[k].get(i) - ref[i]);
+        keep_packed(p[k]);
         __builtin_amdgcn_sched_barrier(0);
       }
+    };
+    {
+      const StridedTeamPlace<E> t(sh, lane_again((int)threadIdx.x), strip);
+      const TI* xs = x + (strip / sh.xtiles) * (int64_t)D * inner;
+      const int last = D - 1 - r0;
+      // the parked packs first, through the registers of the last L packs, which are requested as
+      // the groups are put away
+      if constexpr (L > 0)
+        strided_team_load<TI, E, 0, L>(xp + (R - L), xs, r0, t.ty, t.TY, t.e0, D, inner);
+      strided_team_load<TI, E, L, V - L>(xp, xs, r0, t.ty, t.TY, t.e0, D, inner);
+      static_for<0, L / GR>([&](auto g) {
+        constexpr int K = decltype(g)::value * GR;
+        Pack<TI, E>* p = xp + (R - L + K);
+        strided_team_fill<TI, E, K, K + GR>(p, last, t.ty, t.TY, -INFINITY);
+        absorb(p, std::integral_constant<int, K>{}, std::integral_constant<int, GR>{});
+#pragma unroll
+        for (int k = 0; k < GR; ++k) park.put(K + k, p[k]);
+        strided_team_load<TI, E, V - L + K, V - L + K + GR>(p, xs, r0, t.ty, t.TY, t.e0, D, inner);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      static_for<0, (R + GR - 1) / GR>([&](auto g) {
+        constexpr int K = decltype(g)::value * GR, K1 = K + GR < R ? K + GR : R;
+        strided_team_fill<TI, E, L + K, L + K1>(xp + K, last, t.ty, t.TY, -INFINITY);
+        absorb(xp + K, std::integral_constant<int, L + K>{}, std::integral_constant<int, K1 - K>{});
+      });
     }
     // (formed here: moved behind the reduction of the maxima it would need a copy of the packs)
 #pragma unroll
@@ -402,15 +445,28 @@ softmax_strided_team_fwd_kernel(const TI* __restrict__ x, TO* __restrict__ y, St
     auto store_rows = [&](auto value) {
       const uint32_t off = ((uint32_t)t.ty * (uint32_t)inner + (uint32_t)t.e0) * (uint32_t)sizeof(TO);
       const int64_t step = (int64_t)t.TY * inner;
-#pragma unroll
-      for (int k = 0; k < V; ++k) {
+      int left = D - r0 - t.ty;  // (counted down pack by pack: a bound each would hold a register each)
+      auto store_row = [&](const Pack<TI, E>& p) {
         Pack<TO, E> out;
 #pragma unroll
-        for (int i = 0; i < E; ++i) out.set(i, value(xp[k].get(i), i));
-        if (full || r0 + t.ty + k * t.TY < D) out.store_stream(global_at(yb, off));
+        for (int i = 0; i < E; ++i) out.set(i, value(p.get(i), i));
+        if (full || left > 0) out.store_stream(global_at(yb, off));
         yb = scalar_again(yb + step);
+        left = lane_again(left - t.TY);
         __builtin_amdgcn_sched_barrier(0);
+      };
+      if constexpr (L > 0) {
+        // (the next parked pack is read while one is worked on)
+        Pack<TI, E> next = park.get(0);
+#pragma unroll
+        for (int k = 0; k < L; ++k) {
+          const Pack<TI, E> p = next;
+          if (k + 1 < L) next = park.get(k + 1);
+          store_row(p);
+        }
       }
+#pragma unroll
+      for (int k = 0; k < R; ++k) store_row(xp[k]);
     };
     if (t.in) {
       if (is_log) {
@@ -432,7 +488,7 @@ softmax_strided_team_fwd_kernel(const TI* __restrict__ x, TO* __restrict__ y, St
 // Backward: V packs a lane of grad and of y; the columns' sums of y * grad (log_softmax: of grad)
 // cross the team.
 template <class TG, class TO, int V>
-__global__ void __launch_bounds__(kTeamBlock, kTeamPerCu * kTeamBlock / 256)
+__global__ void __launch_bounds__(kTeamBlock, strided_team_per_cu(true, V) * kTeamBlock / 256)
 softmax_strided_team_bwd_kernel(const TG* __restrict__ grad, const TG* __restrict__ y,
                                 TO* __restrict__ gi, StridedTeamShape sh, int flags,
                                 TeamColumns* slot, unsigned int call_id,
@@ -440,10 +496,14 @@ softmax_strided_team_bwd_kernel(const TG* __restrict__ grad, const TG* __restric
   constexpr int E = elems_per_pack<TG>::value;
   constexpr bool PRECISE = sizeof(TO) == 4 && sizeof(TG) == 4;
   constexpr int NW = kTeamBlock / 64;
+  constexpr int L = strided_team_parked(true, V), R = V - L;  // as in the forward, of each tensor
+  constexpr int GR = kStridedTeamGroup;
+  static_assert(L % GR == 0 && L <= R, "parked packs pass through registers group by group");
   __shared__ float ws[NW * kTeamColumns];
   __shared__ int votes[2][kTeamBlock / 64 + 1];
   __shared__ float gs[kTeamBlock];
   __shared__ __align__(16) float fs[kTeamColumns];
+  __shared__ StridedTeamPark<TG, E, L> gpark, ypark;
   const bool is_log = (flags & kSoftmaxLog) != 0;
   const int D = sh.D, inner = sh.inner, team = sh.team;
   const int TX = 1 << sh.tx_log2, C = TX * E;
@@ -454,24 +514,56 @@ softmax_strided_team_bwd_kernel(const TG* __restrict__ grad, const TG* __restric
   bool lost = false;
   unsigned int round = 0;
   for (int64_t strip = tm; strip < sh.strips; strip += teams, ++round) {
-    Pack<TG, E> gp[V], yp[V];
-    {
-      const StridedTeamPlace<E> t(sh, lane_again((int)threadIdx.x), strip);
-      const int64_t slab = (strip / sh.xtiles) * (int64_t)D * inner;
-      strided_team_load<TG, E, V>(gp, grad + slab, r0, t.ty, t.TY, t.e0, D, inner, 0.0f);
-      strided_team_load<TG, E, V>(yp, y + slab, r0, t.ty, t.TY, t.e0, D, inner, 0.0f);
-    }
+    Pack<TG, E> gp[R], yp[R];
     float s[E];
 #pragma unroll
     for (int i = 0; i < E; ++i) s[i] = 0.0f;
     // (no branch on the variant: two arms would each want the packs in registers of their own)
+    {
+      const StridedTeamPlace<E> t(sh, lane_again((int)threadIdx.x), strip);
+      const int64_t slab = (strip / sh.xtiles) * (int64_t)D * inner;
+      const TG *gs_ = grad + slab, *ys_ = y + slab;
+      auto load = [&](int at, auto k0, auto k1) {
+        constexpr int K0 = decltype(k0)::value, K1 = decltype(k1)::value;
+        strided_team_load<TG, E, K0, K1>(gp + at, gs_, r0, t.ty, t.TY, t.e0, D, inner);
+        strided_team_load<TG, E, K0, K1>(yp + at, ys_, r0, t.ty, t.TY, t.e0, D, inner);
+      };
+      int left = D - r0 - t.ty;  // (as in the stores below)
+      auto absorb = [&](Pack<TG, E>& g, Pack<TG, E>& v) {
 #pragma unroll
-    for (int k = 0; k < V; ++k) {
-#pragma unroll
-      for (int i = 0; i < E; ++i) s[i] = fmaf(is_log ? 1.0f : yp[k].get(i), gp[k].get(i), s[i]);
-      keep_packed(gp[k]);
-      keep_packed(yp[k]);
-      __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < E; ++i) {
+          const float sum = fmaf(is_log ? 1.0f : v.get(i), g.get(i), s[i]);
+          s[i] = left > 0 ? sum : s[i];
+        }
+        left = lane_again(left - t.TY);
+        keep_packed(g);
+        keep_packed(v);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      // the parked packs first, as in the forward; the two tensors group by group where there are
+      // many packs, so that sums are formed while the rest is on its way
+      static_for<0, L / GR>([&](auto g) {
+        constexpr int K = decltype(g)::value * GR;
+        load(R - L + K, std::integral_constant<int, K>{}, std::integral_constant<int, K + GR>{});
+      });
+      constexpr int LG = V > strided_team_max_v(true) ? GR : R;
+      static_assert((R - L) % LG == 0, "whole groups");
+      static_for<0, (R - L) / LG>([&](auto g) {
+        constexpr int K = decltype(g)::value * LG;
+        load(K, std::integral_constant<int, L + K>{}, std::integral_constant<int, L + K + LG>{});
+      });
+      static_for<0, L / GR>([&](auto g) {
+        constexpr int K = decltype(g)::value * GR, AT = R - L + K, K1 = V - L + K;
+        static_for<0, GR>([&](auto k) {
+          constexpr int J = decltype(k)::value;
+          absorb(gp[AT + J], yp[AT + J]);
+          gpark.put(K + J, gp[AT + J]);
+          ypark.put(K + J, yp[AT + J]);
+        });
+        load(AT, std::integral_constant<int, K1>{}, std::integral_constant<int, K1 + GR>{});
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      static_for<0, R>([&](auto k) { absorb(gp[decltype(k)::value], yp[decltype(k)::value]); });
     }
 #pragma unroll
     for (int i = 0; i < E; ++i) asm volatile("" : "+v"(s[i]));
@@ -539,15 +631,30 @@ softmax_strided_team_bwd_kernel(const TG* __restrict__ grad, const TG* __restric
     auto store_rows = [&](auto value) {
       const uint32_t off = ((uint32_t)t.ty * (uint32_t)inner + (uint32_t)t.e0) * (uint32_t)sizeof(TO);
       const int64_t step = (int64_t)t.TY * inner;
-#pragma unroll
-      for (int k = 0; k < V; ++k) {
+      int left = D - r0 - t.ty;  // (counted down pack by pack: a bound each would hold a register each)
+      auto store_row = [&](const Pack<TG, E>& g, const Pack<TG, E>& v) {
         Pack<TO, E> out;
 #pragma unroll
-        for (int i = 0; i < E; ++i) out.set(i, value(gp[k].get(i), yp[k].get(i), s[i]));
-        if (full || r0 + t.ty + k * t.TY < D) out.store_stream(global_at(ob, off));
+        for (int i = 0; i < E; ++i) out.set(i, value(g.get(i), v.get(i), s[i]));
+        if (full || left > 0) out.store_stream(global_at(ob, off));
         ob = scalar_again(ob + step);
+        left = lane_again(left - t.TY);
         __builtin_amdgcn_sched_barrier(0);
+      };
+      if constexpr (L > 0) {
+        Pack<TG, E> ng = gpark.get(0), nv = ypark.get(0);
+#pragma unroll
+        for (int k = 0; k < L; ++k) {
+          const Pack<TG, E> g = ng, v = nv;
+          if (k + 1 < L) {
+            ng = gpark.get(k + 1);
+            nv = ypark.get(k + 1);
+          }
+          store_row(g, v);
+        }
       }
+#pragma unroll
+      for (int k = 0; k < R; ++k) store_row(gp[k], yp[k]);
     };
     if (t.in) {
       if (is_log) {
