@@ -109,16 +109,14 @@ template <class WT>
 struct UniformElem {
   uint32_t word;
   uint32_t shift;
+  // (The word's address is formed by clearing bits of the whole sum.  Written as the element's address less
+  // its odd half word, a constant i goes into the instruction's offset field and the base is left two bytes
+  // off a word; the scalar unit drops the low bits of either by itself and reads the word before.)
   __device__ __forceinline__ static UniformElem load(const WT* w, int64_t i) {
-    const char* p = reinterpret_cast<const char*>(w + i);
+    const uintptr_t a = reinterpret_cast<uintptr_t>(w + i);
     UniformElem r;
-    r.shift = 0;
-    if constexpr (sizeof(WT) == 2) {
-      const uint32_t odd = (uint32_t)(reinterpret_cast<uintptr_t>(p) & 2);
-      p -= odd;
-      r.shift = odd * 8u;
-    }
-    r.word = uniform_load<uint32_t>(p);
+    r.shift = sizeof(WT) == 2 ? (uint32_t)(a & 2) * 8u : 0u;
+    r.word = uniform_load<uint32_t>(reinterpret_cast<const void*>(a & ~(uintptr_t)3));
     return r;
   }
   __device__ __forceinline__ float value() const {
