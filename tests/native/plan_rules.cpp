@@ -36,6 +36,17 @@ void rule_strided_large(int backward, int64_t outer, int64_t D, int64_t inner, i
   out[0] = p.large_team, out[1] = p.large_v, out[2] = 1 << p.large_tx_log2, out[3] = p.large_grid;
 }
 
+// the whole-wavefront layout of a norm call: wavefronts a row, packs a lane, rows in registers, threads the
+// instance is built for, rows a workgroup works on, workgroups; then the rows of the resident plan's partial sums
+void rule_norm_waves(int backward, int64_t M, int64_t N, int esize, int layer_norm, int wide, int want_dx, int64_t out[7]) {
+  Plan p;
+  make_plan(backward ? OC_NORM_BWD : OC_NORM_FWD, M, N, esize, 256, Override{}, backward != 0, &p, false, layer_norm != 0,
+            wide != 0, false, false, false, want_dx != 0);
+  const WavesLayout& l = p.waves;
+  out[0] = l.waves, out[1] = l.v, out[2] = l.depth, out[3] = l.threads, out[4] = l.slots, out[5] = l.grid;
+  out[6] = p.partial_rows;
+}
+
 // one table of slots for streams, as the library keeps one per device
 int rule_team_slots() { return kTeamSlots; }
 void* rule_slots_new() { return new StreamSlots<kTeamSlots>(); }

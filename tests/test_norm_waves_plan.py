@@ -1,0 +1,59 @@
+"""The rule that lays norm rows out on whole wavefronts (norm_waves_layout() in plan.hpp), on the CPU."""
+import ctypes
+import random
+
+from test_plan_rules import rules  # noqa: F401
+
+i64 = ctypes.c_int64
+INSTANCES = {(0, 2): {(1, 3, 1024), (2, 3, 1024)}, (0, 4): {(3, 2, 512)},
+             (1, 2): {(1, 3, 1024), (2, 2, 768)}, (1, 4): {(3, 3, 512), (3, 2, 768)}}
+FOLD_FLOATS = 8192
+
+
+def _layout(rules, backward, M, N, esize, ln=1, wide=0, want_dx=1):  # noqa: F811
+    out = (i64 * 7)()
+    rules.rule_norm_waves(backward, i64(M), i64(N), esize, ln, wide, want_dx, out)
+    return dict(zip(("waves", "v", "depth", "threads", "slots", "grid", "partial"), list(out)))
+
+
+def test_rows_on_whole_wavefronts(rules):  # noqa: F811
+    """Every row is held, only a lane's last pack may reach past it, the workgroup fits its instance, the column
+    sums fit the memory they are folded through and the caller's partial rows, every workgroup has a row."""
+    rng = random.Random(11)
+    taken = {k: 0 for k in INSTANCES}
+    for _ in range(20000):
+        M = int(2 ** rng.uniform(0, 18))
+        N = int(2 ** rng.uniform(6, 14.2))
+        N = N // 8 * 8 if rng.random() < 0.3 else N
+        esize, backward = rng.choice((2, 4)), rng.randint(0, 1)
+        a = (backward, M, N, esize, rng.randint(0, 1), rng.randint(0, 1) if esize == 2 else 0)
+        l = _layout(rules, *a)
+        if l["waves"] == 0:
+            continue
+        taken[(backward, esize)] += 1
+        E = 16 // esize
+        packs = -(-N // E)
+        assert (l["v"], l["depth"], l["threads"]) in INSTANCES[(backward, esize)]
+        lanes = 64 * l["waves"]
+        assert lanes * l["v"] >= packs and (l["v"] - 1) * lanes * E <= N and N >= E, (a, l)
+        assert 1 <= l["slots"] and l["slots"] * lanes <= l["threads"] <= 1024
+        assert 1 <= l["grid"] and (l["grid"] - 1) * l["slots"] < M, "a workgroup without a row"
+        if backward:
+            assert l["grid"] <= l["partial"]
+            assert l["slots"] == 1 or 2 * lanes * l["v"] * E <= FOLD_FLOATS
+            # the column sums alone run on the same layout
+            assert _layout(rules, *a, want_dx=0) == dict(l, partial=_layout(rules, *a, want_dx=0)["partial"]) or N % E == 0
+    assert all(n > 100 for n in taken.values()), taken
+
+
+def test_rows_that_keep_their_layout(rules):  # noqa: F811
+    """Widths an exact layout or a power of two of lanes serves as well, and rows too short or too long."""
+    for N in (1024, 2048, 4096, 5120, 8192, 16384):
+        for ln in (0, 1):
+            for b in (0, 1):
+                assert _layout(rules, b, 16384, N, 2, ln)["waves"] == 0 and _layout(rules, b, 16384, N, 4, ln)["waves"] == 0
+    assert _layout(rules, 1, 8192, 16383, 2)["waves"] == 0 and _layout(rules, 0, 8192, 8195, 2)["waves"] == 0
+    assert _layout(rules, 0, 8192, 4097, 4, 0)["waves"] == 0 and _layout(rules, 0, 1024, 4097, 4)["waves"] == 0
+    assert _layout(rules, 1, 8192, 509, 2)["waves"] == 0 and _layout(rules, 0, 8192, 1021, 4)["waves"] == 0
+    assert _layout(rules, 1, 8192, 4097, 2) == dict(waves=9, v=1, depth=3, threads=1024, slots=1, grid=256, partial=512)
+    assert _layout(rules, 0, 8192, 4097, 2)["waves"] == 5

@@ -128,6 +128,22 @@ struct UniformElem {
   }
 };
 
+// A pointer into global memory, byte offset added per lane (an address made from an integer is
+// otherwise a generic one, whose accesses wait for everything outstanding).
+template <class P>
+__device__ __forceinline__ P* global_at(P* p, uint32_t off) {
+  typedef __attribute__((address_space(1))) P* GlobalPtr;
+  return (P*)reinterpret_cast<GlobalPtr>(reinterpret_cast<uintptr_t>(p) + off);
+}
+
+// A wavefront-uniform pointer the compiler cannot trace back: the V row pointers of a chunk are
+// formed one after the other, not held in registers all at once.
+template <class P>
+__device__ __forceinline__ P* scalar_again(P* p) {
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
 // The lane index as a value the compiler cannot trace back to threadIdx, and
 // that exists only once `after` does: the pack offsets derived from it are then
 // computed where they are used (after a reduction, say) instead of ahead of the

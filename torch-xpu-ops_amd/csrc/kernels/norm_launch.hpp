@@ -2,6 +2,7 @@
 #pragma once
 #include "launch.hpp"
 #include "norm_kernels.hpp"
+#include "norm_waves_kernels.hpp"
 
 namespace rownorm {
 
@@ -102,6 +103,24 @@ bool launch_norm_fwd_flat(FlatLayout f, const NormFwdArgs& a, hipStream_t stream
   return false;
 }
 
+// Rows on whole wavefronts (norm_waves_kernels.hpp): calls go(packs, rows in registers, threads) with the
+// plan's instance; false if there is none.
+template <class T, bool BACKWARD, class Go>
+inline bool launch_norm_waves(const WavesLayout& l, Go go) {
+  constexpr auto& list = [] () -> auto& {
+    if constexpr (sizeof(T) == 2) return BACKWARD ? kWavesBwd16 : kWavesFwd16;
+    else return BACKWARD ? kWavesBwd32 : kWavesFwd32;
+  }();
+  auto at = [&](auto i) {
+    constexpr WavesInstance in = list[decltype(i)::value];
+    if (l.v != in.v || l.depth != in.depth || l.threads != in.threads) return false;
+    go(std::integral_constant<int, in.v>{}, std::integral_constant<int, in.depth>{},
+       std::integral_constant<int, in.threads>{});
+    return true;
+  };
+  return at(std::integral_constant<int, 0>{}) || at(std::integral_constant<int, 1>{});
+}
+
 template <class T, class WT, bool RMS, class TY, bool ADD>
 int launch_norm_fwd(const Plan& plan, const NormFwdArgs& a, hipStream_t stream) {
   const T* res = ADD ? (const T*)a.res : nullptr;
@@ -112,6 +131,18 @@ int launch_norm_fwd(const Plan& plan, const NormFwdArgs& a, hipStream_t stream) 
       const FlatLayout f = flat_layout<T>(plan, a.M, a.N, a.x, a.y, nullptr);
       if (f.g != 0 && launch_norm_fwd_flat<T, WT, RMS>(f, a, stream))
         return (int)hipGetLastError();
+    }
+  }
+  if constexpr (!ADD && std::is_same<T, TY>::value) {
+    if (plan.waves.waves > 0 && a.res == nullptr) {
+      const bool ok = launch_norm_waves<T, false>(plan.waves, [&](auto v, auto d, auto threads) {
+        hipLaunchKernelGGL((norm_fwd_waves_kernel<T, WT, decltype(v)::value, decltype(d)::value,
+                                                  decltype(threads)::value, RMS>),
+                           dim3((unsigned)plan.waves.grid), dim3(plan.waves.waves * plan.waves.slots * 64), 0,
+                           stream, (const T*)a.x, (const WT*)a.gamma, (const WT*)a.beta, (T*)a.y, a.mean,
+                           a.rstd, (int)a.M, a.N, a.eps, plan.waves.waves);
+      });
+      return ok ? (int)hipGetLastError() : (int)hipErrorInvalidConfiguration;
     }
   }
   if (norm_fwd_team_serves<T, TY, ADD>(plan, a) && plan.team_r > 0) {
@@ -320,7 +351,27 @@ int launch_norm_bwd(const Plan& plan, const NormBwdArgs& a, hipStream_t stream) 
              launch_norm_bwd_flat<T, WT, RMS>(plan, f, a, stream, &partial_rows);
     }
   }
-  if (flat) {
+  bool waves = false;
+  if constexpr (!ADD) {
+    if (!flat && plan.waves.waves > 0) {
+      waves = launch_norm_waves<T, true>(plan.waves, [&](auto v, auto d, auto threads) {
+        auto go = [&](auto kernel) {
+          hipLaunchKernelGGL(kernel, dim3((unsigned)plan.waves.grid),
+                             dim3(plan.waves.waves * plan.waves.slots * 64), 0, stream, (const T*)a.dy,
+                             (const T*)a.x, a.mean, a.rstd, (const WT*)a.gamma, (T*)a.dx, a.part_dg, a.part_db,
+                             (int)a.M, a.N, plan.waves.waves);
+        };
+        constexpr int V = decltype(v)::value, D = decltype(d)::value, THREADS = decltype(threads)::value;
+        if (a.dx != nullptr)
+          go(norm_bwd_waves_kernel<T, WT, V, D, THREADS, RMS, true>);
+        else
+          go(norm_bwd_waves_kernel<T, WT, V, D, THREADS, RMS, false>);
+      });
+      if (!waves) return (int)hipErrorInvalidConfiguration;
+      partial_rows = plan.waves.grid;
+    }
+  }
+  if (flat || waves) {
     // (launched above)
   } else if (plan.resident && plan.exact_depth > 0) {
     static_assert(kNormBwdExactCount == 15, "one index per table entry below");

@@ -43,6 +43,13 @@ struct Override {
   int G = 0, V = 0, block = 0, bpc = 0;
 };
 
+// Rows on whole wavefronts, as many as they need (norm_waves_kernels.hpp): wavefronts a row, packs a
+// lane, rows a lane has in its registers, threads the instance is built for, rows a workgroup works on
+// at a time, workgroups.  waves 0: not this call.
+struct WavesLayout {
+  int waves = 0, v = 0, depth = 0, threads = 0, slots = 0, grid = 0;
+};
+
 struct Plan {
   bool resident = true;
   bool fast = true;  // N % E == 0: branch-free row access
@@ -78,6 +85,9 @@ struct Plan {
   // forward: 1); GroupNorm on an exact layout (gn_*_exact_kernel): 1; 0 = the
   // general resident kernel
   int exact_depth = 0;
+  // what serves the call instead of the resident layout where the row is written in its own type
+  // (norm backward: no residual gradient)
+  WavesLayout waves;
   // ragged 16-bit norm rows addressed through the 16-byte aligned window that holds
   // each row (norm_row_window()): G * V holds the packs of that window, and a
   // workgroup that walks several row blocks strides by a multiple of 8 rows
@@ -644,6 +654,79 @@ inline int ragged_norm_fwd_lanes(int64_t packs, const Override& ov) {
   return G;
 }
 
+// The layouts on whole wavefronts: instances (packs a lane, rows in registers, threads), forward and
+// backward, 16-bit and float32 rows.
+struct WavesInstance {
+  int v, depth, threads;
+};
+constexpr WavesInstance kWavesFwd16[] = {{1, 3, 1024}, {2, 3, 1024}};
+constexpr WavesInstance kWavesFwd32[] = {{3, 2, 512}, {3, 2, 512}};
+constexpr WavesInstance kWavesBwd16[] = {{1, 3, 1024}, {2, 2, 768}};
+constexpr WavesInstance kWavesBwd32[] = {{3, 3, 512}, {3, 2, 768}};
+constexpr int kWavesMax = 16;  // wavefronts a workgroup at most
+// LDS floats the backward folds its row slots' column sums through (two slots or more of one pack a lane
+// in 16 bits, three in float32, beside a second set of sums)
+constexpr int kWavesFoldFloats = 8192;
+
+// Which rows take them.  One pack a lane and three rows in registers in 16 bits, with one workgroup of up to
+// sixteen wavefronts a compute unit: what is idle of a row's slots is less than a wavefront, and every row
+// slot has two rows on their way.  Beyond 1024 packs the backward holds two packs a lane and two rows (ragged
+// rows to 1536 packs); float32 rows three packs.  Measured against the general layouts, us, 8192 fp16 rows
+// that start 4 bytes off a boundary: LayerNorm backward N = 521 16.6 -> 15.8, 1401 24.9 -> 21.4, 2049 35.6 ->
+// 27.0, 4097 57.2 -> 47.2, 8191 103 -> 86, 8193 128 -> 97, 12001 175 -> 131, RMSNorm (bf16) 2049 29.0 -> 25.6,
+// 8191 97 -> 82, 1024 rows of 4097 22.8 -> 16.5; LayerNorm forward 1401 14.8 -> 13.8, 2049 19.6 -> 17.6, 4097
+// 34.3 -> 27.9, 8191 60.4 -> 48.5; fp32 LayerNorm 2049 forward / backward 33.0 / 46.1 -> 26.7 / 42.6, 4097 55.6
+// / 80.9 -> 50.2 / 77.7.  Whole-pack rows that no exact layout serves gain in the backward, where theirs
+// leave lanes idle (16384 rows of 2304 48.9 -> 43.6, 4608 84.8 -> 77.9, 6656 117 -> 113; from 513 packs also
+// few rows, 2048 of 4608 21.4 -> 19.6, below only many: 2048 of 2560 14.0 -> 14.6).  The other sides of the
+// lines: forward rows of 1025 12.1 -> 12.8, RMSNorm 1401 11.8 -> 12.6 and, in float32, 2305 28.3 -> 30.1 (no
+// second reduction to wait for); 1024 float32 rows of 4001 8.6 -> 9.4, which are too few to fill three row
+// slots a workgroup; whole-pack forward rows, which four times as many small workgroups serve as well.
+// Forward rows of 513 to 640 packs would leave seven of sixteen wavefronts without a row: two packs a lane,
+// three row slots (4097 30.6 -> 27.9).
+inline WavesLayout norm_waves_layout(bool backward, int esize, int64_t M, int64_t N, bool whole_packs,
+                                     bool layer_norm, int64_t partial_rows, int num_cus) {
+  WavesLayout l;
+  const int E = 16 / esize;
+  const int64_t packs = (N + E - 1) / E;
+  int which = -1;
+  if (esize == 2) {
+    if (backward) {
+      if (whole_packs ? packs > 256 && packs <= 1024 && (packs > 512 || M >= 8192) : packs > 64 && packs <= 1024)
+        which = 0;
+      else if (!whole_packs && packs > 1024 && packs <= 1536)
+        which = 1;
+    } else if (!whole_packs && packs > (layer_norm ? 160 : 320) && packs <= 1024) {
+      which = packs > 512 && packs <= 640 && M >= 16 * (int64_t)num_cus ? 1 : 0;
+    }
+  } else if (!whole_packs && packs > 256) {
+    if (backward)
+      which = packs <= 1536 ? 0 : packs <= 2304 ? 1 : -1;
+    else if (layer_norm && M >= 16 * (int64_t)num_cus && packs <= 1152)
+      which = 0;
+  }
+  if (which < 0 || M > 0x7fffffff / 2) return l;
+  const WavesInstance& in =
+      esize == 2 ? (backward ? kWavesBwd16 : kWavesFwd16)[which] : (backward ? kWavesBwd32 : kWavesFwd32)[which];
+  const int64_t waves = (packs + 64 * in.v - 1) / (64 * in.v);
+  const int most = in.threads / 64;
+  // (only the last of a lane's packs may reach past the row)
+  if (waves > most || (in.v - 1) * 64 * waves * E > N) return l;
+  int64_t grid = (int64_t)num_cus * (!backward && in.threads == 512 ? 2 : 1);
+  if (backward && partial_rows > 0 && grid > partial_rows) grid = partial_rows;
+  int64_t slots = most / waves;
+  const int64_t want = (M + grid - 1) / grid;
+  if (slots > want) slots = want;
+  const int64_t nrb = (M + slots - 1) / slots;
+  l.waves = (int)waves;
+  l.v = in.v;
+  l.depth = in.depth;
+  l.threads = in.threads;
+  l.slots = (int)slots;
+  l.grid = (int)(grid < nrb ? grid : nrb);
+  return l;
+}
+
 // Returns 0, or -5 (ROWNORM_ERR_OVERRIDE) when a forced variant cannot hold the row.
 // force_general: take the general (ragged-row) kernels even when N % E == 0.
 // layer_norm: the norm op is LayerNorm (statistics of two sums, beta), not RMSNorm.
@@ -954,6 +1037,11 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
       p.partial_rows = pr < 1 ? 1 : pr;
     }
   }
+  // (the column sums alone run on the layout they run on beside dX: the same bits)
+  if ((oc == OC_NORM_FWD || oc == OC_NORM_BWD) && p.resident && p.exact_depth == 0 && !fused_add &&
+      !force_general && !p.forced && ov.bpc == 0 &&
+      !(oc == OC_NORM_BWD && p.fast && norm_bwd_exact_index(esize, packs, M, layer_norm, wide_weights, false) >= 0))
+    p.waves = norm_waves_layout(oc == OC_NORM_BWD, esize, M, N, p.fast, layer_norm, p.partial_rows, num_cus);
   // Rows beyond the registers, and too few of them to give every compute unit a
   // workgroup (the regime of the reference's split-row kernels, Norm.h:632-812):
   // cut each row into chunks so that about four workgroups per compute unit

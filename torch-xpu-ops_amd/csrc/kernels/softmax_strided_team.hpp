@@ -65,22 +65,6 @@ struct StridedTeamPlace {
   }
 };
 
-// A pointer into global memory, byte offset added per lane (an address made from an integer is
-// otherwise a generic one, whose accesses wait for everything outstanding).
-template <class P>
-__device__ __forceinline__ P* global_at(P* p, uint32_t off) {
-  typedef __attribute__((address_space(1))) P* GlobalPtr;
-  return (P*)reinterpret_cast<GlobalPtr>(reinterpret_cast<uintptr_t>(p) + off);
-}
-
-// A wavefront-uniform pointer the compiler cannot trace back: the V row pointers of a chunk are
-// formed one after the other, not held in registers all at once.
-template <class P>
-__device__ __forceinline__ P* scalar_again(P* p) {
-  asm volatile("" : "+s"(p));
-  return p;
-}
-
 // Packs [K0, K1) of this thread's V: rows r0 + ty + k * TY, pack column e0 (an element index inside
 // the row), into p[0 .. K1 - K0).  One straight line for every workgroup (two versions of it would
 // each want the packs in registers of their own): rows past D - 1 read row D - 1;
