@@ -18,6 +18,8 @@ void rule_gn_bwd_team(int64_t rows, int64_t D, int64_t cp, int esize, int64_t ou
   out[0] = t.team, out[1] = t.wpc, out[2] = t.v, out[3] = t.ahead, out[4] = t.grid;
 }
 
+int rule_gn_team_sums(int64_t rows, int64_t groups, int64_t teams) { return gn_team_sums_columns(rows, groups, teams); }
+
 // out: workgroups a team, packs a lane, lanes along inner, workgroups launched; then whether the tile
 // kernel holds D, its lanes along inner and along D, rows a lane and workgroups, chunks
 void rule_strided_plan(int backward, int64_t outer, int64_t D, int64_t inner, int esize, int64_t out[10]) {

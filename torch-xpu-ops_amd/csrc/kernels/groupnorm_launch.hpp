@@ -205,20 +205,29 @@ int launch_group_norm_bwd(const Plan& plan, const GroupNormBwdArgs& a, hipStream
   const int C = a.groups * a.D;
   int err = 0;
   const bool teams = !plan.resident && a.team > 0 && a.team_slot != nullptr && a.dx != nullptr;
+  bool team_cols = false;  // the teams write dgamma / dbeta themselves
   if (teams) {
     // slabs beyond the registers, dY and X read once: teams of workgroups
     GroupNormBwdArgs k = a;
     if (!want_cols) k.part_dg = k.part_db = nullptr;
-    auto go = [&](auto kernel) {
+    team_cols = want_cols && !a.team_ahead && gn_team_sums_columns(a.rows, a.groups, a.team_grid / a.team);
+    auto launch = [&](auto kernel, auto... outs) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)a.team_grid), dim3(kTeamBlock), 0, stream,
                          (const T*)a.dy, (const T*)a.x, (const WT*)a.mean, (const WT*)a.rstd,
-                         (const WT*)a.gamma, (T*)a.dx, k.part_dg, k.part_db, a.rows, shape, a.team,
+                         (const WT*)a.gamma, (T*)a.dx, k.part_dg, k.part_db, outs..., a.rows, shape, a.team,
                          a.team_wpc, (TeamSlot*)a.team_slot, a.team_id, a.team_wait_ticks);
     };
+    auto go = [&](auto v) {
+      constexpr int V = decltype(v)::value;
+      if (team_cols)
+        launch(gn_bwd_team_kernel<T, WT, V, true>, (WT*)a.dgamma, (WT*)a.dbeta);
+      else
+        launch(gn_bwd_team_kernel<T, WT, V, false>, (WT*)a.dgamma, (WT*)a.dbeta);
+    };
     switch (a.team_ahead ? 0 : a.team_v) {
-      case 0: go(gn_bwd_team_ahead_kernel<T, WT>); break;
-      case 4: go(gn_bwd_team_kernel<T, WT, 4>); break;
-      case 8: go(gn_bwd_team_kernel<T, WT, 8>); break;
+      case 0: launch(gn_bwd_team_ahead_kernel<T, WT>); break;
+      case 4: go(std::integral_constant<int, 4>{}); break;
+      case 8: go(std::integral_constant<int, 8>{}); break;
       default: return (int)hipErrorInvalidConfiguration;
     }
   } else if (need_sums && !fused_cols) {
@@ -277,7 +286,7 @@ int launch_group_norm_bwd(const Plan& plan, const GroupNormBwdArgs& a, hipStream
                        (const float*)a.part_db, (T*)a.dx, a.rows, shape, chunks);
   }
   err = (int)hipGetLastError();
-  if (err != 0 || !want_cols) return err;
+  if (err != 0 || !want_cols || team_cols) return err;
   const unsigned gx = (unsigned)((C + kFinalizeCols - 1) / kFinalizeCols);
   // one partial row a sample: with very many samples under few channels the rows are first
   // folded in place, kGnFoldRows at a time, by as many workgroups as that gives (bf16
