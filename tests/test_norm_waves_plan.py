@@ -22,12 +22,13 @@ def test_rows_on_whole_wavefronts(rules):  # noqa: F811
     rng = random.Random(11)
     taken = {k: 0 for k in INSTANCES}
     for _ in range(20000):
-        M = int(2 ** rng.uniform(0, 18))
+        M = int(2 ** rng.uniform(6, 18))
         N = int(2 ** rng.uniform(6, 14.2))
         N = N // 8 * 8 if rng.random() < 0.3 else N
         esize, backward = rng.choice((2, 4)), rng.randint(0, 1)
         a = (backward, M, N, esize, rng.randint(0, 1), rng.randint(0, 1) if esize == 2 else 0)
         l = _layout(rules, *a)
+        assert l["waves"] == 0 or M >= 256
         if l["waves"] == 0:
             continue
         taken[(backward, esize)] += 1

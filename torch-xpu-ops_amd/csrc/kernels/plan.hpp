@@ -705,7 +705,9 @@ inline WavesLayout norm_waves_layout(bool backward, int esize, int64_t M, int64_
     else if (layer_norm && M >= 16 * (int64_t)num_cus && packs <= 1152)
       which = 0;
   }
-  if (which < 0 || M > 0x7fffffff / 2) return l;
+  // (a row for every compute unit at least: fewer are as fast on either layout, and keep the bits they have in
+  // common with the fused add, which has the general one -- 130 rows within 3 % of one another up to 8191)
+  if (which < 0 || M < num_cus || M > 0x7fffffff / 2) return l;
   const WavesInstance& in =
       esize == 2 ? (backward ? kWavesBwd16 : kWavesFwd16)[which] : (backward ? kWavesBwd32 : kWavesFwd32)[which];
   const int64_t waves = (packs + 64 * in.v - 1) / (64 * in.v);
