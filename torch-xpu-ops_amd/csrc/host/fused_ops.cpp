@@ -19,13 +19,6 @@ Tensor defined_or_empty(const std::optional<Tensor>& t) {
   return (t.has_value() && t->defined()) ? *t : Tensor();
 }
 
-std::vector<int64_t> stat_shape_of(const Tensor& input, size_t normalized_ndim) {
-  const size_t axis = input.dim() - normalized_ndim;
-  std::vector<int64_t> shape(input.sizes().begin(), input.sizes().begin() + axis);
-  shape.resize(input.dim(), 1);
-  return shape;
-}
-
 rownorm_dtype weight_dtype(const Tensor& X, const Tensor& gamma, const Tensor& beta,
                            const char* op) {
   const Tensor& w = gamma.defined() ? gamma : beta;
@@ -90,10 +83,9 @@ Forward prepare_forward(const Tensor& input, const Tensor& residual,
     f.H = residual;
   } else {
     f.R = residual.contiguous();
-    f.H = at::empty_like(f.X, f.X.options(), at::MemoryFormat::Contiguous);
+    f.H = new_like(f.X);
   }
-  f.Y = at::empty_like(f.X, f.X.options().dtype(check_out_dtype(input, out_dtype, op)),
-                       at::MemoryFormat::Contiguous);
+  f.Y = new_tensor(f.X.sizes(), check_out_dtype(input, out_dtype, op), f.X);
   return f;
 }
 
@@ -113,8 +105,9 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> add_layer_norm_impl(
   Forward f = prepare_forward(input, residual, out_dtype, inplace, op);
   const Tensor gamma = weight.defined() ? weight.contiguous() : weight;
   const Tensor beta = bias.defined() ? bias.contiguous() : bias;
-  Tensor mean = at::empty({M}, f.X.options().dtype(at::kFloat));
-  Tensor rstd = at::empty({M}, f.X.options().dtype(at::kFloat));
+  const auto stat_shape = stat_shape_of(input, normalized_shape.size());
+  Tensor mean = new_tensor(stat_shape, at::kFloat, f.X);
+  Tensor rstd = new_tensor(stat_shape, at::kFloat, f.X);
   if (M > 0 && N > 0) {
     check_status(
         mi355x_add_layer_norm_fwd(f.X.const_data_ptr(), f.R.const_data_ptr(), ptr_or_null(gamma),
@@ -129,9 +122,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> add_layer_norm_impl(
     mean.zero_();
     rstd.fill_(std::numeric_limits<float>::quiet_NaN());
   }
-  const auto stat_shape = stat_shape_of(input, normalized_shape.size());
-  return std::make_tuple(std::move(f.Y), std::move(f.H), mean.view(stat_shape),
-                         rstd.view(stat_shape));
+  return std::make_tuple(std::move(f.Y), std::move(f.H), std::move(mean), std::move(rstd));
 }
 
 std::tuple<Tensor, Tensor, Tensor> add_rms_norm_impl(const Tensor& input, const Tensor& residual,
@@ -150,7 +141,7 @@ std::tuple<Tensor, Tensor, Tensor> add_rms_norm_impl(const Tensor& input, const 
   Forward f = prepare_forward(input, residual, out_dtype, inplace, op);
   const Tensor gamma = weight.defined() ? weight.contiguous() : weight;
   const double eps = eps_opt.value_or((double)std::numeric_limits<float>::epsilon());
-  Tensor rstd = at::empty({M}, f.X.options().dtype(at::kFloat));
+  Tensor rstd = new_tensor(stat_shape_of(input, normalized_shape.size()), at::kFloat, f.X);
   if (M > 0 && N > 0) {
     check_status(
         mi355x_add_rms_norm_fwd(f.X.const_data_ptr(), f.R.const_data_ptr(), ptr_or_null(gamma),
@@ -163,8 +154,7 @@ std::tuple<Tensor, Tensor, Tensor> add_rms_norm_impl(const Tensor& input, const 
   } else if (M > 0) {
     rstd.fill_(std::numeric_limits<float>::quiet_NaN());
   }
-  return std::make_tuple(std::move(f.Y), std::move(f.H),
-                         rstd.view(stat_shape_of(input, normalized_shape.size())));
+  return std::make_tuple(std::move(f.Y), std::move(f.H), std::move(rstd));
 }
 
 }  // namespace
@@ -250,18 +240,17 @@ std::tuple<Tensor, Tensor, Tensor> add_layer_norm_backward(
   const rownorm_dtype xd = to_rownorm_dtype(H.scalar_type(), op);
   const rownorm_dtype wd = weight_dtype(H, gamma, bias, op);
   Tensor dH, dgamma, dbeta;
-  if (output_mask[0]) dH = at::empty_like(H, H.options(), at::MemoryFormat::Contiguous);
+  if (output_mask[0]) dH = new_like(H);
   if (output_mask[1] && gamma.defined())
-    dgamma = M > 0 ? at::empty_like(gamma, at::MemoryFormat::Contiguous)
+    dgamma = M > 0 ? new_like(gamma)
                    : at::zeros_like(gamma, at::MemoryFormat::Contiguous);
   if (output_mask[2] && bias.defined())
-    dbeta = M > 0 ? at::empty_like(bias, at::MemoryFormat::Contiguous)
+    dbeta = M > 0 ? new_like(bias)
                   : at::zeros_like(bias, at::MemoryFormat::Contiguous);
   if (M > 0 && N > 0) {
     const size_t ws_bytes = mi355x_layer_norm_bwd_workspace_bytes(M, N, xd, wd, dgamma.defined(),
                                                                   dbeta.defined());
-    Tensor ws;
-    if (ws_bytes > 0) ws = at::empty({(int64_t)ws_bytes}, H.options().dtype(at::kByte));
+    Tensor ws = new_workspace(ws_bytes, H);
     check_status(mi355x_add_layer_norm_bwd(
                      dY.const_data_ptr(), ptr_or_null(dHin), H.const_data_ptr(),
                      (const float*)mc.const_data_ptr(), (const float*)rc.const_data_ptr(),
@@ -295,14 +284,13 @@ std::tuple<Tensor, Tensor> add_rms_norm_backward(const Tensor& grad_y,
   const rownorm_dtype xd = to_rownorm_dtype(H.scalar_type(), op);
   const rownorm_dtype wd = weight_dtype(H, gamma, Tensor(), op);
   Tensor dH, dgamma;
-  if (output_mask[0]) dH = at::empty_like(H, H.options(), at::MemoryFormat::Contiguous);
+  if (output_mask[0]) dH = new_like(H);
   if (output_mask[1] && gamma.defined())
-    dgamma = M > 0 ? at::empty_like(gamma, at::MemoryFormat::Contiguous)
+    dgamma = M > 0 ? new_like(gamma)
                    : at::zeros_like(gamma, at::MemoryFormat::Contiguous);
   if (M > 0 && N > 0) {
     const size_t ws_bytes = mi355x_rms_norm_bwd_workspace_bytes(M, N, xd, wd, dgamma.defined());
-    Tensor ws;
-    if (ws_bytes > 0) ws = at::empty({(int64_t)ws_bytes}, H.options().dtype(at::kByte));
+    Tensor ws = new_workspace(ws_bytes, H);
     check_status(mi355x_add_rms_norm_bwd(dY.const_data_ptr(), ptr_or_null(dHin),
                                          H.const_data_ptr(), (const float*)rc.const_data_ptr(),
                                          ptr_or_null(gamma), mut_ptr_or_null(&dH),

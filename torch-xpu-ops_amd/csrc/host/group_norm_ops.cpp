@@ -155,8 +155,7 @@ void group_norm_backward_kernel(const Tensor& dY, const Tensor& X, const Tensor&
   c10::DeviceGuard guard(X.device());
   const size_t nbytes = mi355x_group_norm_bwd_workspace_bytes(N, C, HxW, group, xd, sd,
                                                               dgamma.defined(), dbeta.defined());
-  Tensor workspace;
-  if (nbytes > 0) workspace = at::empty({(int64_t)nbytes}, X.options().dtype(at::kByte));
+  Tensor workspace = new_workspace(nbytes, X);
   check_status(
       mi355x_group_norm_bwd(dYc.const_data_ptr(), Xc.const_data_ptr(), mc.const_data_ptr(),
                             rc.const_data_ptr(), ptr_or_null(gc), mut_ptr_or_null(&dX),
@@ -199,9 +198,9 @@ std::tuple<Tensor, Tensor, Tensor> native_group_norm(const Tensor& X,
   check_same_device(X, beta, op, "bias");
   const rownorm_dtype sd = stat_dtype(X, gamma, beta, op);
   (void)to_rownorm_dtype(X.scalar_type(), op);
-  Tensor Y = at::empty_like(X, X.options(), at::MemoryFormat::Contiguous);
-  Tensor mean = at::empty({N, group}, X.options().dtype(to_scalar_type(sd)));
-  Tensor rstd = at::empty({N, group}, X.options().dtype(to_scalar_type(sd)));
+  Tensor Y = new_like(X);
+  Tensor mean = new_tensor({N, group}, to_scalar_type(sd), X);
+  Tensor rstd = new_tensor({N, group}, to_scalar_type(sd), X);
   group_norm_kernel(X, gamma, beta, N, C, HxW, group, eps, Y, mean, rstd);
   return std::make_tuple(std::move(Y), std::move(mean), std::move(rstd));
 }
@@ -226,9 +225,9 @@ std::tuple<Tensor, Tensor, Tensor> native_group_norm_backward(
   check_same_device(X, rstd, op, "rstd");
   check_same_device(X, gamma, op, "weight");
   Tensor dX, dgamma, dbeta;
-  if (output_mask[0]) dX = at::empty_like(X, X.options(), at::MemoryFormat::Contiguous);
-  if (output_mask[1]) dgamma = at::empty({C}, X.options().dtype(mean.scalar_type()));
-  if (output_mask[2]) dbeta = at::empty({C}, X.options().dtype(mean.scalar_type()));
+  if (output_mask[0]) dX = new_like(X);
+  if (output_mask[1]) dgamma = new_tensor({C}, mean.scalar_type(), X);
+  if (output_mask[2]) dbeta = new_tensor({C}, mean.scalar_type(), X);
   group_norm_backward_kernel(dY, X, mean, rstd, gamma, N, C, HxW, group, dX, dgamma, dbeta);
   return std::make_tuple(std::move(dX), std::move(dgamma), std::move(dbeta));
 }

@@ -22,19 +22,6 @@ Tensor defined_or_empty(const std::optional<Tensor>& t) {
   return (t.has_value() && t->defined()) ? *t : Tensor();
 }
 
-// input.shape[:axis] + [1] * len(normalized_shape): the shape mean/rstd are
-// returned in (LayerNorm.cpp:82-94, 239-250).
-std::vector<int64_t> stat_shape_of(const Tensor& input, size_t normalized_ndim) {
-  const size_t axis = input.dim() - normalized_ndim;
-  std::vector<int64_t> shape(input.sizes().begin(), input.sizes().begin() + axis);
-  shape.resize(input.dim(), 1);
-  return shape;
-}
-
-Tensor contiguous_like(const Tensor& t) {
-  return at::empty_like(t, t.options(), at::MemoryFormat::Contiguous);
-}
-
 // gamma/beta may be the row dtype, or float32 next to 16-bit rows.
 rownorm_dtype weight_dtype(const Tensor& X, const Tensor& gamma, const Tensor& beta,
                            const char* op) {
@@ -148,8 +135,7 @@ void layer_norm_backward_kernel(const Tensor& dY, const Tensor& X, const Tensor&
   c10::DeviceGuard guard(X.device());
   const size_t ws_bytes =
       mi355x_layer_norm_bwd_workspace_bytes(M, N, xd, wd, dg_p != nullptr, db_p != nullptr);
-  Tensor ws;
-  if (ws_bytes > 0) ws = at::empty({(int64_t)ws_bytes}, X.options().dtype(at::kByte));
+  Tensor ws = new_workspace(ws_bytes, X);
   check_status(mi355x_layer_norm_bwd(dYc.const_data_ptr(), Xc.const_data_ptr(),
                                      (const float*)mc.const_data_ptr(),
                                      (const float*)rc.const_data_ptr(), ptr_or_null(gamma), dx_p,
@@ -192,8 +178,7 @@ void rms_norm_backward_kernel(const Tensor& dY, const Tensor& X, const Tensor& r
   }
   c10::DeviceGuard guard(X.device());
   const size_t ws_bytes = mi355x_rms_norm_bwd_workspace_bytes(M, N, xd, wd, dg_p != nullptr);
-  Tensor ws;
-  if (ws_bytes > 0) ws = at::empty({(int64_t)ws_bytes}, X.options().dtype(at::kByte));
+  Tensor ws = new_workspace(ws_bytes, X);
   check_status(mi355x_rms_norm_bwd(dYc.const_data_ptr(), Xc.const_data_ptr(),
                                    (const float*)rc.const_data_ptr(), ptr_or_null(gamma), dx_p,
                                    dg_p, ws.defined() ? ws.mutable_data_ptr() : nullptr, ws_bytes,
@@ -224,13 +209,13 @@ std::tuple<Tensor, Tensor, Tensor> native_layer_norm(const Tensor& input,
   const auto [M, N] = at::native::_check_layer_norm_inputs(input, normalized_shape, weight, bias);
   check_gpu(input, op, "input");
   (void)to_rownorm_dtype(input.scalar_type(), op);
-  c10::DeviceGuard guard(input.device());
   const Tensor X = input.contiguous();
   const Tensor gamma = weight.defined() ? weight.contiguous() : weight;
   const Tensor beta = bias.defined() ? bias.contiguous() : bias;
-  Tensor Y = contiguous_like(X);
-  Tensor mean = at::empty({M}, X.options().dtype(at::kFloat));
-  Tensor rstd = at::empty({M}, X.options().dtype(at::kFloat));
+  Tensor Y = new_like(X);
+  const auto stat_shape = stat_shape_of(input, normalized_shape.size());
+  Tensor mean = new_tensor(stat_shape, at::kFloat, X);
+  Tensor rstd = new_tensor(stat_shape, at::kFloat, X);
   if (M > 0 && N > 0) {
     layer_norm_kernel(X, gamma, beta, M, N, epsilon, &Y, &mean, &rstd);
   } else if (M > 0) {
@@ -238,8 +223,7 @@ std::tuple<Tensor, Tensor, Tensor> native_layer_norm(const Tensor& input,
     mean.zero_();
     rstd.fill_(std::numeric_limits<float>::quiet_NaN());
   }
-  const auto stat_shape = stat_shape_of(input, normalized_shape.size());
-  return std::make_tuple(std::move(Y), mean.view(stat_shape), rstd.view(stat_shape));
+  return std::make_tuple(std::move(Y), std::move(mean), std::move(rstd));
 }
 
 // native_layer_norm_backward: LayerNorm.cpp:99-196.  Only the outputs whose
@@ -265,17 +249,16 @@ std::tuple<Tensor, Tensor, Tensor> native_layer_norm_backward(
   const auto [M, N] = at::native::_check_layer_norm_inputs(input, normalized_shape, weight, bias);
   check_gpu(input, op, "input");
   (void)to_rownorm_dtype(input.scalar_type(), op);
-  c10::DeviceGuard guard(input.device());
   const Tensor X = input.contiguous();
   const Tensor gamma = weight.defined() ? weight.contiguous() : weight;
   const Tensor beta = bias.defined() ? bias.contiguous() : bias;
 
   Tensor dX, dgamma, dbeta;
-  if (grad_input_mask[0]) dX = contiguous_like(X);
+  if (grad_input_mask[0]) dX = new_like(X);
   if (grad_input_mask[1] && gamma.defined())
-    dgamma = M > 0 ? contiguous_like(gamma) : at::zeros_like(gamma, at::MemoryFormat::Contiguous);
+    dgamma = M > 0 ? new_like(gamma) : at::zeros_like(gamma, at::MemoryFormat::Contiguous);
   if (grad_input_mask[2] && beta.defined())
-    dbeta = M > 0 ? contiguous_like(beta) : at::zeros_like(beta, at::MemoryFormat::Contiguous);
+    dbeta = M > 0 ? new_like(beta) : at::zeros_like(beta, at::MemoryFormat::Contiguous);
   if (M > 0 && N > 0)
     layer_norm_backward_kernel(grad_output, X, mean, rstd, gamma, M, N, &dX, &dgamma, &dbeta);
   return std::make_tuple(std::move(dX), std::move(dgamma), std::move(dbeta));
@@ -297,18 +280,17 @@ std::tuple<Tensor, Tensor> _fused_rms_norm(const Tensor& input, at::IntArrayRef 
       at::native::_check_layer_norm_inputs(input, normalized_shape, weight, weight);
   check_gpu(input, op, "input");
   (void)to_rownorm_dtype(input.scalar_type(), op);
-  c10::DeviceGuard guard(input.device());
   const Tensor X = input.contiguous();
   const Tensor gamma = weight.defined() ? weight.contiguous() : weight;
   const double eps = eps_opt.value_or((double)std::numeric_limits<float>::epsilon());
-  Tensor Y = contiguous_like(X);
-  Tensor rstd = at::empty({M}, X.options().dtype(at::kFloat));
+  Tensor Y = new_like(X);
+  Tensor rstd = new_tensor(stat_shape_of(input, normalized_shape.size()), at::kFloat, X);
   if (M > 0 && N > 0) {
     rms_norm_kernel(X, gamma, M, N, eps, &Y, &rstd);
   } else if (M > 0) {
     rstd.fill_(std::numeric_limits<float>::quiet_NaN());  // the mean of no squares, as on the CPU
   }
-  return std::make_tuple(std::move(Y), rstd.view(stat_shape_of(input, normalized_shape.size())));
+  return std::make_tuple(std::move(Y), std::move(rstd));
 }
 
 // _fused_rms_norm_backward: LayerNorm.cpp:255-305.
@@ -331,13 +313,12 @@ std::tuple<Tensor, Tensor> _fused_rms_norm_backward(const Tensor& dY, const Tens
       at::native::_check_layer_norm_inputs(input, normalized_shape, weight, weight);
   check_gpu(input, op, "input");
   (void)to_rownorm_dtype(input.scalar_type(), op);
-  c10::DeviceGuard guard(input.device());
   const Tensor X = input.contiguous();
   const Tensor gamma = weight.defined() ? weight.contiguous() : weight;
   Tensor dX, dgamma;
-  if (grad_input_mask[0]) dX = contiguous_like(X);
+  if (grad_input_mask[0]) dX = new_like(X);
   if (grad_input_mask[1] && gamma.defined())
-    dgamma = M > 0 ? contiguous_like(gamma) : at::zeros_like(gamma, at::MemoryFormat::Contiguous);
+    dgamma = M > 0 ? new_like(gamma) : at::zeros_like(gamma, at::MemoryFormat::Contiguous);
   if (M > 0 && N > 0) rms_norm_backward_kernel(dY, X, rstd, gamma, M, N, &dX, &dgamma);
   return std::make_tuple(std::move(dX), std::move(dgamma));
 }

@@ -128,8 +128,7 @@ void softmax_backward_entry(const Tensor& grad_, const Tensor& output_, int64_t 
 }
 
 Tensor alloc_forward_output(const Tensor& self, bool half_to_float) {
-  return at::empty_like(self, self.options().dtype(half_to_float ? at::kFloat : self.scalar_type()),
-                        at::MemoryFormat::Contiguous);
+  return new_tensor(self.sizes(), half_to_float ? at::kFloat : self.scalar_type(), self);
 }
 
 // SoftMax.cpp:44-55: half_to_float is implied by grad.dtype != input_dtype and
@@ -214,7 +213,7 @@ Tensor masked_softmax_kernel(const Tensor& input_, const Tensor& mask_,
   check_gpu(input_, op, "input");
   check_same_device(input_, mask_, op, "mask");
   const rownorm_dtype dt = to_rownorm_dtype(input_.scalar_type(), op);
-  Tensor output = at::empty_like(input_, input_.options(), at::MemoryFormat::Contiguous);
+  Tensor output = new_like(input_);
   Tensor input = input_.dim() == 0 ? input_.view(1) : input_;
   Tensor mask = mask_.dim() == 0 ? mask_.view(1) : mask_;
   Tensor out = output.dim() == 0 ? output.view(1) : output;
@@ -252,7 +251,7 @@ Tensor masked_softmax_backward_kernel(const Tensor& grad_, const Tensor& output_
   check_gpu(grad_, op, "grad_output");
   check_same_device(grad_, output_, op, "output");
   check_same_device(grad_, mask_, op, "mask");
-  Tensor grad_input = at::empty_like(grad_, grad_.options(), at::MemoryFormat::Contiguous);
+  Tensor grad_input = new_like(grad_);
   if (grad_.numel() == 0) return grad_input;
   Tensor grad = grad_.contiguous();
   Tensor output = output_.contiguous();
@@ -377,8 +376,7 @@ Tensor _softmax_backward_data(const Tensor& grad_output, const Tensor& output, i
   }
   const bool h2f = backward_half_to_float(grad_output, input_dtype);
   check_gpu(grad_output, "mi355x::_softmax_backward_data", "grad_output");
-  Tensor gi = at::empty_like(grad_output, grad_output.options().dtype(input_dtype),
-                             at::MemoryFormat::Contiguous);
+  Tensor gi = new_tensor(grad_output.sizes(), input_dtype, grad_output);
   _softmax_backward_kernel(grad_output, output, dim, h2f, gi);
   return gi;
 }
@@ -390,8 +388,7 @@ Tensor _log_softmax_backward_data(const Tensor& grad_output, const Tensor& outpu
   }
   const bool h2f = backward_half_to_float(grad_output, input_dtype);
   check_gpu(grad_output, "mi355x::_log_softmax_backward_data", "grad_output");
-  Tensor gi = at::empty_like(grad_output, grad_output.options().dtype(input_dtype),
-                             at::MemoryFormat::Contiguous);
+  Tensor gi = new_tensor(grad_output.sizes(), input_dtype, grad_output);
   _log_softmax_backward_kernel(grad_output, output, dim, h2f, gi);
   return gi;
 }
