@@ -49,6 +49,13 @@ void rule_norm_waves(int backward, int64_t M, int64_t N, int esize, int layer_no
   out[6] = p.partial_rows;
 }
 
+// the team of a long norm forward row on a machine of 256 compute units: workgroups, packs a lane, teams
+void rule_norm_team(int64_t M, int64_t N, int esize, int wide, int64_t out[3]) {
+  Plan p;
+  make_plan(OC_NORM_FWD, M, N, esize, 256, Override{}, false, &p, false, true, wide != 0);
+  out[0] = p.team, out[1] = p.team_r ? 0 : p.team_v, out[2] = p.team ? p.team_grid / p.team : 0;
+}
+
 // one table of slots for streams, as the library keeps one per device
 int rule_team_slots() { return kTeamSlots; }
 void* rule_slots_new() { return new StreamSlots<kTeamSlots>(); }

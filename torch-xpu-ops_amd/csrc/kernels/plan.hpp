@@ -1102,10 +1102,28 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
     if (teams >= kTeamMinTeams || ((oc == OC_GROUP_FWD || few_rows) && teams >= 1 && teams == M)) {
       // a chunk is a whole number of workgroup strides, exactly the packs a lane the
       // kernel is compiled for: every workgroup but a row's last runs straight-line code
-      int64_t team_max = cus / teams;
       const int64_t strides = (packs + kTeamBlock - 1) / kTeamBlock;
-      if (team_max > strides) team_max = strides;
-      const int64_t v = (strides + team_max - 1) / team_max;
+      auto packs_a_lane = [&](int64_t n) {
+        const int64_t most = cus / n < strides ? cus / n : strides;
+        return (strides + most - 1) / most;
+      };
+      // Two or three rounds, the last of them not full: as many teams as give every round the same rows, each
+      // row over more workgroups (norm forward, bf16 LayerNorm: [140, 216576] 128 teams of 4 -> 70 of 7 35.3 ->
+      // 28.5 us, [33, 1103488] 44.8 -> 36.5, [256, 188416] 52.3 -> 42.5, [358, 163840] 58.5 -> 52.2, [64, 1345664]
+      // 92.0 -> 80.8, RMSNorm [100, 536704] 47.0 -> 42.3).  The other sides of the lines: a row that would not
+      // spread further ([389, 188800] 66.9 -> 74.5); four rounds or more, where the last leaves little idle
+      // ([216, 468864] 84.5 -> 89.0, [110, 1526656] 143 -> 181); less than 15 of 16 workgroups used in every
+      // round where the last one was a quarter full or more ([148, 291328] 39.4 -> 44.1); an odd team, whose
+      // chunks of the weights every XCD reads, where gamma and beta fill three quarters of its L2 ([71, 1284480]
+      // teams of 20 -> 21 79.7 -> 94.4, [65, 1213312] 19 -> 23 76.5 -> 82.9).
+      const int64_t rounds = (M + teams - 1) / teams;
+      if (oc == OC_NORM_FWD && (rounds == 2 || rounds == 3)) {
+        const int64_t even = (M + rounds - 1) / rounds, ve = packs_a_lane(even), members = (strides + ve - 1) / ve;
+        const bool fills = 16 * even * members >= 15 * cus || 4 * (M - (rounds - 1) * teams) < teams;
+        const bool in_l2 = members % 2 == 0 || 2 * (wide_weights ? 32 : 16) * packs <= (3 << 20);
+        if (even >= kTeamMinTeams && ve < packs_a_lane(teams) && fills && in_l2) teams = even;
+      }
+      const int64_t v = packs_a_lane(teams);
       const int64_t team = (strides + v - 1) / v;
       p.team = (int)team;
       p.team_v = (int)v;
