@@ -363,8 +363,7 @@ int mi355x_softmax_strided_plan(int backward, int64_t outer, int64_t dim_size, i
  * that bound, and reads the whole strip itself if it runs out.  They need an output that overlaps no
  * input; such a call in place, on a stream under capture, or on a stream beyond the eight takes
  * mi355x_softmax_strided_plan's layout.  A team of one waits for nobody and has none of these
- * conditions.  Where a team with a compute unit a workgroup is reported (it holds twice the strip), a
- * call that cannot have it runs on the team it replaced, if that is a team of one. */
+ * conditions. */
 int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_size, int64_t inner,
                                      rownorm_dtype dtype, rownorm_plan* out);
 

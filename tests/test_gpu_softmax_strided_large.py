@@ -62,3 +62,42 @@ def test_large_teams_against_oracle_and_the_give_up_path(cabi, oracle, gpu, dtyp
         assert_close(pick(gi), ogi, dtype, what + " backward", slack=sl)
         assert torch.equal(gi.view(torch.uint8), bwd().view(torch.uint8)), what + ": run to run"
         assert_close(pick(given_up(bwd)), ogi, dtype, what + " backward, every wait given up", slack=sl)
+
+
+@pytest.mark.parametrize("dtype,shape", [(torch.float32, (112, 497, 51)), (torch.bfloat16, (6, 323, 1285))], ids=str)
+def test_a_team_of_one_has_no_conditions(cabi, gpu, dtype, shape):
+    """A backward whose strips one workgroup holds runs on it in place, under capture and on any stream, with the
+    bits of the plain call, and its inputs may be the outputs."""
+    outer, D, packs = shape
+    inner = packs * (4 if dtype == torch.float32 else 8)
+    print("case strided softmax, large teams of one", dtype, (outer, D, inner), flush=True)
+    p = cabi.strided_team_plan(1, outer, D, inner, cabi.dtype_code(dtype))
+    assert p["team"] == 1 and p["packs_per_lane"] > 8, p
+    g = torch.Generator(device=gpu).manual_seed(D)
+    grad = torch.empty(outer, D, inner, device=gpu, dtype=dtype).normal_(0, 1.0, generator=g)
+    y = torch.softmax(torch.empty(outer, D, inner, device=gpu).normal_(0, 3.0, generator=g), 1).to(dtype)
+    for mode in (cabi.SOFTMAX, cabi.LOG_SOFTMAX):
+        want = cabi.softmax_strided_bwd(grad, y, 1, mode)
+        yd, gd = y.double(), grad.double()
+        ref = gd - yd.exp() * gd.sum(1, keepdim=True) if mode else yd * (gd - (yd * gd).sum(1, keepdim=True))
+        # (a few ulps of the magnitudes' sum, as for any float32 sum in another order)
+        mag = yd.exp() * gd.abs().sum(1, keepdim=True) if mode else yd * (yd * gd).abs().sum(1, keepdim=True)
+        assert_close(want, ref.float().cpu().numpy(), dtype, "mode %d" % mode, slack=(mag * 2.0 ** -21).float().cpu())
+        del yd, gd, ref, mag
+        for over in (0, 1):
+            a, b = grad.clone(), y.clone()
+            assert torch.equal(cabi.softmax_strided_bwd(a, b, 1, mode, gi=(a, b)[over]), want), "in place over %d" % over
+        s = torch.cuda.Stream()
+        s.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            assert torch.equal(cabi.softmax_strided_bwd(grad, y, 1, mode), want)
+        torch.cuda.current_stream().wait_stream(s)
+        gi = torch.empty_like(grad)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            cabi.softmax_strided_bwd(grad, y, 1, mode, gi=gi)
+        for _ in range(3):
+            gi.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(gi, want), "replayed"

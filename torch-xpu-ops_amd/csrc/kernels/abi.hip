@@ -890,7 +890,7 @@ int mi355x_softmax_strided_fwd(const void* x, void* y, int64_t outer, int64_t di
   // (a workgroup whose team does not come together reads the whole strip again; a team of one
   // has nobody to wait for)
   const int64_t n = outer * dim_size * inner;
-  if ((plan.team > 1 || plan.large_team > 1) && regions_disjoint(y, n * esize_of(od), x, n * esize_of(id))) {
+  if (plan.team_size() > 1 && regions_disjoint(y, n * esize_of(od), x, n * esize_of(id))) {
     a.team_slot = team_columns_for_call(s, &a.team_id);
     a.team_wait_ticks = g_team_wait_ticks.load(std::memory_order_relaxed);
   }
@@ -920,8 +920,7 @@ int mi355x_softmax_strided_bwd(const void* grad, const void* y, void* gi, int64_
   SoftmaxStridedBwdArgs a{grad, y, gi, outer, (int)dim_size, (int)inner, flags};
   hipStream_t s = (hipStream_t)stream;
   const int64_t n = outer * dim_size * inner;
-  if ((plan.team > 1 || plan.large_team > 1) &&
-      regions_disjoint(gi, n * esize_of(od), grad, n * esize_of(gd)) &&
+  if (plan.team_size() > 1 && regions_disjoint(gi, n * esize_of(od), grad, n * esize_of(gd)) &&
       regions_disjoint(gi, n * esize_of(od), y, n * esize_of(gd))) {
     a.team_slot = team_columns_for_call(s, &a.team_id);
     a.team_wait_ticks = g_team_wait_ticks.load(std::memory_order_relaxed);
@@ -963,8 +962,8 @@ int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_si
     return e;
   const bool large = plan.large_team > 0;
   const int tx_log2 = large ? plan.large_tx_log2 : plan.team_tx_log2;
-  out->reserved = large ? plan.large_team : plan.team;
-  if (plan.team == 0) return 0;
+  out->reserved = plan.team_size();
+  if (plan.team_size() == 0) return 0;
   out->resident = 1;
   out->lanes_per_row = 1 << tx_log2;
   out->packs_per_lane = large ? plan.large_v : plan.team_v;

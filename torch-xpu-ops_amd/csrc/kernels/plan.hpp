@@ -1328,6 +1328,8 @@ struct StridedPlan {
   // large_team 0: two a compute unit
   int large_team = 0, large_v = 0, large_tx_log2 = 0;
   int64_t large_grid = 0;
+  // Workgroups of the team a call by teams runs on (0: no teams): one waits for nobody, more exchange.
+  int team_size() const { return large_team > 0 ? large_team : team; }
 };
 
 // The packs a lane the strided team kernels are built for: the forward holds one tensor, the

@@ -23,8 +23,8 @@ bool launch_strided_team_v(int v, Go go) {
   return false;
 }
 template <bool BACKWARD, int E, class Go>
-bool launch_strided_team(const StridedPlan& p, int64_t outer, int D, int inner, bool exchange, Go go) {
-  const bool large = p.large_team == 1 || (p.large_team > 1 && exchange);
+bool launch_strided_team(const StridedPlan& p, int64_t outer, int D, int inner, Go go) {
+  const bool large = p.large_team > 0;
   const int tx_log2 = large ? p.large_tx_log2 : p.team_tx_log2;
   const int64_t xtiles = (inner / E + (1 << tx_log2) - 1) >> tx_log2;
   const StridedTeamShape sh{outer * xtiles, xtiles, D, inner, tx_log2, large ? p.large_team : p.team};
@@ -59,9 +59,9 @@ bool launch_strided_fwd_f(const StridedPlan& p, const SoftmaxStridedFwdArgs& a, 
 template <class TI, class TO>
 int launch_softmax_strided_fwd(const StridedPlan& p, const SoftmaxStridedFwdArgs& a,
                                hipStream_t s) {
-  if (p.team == 1 || (p.team > 1 && a.team_slot != nullptr)) {
+  if (p.team_size() == 1 || (p.team_size() > 1 && a.team_slot != nullptr)) {
     const bool ok = launch_strided_team<false, elems_per_pack<TI>::value>(
-        p, a.outer, a.D, a.inner, a.team_slot != nullptr, [&](auto v, const StridedTeamShape& sh, dim3 grid) {
+        p, a.outer, a.D, a.inner, [&](auto v, const StridedTeamShape& sh, dim3 grid) {
           hipLaunchKernelGGL((softmax_strided_team_fwd_kernel<TI, TO, decltype(v)::value>), grid,
                              dim3(kTeamBlock), 0, s, (const TI*)a.x, (TO*)a.y, sh, a.flags,
                              (TeamColumns*)a.team_slot, a.team_id, a.team_wait_ticks);
@@ -123,9 +123,9 @@ bool launch_strided_bwd_f(const StridedPlan& p, const SoftmaxStridedBwdArgs& a, 
 template <class TG, class TO>
 int launch_softmax_strided_bwd(const StridedPlan& p, const SoftmaxStridedBwdArgs& a,
                                hipStream_t s) {
-  if (p.team == 1 || (p.team > 1 && a.team_slot != nullptr)) {
+  if (p.team_size() == 1 || (p.team_size() > 1 && a.team_slot != nullptr)) {
     const bool ok = launch_strided_team<true, elems_per_pack<TG>::value>(
-        p, a.outer, a.D, a.inner, a.team_slot != nullptr, [&](auto v, const StridedTeamShape& sh, dim3 grid) {
+        p, a.outer, a.D, a.inner, [&](auto v, const StridedTeamShape& sh, dim3 grid) {
           hipLaunchKernelGGL((softmax_strided_team_bwd_kernel<TG, TO, decltype(v)::value>), grid,
                              dim3(kTeamBlock), 0, s, (const TG*)a.grad, (const TG*)a.y, (TO*)a.gi,
                              sh, a.flags, (TeamColumns*)a.team_slot, a.team_id, a.team_wait_ticks);
