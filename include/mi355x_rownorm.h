@@ -363,7 +363,8 @@ int mi355x_softmax_strided_plan(int backward, int64_t outer, int64_t dim_size, i
  * that bound, and reads the whole strip itself if it runs out.  They need an output that overlaps no
  * input; such a call in place, on a stream under capture, or on a stream beyond the eight takes
  * mi355x_softmax_strided_plan's layout.  A team of one waits for nobody and has none of these
- * conditions. */
+ * conditions.  Reported is the call whose output has the input's type: a float16 forward with a float32
+ * output keeps to teams of which a compute unit holds two (packs_per_lane <= 16). */
 int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_size, int64_t inner,
                                      rownorm_dtype dtype, rownorm_plan* out);
 

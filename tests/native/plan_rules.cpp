@@ -32,9 +32,9 @@ void rule_strided_plan(int backward, int64_t outer, int64_t D, int64_t inner, in
 
 // the same call's teams of workgroups that have a compute unit each: workgroups a team, packs a lane, lanes
 // along inner, workgroups launched
-void rule_strided_large(int backward, int64_t outer, int64_t D, int64_t inner, int esize, int64_t out[4]) {
+void rule_strided_large(int backward, int64_t outer, int64_t D, int64_t inner, int esize, int64_t out[4], int widened) {
   StridedPlan p;
-  make_strided_plan(backward != 0, outer, D, inner, esize, 256, Override{}, &p);
+  make_strided_plan(backward != 0, outer, D, inner, esize, 256, Override{}, &p, widened != 0);
   out[0] = p.large_team, out[1] = p.large_v, out[2] = 1 << p.large_tx_log2, out[3] = p.large_grid;
 }
 

@@ -8,9 +8,9 @@ from test_plan_rules import _strided, rules  # noqa: F401
 i64 = ctypes.c_int64
 
 
-def _large(rules, backward, outer, D, inner, esize):  # noqa: F811
+def _large(rules, backward, outer, D, inner, esize, widened=0):  # noqa: F811
     out = (i64 * 4)()
-    rules.rule_strided_large(backward, i64(outer), i64(D), i64(inner), esize, out)
+    rules.rule_strided_large(backward, i64(outer), i64(D), i64(inner), esize, out, widened)
     return dict(zip(("team", "v", "tx", "grid"), list(out)))
 
 
@@ -42,3 +42,13 @@ def test_large_teams(rules):  # noqa: F811
     # where two a compute unit measured faster
     for a in ((0, 50, 954, 920, 2), (0, 6, 820, 10296, 2), (0, 4, 3419, 3912, 2), (1, 36, 2844, 384, 2), (0, 8, 2048, 2048, 2)):
         assert _large(rules, *a)["team"] == 0, a
+
+
+def test_not_for_an_output_wider_than_the_input(rules):  # noqa: F811
+    """A float16 forward with a float32 output is slower on them at every size."""
+    rng, plain = random.Random(8), 0
+    for _ in range(3000):
+        a = (0, rng.randint(1, 64), int(2 ** rng.uniform(8, 15)), 8 * int(2 ** rng.uniform(1, 12)), 2)
+        plain += _large(rules, *a)["team"] > 0
+        assert _large(rules, *a, widened=1)["team"] == 0, a
+    assert plain > 300

@@ -883,7 +883,7 @@ int mi355x_softmax_strided_fwd(const void* x, void* y, int64_t outer, int64_t di
   if (!x || !y) return ROWNORM_ERR_NULL;
   StridedPlan plan;
   if (int e = make_strided_plan(false, outer, dim_size, inner, esize_of(id), current_num_cus(),
-                                g_override[ROWNORM_OP_SOFTMAX_STRIDED_FWD], &plan))
+                                g_override[ROWNORM_OP_SOFTMAX_STRIDED_FWD], &plan, od != id))
     return e;
   SoftmaxStridedFwdArgs a{x, y, outer, (int)dim_size, (int)inner, flags};
   hipStream_t s = (hipStream_t)stream;

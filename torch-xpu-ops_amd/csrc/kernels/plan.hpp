@@ -1469,9 +1469,13 @@ inline StridedTeam strided_team(bool backward, int64_t outer, int64_t D, int64_t
 // from teams of 24 on (forward of [4, 3419, 3912], 16 members, 58.5 / 67.9, of [2, 13960, 1272], 44, 57.0
 // / 47.6).  A backward whose strips then need no exchange and make one round gains whatever the teams
 // were ([6, 323, 10280] 31.8 / 29.3, fp32 [4, 325, 7136] 24.7 / 18.4).
+// Never a float16 forward with a float32 output (widened): its stores are twice the bytes of its loads and its
+// exponentials are the long ones, and with one workgroup a compute unit neither runs under the other's reads
+// (560 shapes of 20 to 600 MB, 1.14 times the time: [59, 3360, 192] 73 / 113, [6, 5912, 1536] 100 / 143, [2,
+// 13179, 6336] 320 / 389).
 inline StridedTeam strided_large_team(bool backward, int64_t outer, int64_t D, int64_t packs, int esize,
-                                      const StridedTeam& t, int num_cus) {
-  if (t.team == 0 || t.rounds < 2) return StridedTeam{};
+                                      const StridedTeam& t, int num_cus, bool widened) {
+  if (t.team == 0 || t.rounds < 2 || widened) return StridedTeam{};
   const StridedTeam l = strided_team_of(backward, outer, D, packs, esize,
                                         packs > kStridedTeamTx ? kStridedTeamWideTx : kStridedTeamTx, num_cus, true);
   if (l.team == 0 || l.rounds >= t.rounds || 8 * l.rounds * l.v > 17 * t.rounds * t.v) return StridedTeam{};
@@ -1516,8 +1520,9 @@ inline bool strided_team_beats_tile(bool backward, int64_t outer, int64_t D, int
 // Override: G = lanes along inner (power of two 1..64; -1 forces the multi-pass
 // kernel, and then V = 1 keeps all D rows of a tile on one workgroup, V > 1 cuts
 // them into that many chunks), V = packs per lane.  Returns 0 or -5.
+// widened: the output's elements are wider than the input's.
 inline int make_strided_plan(bool backward, int64_t outer, int64_t D, int64_t inner, int esize,
-                             int num_cus, const Override& ov, StridedPlan* out) {
+                             int num_cus, const Override& ov, StridedPlan* out, bool widened = false) {
   StridedPlan p;
   const int E = 16 / esize;
   const int64_t packs = (inner + E - 1) / E;
@@ -1608,7 +1613,7 @@ inline int make_strided_plan(bool backward, int64_t outer, int64_t D, int64_t in
       p.team_v = t.v;
       p.team_tx_log2 = log2_of_pow2(t.tx);
       p.team_grid = t.grid;
-      const StridedTeam l = strided_large_team(backward, outer, D, packs, esize, t, num_cus);
+      const StridedTeam l = strided_large_team(backward, outer, D, packs, esize, t, num_cus, widened);
       p.large_team = l.team;
       p.large_v = l.v;
       p.large_tx_log2 = log2_of_pow2(l.tx);

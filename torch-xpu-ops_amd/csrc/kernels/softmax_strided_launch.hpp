@@ -22,15 +22,19 @@ bool launch_strided_team_v(int v, Go go) {
     return launch_strided_team_v<BACKWARD, LARGE, I + 1>(v, go);
   return false;
 }
-template <bool BACKWARD, int E, class Go>
+// (LARGE: the instances with a compute unit a workgroup are built, see strided_large_team())
+template <bool BACKWARD, int E, bool LARGE, class Go>
 bool launch_strided_team(const StridedPlan& p, int64_t outer, int D, int inner, Go go) {
   const bool large = p.large_team > 0;
   const int tx_log2 = large ? p.large_tx_log2 : p.team_tx_log2;
   const int64_t xtiles = (inner / E + (1 << tx_log2) - 1) >> tx_log2;
   const StridedTeamShape sh{outer * xtiles, xtiles, D, inner, tx_log2, large ? p.large_team : p.team};
   const dim3 grid((unsigned)(large ? p.large_grid : p.team_grid));
-  if (large)
-    return launch_strided_team_v<BACKWARD, true>(p.large_v, [&](auto v) { go(v, sh, grid); });
+  if (large) {
+    if constexpr (LARGE)
+      return launch_strided_team_v<BACKWARD, true>(p.large_v, [&](auto v) { go(v, sh, grid); });
+    return false;
+  }
   return launch_strided_team_v<BACKWARD, false>(p.team_v, [&](auto v) { go(v, sh, grid); });
 }
 
@@ -60,7 +64,7 @@ template <class TI, class TO>
 int launch_softmax_strided_fwd(const StridedPlan& p, const SoftmaxStridedFwdArgs& a,
                                hipStream_t s) {
   if (p.team_size() == 1 || (p.team_size() > 1 && a.team_slot != nullptr)) {
-    const bool ok = launch_strided_team<false, elems_per_pack<TI>::value>(
+    const bool ok = launch_strided_team<false, elems_per_pack<TI>::value, sizeof(TO) <= sizeof(TI)>(
         p, a.outer, a.D, a.inner, [&](auto v, const StridedTeamShape& sh, dim3 grid) {
           hipLaunchKernelGGL((softmax_strided_team_fwd_kernel<TI, TO, decltype(v)::value>), grid,
                              dim3(kTeamBlock), 0, s, (const TI*)a.x, (TO*)a.y, sh, a.flags,
@@ -124,7 +128,7 @@ template <class TG, class TO>
 int launch_softmax_strided_bwd(const StridedPlan& p, const SoftmaxStridedBwdArgs& a,
                                hipStream_t s) {
   if (p.team_size() == 1 || (p.team_size() > 1 && a.team_slot != nullptr)) {
-    const bool ok = launch_strided_team<true, elems_per_pack<TG>::value>(
+    const bool ok = launch_strided_team<true, elems_per_pack<TG>::value, true>(
         p, a.outer, a.D, a.inner, [&](auto v, const StridedTeamShape& sh, dim3 grid) {
           hipLaunchKernelGGL((softmax_strided_team_bwd_kernel<TG, TO, decltype(v)::value>), grid,
                              dim3(kTeamBlock), 0, s, (const TG*)a.grad, (const TG*)a.y, (TO*)a.gi,
