@@ -42,6 +42,10 @@ def test_large_teams(rules):  # noqa: F811
     # where two a compute unit measured faster
     for a in ((0, 50, 954, 920, 2), (0, 6, 820, 10296, 2), (0, 4, 3419, 3912, 2), (1, 36, 2844, 384, 2), (0, 8, 2048, 2048, 2)):
         assert _large(rules, *a)["team"] == 0, a
+    # strips no wider than the small teams', in a float32 forward also rows of 16 packs at most
+    for a in ((0, 48, 3983, 592, 2), (0, 18, 4088, 2736, 2), (0, 47, 3854, 472, 4), (1, 14, 3068, 1336, 2), (1, 45, 3068, 488, 4),
+              (0, 34, 12457, 60, 4), (0, 62, 14919, 56, 4)):
+        assert _large(rules, *a)["team"] == 0, a
 
 
 def test_not_for_an_output_wider_than_the_input(rules):  # noqa: F811

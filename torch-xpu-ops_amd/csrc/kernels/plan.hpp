@@ -1363,9 +1363,9 @@ inline int log2_of_pow2(int v) {
   return l;
 }
 
-// Strips of tx packs held by teams (large: on workgroups that have a compute unit each): as few workgroups a strip as hold its D rows, as many teams as
-// strips and compute units allow, evened out over the rounds; then a strip is spread over the
-// workgroups its team can have.
+// Strips of tx packs held by teams (large: on workgroups that have a compute unit each): as few workgroups
+// a strip as hold its D rows, as many teams as strips and compute units allow, evened out over the rounds;
+// then a strip is spread over the workgroups its team can have.
 struct StridedTeam {
   int team = 0, v = 0, tx = 0;
   bool capped = false;  // there were workgroups for a larger team
@@ -1465,10 +1465,17 @@ inline StridedTeam strided_team(bool backward, int64_t outer, int64_t D, int64_t
 // of step do as well as fewer rounds (us, two a compute unit / one: bf16 forward of [1, 8192, 8192]
 // 70.5 / 59.1, [1, 12899, 3872] 58.4 / 50.1, but [50, 954, 920], teams of 5, 50.5 / 59.4 and [6, 820,
 // 10296], of 4, 58.3 / 61.1; backward of [1, 8192, 8192] 103.7 / 82.9, [12, 9602, 200] 46.2 / 30.0,
-// [92, 2206, 256] 66.2 / 60.5, but [36, 2844, 384] with 4/3 of the packs 48.1 / 51.5).  Rows of an odd number of packs, whose 512-byte pieces start off 32 bytes, gain
-// from teams of 24 on (forward of [4, 3419, 3912], 16 members, 58.5 / 67.9, of [2, 13960, 1272], 44, 57.0
-// / 47.6).  A backward whose strips then need no exchange and make one round gains whatever the teams
-// were ([6, 323, 10280] 31.8 / 29.3, fp32 [4, 325, 7136] 24.7 / 18.4).
+// [92, 2206, 256] 66.2 / 60.5, but [36, 2844, 384] with 4/3 of the packs 48.1 / 51.5).  Rows of an odd
+// number of packs, whose 512-byte pieces start off 32 bytes, gain from teams of 24 on (forward of [4,
+// 3419, 3912], 16 members, 58.5 / 67.9, of [2, 13960, 1272], 44, 57.0 / 47.6).  A backward whose strips
+// then need no exchange and make one round gains whatever the teams were ([6, 323, 10280] 31.8 / 29.3,
+// fp32 [4, 325, 7136] 24.7 / 18.4).
+// Part of the gain is the wider strip, 32 packs for 16, half as many strips to exchange.  Where the small
+// teams have strips of 32 packs as well there is none in the forward (560 shapes of 20 to 600 MB each: bf16
+// 0.97 of the time, a quarter of them slower: [48, 3983, 592] 126 / 149, [18, 4088, 2736] 219 / 239; fp32
+// 1.03: [47, 3854, 472] 189 / 218), and in the backward only from eight members on (below: bf16 [14, 3068,
+// 1336] 85 / 93, fp32 [45, 3068, 488] 177 / 197).  Nor in a float32 forward of rows of 16 packs at most, whose
+// strips stay as they are ([34, 12457, 60] 52 / 59, [62, 14919, 56] 112 / 123).
 // Never a float16 forward with a float32 output (widened): its stores are twice the bytes of its loads and its
 // exponentials are the long ones, and with one workgroup a compute unit neither runs under the other's reads
 // (560 shapes of 20 to 600 MB, 1.14 times the time: [59, 3360, 192] 73 / 113, [6, 5912, 1536] 100 / 143, [2,
@@ -1480,6 +1487,8 @@ inline StridedTeam strided_large_team(bool backward, int64_t outer, int64_t D, i
                                         packs > kStridedTeamTx ? kStridedTeamWideTx : kStridedTeamTx, num_cus, true);
   if (l.team == 0 || l.rounds >= t.rounds || 8 * l.rounds * l.v > 17 * t.rounds * t.v) return StridedTeam{};
   if (l.team == 1) return backward && l.rounds == 1 ? l : StridedTeam{};
+  if (t.tx > kStridedTeamTx && (!backward || l.team < 8)) return StridedTeam{};
+  if (!backward && esize == 4 && packs <= kStridedTeamTx) return StridedTeam{};
   return t.team >= (packs % 2 == 0 ? 12 : 24) ? l : StridedTeam{};
 }
 
