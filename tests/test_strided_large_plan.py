@@ -46,6 +46,9 @@ def test_large_teams(rules):  # noqa: F811
     for a in ((0, 48, 3983, 592, 2), (0, 18, 4088, 2736, 2), (0, 47, 3854, 472, 4), (1, 14, 3068, 1336, 2), (1, 45, 3068, 488, 4),
               (0, 34, 12457, 60, 4), (0, 62, 14919, 56, 4)):
         assert _large(rules, *a)["team"] == 0, a
+    # forward rows of whole lines, several rounds
+    for a in ((0, 62, 6587, 256, 2), (0, 4, 9431, 2304, 2), (0, 40, 10726, 128, 4)):
+        assert _large(rules, *a)["team"] == 0, a
 
 
 def test_not_for_an_output_wider_than_the_input(rules):  # noqa: F811

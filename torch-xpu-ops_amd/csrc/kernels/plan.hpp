@@ -1476,6 +1476,10 @@ inline StridedTeam strided_team(bool backward, int64_t outer, int64_t D, int64_t
 // 1.03: [47, 3854, 472] 189 / 218), and in the backward only from eight members on (below: bf16 [14, 3068,
 // 1336] 85 / 93, fp32 [45, 3068, 488] 177 / 197).  Nor in a float32 forward of rows of 16 packs at most, whose
 // strips stay as they are ([34, 12457, 60] 52 / 59, [62, 14919, 56] 112 / 123).
+// The other part is the lines of 128 bytes that neighbouring strips of other rows share, and that are read
+// twice.  Forward rows of whole lines share none: they take large teams for a single round only, with no other
+// to be out of step with (bf16 0.90 of the time, fp32 0.95; of several rounds 1.02 and 1.00: bf16 [62, 6587, 256]
+// 90 / 99, [4, 9431, 2304] 80 / 84, fp32 [40, 10726, 128] 94 / 107).
 // Never a float16 forward with a float32 output (widened): its stores are twice the bytes of its loads and its
 // exponentials are the long ones, and with one workgroup a compute unit neither runs under the other's reads
 // (560 shapes of 20 to 600 MB, 1.14 times the time: [59, 3360, 192] 73 / 113, [6, 5912, 1536] 100 / 143, [2,
@@ -1489,6 +1493,7 @@ inline StridedTeam strided_large_team(bool backward, int64_t outer, int64_t D, i
   if (l.team == 1) return backward && l.rounds == 1 ? l : StridedTeam{};
   if (t.tx > kStridedTeamTx && (!backward || l.team < 8)) return StridedTeam{};
   if (!backward && esize == 4 && packs <= kStridedTeamTx) return StridedTeam{};
+  if (!backward && packs % 8 == 0 && l.rounds > 1) return StridedTeam{};
   return t.team >= (packs % 2 == 0 ? 12 : 24) ? l : StridedTeam{};
 }
 
