@@ -41,3 +41,6 @@ def test_rounds_of_the_same_rows(rules):  # noqa: F811
     assert _team(rules, 64, 115200)[2] == 64 and _team(rules, 512, 401408) == (7, 14, 73)
     assert _team(rules, 389, 188800)[2] == 170 and _team(rules, 148, 291328)[2] == 102
     assert _team(rules, 71, 1284480)[2] == 25
+    # packs that do not go down as far as the last round was short, weights an XCD's L2 does not hold
+    assert _team(rules, 112, 686560)[2] == 46 and _team(rules, 241, 133440, wide=1)[2] == 170
+    assert _team(rules, 20, 2036640, wide=1)[2] == 16 and _team(rules, 35, 2034192, wide=1)[2] == 16

@@ -1108,20 +1108,27 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
         return (strides + most - 1) / most;
       };
       // Two or three rounds, the last of them not full: as many teams as give every round the same rows, each
-      // row over more workgroups (norm forward, bf16 LayerNorm: [140, 216576] 128 teams of 4 -> 70 of 7 35.3 ->
-      // 28.5 us, [33, 1103488] 44.8 -> 36.5, [256, 188416] 52.3 -> 42.5, [358, 163840] 58.5 -> 52.2, [64, 1345664]
-      // 92.0 -> 80.8, RMSNorm [100, 536704] 47.0 -> 42.3).  The other sides of the lines: a row that would not
-      // spread further ([389, 188800] 66.9 -> 74.5); four rounds or more, where the last leaves little idle
-      // ([216, 468864] 84.5 -> 89.0, [110, 1526656] 143 -> 181); less than 15 of 16 workgroups used in every
-      // round where the last one was a quarter full or more ([148, 291328] 39.4 -> 44.1); an odd team, whose
-      // chunks of the weights every XCD reads, where gamma and beta fill three quarters of its L2 ([71, 1284480]
-      // teams of 20 -> 21 79.7 -> 94.4, [65, 1213312] 19 -> 23 76.5 -> 82.9).
+      // row over more workgroups, where that is less work in a row.  A last round of at most half the teams
+      // takes about three tenths of a round's time (two tenths beside float32 weights of 16-bit rows), its
+      // workgroups having a compute unit's bandwidth each; a fuller one nine (norm forward, bf16 LayerNorm:
+      // [140, 216576] 128 teams of 4 -> 70 of 7 35.3 -> 28.5 us, [33, 1103488] 44.8 -> 36.5, [256, 188416] 52.3
+      // -> 42.5, [358, 163840] 58.5 -> 52.2, [64, 1345664] 92.0 -> 80.8; 0.90 of the time over 900 shapes that the
+      // rule takes, at worst 1.07).  The other sides of the lines: more packs than that ([389, 188800] 66.9
+      // -> 74.5, [112, 686560] 3 x 16 -> 3 x 13 packs 68 -> 77, fp16 with fp32 weights [241, 133440] 35 -> 40); four
+      // rounds or more, where the last leaves little idle ([216, 468864] 84.5 -> 89.0, [110, 1526656] 143 -> 181);
+      // less than 15 of 16 workgroups used in every round where the last one was a quarter full or more ([148,
+      // 291328] 39.4 -> 44.1).  And the weights: workgroup b runs on XCD b % 8, which so meets every gcd(team,
+      // 8)-th chunk of gamma and beta; beyond three quarters of its L2 they come from further out every round
+      // ([71, 1284480] teams of 20 -> 21 79.7 -> 94.4; fp16 with fp32 weights [20, 2036640] 32 -> 50 41 -> 62).
       const int64_t rounds = (M + teams - 1) / teams;
       if (oc == OC_NORM_FWD && (rounds == 2 || rounds == 3)) {
         const int64_t even = (M + rounds - 1) / rounds, ve = packs_a_lane(even), members = (strides + ve - 1) / ve;
-        const bool fills = 16 * even * members >= 15 * cus || 4 * (M - (rounds - 1) * teams) < teams;
-        const bool in_l2 = members % 2 == 0 || 2 * (wide_weights ? 32 : 16) * packs <= (3 << 20);
-        if (even >= kTeamMinTeams && ve < packs_a_lane(teams) && fills && in_l2) teams = even;
+        const int64_t last = M - (rounds - 1) * teams, tenths = 2 * last > teams ? 9 : wide_weights ? 2 : 3;
+        const bool less = 10 * rounds * ve <= packs_a_lane(teams) * (10 * (rounds - 1) + tenths);
+        const bool fills = 16 * even * members >= 15 * cus || 4 * last < teams;
+        const int64_t shared = members % 8 == 0 ? 8 : members % 4 == 0 ? 4 : members % 2 == 0 ? 2 : 1;
+        const int64_t weights = (layer_norm || shared == 1 ? 2 : 1) * (wide_weights ? 32 : 16) * packs;
+        if (even >= kTeamMinTeams && less && fills && weights <= shared * (3 << 20)) teams = even;
       }
       const int64_t v = packs_a_lane(teams);
       const int64_t team = (strides + v - 1) / v;
