@@ -92,6 +92,23 @@ def test_group_norm_backward_teams(rules):
         assert _gn_team(rules, N, C, side, esize)["ahead"], (N, C, side)
 
 
+def test_group_norm_backward_teams_that_sum_their_channels(rules):
+    """Whole groups a team make no more rounds than slabs dealt out one by one, and of no more teams: a last round
+    of at most half the teams keeps the second stage."""
+    i64 = ctypes.c_int64
+    f = lambda N, groups, teams: bool(rules.rule_gn_team_sums(i64(N * groups), i64(groups), i64(teams)))  # noqa: E731
+    for groups in (1, 4, 8, 12, 32, 64):
+        for N in range(1, 9):
+            for teams in range(1, 513):
+                rounds = -(-N * groups // teams)
+                last = N * groups - (rounds - 1) * teams
+                if f(N, groups, teams):
+                    assert teams <= groups and -(-groups // teams) * N <= rounds
+                    assert N == 1 or 2 * last > teams
+    assert f(1, 32, 25) and f(2, 32, 32) and f(3, 32, 32)
+    assert not f(2, 64, 25) and not f(2, 8, 5) and not f(2, 64, 42) and not f(4, 32, 64)
+
+
 def test_every_stream_has_its_own_exchange_memory(rules):
     """Slots are handed out by stream, whatever the order and the number of calls: one stream always gets
     the same, two never share one, a stream beyond the last slot gets none; also from several threads."""

@@ -1299,12 +1299,15 @@ inline GnBwdTeam gn_bwd_team(int64_t rows, int64_t D, int64_t cp, int esize, int
 }
 
 // Whether the teams of gn_bwd_team_kernel write dgamma / dbeta themselves: a team then takes whole groups, all
-// samples of one after the other, which must not make more rounds than slabs dealt out one by one.  (The
-// kernel that has the next slab on its way lost what it gained: [4, 256, 128, 128] 24.0 -> 25.3 us.)
+// samples of one after the other, which must not make more rounds than slabs dealt out one by one, nor rounds
+// of more teams: a last round of at most half the teams is a cheap one, and whole groups put all of a group's
+// samples behind it (fp16 [2, 128, 560, 560] in 64 groups, 25 teams, 107 -> 116 us, [2, 256, 296, 296] in 8, 5
+// teams, 69 -> 73, bf16 [2, 256, 304, 304] in 64, 42 teams, 66 -> 70; the shapes taken 0.90 to 1.005 of the time).
+// (The kernel that has the next slab on its way lost what it gained: [4, 256, 128, 128] 24.0 -> 25.3 us.)
 inline bool gn_team_sums_columns(int64_t rows, int64_t groups, int64_t teams) {
-  const int64_t samples = rows / groups;
-  return teams <= groups && samples <= 0xffffff &&
-         (groups + teams - 1) / teams * samples <= (rows + teams - 1) / teams;
+  const int64_t samples = rows / groups, rounds = (rows + teams - 1) / teams;
+  if (teams > groups || samples > 0xffffff || (groups + teams - 1) / teams * samples > rounds) return false;
+  return samples == 1 || 2 * (rows - (rounds - 1) * teams) > teams;
 }
 
 // ---- softmax over a non-innermost dimension: [outer, D, inner] ----------------
