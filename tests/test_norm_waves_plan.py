@@ -58,3 +58,14 @@ def test_rows_that_keep_their_layout(rules):  # noqa: F811
     assert _layout(rules, 1, 8192, 509, 2)["waves"] == 0 and _layout(rules, 0, 8192, 1021, 4)["waves"] == 0
     assert _layout(rules, 1, 8192, 4097, 2) == dict(waves=9, v=1, depth=3, threads=1024, slots=1, grid=256, partial=512)
     assert _layout(rules, 0, 8192, 4097, 2)["waves"] == 5
+
+
+def test_short_rows_need_many_of_them(rules):  # noqa: F811
+    """A ragged 16-bit backward whose row slots see a row or two each measured slower on whole wavefronts."""
+    taken = lambda M, N, ln: _layout(rules, 1, M, N, 2, ln)["waves"] > 0  # noqa: E731
+    for ln in (0, 1):
+        assert not taken(881, 739, ln) and not taken(1830, 869, ln) and not taken(2395, 547, ln) and taken(3100, 850, ln)
+        assert not taken(910, 1807, ln) and taken(1100, 1807, ln)
+    assert not taken(1997, 1317, 0) and taken(2100, 1317, 0) and taken(600, 1317, 1)
+    assert not taken(538, 2249, 0) and taken(800, 2249, 0) and taken(600, 2201, 1)
+    assert not taken(412, 3791, 0) and taken(600, 3791, 0) and taken(300, 4097, 0)

@@ -668,6 +668,22 @@ constexpr int kWavesMax = 16;  // wavefronts a workgroup at most
 // in 16 bits, three in float32, beside a second set of sums)
 constexpr int kWavesFoldFloats = 8192;
 
+// Whether a ragged 16-bit backward call has rows enough for them: a workgroup of sixteen wavefronts holds
+// several short rows at a time, and where its slots see a row or two each there is nothing to have on its way,
+// while the general layout spreads the rows over up to four times as many workgroups.  us, general layout /
+// whole wavefronts: up to 128 packs (eight slots) fp16 LayerNorm [881, 739] 8.8 / 9.6, [1830, 869] 10.3 / 11.1,
+// bf16 RMSNorm [2395, 547] 10.3 / 11.0, from twelve rows a compute unit on [3100, 850] 13.5 / 13.0; up to 192 (five)
+// RMSNorm [1213, 1401] 9.6 / 10.6, fp32 weights [1997, 1317] 10.6 / 11.0, eight rows; up to 256 (four) LayerNorm
+// [910, 1807] 11.0 / 11.5, a row for every slot; beyond (three and two) RMSNorm [538, 2249] 9.5 / 10.1, [412, 3791]
+// 10.5 / 10.9, likewise.  The LayerNorm, which waits for two sums, gains with five, three and two slots whatever
+// the rows ([600, 2201] 12.6 / 10.3).
+inline bool norm_waves_bwd_rows(int64_t M, int64_t packs, bool layer_norm, int num_cus) {
+  const int64_t waves = (packs + 63) / 64;
+  if (waves == 2) return M >= 12 * (int64_t)num_cus;
+  if (waves != 4 && layer_norm) return true;
+  return M >= (waves == 3 ? 8 : 16 / waves) * num_cus;
+}
+
 // Which rows take them.  One pack a lane and three rows in registers in 16 bits, with one workgroup of up to
 // sixteen wavefronts a compute unit: what is idle of a row's slots is less than a wavefront, and every row
 // slot has two rows on their way.  Beyond 1024 packs the backward holds two packs a lane and two rows (ragged
@@ -692,7 +708,8 @@ inline WavesLayout norm_waves_layout(bool backward, int esize, int64_t M, int64_
   int which = -1;
   if (esize == 2) {
     if (backward) {
-      if (whole_packs ? packs > 256 && packs <= 1024 && (packs > 512 || M >= 8192) : packs > 64 && packs <= 1024)
+      if (whole_packs ? packs > 256 && packs <= 1024 && (packs > 512 || M >= 8192)
+                      : packs > 64 && packs <= 1024 && norm_waves_bwd_rows(M, packs, layer_norm, num_cus))
         which = 0;
       else if (!whole_packs && packs > 1024 && packs <= 1536)
         which = 1;
