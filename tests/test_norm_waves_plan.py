@@ -69,3 +69,17 @@ def test_short_rows_need_many_of_them(rules):  # noqa: F811
     assert not taken(1997, 1317, 0) and taken(2100, 1317, 0) and taken(600, 1317, 1)
     assert not taken(538, 2249, 0) and taken(800, 2249, 0) and taken(600, 2201, 1)
     assert not taken(412, 3791, 0) and taken(600, 3791, 0) and taken(300, 4097, 0)
+
+
+def test_whole_packs_of_large_tensors(rules):  # noqa: F811
+    """Backward rows of 513 to 768 whole packs beyond 50 million elements, and LayerNorm rows just below 512 beyond
+    200 million, keep their layout, except LayerNorm rows that leave half of its lanes idle."""
+    taken = lambda M, N, ln: _layout(rules, 1, M, N, 2, ln)["waves"] > 0  # noqa: E731
+    for ln in (0, 1):
+        for N in (4616, 4968, 5288, 5448, 6136):
+            assert taken(8000, N, ln) and not taken(11000, N, ln) and not taken(100000, N, ln)
+        for N in (6152, 7000, 8184):
+            assert taken(300, N, ln) and taken(60000, N, ln)
+        assert taken(60000, 3200, ln) and not taken(8191, 3200, ln)
+    assert taken(100000, 4184, 1) and not taken(100000, 4184, 0)
+    assert taken(40000, 4072, 1) and not taken(104347, 4072, 1) and taken(104347, 4072, 0)

@@ -684,6 +684,20 @@ inline bool norm_waves_bwd_rows(int64_t M, int64_t packs, bool layer_norm, int n
   return M >= (waves == 3 ? 8 : 16 / waves) * num_cus;
 }
 
+// Whether a 16-bit backward call of whole packs, 257 to 1024 of them, takes them (us, general layout / whole
+// wavefronts).  From 8192 rows on below 513 packs, see below, the LayerNorm beyond 448 up to 200 million elements
+// (fp32 weights [40000, 3968] 165 / 163, [104347, 4072] 455 / 478).  Of 513 to 768 packs, where nine to twelve
+// wavefronts work of the sixteen that a compute unit's one workgroup has room for, and the general layout has its
+// three packs on 256 lanes, calls of up to 50 million elements: beyond, memory is the bound and more wavefronts
+// keep it busier (bf16 LayerNorm [8192, 5448] 54 / 53, [36503, 5360] 201 / 215, [52273, 5288] 291 / 320, RMSNorm with
+// fp32 weights [104044, 5160] 565 / 636); but not the LayerNorm up to 544, which leaves nearly half of those
+// lanes idle ([52000, 4184] 238 / 210).
+inline bool norm_waves_bwd_whole(int64_t M, int64_t N, int64_t packs, bool layer_norm) {
+  const int64_t n = M * N;
+  if (packs <= 512) return M >= 8192 && !(layer_norm && packs > 448 && n > 200000000);
+  return packs > 768 || n <= 50000000 || (layer_norm && packs <= 544);
+}
+
 // Which rows take them.  One pack a lane and three rows in registers in 16 bits, with one workgroup of up to
 // sixteen wavefronts a compute unit: what is idle of a row's slots is less than a wavefront, and every row
 // slot has two rows on their way.  Beyond 1024 packs the backward holds two packs a lane and two rows (ragged
@@ -708,7 +722,7 @@ inline WavesLayout norm_waves_layout(bool backward, int esize, int64_t M, int64_
   int which = -1;
   if (esize == 2) {
     if (backward) {
-      if (whole_packs ? packs > 256 && packs <= 1024 && (packs > 512 || M >= 8192)
+      if (whole_packs ? packs > 256 && packs <= 1024 && norm_waves_bwd_whole(M, N, packs, layer_norm)
                       : packs > 64 && packs <= 1024 && norm_waves_bwd_rows(M, packs, layer_norm, num_cus))
         which = 0;
       else if (!whole_packs && packs > 1024 && packs <= 1536)
