@@ -21,7 +21,7 @@ def test_rows_on_whole_wavefronts(rules):  # noqa: F811
     sums fit the memory they are folded through and the caller's partial rows, every workgroup has a row."""
     rng = random.Random(11)
     taken = {k: 0 for k in INSTANCES}
-    for _ in range(20000):
+    for _ in range(60000):
         M = int(2 ** rng.uniform(6, 18))
         N = int(2 ** rng.uniform(6, 14.2))
         N = N // 8 * 8 if rng.random() < 0.3 else N
@@ -83,3 +83,17 @@ def test_whole_packs_of_large_tensors(rules):  # noqa: F811
         assert taken(60000, 3200, ln) and not taken(8191, 3200, ln)
     assert taken(100000, 4184, 1) and not taken(100000, 4184, 0)
     assert taken(40000, 4072, 1) and not taken(104347, 4072, 1) and taken(104347, 4072, 0)
+
+
+def test_float_rows(rules):  # noqa: F811
+    """Ragged float32 rows keep their layout in tensors far beyond the caches, and in the backward where a compute
+    unit would get one long row or two."""
+    fwd = lambda M, N: _layout(rules, 0, M, N, 4)["waves"] > 0  # noqa: E731
+    for N in (1027, 2051, 2999, 4095):
+        assert fwd(12000, N) and not fwd(70000, N) and not fwd(4000, N)
+    assert fwd(9000, 1999) and not fwd(13000, 1999) and fwd(60000, 4097) and fwd(60000, 4607)
+    bwd = lambda M, N, ln: _layout(rules, 1, M, N, 4, ln)["waves"] > 0  # noqa: E731
+    for ln in (0, 1):
+        assert bwd(65000, 3071, ln) and bwd(24000, 4097, ln) and not bwd(25000, 4097, ln) and not bwd(55957, 3777, ln)
+        assert bwd(300, 6143, ln) and not bwd(300, 6145, ln) and bwd(400, 6145, ln)
+        assert not bwd(485, 8743, ln) and bwd(700, 8743, ln) and not bwd(27414, 8269, ln)

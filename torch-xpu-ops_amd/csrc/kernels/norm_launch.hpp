@@ -108,8 +108,10 @@ bool launch_norm_fwd_flat(FlatLayout f, const NormFwdArgs& a, hipStream_t stream
 template <class T, bool BACKWARD, class Go>
 inline bool launch_norm_waves(const WavesLayout& l, Go go) {
   constexpr auto& list = [] () -> auto& {
-    if constexpr (sizeof(T) == 2) return BACKWARD ? kWavesBwd16 : kWavesFwd16;
-    else return BACKWARD ? kWavesBwd32 : kWavesFwd32;
+    if constexpr (sizeof(T) == 2 && BACKWARD) return kWavesBwd16;
+    else if constexpr (sizeof(T) == 2) return kWavesFwd16;
+    else if constexpr (BACKWARD) return kWavesBwd32;
+    else return kWavesFwd32;
   }();
   auto at = [&](auto i) {
     constexpr WavesInstance in = list[decltype(i)::value];
@@ -118,7 +120,9 @@ inline bool launch_norm_waves(const WavesLayout& l, Go go) {
        std::integral_constant<int, in.threads>{});
     return true;
   };
-  return at(std::integral_constant<int, 0>{}) || at(std::integral_constant<int, 1>{});
+  if (at(std::integral_constant<int, 0>{})) return true;
+  if constexpr (sizeof(list) / sizeof(list[0]) > 1) return at(std::integral_constant<int, 1>{});
+  return false;
 }
 
 template <class T, class WT, bool RMS, class TY, bool ADD>

@@ -660,7 +660,7 @@ struct WavesInstance {
   int v, depth, threads;
 };
 constexpr WavesInstance kWavesFwd16[] = {{1, 3, 1024}, {2, 3, 1024}};
-constexpr WavesInstance kWavesFwd32[] = {{3, 2, 512}, {3, 2, 512}};
+constexpr WavesInstance kWavesFwd32[] = {{3, 2, 512}};
 constexpr WavesInstance kWavesBwd16[] = {{1, 3, 1024}, {2, 2, 768}};
 constexpr WavesInstance kWavesBwd32[] = {{3, 3, 512}, {3, 2, 768}};
 constexpr int kWavesMax = 16;  // wavefronts a workgroup at most
@@ -698,6 +698,28 @@ inline bool norm_waves_bwd_whole(int64_t M, int64_t N, int64_t packs, bool layer
   return packs > 768 || n <= 50000000 || (layer_norm && packs <= 544);
 }
 
+// Whether a call on ragged float32 rows of more than 256 packs takes them (us, general layout / whole
+// wavefronts).  The forward is the LayerNorm's, from sixteen rows a compute unit on; beyond 60 million elements
+// memory is the bound, and four times as many small workgroups out of phase keep it busier ([37590, 4065]
+// 228 / 250, [91025, 2949] 388 / 424; up to there 0.78 to 0.98 of the time: [12000, 4097] 73 / 66); of 385 to 512
+// packs, which the general layout's 128 lanes hold without a gap, beyond 20 million ([47928, 1559] 116 / 125,
+// [8192, 1999] 22.6 / 21.2); not so from 1025 packs on, which leave a third of that layout idle.
+// The backward gains up to 100 million elements (0.75 to 0.97 of the time), and up to 768 packs beyond; with more,
+// there, the general layout's loads in several workgroups again ([55957, 3777] 483 / 504, [27414, 8269] 521 / 542).
+// Rows of more than 1536 packs, one at a time on a compute unit, need a round and a half of them, beyond 2048
+// packs two and a half: the general layout works on two at a time ([279, 8061] 21.0 / 21.8, [485, 8743] 25.6 / 27.4,
+// RMSNorm [259, 6521] 12.6 / 13.4; [700, 8743] 37.3 / 35.5).
+inline bool norm_waves_float_rows(bool backward, int64_t M, int64_t N, int64_t packs, bool layer_norm,
+                                  int num_cus) {
+  const int64_t n = M * N;
+  if (!backward) {
+    if (!layer_norm || M < 16 * (int64_t)num_cus) return false;
+    return packs > 1024 || n <= (packs > 384 && packs <= 512 ? 20000000 : 60000000);
+  }
+  if (packs > 1536 && 2 * M < (packs > 2048 ? 5 : 3) * (int64_t)num_cus) return false;
+  return packs <= 768 || n <= 100000000;
+}
+
 // Which rows take them.  One pack a lane and three rows in registers in 16 bits, with one workgroup of up to
 // sixteen wavefronts a compute unit: what is idle of a row's slots is less than a wavefront, and every row
 // slot has two rows on their way.  Beyond 1024 packs the backward holds two packs a lane and two rows (ragged
@@ -730,11 +752,9 @@ inline WavesLayout norm_waves_layout(bool backward, int esize, int64_t M, int64_
     } else if (!whole_packs && packs > (layer_norm ? 160 : 320) && packs <= 1024) {
       which = packs > 512 && packs <= 640 && M >= 16 * (int64_t)num_cus ? 1 : 0;
     }
-  } else if (!whole_packs && packs > 256) {
-    if (backward)
-      which = packs <= 1536 ? 0 : packs <= 2304 ? 1 : -1;
-    else if (layer_norm && M >= 16 * (int64_t)num_cus && packs <= 1152)
-      which = 0;
+  } else if (!whole_packs && packs > 256 && packs <= (backward ? 2304 : 1152) &&
+             norm_waves_float_rows(backward, M, N, packs, layer_norm, num_cus)) {
+    which = packs <= 1536 ? 0 : 1;
   }
   // (a row for every compute unit at least: fewer are as fast on either layout, and keep the bits they have in
   // common with the fused add, which has the general one -- 130 rows within 3 % of one another up to 8191)
