@@ -97,3 +97,17 @@ def test_float_rows(rules):  # noqa: F811
         assert bwd(65000, 3071, ln) and bwd(24000, 4097, ln) and not bwd(25000, 4097, ln) and not bwd(55957, 3777, ln)
         assert bwd(300, 6143, ln) and not bwd(300, 6145, ln) and bwd(400, 6145, ln)
         assert not bwd(485, 8743, ln) and bwd(700, 8743, ln) and not bwd(27414, 8269, ln)
+
+
+def test_forward_rows(rules):  # noqa: F811
+    """RMSNorm rows of 577 to 768 packs in calls of a middling number of rows, its longest rows, and LayerNorm rows
+    whose slots leave wavefronts idle in large tensors, keep their layout."""
+    taken = lambda M, N, ln, wide=0: _layout(rules, 0, M, N, 2, ln, wide)["waves"] > 0  # noqa: E731
+    for wide in (0, 1):
+        for N in (4617, 5001, 6143):
+            assert taken(1000, N, 0, wide) and not taken(1100, N, 0, wide) and not taken(8000, N, 0, wide)
+            assert taken(8192, N, 0, wide) and taken(4000, N, 1, wide)
+        assert taken(4000, 4603, 0, wide) and taken(4000, 6151, 0, wide)
+        assert taken(1000, 8001, 0, wide) and taken(30000, 8001, 0, wide) == (wide == 1) and taken(30000, 8001, 1, wide)
+        assert taken(68064, 2577, 1, wide) == (wide == 1) and taken(94118, 1293, 1, wide) == (wide == 1)
+        assert taken(30000, 1401, 1, wide) and taken(16821, 2669, 1, wide) and taken(100000, 2051, 1, wide)

@@ -720,6 +720,21 @@ inline bool norm_waves_float_rows(bool backward, int64_t M, int64_t N, int64_t p
   return packs <= 768 || n <= 100000000;
 }
 
+// Whether a ragged 16-bit forward call takes them (us, general layout / whole wavefronts).  The RMSNorm of 577 to
+// 768 packs, ten to twelve wavefronts of sixteen, not from four to 31 rows a compute unit ([4832, 4667] 19.3 / 21.3,
+// fp32 weights [2687, 5681] 13.8 / 14.8, but [600, 5001] 6.5 / 6.1 and [16384, 4801] 61 / 57), and that of more than
+// 896, whose window the general layout's 512 lanes hold without a gap, below four only, with fp32 weights always
+// ([21154, 7883] 121 / 129).  The LayerNorm with weights of the rows' type not beyond 60 million elements where row
+// slots leave wavefronts of a workgroup idle (161 to 192 and 321 to 384 packs: [30825, 2565] 66 / 72, [94118,
+// 1293] 103 / 110, but [16821, 2669] 45 / 40).
+inline bool norm_waves_fwd_rows(int64_t M, int64_t N, int64_t packs, bool layer_norm, bool wide_weights,
+                                int num_cus) {
+  if (layer_norm)
+    return wide_weights || M * N <= 60000000 || !(packs <= 192 || (packs > 320 && packs <= 384));
+  if (packs > 576 && packs <= 768) return M < 4 * (int64_t)num_cus || M >= 32 * (int64_t)num_cus;
+  return packs <= 896 || wide_weights || M < 4 * (int64_t)num_cus;
+}
+
 // Which rows take them.  One pack a lane and three rows in registers in 16 bits, with one workgroup of up to
 // sixteen wavefronts a compute unit: what is idle of a row's slots is less than a wavefront, and every row
 // slot has two rows on their way.  Beyond 1024 packs the backward holds two packs a lane and two rows (ragged
@@ -737,7 +752,7 @@ inline bool norm_waves_float_rows(bool backward, int64_t M, int64_t N, int64_t p
 // Forward rows of 513 to 640 packs would leave seven of sixteen wavefronts without a row: two packs a lane,
 // three row slots (4097 30.6 -> 27.9).
 inline WavesLayout norm_waves_layout(bool backward, int esize, int64_t M, int64_t N, bool whole_packs,
-                                     bool layer_norm, int64_t partial_rows, int num_cus) {
+                                     bool layer_norm, bool wide_weights, int64_t partial_rows, int num_cus) {
   WavesLayout l;
   const int E = 16 / esize;
   const int64_t packs = (N + E - 1) / E;
@@ -749,7 +764,8 @@ inline WavesLayout norm_waves_layout(bool backward, int esize, int64_t M, int64_
         which = 0;
       else if (!whole_packs && packs > 1024 && packs <= 1536)
         which = 1;
-    } else if (!whole_packs && packs > (layer_norm ? 160 : 320) && packs <= 1024) {
+    } else if (!whole_packs && packs > (layer_norm ? 160 : 320) && packs <= 1024 &&
+               norm_waves_fwd_rows(M, N, packs, layer_norm, wide_weights, num_cus)) {
       which = packs > 512 && packs <= 640 && M >= 16 * (int64_t)num_cus ? 1 : 0;
     }
   } else if (!whole_packs && packs > 256 && packs <= (backward ? 2304 : 1152) &&
@@ -1094,7 +1110,8 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
   if ((oc == OC_NORM_FWD || oc == OC_NORM_BWD) && p.resident && p.exact_depth == 0 && !fused_add &&
       !force_general && !p.forced && ov.bpc == 0 &&
       !(oc == OC_NORM_BWD && p.fast && norm_bwd_exact_index(esize, packs, M, layer_norm, wide_weights, false) >= 0))
-    p.waves = norm_waves_layout(oc == OC_NORM_BWD, esize, M, N, p.fast, layer_norm, p.partial_rows, num_cus);
+    p.waves = norm_waves_layout(oc == OC_NORM_BWD, esize, M, N, p.fast, layer_norm, wide_weights, p.partial_rows,
+                                num_cus);
   // Rows beyond the registers, and too few of them to give every compute unit a
   // workgroup (the regime of the reference's split-row kernels, Norm.h:632-812):
   // cut each row into chunks so that about four workgroups per compute unit
