@@ -379,12 +379,15 @@ int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_si
  * of packs) of at most 2048 16-bit / 1024 float32 elements, and on rows of up to
  * 12 whole packs that fit the reported layout badly, with 16-byte aligned
  * tensors and one dtype, run through LDS-staged kernels instead of the layout
- * reported here (a forced layout keeps the reported kernels).  The query
+ * reported here (a forced layout keeps the reported kernels); so do norm calls on ragged rows of such
+ * tensors, forwards of that length, backwards of up to 192 16-bit / 1024 float32 elements.  The query
  * describes the plain call: the fused residual add keeps 1024 lanes for 16-bit
  * rows of 16392..24576 elements and takes the multi-pass kernel beyond 12 packs a
  * lane (float32 LayerNorm: 10), and the masked softmax calls beyond 32 elements a
  * lane on 1024 lanes (rows of more than 32768 elements; a forced layout beyond
- * that is ROWNORM_ERR_OVERRIDE for a masked call). */
+ * that is ROWNORM_ERR_OVERRIDE for a masked call).
+ * Norm calls that mi355x_rownorm_waves_plan reports a layout for run on that one instead; the one
+ * reported here then serves the same call with a residual add or gradient, an output cast, or a forced field. */
 int mi355x_rownorm_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_dtype,
                         rownorm_dtype w_dtype, rownorm_plan* out);
 
@@ -394,6 +397,16 @@ int mi355x_rownorm_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_dty
  * off_line == 0 is mi355x_rownorm_plan. */
 int mi355x_rownorm_plan_at(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_dtype,
                            rownorm_dtype w_dtype, int off_line, rownorm_plan* out);
+
+/* The layout of a norm call on whole wavefronts: rows that fit no power of two of lanes, each held by
+ * `reserved` wavefronts (lanes_per_row = 64 times those, packs_per_lane packs a lane), rows_per_block rows a
+ * workgroup at a time.  `reserved` == 0: not this call, the rest is what mi355x_rownorm_plan reports.
+ * Taken by calls of at least a row for every compute unit without a residual add or gradient, an output
+ * cast and forced fields (and behind the LDS-staged kernels), where it measured faster: which lengths depends on the number of rows.  So
+ * the results of a row agree to rounding, but not bit for bit, with those it has in a call of another
+ * number of rows, or with the fused add in place of an add and the norm; equal calls give equal bits. */
+int mi355x_rownorm_waves_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_dtype,
+                              rownorm_dtype w_dtype, rownorm_plan* out);
 
 /* Test and tuning hook: force lanes_per_row / packs_per_lane / threads per
  * workgroup / workgroups per compute unit for one op (0 keeps the automatic

@@ -51,6 +51,7 @@ DECL(mi355x_group_norm_bwd);
 DECL(mi355x_group_norm_plan);
 DECL(mi355x_rownorm_plan);
 DECL(mi355x_rownorm_plan_at);
+DECL(mi355x_rownorm_waves_plan);
 DECL(mi355x_rownorm_set_override);
 
 static int failures = 0;
@@ -101,6 +102,7 @@ static bool load_all(void* lib) {
   LOAD(mi355x_group_norm_plan);
   LOAD(mi355x_rownorm_plan);
   LOAD(mi355x_rownorm_plan_at);
+  LOAD(mi355x_rownorm_waves_plan);
   LOAD(mi355x_rownorm_set_override);
   return ok;
 }

@@ -111,3 +111,40 @@ def test_forward_rows(rules):  # noqa: F811
         assert taken(1000, 8001, 0, wide) and taken(30000, 8001, 0, wide) == (wide == 1) and taken(30000, 8001, 1, wide)
         assert taken(68064, 2577, 1, wide) == (wide == 1) and taken(94118, 1293, 1, wide) == (wide == 1)
         assert taken(30000, 1401, 1, wide) and taken(16821, 2669, 1, wide) and taken(100000, 2051, 1, wide)
+
+
+def test_the_plan_query_reports_them(cabi, rules):  # noqa: F811
+    """mi355x_rownorm_waves_plan says what runs: lanes, packs, rows a workgroup works on, workgroups, and the partial
+    rows of a backward, which fit the workspace that the call asks for; nothing for forced fields, mi355x_rownorm_plan's
+    layout where it reports none."""
+    rng, taken = random.Random(13), 0
+    for _ in range(4000):
+        M, N = int(2 ** rng.uniform(7, 17)), int(2 ** rng.uniform(9, 14))
+        dt, wd = rng.choice(((cabi.F32, cabi.F32), (cabi.F16, cabi.F16), (cabi.BF16, cabi.F32)))
+        esize = 4 if dt == cabi.F32 else 2
+        ln, backward = rng.randint(0, 1), rng.randint(0, 1)
+        l = _layout(rules, backward, M, N, esize, ln, int(wd == cabi.F32 and esize == 2))
+        op = ((cabi.OP_RMS_NORM_FWD, cabi.OP_LAYER_NORM_FWD), (cabi.OP_RMS_NORM_BWD, cabi.OP_LAYER_NORM_BWD))[backward][ln]
+        p = cabi.waves_plan(op, M, N, dt, wd)
+        assert p.pop("waves") == l["waves"]
+        if l["waves"] == 0:
+            q = cabi.plan(op, M, N, dt, wd)
+            q.pop("row_chunks")
+            assert p == q
+            continue
+        taken += 1
+        assert p["resident"] == 1 and p["lanes_per_row"] == 64 * l["waves"]
+        assert (p["packs_per_lane"], p["rows_per_block"], p["grid_blocks"]) == (l["v"], l["slots"], l["grid"])
+        assert p["block_threads"] == 64 * l["waves"] * l["slots"]
+        assert p["partial_rows"] == (l["grid"] if backward else 0)
+        if backward:
+            f = cabi.lib().mi355x_layer_norm_bwd_workspace_bytes if ln else cabi.lib().mi355x_rms_norm_bwd_workspace_bytes
+            assert f(M, N, dt, wd, *((1, 1) if ln else (1,))) >= p["partial_rows"] * N * 4 * (1 + ln)
+    assert taken > 300
+    assert cabi.waves_plan(cabi.OP_SOFTMAX_FWD, 8192, 4097, cabi.F16, cabi.F16)["waves"] == 0
+    try:
+        cabi.set_override(cabi.OP_LAYER_NORM_BWD, 0, 0, 0, 3)
+        assert cabi.waves_plan(cabi.OP_LAYER_NORM_BWD, 8192, 4097, cabi.F16, cabi.F16)["waves"] == 0
+    finally:
+        cabi.clear_overrides()
+    assert cabi.waves_plan(cabi.OP_LAYER_NORM_BWD, 8192, 4097, cabi.F16, cabi.F16)["waves"] == 9

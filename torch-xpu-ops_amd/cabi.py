@@ -28,7 +28,7 @@ EXPORTED_SYMBOLS = (
     "mi355x_masked_softmax_bwd", "mi355x_softmax_strided_fwd", "mi355x_softmax_strided_bwd",
     "mi355x_softmax_strided_plan", "mi355x_softmax_strided_team_plan", "mi355x_group_norm_fwd",
     "mi355x_group_norm_bwd_workspace_bytes", "mi355x_group_norm_bwd", "mi355x_group_norm_plan",
-    "mi355x_rownorm_plan", "mi355x_rownorm_plan_at", "mi355x_rownorm_set_override",
+    "mi355x_rownorm_plan", "mi355x_rownorm_plan_at", "mi355x_rownorm_waves_plan", "mi355x_rownorm_set_override",
     "mi355x_rownorm_stream_probe", "mi355x_rownorm_set_team_wait_us",
 )
 
@@ -108,6 +108,8 @@ def lib():
         L.mi355x_rownorm_plan.argtypes = [_int, _i64, _i64, _int, _int, ctypes.POINTER(Plan)]
         L.mi355x_rownorm_plan_at.argtypes = [_int, _i64, _i64, _int, _int, _int,
                                              ctypes.POINTER(Plan)]
+        L.mi355x_rownorm_waves_plan.argtypes = [_int, _i64, _i64, _int, _int, ctypes.POINTER(Plan)]
+        L.mi355x_rownorm_waves_plan.restype = _int
         L.mi355x_rownorm_set_override.argtypes = [_int, _int, _int, _int, _int]
         L.mi355x_rownorm_stream_probe.argtypes = [_vp, _vp, _vp, ctypes.c_size_t, _int, _vp]
         L.mi355x_rownorm_stream_probe.restype = _int
@@ -153,6 +155,15 @@ def plan(op, M, N, x_dtype=F32, w_dtype=F32, off_line=False):
                                         ctypes.byref(p)), "plan")
     d = p.as_dict()
     d["row_chunks"] = p.reserved  # workgroups a row is split over (0: not split)
+    return d
+
+
+def waves_plan(op, M, N, x_dtype=F32, w_dtype=F32):
+    """The layout of a norm call on whole wavefronts; "waves" 0: not this call, the rest is plan()'s."""
+    p = Plan()
+    _check(lib().mi355x_rownorm_waves_plan(op, M, N, x_dtype, w_dtype, ctypes.byref(p)), "waves_plan")
+    d = p.as_dict()
+    d["waves"] = p.reserved
     return d
 
 

@@ -1018,6 +1018,30 @@ int mi355x_rownorm_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_dty
   return mi355x_rownorm_plan_at(op, M, N, x_dtype, w_dtype, 0, out);
 }
 
+int mi355x_rownorm_waves_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_dtype,
+                              rownorm_dtype w_dtype, rownorm_plan* out) {
+  if (int e = mi355x_rownorm_plan(op, M, N, x_dtype, w_dtype, out)) return e;
+  const OpClass oc = class_of((int)op);
+  out->reserved = 0;
+  if (oc != OC_NORM_FWD && oc != OC_NORM_BWD) return 0;
+  Plan plan;
+  if (int e = make_plan(oc, M, N, esize_of((int)x_dtype), current_num_cus(), g_override[(int)op],
+                        oc == OC_NORM_BWD, &plan, false,
+                        op == ROWNORM_OP_LAYER_NORM_FWD || op == ROWNORM_OP_LAYER_NORM_BWD,
+                        esize_of((int)w_dtype) > esize_of((int)x_dtype)))
+    return e;
+  const WavesLayout& l = plan.waves;
+  if (l.waves == 0) return 0;
+  out->reserved = l.waves;
+  out->lanes_per_row = 64 * l.waves;
+  out->packs_per_lane = l.v;
+  out->block_threads = 64 * l.waves * l.slots;
+  out->rows_per_block = l.slots;
+  out->grid_blocks = l.grid;
+  out->partial_rows = oc == OC_NORM_BWD ? l.grid : 0;
+  return 0;
+}
+
 int mi355x_rownorm_set_override(rownorm_op op, int lanes_per_row, int packs_per_lane,
                                 int block_threads, int blocks_per_cu) {
   if ((int)op < 0 || (int)op >= ROWNORM_OP_COUNT) return ROWNORM_ERR_SHAPE;
