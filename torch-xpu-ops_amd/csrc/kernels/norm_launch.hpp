@@ -244,7 +244,7 @@ struct NormBwdLauncher {
                                c.a.rstd, (const WT*)c.a.gamma, (T*)c.a.dx, c.a.part_dg,
                                c.a.part_db, c.a.M, c.a.N);
           };
-          if constexpr (!FAST && norm_bwd_reads_elements_built(sizeof(T), G, V, RMS)) {
+          if constexpr (!FAST && norm_bwd_reads_elements_built(sizeof(T), G, V, RMS, ADD)) {
             if (norm_bwd_reads_elements(sizeof(T), sizeof(WT), G, V, RMS, c.a.M, c.a.N)) {
               go(norm_bwd_resident_kernel<T, WT, G, V, BLOCK, 1, RMS, FAST, ADD, kReadElements>);
               return true;

@@ -455,24 +455,29 @@ constexpr NormBwdRead norm_bwd_read(int esize, int G, bool fast, bool rms) {
   if (!norm_bwd_clamps(G, fast)) return kReadElements;
   return esize == 2 && G >= kMaxG && !rms ? kReadClamped : kReadClampedInside;
 }
-// The instances that exist with element loads as well, and the calls those serve because they
-// measured faster (us, element loads / whole packs):
+// The instances that exist with element loads as well, and the calls those serve (us, element loads /
+// whole packs):
 //   16-bit LayerNorm rows that leave much of 1024 lanes idle -- a wavefront wholly past the row has
-//   next to nothing to do there, while the clamped form clears its packs: 16384 fp16 rows of 8193
-//   241 / 276, 12289 324 / 339, 13001 369 / 354; with fp32 weights 4096 rows of 8193 79.2 / 81.0,
-//   9001 89.3 / 84.0.  In 32nds of the pack slots.
+//   next to nothing to do there, while the clamped form clears its packs: 16384 fp16 rows of 12289
+//   324 / 339, 13001 369 / 354.  In 32nds of the pack slots.  (Plain calls of 1537 to 1600 packs;
+//   shorter rows run on whole wavefronts.)
 //   Tensors far beyond the caches, rows that fill most of their lanes -- memory-bound, and the
 //   requests of the next rows keep the memory busy while one wavefront waits for its elements: fp32
-//   LayerNorm [32768, 6143] 456 / 490, RMSNorm 450 / 484, LayerNorm [8192, 6143] 122.2 / 123.9 but
-//   [4096, 6143] 70.4 / 68.2 and [16384, 4097], half the slots idle, 157 / 149; fp16 RMSNorm on 512
-//   lanes x 3 packs [16384, 8193] 183 / 191, [4096, 8193] 57.0 / 56.6.
-constexpr bool norm_bwd_reads_elements_built(int esize, int G, int V, bool rms) {
+//   LayerNorm [32768, 6143] 460 / 491, [30000, 5001] 341 / 358, RMSNorm [32768, 6143] 454 / 487, [30000,
+//   7777] 531 / 567.  (Plain calls beyond 100 million elements; below, whole wavefronts.)
+// Calls with a residual gradient go by the same lines, drawn for the plain calls that had these layouts before
+// the whole wavefronts did.  There a third tensor is read as well, and the element loads are the faster ones in
+// float32 RMSNorm only ([32768, 6143] 634 / 642, [20000, 7777] 485 / 504, but LayerNorm 676 / 599 and [8192, 6143] 180 /
+// 157; fp16 LayerNorm [16384, 8193] 648 / 622, [4096, 12289] 213 / 200, with fp32 weights [4096, 8193] 149 / 154; fp16
+// RMSNorm on 512 lanes x 3 packs, which no plain call has, [16384, 8193] 311 / 299, [16384, 10001] 395 / 341).
+// (add: the call has a residual gradient)
+constexpr bool norm_bwd_reads_elements_built(int esize, int G, int V, bool rms, bool add) {
   if (esize == 4) return G == 256 || G == 512;
-  return rms ? G == 512 && V == 3 : G >= kMaxG;
+  return rms ? add && G == 512 && V == 3 : G >= kMaxG;
 }
 inline bool norm_bwd_reads_elements(int esize, int wsize, int G, int V, bool rms, int64_t M,
                                     int64_t N) {
-  if (!norm_bwd_reads_elements_built(esize, G, V, rms)) return false;
+  if (!norm_bwd_reads_elements_built(esize, G, V, rms, true)) return false;
   const int64_t packs = (N * esize + 15) / 16, slots = (int64_t)G * V;
   if (esize == 4) return packs * 16 > slots * 9 && M * N > 50000000;
   return rms ? M * N > 100000000 : packs * 32 <= slots * (wsize > 2 ? 17 : 25);
