@@ -61,9 +61,46 @@ def test_ragged_rows_off_a_boundary(cabi, oracle, gpu, dtype, offs):
                                        (270, 16383, torch.float16), (270, 12289, torch.float32),
                                        (8150, 6145, torch.float32)], ids=str)
 def test_both_ways_of_reading_a_ragged_row(cabi, oracle, gpu, M, N, dtype):
-    """Rows on 1024 lanes on both sides of the line between whole packs and element loads, and a
-    float32 tensor of more than 50 million elements, whose long rows keep the element loads."""
+    """Rows on 1024 lanes on both sides of the line between whole packs and element loads; two of the calls run on
+    whole wavefronts, whose last pack is the row's last whole pack."""
+    code = cabi.dtype_code(dtype)
+    w = cabi.waves_plan(cabi.OP_LAYER_NORM_BWD, M, N, code, code)["waves"]
+    assert (w > 0) == ((M, N) in ((300, 10005), (8150, 6145)))
     _check(cabi, oracle, gpu, M, N, dtype, (1, 3))
+
+
+@pytest.mark.parametrize("M,N", [(33000, 3071 + 64), (16500, 6145), (13100, 7777)], ids=str)
+def test_element_loads_of_float_tensors_beyond_100_million_elements(cabi, gpu, M, N):
+    """Float32 rows that fill most of their lanes, in tensors far beyond the caches, keep the element loads: against
+    float64 on the GPU, NaN on both sides of the inputs."""
+    print("case float32 element loads", (M, N), flush=True)
+    for op in (cabi.OP_LAYER_NORM_BWD, cabi.OP_RMS_NORM_BWD):
+        p = cabi.plan(op, M, N, cabi.F32, cabi.F32)
+        assert cabi.waves_plan(op, M, N, cabi.F32, cabi.F32)["waves"] == 0 and M * N > 100000000
+        assert p["lanes_per_row"] in (256, 512) and 16 * N * 4 > 9 * 16 * p["lanes_per_row"] * p["packs_per_lane"]
+    g = torch.Generator(device=gpu).manual_seed(2570 + N)
+    x, dy = (_inside(torch.empty(M, N, device=gpu).normal_(generator=g), o, gpu) for o in (1, 3))
+    w = _inside(1 + 0.1 * torch.empty(N, device=gpu).normal_(generator=g), 1, gpu)
+    for rms in (False, True):
+        # (a slab of columns or rows at a time in float64)
+        xd = x.double()
+        mu = xd.new_zeros(M, 1) if rms else xd.mean(1, keepdim=True)
+        rs = (xd.sub_(mu).square().mean(1, keepdim=True) + 1e-5).rsqrt()
+        xh = xd.mul_(rs)
+        stats = rs.view(-1).float(), mu.view(-1).float()
+        out = cabi.rms_norm_bwd(dy, x, stats[0], w) if rms else cabi.layer_norm_bwd(dy, x, stats[1], stats[0], w)
+        terms = dy.double().mul_(xh)
+        # (float32 sums over the rows of terms with the statistics' own rounding: a few ulps of the magnitudes' sum)
+        assert_close(out[1], to_np32(terms.sum(0)), torch.float32, "dgamma", slack=(terms.abs().sum(0) * 2.0 ** -20).cpu())
+        s2 = terms.mul_(w.double()).mean(1, keepdim=True)
+        del terms
+        if not rms:
+            assert_close(out[2], to_np32(dy.double().sum(0)), torch.float32, "dbeta", slack=(dy.abs().sum(0) * 2.0 ** -21).cpu())
+        gy = dy.double().mul_(w.double())
+        want = gy.sub_(0 if rms else gy.mean(1, keepdim=True)).sub_(xh.mul_(s2)).mul_(rs)
+        for r in range(0, M, 4096):
+            assert_close(out[0][r:r + 4096], to_np32(want[r:r + 4096]), torch.float32, "dx from row %d" % r)
+        del xd, xh, gy, want, out
 
 
 @pytest.mark.parametrize("N,dtype", [(5, torch.float16), (7, torch.bfloat16), (3, torch.float32)],

@@ -1,5 +1,5 @@
-"""Long norm forward rows whose teams share the rows out evenly over two or three rounds: full and nearly empty
-last chunks, against float64."""
+"""Long norm forward rows whose teams share the rows out evenly over two or three rounds, beside calls whose teams
+are as many as fit: full and nearly empty last chunks, against float64."""
 import pytest
 import torch
 
@@ -12,10 +12,16 @@ EPS = 1e-5
 
 @pytest.mark.parametrize("dtype,wdtype", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32),
                                           (torch.float32, torch.float32)], ids=str)
-@pytest.mark.parametrize("M,packs", [(140, 27072), (139, 27073), (131, 3 * 8192 - 511), (259, 16385)])
-def test_even_rounds(cabi, gpu, dtype, wdtype, M, packs):
+@pytest.mark.parametrize("M,packs,even", [(140, 27072, "all"), (139, 27073, "all"), (131, 3 * 8192 - 511, ""),
+                                          (259, 16385, ""), (33, 137936, "same"), (358, 20480, "all")])
+def test_even_rounds(cabi, gpu, dtype, wdtype, M, packs, even):
+    """even: whether the rule takes the call, with all weights or only those of the rows' type."""
     N = packs * (4 if dtype == torch.float32 else 8)
     print("case even rounds of teams", dtype, wdtype, (M, N), flush=True)
+    p = cabi.plan(cabi.OP_LAYER_NORM_FWD, M, N, cabi.dtype_code(dtype), cabi.dtype_code(wdtype))
+    teams, most = p["grid_blocks"] // p["row_chunks"], min(M, 512 // -(-packs // 8192))
+    assert (teams < most) == (even == "all" or (even == "same" and dtype == wdtype)), (p, most)
+    assert -(-M // teams) == -(-M // most)
     g = gen(M + packs)
     base = (torch.randn(M, 997, generator=g) + 0.5).to(gpu)
     x = base.repeat(1, -(-N // 997))[:, :N].mul(torch.linspace(0.5, 1.5, N, device=gpu)).to(dtype).contiguous()

@@ -29,9 +29,10 @@ def _untouched(buf, off, numel, fill=-77.0):
     return bool((head == fill).all()) and bool((tail == fill).all())
 
 
-# (rows, N): one row block a workgroup (grid = rows); three row blocks a workgroup at a stride of
-# 1024 rows; 512 and 1024 lanes; a row whose window holds one pack more than the row itself
+# (rows, N): one row block a workgroup (grid = rows); 512 and 1024 lanes; a row whose window holds one pack
+# more than the row itself; and calls that run on whole wavefronts, the LayerNorm forward at least
 SHAPES = [(37, 4097), (3000, 4097), (1100, 5121), (600, 8193), (300, 12289), (520, 3071), (64, 4103)]
+ON_WAVEFRONTS = {(3000, 4097), (1100, 5121), (520, 3071)}
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=str)
@@ -41,6 +42,9 @@ def test_windowed_forward_against_oracle(cabi, oracle, gpu, dtype, offs):
     code = cabi.dtype_code(dtype)
     for i, (M, N) in enumerate(SHAPES):
         print("case ragged norm rows", dtype, offs, (M, N), flush=True)
+        w = cabi.waves_plan(cabi.OP_LAYER_NORM_FWD, M, N, code, code)
+        assert (w["waves"] > 0) == ((M, N) in ON_WAVEFRONTS), w
+        # (the layout of the call with a residual add, where this one runs on wavefronts)
         p = cabi.plan(cabi.OP_LAYER_NORM_FWD, M, N, code, code)
         nrb = -(-M // p["rows_per_block"])
         assert p["resident"] == 1 and p["lanes_per_row"] >= 256, p
@@ -82,8 +86,12 @@ def test_windowed_forward_against_oracle(cabi, oracle, gpu, dtype, offs):
             assert _untouched(xbuf, ox, M * N), "in-place layer_norm wrote outside x " + what
 
 
-def test_windowed_forward_with_fp32_weights_and_special_rows(cabi, oracle, gpu):
-    M, N = 700, 4097
+@pytest.mark.parametrize("M", [250, 700])
+def test_windowed_forward_with_fp32_weights_and_special_rows(cabi, oracle, gpu, M):
+    """On the windowed kernel and, with more rows, on whole wavefronts."""
+    N = 4097
+    for op in (cabi.OP_LAYER_NORM_FWD, cabi.OP_RMS_NORM_FWD):
+        assert (cabi.waves_plan(op, M, N, cabi.BF16, cabi.F32)["waves"] > 0) == (M == 700)
     g = gen(1750)
     x = (0.25 + torch.randn(M, N, generator=g)).bfloat16()
     x[3, 4096] = float("inf")   # the last element of a row: the window's ragged end pack
@@ -105,6 +113,45 @@ def test_windowed_forward_with_fp32_weights_and_special_rows(cabi, oracle, gpu):
     assert float(rr[3]) == 0.0 and bool(torch.isnan(rr[5]))
     roy, ror = oracle.rms_norm_fwd(to_np32(x[fin]), (N,), to_np32(gamma), 1e-6)
     assert_close(ry[fin], roy, torch.bfloat16, "rms_norm, finite rows")
+
+
+@pytest.mark.parametrize("dtype,wdtype", [(torch.float16, torch.float16), (torch.bfloat16, torch.float32)], ids=str)
+def test_workgroups_that_walk_windowed_rows(cabi, gpu, dtype, wdtype):
+    """Three row blocks a workgroup at a stride of 1024 rows (512 at 512 lanes), so that every row of a workgroup has
+    the same window head: the fused add, which has no other layout, and a forced grid."""
+    for M, N in ((3000, 4097), (2900, 3071), (1500, 8193)):
+        print("case windowed rows walked", dtype, wdtype, (M, N), flush=True)
+        code, wcode = cabi.dtype_code(dtype), cabi.dtype_code(wdtype)
+        p = cabi.plan(cabi.OP_LAYER_NORM_FWD, M, N, code, wcode)
+        assert p["grid_blocks"] in (1024, 512) and 2 * p["grid_blocks"] < M * p["rows_per_block"]
+        g = torch.Generator(device=gpu).manual_seed(1770 + N)
+        rand = lambda *s: torch.empty(*s, device=gpu).normal_(generator=g)  # noqa: E731
+        _, x = _view(rand(M, N).to(dtype), 3)
+        _, res = _view((0.5 + rand(M, N)).to(dtype), 6)
+        _, w = _view((1 + 0.1 * rand(N)).to(wdtype), 1)
+        _, b = _view((0.1 * rand(N)).to(wdtype), 2)
+        hbuf, h = _view(torch.zeros_like(x), 5)
+        ybuf, y = _view(torch.zeros_like(x), 2)
+        cabi.add_layer_norm_fwd(x, res, w, b, 1e-5, h=h, y=y)
+        assert torch.equal(h, (x.float() + res.float()).to(dtype))
+        assert _untouched(hbuf, 5, M * N) and _untouched(ybuf, 2, M * N)
+        yr = cabi.add_rms_norm_fwd(x, res, w, 1e-6)[0]
+
+        def check(t, y, yr, what):
+            t, mu = t.double(), t.double().mean(1, keepdim=True)
+            want = (t - mu) * ((t - mu).square().mean(1, keepdim=True) + 1e-5).rsqrt() * w.double() + b.double()
+            assert_close(y, want.float().cpu().numpy(), dtype, "layer_norm, " + what)
+            want = t * (t.square().mean(1, keepdim=True) + 1e-6).rsqrt() * w.double()
+            assert_close(yr, want.float().cpu().numpy(), dtype, "rms_norm, " + what)
+
+        check(h, y, yr, "fused add [%d, %d]" % (M, N))
+        try:
+            for op in (cabi.OP_LAYER_NORM_FWD, cabi.OP_RMS_NORM_FWD):
+                cabi.set_override(op, 0, 0, 0, 2)
+                assert cabi.waves_plan(op, M, N, code, wcode)["waves"] == 0
+            check(x, cabi.layer_norm_fwd(x, w, b, 1e-5)[0], cabi.rms_norm_fwd(x, w, 1e-6)[0], "forced grid [%d, %d]" % (M, N))
+        finally:
+            cabi.clear_overrides()
 
 
 def test_fused_add_and_forced_layouts_on_windowed_rows(cabi, oracle, gpu):

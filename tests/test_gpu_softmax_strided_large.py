@@ -101,3 +101,52 @@ def test_a_team_of_one_has_no_conditions(cabi, gpu, dtype, shape):
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(gi, want), "replayed"
+
+
+@pytest.mark.parametrize("shape", [(1, 8191, 1024), (40, 4286, 28), (1, 12899, 484)], ids=str)
+def test_safe_softmax_and_outputs_of_another_type(cabi, gpu, shape):
+    """Safe softmax and float32 gradients with a float16 grad_input on large teams, and a float16 forward with a
+    float32 output, which keeps to small ones, at the same sizes: against float64 on the GPU, and with every wait
+    given up."""
+    outer, D, packs = shape
+    print("case strided softmax, large teams, other types", shape, flush=True)
+    g = torch.Generator(device=gpu).manual_seed(D + 5)
+
+    def both(fn):
+        a = fn()
+        try:
+            cabi.set_team_wait_us(0)
+            return a, fn()
+        finally:
+            cabi.set_team_wait_us()
+
+    for dtype in (torch.float16, torch.float32):
+        inner = packs * (4 if dtype == torch.float32 else 8)
+        x = torch.empty(outer, D, inner, device=gpu, dtype=dtype).normal_(0, 3.0, generator=g)
+        x[0, D // 3:, 0] = float("-inf")
+        x[-1, :, 1] = float("-inf")
+        assert cabi.strided_team_plan(0, outer, D, inner, cabi.dtype_code(dtype))["packs_per_lane"] > 16
+        want = torch.softmax(x.double(), 1)
+        nan = want.isnan()
+        assert int(nan.sum()) == D
+        for y in both(lambda: cabi.softmax_strided_fwd(x, 1, cabi.SAFE_SOFTMAX)):
+            assert bool((y[-1, :, 1] == 0).all()), "zeros for a column without a finite element"
+            assert_close(y, want.masked_fill(nan, 0).float().cpu().numpy(), dtype, "safe softmax")
+        if dtype == torch.float16:
+            for y in both(lambda: cabi.softmax_strided_fwd(x, 1, cabi.SOFTMAX, out_dtype=torch.float32)):
+                assert_close(y, want.float().cpu().numpy(), torch.float32, "float16 -> float32")
+            for y in both(lambda: cabi.softmax_strided_fwd(x, 1, cabi.LOG_SOFTMAX, out_dtype=torch.float32)):
+                ref = torch.log_softmax(x.double(), 1)
+                assert_close(y, ref.float().cpu().numpy(), torch.float32, "float16 -> float32, log")
+            continue
+        y = torch.softmax(torch.empty(outer, D, inner, device=gpu).normal_(0, 3.0, generator=g), 1)
+        grad = torch.empty(outer, D, inner, device=gpu).normal_(generator=g)
+        assert cabi.strided_team_plan(1, outer, D, inner, cabi.F32)["packs_per_lane"] > 8
+        yd, gd = y.double(), grad.double()
+        for mode in (cabi.SOFTMAX, cabi.LOG_SOFTMAX):
+            want = gd - yd.exp() * gd.sum(1, keepdim=True) if mode else yd * (gd - (yd * gd).sum(1, keepdim=True))
+            mag = yd.exp() * gd.abs().sum(1, keepdim=True) if mode else yd * (yd * gd).abs().sum(1, keepdim=True)
+            # (a few ulps of the magnitudes' sum, as for any float32 sum in another order)
+            for gi in both(lambda: cabi.softmax_strided_bwd(grad, y, 1, mode, gi_dtype=torch.float16)):
+                assert_close(gi, want.float().cpu().numpy(), torch.float16, "float32 -> float16 mode %d" % mode,
+                             slack=(mag * 2.0 ** -21).float().cpu())
