@@ -399,12 +399,13 @@ int mi355x_rownorm_plan_at(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_
                            rownorm_dtype w_dtype, int off_line, rownorm_plan* out);
 
 /* The layout of a norm call on whole wavefronts: rows that fit no power of two of lanes, each held by
- * `reserved` wavefronts (lanes_per_row = 64 times those, packs_per_lane packs a lane), rows_per_block rows a
- * workgroup at a time.  `reserved` == 0: not this call, the rest is what mi355x_rownorm_plan reports.
- * Taken by calls of at least a row for every compute unit without a residual add or gradient, an output
- * cast and forced fields (and behind the LDS-staged kernels), where it measured faster: which lengths depends on the number of rows.  So
- * the results of a row agree to rounding, but not bit for bit, with those it has in a call of another
- * number of rows, or with the fused add in place of an add and the norm; equal calls give equal bits. */
+ * `reserved` wavefronts (lanes_per_row = 64 times those, packs_per_lane packs a lane), rows_per_block
+ * rows a workgroup at a time.  `reserved` == 0: not this call, the rest is what mi355x_rownorm_plan
+ * reports.  Taken by calls of at least a row for every compute unit without a residual add or gradient,
+ * an output cast and forced fields (and behind the LDS-staged kernels), where it measured faster: which
+ * lengths depends on the number of rows.  So the results of a row agree to rounding, but not bit for bit,
+ * with those it has in a call of another number of rows, or with the fused add in place of an add and the
+ * norm; equal calls give equal bits. */
 int mi355x_rownorm_waves_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_dtype,
                               rownorm_dtype w_dtype, rownorm_plan* out);
 

@@ -55,7 +55,9 @@ inline void check_same_device(const at::Tensor& ref, const at::Tensor& t, const 
 // A new tensor on the GPU of `like`, straight from the caching allocator.  at::empty reaches the same
 // function through the dispatcher; a call of a norm makes three to four of them, and small calls are bound by
 // the host (us a call, back to back, with the statistics made in their final shape instead of viewed in it:
-// add_rms_norm of [8, 4096] 8.6 -> 7.5).  A tensor that is on no GPU is refused later, as it is with at::empty.
+// add_rms_norm of [8, 4096] 8.6 -> 7.5).  Unlike at::empty it leaves the memory as it is under deterministic
+// algorithms, which fill new memory with NaN there: every output made here is written in full.  A tensor that
+// is on no GPU is refused later, as it is with at::empty.
 inline at::Tensor new_tensor(at::IntArrayRef sizes, at::ScalarType dtype, const at::Tensor& like) {
   if (!like.is_cuda()) return at::empty(sizes, like.options().dtype(dtype));
   return at::Tensor(at::detail::empty_cuda(sizes, dtype, like.device(), std::nullopt));

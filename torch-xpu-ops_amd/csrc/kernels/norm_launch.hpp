@@ -137,7 +137,8 @@ int launch_norm_fwd(const Plan& plan, const NormFwdArgs& a, hipStream_t stream) 
         return (int)hipGetLastError();
     }
   }
-  if constexpr (!ADD && std::is_same<T, TY>::value) {
+  // (float32 rows: the LayerNorm's only, see norm_waves_float_rows())
+  if constexpr (!ADD && std::is_same<T, TY>::value && !(RMS && sizeof(T) == 4)) {
     if (plan.waves.waves > 0 && a.res == nullptr) {
       const bool ok = launch_norm_waves<T, false>(plan.waves, [&](auto v, auto d, auto threads) {
         hipLaunchKernelGGL((norm_fwd_waves_kernel<T, WT, decltype(v)::value, decltype(d)::value,

@@ -1422,7 +1422,9 @@ constexpr int kStridedLargeV[2][4] = {{40, 48, 56, 64}, {20, 24, 28, 32}};
 constexpr int strided_team_max_v(bool backward) { return backward ? 8 : 16; }
 constexpr int strided_large_max_v(bool backward) { return backward ? 32 : 64; }
 // Workgroups of an instance a compute unit holds, and the packs a lane keeps in LDS: up to 48 packs
-// of a lane (the backward 24 of each tensor) fit 256 registers, the rest 16 bytes a thread each.
+// of a lane (the backward 24 of each tensor) fit 256 registers, the rest 16 bytes a thread each.  (Beside
+// 16 packs in LDS the forward spills 9 to 11 registers, in bfloat16 beside 8 packs 3, outside the loops over the
+// packs.)
 constexpr int strided_team_per_cu(bool backward, int v) {
   return v > strided_team_max_v(backward) ? 1 : kTeamPerCu;
 }

@@ -4,8 +4,8 @@
 //
 // The tensor is [outer, D, inner], inner a whole number of 16-byte packs (any alignment); a strip is
 // TX consecutive packs of `inner` (up to 32: 512 bytes) and all D rows under them.  A team of `team`
-// workgroups of 512 threads holds a strip in
-// registers (and, one workgroup a compute unit, in LDS: strided_large_team()): workgroup c the rows [c * TY * V, (c + 1) * TY * V), thread (ty, tx) the V packs
+// workgroups of 512 threads holds a strip in registers (and, one workgroup a compute unit, in LDS:
+// strided_large_team()): workgroup c the rows [c * TY * V, (c + 1) * TY * V), thread (ty, tx) the V packs
 // of rows ty, ty + TY, ... of pack column tx.  A workgroup reduces its rows per column (each
 // lane over its packs, a wavefront by shuffles, the eight wavefronts through LDS), publishes the
 // C = TX * E columns' numbers -- running maximum and sum of exp(x - maximum), or the sum the
@@ -18,12 +18,12 @@
 // [8192, 8192] call) and the exchange, whose rounds run in step.  Two workgroups a compute unit hold
 // 64 MB in registers, so that call made two (forward) or four rounds; one workgroup of 256 registers a
 // lane with 16 packs a lane more in LDS holds 128 MB: one or two rounds of teams a quarter as large,
-// 70.5 / 103.7 -> 59.1 / 82.9 us (of the 59, reads 24, the exponentials 4 + 4 beside reads and writes,
-// the exchange 6).  The exponentials of a group of packs are formed while the next groups are on their
-// way: the rows past D are replaced group by group, not all at once, which waited for every load (71 ->
-// 68 us).  bf16 forward / backward us, without -> with teams of two workgroups a compute unit: [8192,
-// 8192] over dim 0 78.3 / 115 -> 67.8 / 102; [4000, 16384] 75.9 / 112 -> 64.6 / 83.6; [8192, 64] 17.6 / 12.1 -> 9.8 / 7.5; [8, 1000, 1024] 22.8 / 17.9 -> 12.0 / 12.3;
-// [35, 1000, 1904] 150 / 176 -> 76.6 / 95.7; [100, 2000, 128] 38.6 / 45.6 -> 22.8 / 32.0.
+// 70.5 / 103.7 -> 59.1 / 82.9 us (of the 59, the loads alone take 28, the exchange 7).  The exponentials of
+// a group of packs are formed while the next groups are on their way: the rows past D are replaced group
+// by group, not all at once, which waited for every load (71 -> 68 us).  bf16 forward / backward us,
+// without -> with teams of two workgroups a compute unit: [8192, 8192] over dim 0 78.3 / 115 -> 67.8 / 102;
+// [4000, 16384] 75.9 / 112 -> 64.6 / 83.6; [8192, 64] 17.6 / 12.1 -> 9.8 / 7.5; [8, 1000, 1024] 22.8 / 17.9 ->
+// 12.0 / 12.3; [35, 1000, 1904] 150 / 176 -> 76.6 / 95.7; [100, 2000, 128] 38.6 / 45.6 -> 22.8 / 32.0.
 // Requesting the next strip ahead of the exchange (half the packs a lane, twice the rounds)
 // measured slower (84-90 us on [8192, 8192]), as did rows dealt out in bands over the team.
 //
@@ -126,7 +126,8 @@ __device__ __forceinline__ void merge_pairs(float& m, float& s, const float (&vm
 }
 
 // Gathers this thread's share of the team: merge(v) is called with v[number][member] for members
-// q, q + Q, ..., B at a time, after reset(); -inf / 0 stand for members past the team's end.  Every thread of the workgroup calls it; the result is uniform: true when
+// q, q + Q, ..., B at a time, after reset(); -inf / 0 stand for members past the team's end.  Every
+// thread of the workgroup calls it; the result is uniform: true when
 // all words of the round were there, false when the wait ran out or the call is lost.
 template <int NF, class Reset, class Merge>
 __device__ __forceinline__ bool columns_gather(TeamColumns* slot, const unsigned long long* mates,
