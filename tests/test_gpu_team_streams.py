@@ -13,6 +13,13 @@ from helpers import assert_close, gen
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(scope="module")
+def streams(gpu):
+    """Three streams for all tests of this file that need exchange memory: a stream keeps its slot of the strided
+    softmax (eight a device) for the process, and calls on one that found none give other bits."""
+    return [torch.cuda.Stream() for _ in range(3)]
+
+
 def _calls(cabi, gpu, seed):
     """Thunks of one stream: strips on 64 workgroups, on a few, forward and backward, and rows of the
     norm and softmax kernels held by teams."""
@@ -27,8 +34,7 @@ def _calls(cabi, gpu, seed):
             lambda: cabi.layer_norm_fwd(r, gamma, None, 1e-5)[0], lambda: cabi.softmax_fwd(r)]
 
 
-def test_calls_on_three_streams_do_not_wait_for_one_another(cabi, gpu):
-    streams = [torch.cuda.Stream() for _ in range(3)]
+def test_calls_on_three_streams_do_not_wait_for_one_another(cabi, gpu, streams):
     calls = [_calls(cabi, gpu, 2600 + i) for i in range(3)]
     alone = [[f() for f in fs] for fs in calls]
     got = [[None] * len(fs) for fs in calls]
@@ -74,10 +80,9 @@ def _large_calls(cabi, gpu, seed):
             lambda: cabi.layer_norm_fwd(many, gamma[:4096], None, 1e-5)[0]]
 
 
-def test_workgroups_that_need_a_whole_compute_unit_on_three_streams(cabi, gpu):
+def test_workgroups_that_need_a_whole_compute_unit_on_three_streams(cabi, gpu, streams):
     """A large team shares the machine with other streams' teams and with kernels whose workgroups take any compute
     unit that has room: nobody's wait runs out."""
-    streams = [torch.cuda.Stream() for _ in range(3)]
     calls = [_large_calls(cabi, gpu, 2700 + i) for i in range(3)]
     alone = [[f() for f in fs] for fs in calls]
     for i, s in enumerate(streams):  # (the streams' slots, the allocator's blocks)
