@@ -46,9 +46,18 @@ def test_large_teams(rules):  # noqa: F811
     for a in ((0, 48, 3983, 592, 2), (0, 18, 4088, 2736, 2), (0, 47, 3854, 472, 4), (1, 14, 3068, 1336, 2), (1, 45, 3068, 488, 4),
               (0, 34, 12457, 60, 4), (0, 62, 14919, 56, 4)):
         assert _large(rules, *a)["team"] == 0, a
-    # forward rows of whole lines, several rounds
-    for a in ((0, 62, 6587, 256, 2), (0, 4, 9431, 2304, 2), (0, 40, 10726, 128, 4)):
+    # in 16 bits rows of 16 packs at most for a single round only
+    for a, one in (((0, 55, 14117, 120, 2), 32), ((0, 56, 15618, 104, 2), 28), ((0, 49, 14836, 80, 2), 24)):
+        assert _large(rules, *a)["team"] == 0 and _large(rules, 0, one, *a[2:])["team"] > 0, a
+    # forward rows of whole lines, several rounds, in float32 any
+    for a in ((0, 62, 6587, 256, 2), (0, 4, 9431, 2304, 2), (0, 40, 10726, 128, 4), (0, 16, 11602, 128, 4), (0, 2, 5884, 1824, 4)):
         assert _large(rules, *a)["team"] == 0, a
+    # float32 forward rows on small teams whose neighbouring strips meet on one XCD
+    for a in ((0, 14, 6942, 376, 4), (0, 4, 8964, 632, 4), (0, 4, 12060, 492, 4)):
+        assert _strided(rules, *a)["team"] % 8 == 0 and _large(rules, *a)["team"] == 0, a
+    # float32 backward strips no wider, of an odd number of packs, rounds not halved
+    for a in ((1, 9, 4084, 524, 4), (1, 53, 3929, 236, 4)):
+        assert _large(rules, *a)["team"] == 0 and _large(rules, *a[:3], a[3] + 4, 4)["team"] > 0, a
 
 
 def test_not_for_an_output_wider_than_the_input(rules):  # noqa: F811

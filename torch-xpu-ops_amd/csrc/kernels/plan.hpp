@@ -1565,12 +1565,20 @@ inline StridedTeam strided_team(bool backward, int64_t outer, int64_t D, int64_t
 // teams have strips of 32 packs as well there is none in the forward (560 shapes of 20 to 600 MB each: bf16
 // 0.97 of the time, a quarter of them slower: [48, 3983, 592] 126 / 149, [18, 4088, 2736] 219 / 239; fp32
 // 1.03: [47, 3854, 472] 189 / 218), and in the backward only from eight members on (below: bf16 [14, 3068,
-// 1336] 85 / 93, fp32 [45, 3068, 488] 177 / 197).  Nor in a float32 forward of rows of 16 packs at most, whose
-// strips stay as they are ([34, 12457, 60] 52 / 59, [62, 14919, 56] 112 / 123).
+// 1336] 85 / 93, fp32 [45, 3068, 488] 177 / 197), in float32 rows of an odd number of packs where it halves the
+// rounds (otherwise 0.98 of the time over 68 shapes, 15 of them slower: [9, 4084, 524] 58.6 / 63.5, [53, 3929,
+// 236] 143 / 154; where it does 0.91).  Nor in a forward of rows of 16 packs at most, whose strips stay as they
+// are: not in float32 ([34, 12457, 60] 52 / 59, [62, 14919, 56] 112 / 123), in 16 bits for a single round only
+// (0.91 of the time; two 1.03: bf16 [55, 14117, 120] 98 / 107, [56, 15618, 104] 99 / 108).
 // The other part is the lines of 128 bytes that neighbouring strips of other rows share, and that are read
-// twice.  Forward rows of whole lines share none: they take large teams for a single round only, with no other
-// to be out of step with (bf16 0.90 of the time, fp32 0.95; of several rounds 1.02 and 1.00: bf16 [62, 6587, 256]
-// 90 / 99, [4, 9431, 2304] 80 / 84, fp32 [40, 10726, 128] 94 / 107).
+// twice.  Forward rows of whole lines share none: they take large teams in 16 bits, for a single round, with no
+// other to be out of step with (0.93 of the time; of several rounds 1.02: bf16 [62, 6587, 256] 90 / 99, [4, 9431,
+// 2304] 80 / 84), and never in float32 (one round 1.00, a quarter of 37 shapes slower: [16, 11602, 128] 44.3 /
+// 48.5, [2, 5884, 1824] 42.3 / 45.3; several 1.00: [40, 10726, 128] 94 / 107).
+// Workgroup b runs on XCD b % 8: in teams of a multiple of eight members the same rows of neighbouring strips, and
+// so the lines they share, meet in one L2.  Float32 forward rows of more than 32 packs on such teams gain from
+// large ones of several rounds and a multiple of eight members alone (0.96 of the time; other teams 1.02 over 93
+// shapes: [14, 6942, 376] 88 / 98; a single round 1.02 over 62: [4, 8964, 632] 50 / 58, [4, 12060, 492] 56 / 60).
 // Never a float16 forward with a float32 output (widened): its stores are twice the bytes of its loads and its
 // exponentials are the long ones, and with one workgroup a compute unit neither runs under the other's reads
 // (560 shapes of 20 to 600 MB, 1.14 times the time: [59, 3360, 192] 73 / 113, [6, 5912, 1536] 100 / 143, [2,
@@ -1583,8 +1591,10 @@ inline StridedTeam strided_large_team(bool backward, int64_t outer, int64_t D, i
   if (l.team == 0 || l.rounds >= t.rounds || 8 * l.rounds * l.v > 17 * t.rounds * t.v) return StridedTeam{};
   if (l.team == 1) return backward && l.rounds == 1 ? l : StridedTeam{};
   if (t.tx > kStridedTeamTx && (!backward || l.team < 8)) return StridedTeam{};
-  if (!backward && esize == 4 && packs <= kStridedTeamTx) return StridedTeam{};
-  if (!backward && packs % 8 == 0 && l.rounds > 1) return StridedTeam{};
+  if (t.tx > kStridedTeamTx && esize == 4 && packs % 2 != 0 && 2 * l.rounds > t.rounds) return StridedTeam{};
+  if (!backward && (packs <= kStridedTeamTx || packs % 8 == 0) && (esize == 4 || l.rounds > 1)) return StridedTeam{};
+  if (!backward && esize == 4 && packs > kStridedTeamWideTx && t.team % 8 == 0 && (l.team % 8 != 0 || l.rounds == 1))
+    return StridedTeam{};
   return t.team >= (packs % 2 == 0 ? 12 : 24) ? l : StridedTeam{};
 }
 
