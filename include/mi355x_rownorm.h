@@ -356,14 +356,15 @@ int mi355x_softmax_strided_plan(int backward, int64_t outer, int64_t dim_size, i
  * 16-byte packs of `inner`, all dim_size rows) in the registers of `reserved` workgroups of
  * block_threads threads, packs_per_lane rows on each of the rows_per_block threads along
  * dim_size; grid_blocks / reserved teams walk the strips.  `reserved` == 0: no teams, the rest is what
- * mi355x_softmax_strided_plan reports.  Teams serve inner sizes of whole packs, any alignment, where
- * they measured faster.  Teams of more than one workgroup pass the columns' partial results through
+ * mi355x_softmax_strided_plan reports.  Teams serve inner sizes of a pack or more, any alignment, where
+ * they measured faster; reported are inner sizes of whole packs, and an inner size between two of those has
+ * the teams of the larger one.  Teams of more than one workgroup pass the columns' partial results through
  * the stream's bookkeeping slot, under the rules of mi355x_rownorm_set_team_wait_us (eight streams
  * can hold a slot of this kind): a workgroup may wait for the others of its team for up to
  * that bound, and reads the whole strip itself if it runs out.  They need an output that overlaps no
  * input; such a call in place, on a stream under capture, or on a stream beyond the eight takes
  * mi355x_softmax_strided_plan's layout.  A team of one waits for nobody and has none of these
- * conditions.  Reported is the call whose output has the input's type: a float16 forward with a float32
+ * conditions, but where inner is not a whole number of packs the output must overlap no input.  Reported is the call whose output has the input's type: a float16 forward with a float32
  * output keeps to teams of which a compute unit holds two (packs_per_lane <= 16). */
 int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_size, int64_t inner,
                                      rownorm_dtype dtype, rownorm_plan* out);

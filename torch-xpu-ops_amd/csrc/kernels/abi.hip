@@ -962,8 +962,8 @@ int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_si
     return e;
   const bool large = plan.large_team > 0;
   const int tx_log2 = large ? plan.large_tx_log2 : plan.team_tx_log2;
-  out->reserved = plan.team_size();
-  if (plan.team_size() == 0) return 0;
+  out->reserved = plan.fast ? plan.team_size() : 0;  // (rows of whole packs: see the header)
+  if (out->reserved == 0) return 0;
   out->resident = 1;
   out->lanes_per_row = 1 << tx_log2;
   out->packs_per_lane = large ? plan.large_v : plan.team_v;

@@ -1720,8 +1720,11 @@ inline int make_strided_plan(bool backward, int64_t outer, int64_t D, int64_t in
     }
   }
   // Strips held by teams of workgroups, where D is beyond the one-workgroup tile or teams are faster
-  // than that.
-  if (p.fast && ov.G == 0 && ov.V == 0 && ov.bpc == 0) {
+  // than that.  Rows of no whole number of packs too (softmax_strided_team.hpp), by the rules of those rounded
+  // up: without teams they were read two and three times, each row's last pack element by element (forward /
+  // backward us: bf16 [93, 616, 723] 160 / 194 -> 52 / 67, [1, 6246, 78] 47.0 / 30.3 -> 10.1 / 8.0, fp16 [28, 3452,
+  // 239] 80.6 / 90.0 -> 33.4 / 31.3; 400 calls of random shapes 0.57 and 0.52 of the time, none slower).
+  if (inner >= E && ov.G == 0 && ov.V == 0 && ov.bpc == 0) {
     const StridedTeam t = strided_team(backward, outer, D, packs, esize, num_cus);
     if (t.team > 0 && (stream || strided_team_beats_tile(backward, outer, D, packs, esize, TX, t))) {
       p.team = t.team;

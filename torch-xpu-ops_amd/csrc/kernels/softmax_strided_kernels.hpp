@@ -83,7 +83,10 @@ struct StridedTile {
   bool valid;    // false: the group has run out of tiles; nothing is loaded or stored
 };
 
-template <int BLOCK, int E>
+// WHOLE: every access is a whole pack.  A pack that would end past the row is the row's last one instead, whose
+// first elements are the neighbouring lane's as well: both store the same result, and the output overlaps no
+// input (the neighbour may be another workgroup's).
+template <int BLOCK, int E, bool WHOLE>
 __device__ __forceinline__ StridedTile strided_tile(int64_t t0, int64_t ntiles, int64_t xtiles,
                                                     int D, int inner, StridedLayout lay) {
   const int TX = 1 << lay.tx_log2;
@@ -99,7 +102,7 @@ __device__ __forceinline__ StridedTile strided_tile(int64_t t0, int64_t ntiles, 
   const int64_t xt = tc - o * xtiles;
   r.slab = o * (int64_t)D * (int64_t)inner;
   const int64_t e = (xt * TX + tx) * (int64_t)E;
-  r.e0 = e < inner ? (int)e : inner;
+  r.e0 = e < inner ? (WHOLE && e + E > inner ? inner - E : (int)e) : inner;
   return r;
 }
 
@@ -123,7 +126,7 @@ softmax_strided_fwd_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t
   const int64_t ntiles = outer * xtiles;
   const int NG = groups_per_block<BLOCK>(lay);
   for (int64_t t0 = (int64_t)blockIdx.x * NG; t0 < ntiles; t0 += (int64_t)gridDim.x * NG) {
-    const StridedTile tile = strided_tile<BLOCK, E>(t0, ntiles, xtiles, D, inner, lay);
+    const StridedTile tile = strided_tile<BLOCK, E, FAST>(t0, ntiles, xtiles, D, inner, lay);
     const int ty = tile.ty, TY = tile.TY;
     // the V packs stay in storage format; each pass widens them again (softmax
     // then evaluates exp twice per element, which measured faster than holding
@@ -224,7 +227,7 @@ softmax_strided_bwd_kernel(const TG* __restrict__ grad, const TG* __restrict__ y
   const int64_t ntiles = outer * xtiles;
   const int NG = groups_per_block<BLOCK>(lay);
   for (int64_t t0 = (int64_t)blockIdx.x * NG; t0 < ntiles; t0 += (int64_t)gridDim.x * NG) {
-    const StridedTile tile = strided_tile<BLOCK, E>(t0, ntiles, xtiles, D, inner, lay);
+    const StridedTile tile = strided_tile<BLOCK, E, FAST>(t0, ntiles, xtiles, D, inner, lay);
     const int ty = tile.ty, TY = tile.TY;
     Pack<TG, E> pg[V], py[V];
 #pragma unroll
@@ -297,7 +300,7 @@ softmax_strided_fwd_stream_kernel(const TI* __restrict__ x, TO* __restrict__ y, 
   const int64_t ntiles = outer * xtiles;
   const int NG = groups_per_block<BLOCK>(lay);
   for (int64_t t0 = (int64_t)blockIdx.x * NG; t0 < ntiles; t0 += (int64_t)gridDim.x * NG) {
-    const StridedTile tile = strided_tile<BLOCK, E>(t0, ntiles, xtiles, D, inner, lay);
+    const StridedTile tile = strided_tile<BLOCK, E, false>(t0, ntiles, xtiles, D, inner, lay);
     const int ty = tile.ty, TY = tile.TY;
     const TI* xs = x + tile.slab;
     TO* ys = y + tile.slab;
@@ -358,7 +361,7 @@ softmax_strided_bwd_stream_kernel(const TG* __restrict__ grad, const TG* __restr
   const int64_t ntiles = outer * xtiles;
   const int NG = groups_per_block<BLOCK>(lay);
   for (int64_t t0 = (int64_t)blockIdx.x * NG; t0 < ntiles; t0 += (int64_t)gridDim.x * NG) {
-    const StridedTile tile = strided_tile<BLOCK, E>(t0, ntiles, xtiles, D, inner, lay);
+    const StridedTile tile = strided_tile<BLOCK, E, false>(t0, ntiles, xtiles, D, inner, lay);
     const int ty = tile.ty, TY = tile.TY;
     const TG* gs = grad + tile.slab;
     const TG* ys = y + tile.slab;
@@ -531,7 +534,7 @@ softmax_strided_split_partial_kernel(const TI* __restrict__ x, TO* __restrict__ 
   int d0, d1;
   split_rows(blockIdx.y, gridDim.y, chunk_rows, D, &d0, &d1);
   for (int64_t t0 = (int64_t)blockIdx.x * NG; t0 < ntiles; t0 += (int64_t)gridDim.x * NG) {
-    const StridedTile tile = strided_tile<BLOCK, E>(t0, ntiles, xtiles, D, inner, lay);
+    const StridedTile tile = strided_tile<BLOCK, E, false>(t0, ntiles, xtiles, D, inner, lay);
     const int ty = tile.ty, TY = tile.TY;
     const TI* xs = x + tile.slab;
     float mx[E], sum[E];
@@ -586,7 +589,7 @@ softmax_strided_split_combine_kernel(TO* __restrict__ y, int64_t outer, int D, i
   const int64_t ntiles = outer * xtiles;
   const int NG = groups_per_block<BLOCK>(lay);
   for (int64_t t0 = (int64_t)blockIdx.x * NG; t0 < ntiles; t0 += (int64_t)gridDim.x * NG) {
-    const StridedTile tile = strided_tile<BLOCK, E>(t0, ntiles, xtiles, D, inner, lay);
+    const StridedTile tile = strided_tile<BLOCK, E, false>(t0, ntiles, xtiles, D, inner, lay);
     const int ty = tile.ty, TY = tile.TY;
     TO* ys = y + tile.slab;
     float a[E], b[E];
@@ -634,7 +637,7 @@ softmax_strided_split_apply_kernel(const TI* __restrict__ x, TO* __restrict__ y,
   int d0, d1;
   split_rows(blockIdx.y, gridDim.y, chunk_rows, D, &d0, &d1);
   for (int64_t t0 = (int64_t)blockIdx.x * NG; t0 < ntiles; t0 += (int64_t)gridDim.x * NG) {
-    const StridedTile tile = strided_tile<BLOCK, E>(t0, ntiles, xtiles, D, inner, lay);
+    const StridedTile tile = strided_tile<BLOCK, E, false>(t0, ntiles, xtiles, D, inner, lay);
     const int ty = tile.ty, TY = tile.TY;
     const TI* xs = x + tile.slab;
     TO* ys = y + tile.slab;
@@ -692,7 +695,7 @@ softmax_strided_split_bwd_partial_kernel(const TG* __restrict__ grad, const TG* 
   int d0, d1;
   split_rows(blockIdx.y, gridDim.y, chunk_rows, D, &d0, &d1);
   for (int64_t t0 = (int64_t)blockIdx.x * NG; t0 < ntiles; t0 += (int64_t)gridDim.x * NG) {
-    const StridedTile tile = strided_tile<BLOCK, E>(t0, ntiles, xtiles, D, inner, lay);
+    const StridedTile tile = strided_tile<BLOCK, E, false>(t0, ntiles, xtiles, D, inner, lay);
     const int ty = tile.ty, TY = tile.TY;
     const TG* gs = grad + tile.slab;
     const TG* ys = y + tile.slab;
@@ -750,7 +753,7 @@ softmax_strided_split_bwd_apply_kernel(const TG* __restrict__ grad, const TG* __
   int d0, d1;
   split_rows(blockIdx.y, gridDim.y, chunk_rows, D, &d0, &d1);
   for (int64_t t0 = (int64_t)blockIdx.x * NG; t0 < ntiles; t0 += (int64_t)gridDim.x * NG) {
-    const StridedTile tile = strided_tile<BLOCK, E>(t0, ntiles, xtiles, D, inner, lay);
+    const StridedTile tile = strided_tile<BLOCK, E, false>(t0, ntiles, xtiles, D, inner, lay);
     const int ty = tile.ty, TY = tile.TY;
     const TG* gs = grad + tile.slab;
     const TG* ys = y + tile.slab;

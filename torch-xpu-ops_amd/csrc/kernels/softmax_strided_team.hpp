@@ -2,7 +2,7 @@
 // tile of softmax_strided_kernels.hpp or teams are faster than that (strided_team_beats_tile()): every
 // element crosses the memory interface once.
 //
-// The tensor is [outer, D, inner], inner a whole number of 16-byte packs (any alignment); a strip is
+// The tensor is [outer, D, inner], inner a 16-byte pack or more (any alignment); a strip is
 // TX consecutive packs of `inner` (up to 32: 512 bytes) and all D rows under them.  A team of `team`
 // workgroups of 512 threads holds a strip in registers (and, one workgroup a compute unit, in LDS:
 // strided_large_team()): workgroup c the rows [c * TY * V, (c + 1) * TY * V), thread (ty, tx) the V packs
@@ -49,8 +49,11 @@ struct StridedTeamShape {
 };
 
 // A thread's place in a strip: pack column tx, rows ty, ty + TY, ...; the element of `inner` its
-// packs start at (where the strip is wider than what is left of `inner`, the row's last pack, which
-// a neighbouring lane reads as well: loaded, never stored).
+// packs start at.  A pack that would end past the row is the row's last whole pack instead: where the row is
+// not a whole number of packs, its first elements are the neighbouring lane's as well, and both store the
+// same result (their columns' numbers are formed alike; the neighbour may be another team's, so the output
+// must then overlap no input); where the strip is wider than what is left of `inner`, the lane has no column
+// of its own and stores nothing (in == false).
 template <int E>
 struct StridedTeamPlace {
   int tx, ty, TY, e0;
@@ -61,7 +64,7 @@ struct StridedTeamPlace {
     TY = kTeamBlock >> s.tx_log2;
     const int64_t e = (((strip % s.xtiles) << s.tx_log2) + tx) * E;
     in = e < s.inner;
-    e0 = in ? (int)e : s.inner - E;
+    e0 = e + E <= s.inner ? (int)e : s.inner - E;
   }
 };
 
