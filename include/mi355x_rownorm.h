@@ -115,7 +115,9 @@ int mi355x_layer_norm_fwd(const void* x, const void* gamma, const void* beta, vo
  * ROWNORM_ERR_WORKSPACE), and, for a few rows far too long for the registers,
  * the partial sums of the split-row dX (the regime of Norm.h:632-812), which
  * follow the column sums.  A workspace that holds the first part only is
- * accepted: every row's dX then stays on one workgroup.  Rows beyond one
+ * accepted: every row's dX then stays on one workgroup, but for up to 128 such rows of
+ * 32 MB at most, which keep the rows' partial sums in the first part (they leave no
+ * partial rows of column sums).  Rows beyond one
  * workgroup's registers in calls of many rows may be held four at a time by teams
  * of workgroups (dY and X read once; whole packs, 16-byte aligned tensors and
  * workspace, dx apart from dy and x, the bookkeeping and the bounded wait of
@@ -387,6 +389,9 @@ int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_si
  * lane (float32 LayerNorm: 10), and the masked softmax calls beyond 32 elements a
  * lane on 1024 lanes (rows of more than 32768 elements; a forced layout beyond
  * that is ROWNORM_ERR_OVERRIDE for a masked call).
+ * Fewer than eight forward rows of whole packs beyond one workgroup's registers are held by teams of at most an
+ * eighth of the machine where the conditions of mi355x_rownorm_set_team_wait_us allow it; reported is the layout
+ * they have otherwise.
  * Norm calls that mi355x_rownorm_waves_plan reports a layout for run on that one instead; the one
  * reported here then serves the same call with a residual add or gradient, an output cast, or a forced field. */
 int mi355x_rownorm_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_dtype,

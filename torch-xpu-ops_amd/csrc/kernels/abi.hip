@@ -994,8 +994,9 @@ int mi355x_rownorm_plan_at(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_
   out->block_threads = plan.block;
   out->rows_per_block = plan.rpb;
   // (a forward row held by a team of workgroups: the team and its grid)
-  out->reserved = plan.team > 0 ? plan.team : (plan.split > 1 ? plan.split : 0);
-  out->grid_blocks = plan.team > 0 ? plan.team_grid : plan.grid;
+  const bool team = plan.team > 0 && !plan.team_small;
+  out->reserved = team ? plan.team : (plan.split > 1 ? plan.split : 0);
+  out->grid_blocks = team ? plan.team_grid : plan.grid;
   out->partial_rows = (int64_t)bwd_partial_rows(plan);
   // (groups of rows held by teams: the workgroup, the packs of a row a lane holds, the rows)
   if (plan.team > 0 && (op == ROWNORM_OP_LAYER_NORM_BWD || op == ROWNORM_OP_RMS_NORM_BWD)) {

@@ -2567,6 +2567,124 @@ norm_bwd_split_dx_colsum_kernel(const T* __restrict__ dy, const T* __restrict__ 
     store_column_sums<WT, E>(db, part_db + (int64_t)blockIdx.y * N, dbeta, direct != 0, e0, N);
 }
 
+// The same for few rows, dgamma and dbeta complete: a wavefront owns 64 packs of columns and every `waves`-th row,
+// U of them at a time; a workgroup holds kFewRowsWaves / waves such pieces of columns.  It adds the rows' chunk sums
+// itself (in the order of norm_bwd_split_totals_kernel), and the column sums of the wavefronts that share a piece
+// meet in LDS, in wavefront order.  So the backward of few long rows is two launches, this one behind
+// norm_bwd_split_sums_kernel, in place of four with a partial row for each row or so (the totals and the
+// second stage in launches of their own), and nothing of the column sums goes through memory.
+//
+// WHOLE: every access is a whole pack; a pack that would end past a ragged row is the row's last whole one
+// instead, over columns that its neighbour holds as well: both store the same dX and the same sums, and dX
+// overlaps no input (the neighbour may be another workgroup's).
+template <class T, class WT, bool RMS, bool ADD, bool WHOLE>
+__global__ void __launch_bounds__(kFewRowsWaves * 64)
+norm_bwd_few_rows_kernel(const T* __restrict__ dy, const T* __restrict__ x, const T* dres,
+                         const float* __restrict__ mean, const float* __restrict__ rstd,
+                         const WT* __restrict__ gamma, const float* __restrict__ split_ws, int chunks, T* dx,
+                         WT* __restrict__ dgamma, WT* __restrict__ dbeta, int M, int N, int waves) {
+  constexpr int E = elems_per_pack<T>::value;
+  constexpr int U = 4;
+  __shared__ float tot[kFewRowsMax][2];
+  __shared__ __align__(16) float sums[kFewRowsWaves][64 * E];
+  const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int first = wave % waves, pieces = kFewRowsWaves / waves;
+  const int64_t e0l = (((int64_t)blockIdx.x * pieces + wave / waves) * 64 + lane) * E;
+  const bool in = e0l < N;
+  const int e0 = WHOLE ? (e0l + E <= N ? (int)e0l : N - E) : in ? (int)e0l : 0;
+  auto load = [&](const auto* row) {
+    using P = Pack<std::remove_cv_t<std::remove_pointer_t<decltype(row)>>, E>;
+    if constexpr (WHOLE) return P::load_stream(row + e0);
+    else return load_row_pack<std::remove_cv_t<std::remove_pointer_t<decltype(row)>>, E, true>(row, e0, N, true, 0.0f);
+  };
+  const Pack<WT, E> pg = gamma ? load(gamma) : Pack<WT, E>::splat(1.0f);
+  Pack<T, E> px[U], pd[U], pu[ADD ? U : 1];
+  // (row numbers past M - 1 read row M - 1 and are left out below)
+  auto fetch = [&](int row0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int row = row0 + u * waves < M ? row0 + u * waves : M - 1;
+      px[u] = load(x + (int64_t)row * N);
+      pd[u] = load(dy + (int64_t)row * N);
+      if constexpr (ADD) pu[u] = load(dres + (int64_t)row * N);
+    }
+  };
+  fetch(first);
+  for (int row = wave; row < M; row += kFewRowsWaves) {
+    const float* sc = split_ws + (int64_t)row * chunks * 2;
+    float s1 = 0.0f, s2 = 0.0f;
+    for (int c = lane; c < chunks; c += 64) {
+      s1 += sc[2 * c];
+      s2 += sc[2 * c + 1];
+    }
+    s1 = wave_group_allreduce<64, SumOp>(s1);
+    s2 = wave_group_allreduce<64, SumOp>(s2);
+    if (lane == 0) {
+      tot[row][0] = s1;
+      tot[row][1] = s2;
+    }
+  }
+  __syncthreads();
+  const float fN = (float)N;
+  float dg[E], db[RMS ? 1 : E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    dg[i] = 0.0f;
+    if constexpr (!RMS) db[i] = 0.0f;
+  }
+  for (int row0 = first; row0 < M; row0 += U * waves) {
+    if (row0 != first) fetch(row0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int row = row0 + u * waves;
+      if (row >= M) break;  // uniform
+      const float mu = RMS ? 0.0f : uniform_load<float>(mean + row), rs = uniform_load<float>(rstd + row);
+      const float s1 = tot[row][0], s2 = tot[row][1];
+      const float term1 = rs / fN;
+      Pack<T, E> o;
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+        const float xh = (px[u].get(i) - mu) * rs;
+        float f = fN * (pd[u].get(i) * pg.get(i));
+        f -= xh * s2;
+        if constexpr (!RMS) f -= s1;
+        f *= term1;
+        if constexpr (ADD) f += pu[u].get(i);
+        o.set(i, f);
+        dg[i] = fmaf(pd[u].get(i), xh, dg[i]);
+        if constexpr (!RMS) db[i] += pd[u].get(i);
+      }
+      if constexpr (WHOLE) {
+        if (in) o.store_stream(dx + (int64_t)row * N + e0);
+      } else {
+        store_row_pack<T, E, true>(dx + (int64_t)row * N, e0, N, in, o);
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < (RMS ? 1 : 2); ++k) {
+    WT* out = k == 0 ? dgamma : dbeta;
+    if (out == nullptr) continue;
+    if (k > 0) __syncthreads();
+#pragma unroll
+    for (int h = 0; h < E; h += 4) {
+      const int b = RMS ? 0 : h;  // (db has one element where there is no dbeta)
+      *reinterpret_cast<float4*>(&sums[wave][lane * E + h]) =
+          k == 0 ? float4{dg[h], dg[h + 1], dg[h + 2], dg[h + 3]}
+                 : float4{db[b], db[RMS ? 0 : b + 1], db[RMS ? 0 : b + 2], db[RMS ? 0 : b + 3]};
+    }
+    __syncthreads();
+    for (int col = (int)threadIdx.x; col < pieces * 64 * E; col += kFewRowsWaves * 64) {
+      const int64_t pack = (int64_t)blockIdx.x * (pieces * 64 * E) + col / E * E;
+      const int64_t at = (WHOLE && pack + E > N ? N - E : pack) + col % E;
+      const int w0 = col / (64 * E) * waves;
+      float t = 0.0f;
+      for (int w = 0; w < waves; ++w) t += sums[w0 + w][col % (64 * E)];
+      if (pack < N && at < N) out[at] = (WT)t;
+    }
+  }
+}
+
 // Column sums for rows too wide for registers: workgroup (bx, by) owns the
 // BLOCK*E columns starting at bx*BLOCK*E and the rows by, by+gridDim.y, ...;
 // it writes row `by` of the [gridDim.y, N] partial buffers.

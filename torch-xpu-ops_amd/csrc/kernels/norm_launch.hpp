@@ -403,6 +403,28 @@ int launch_norm_bwd(const Plan& plan, const NormBwdArgs& a, hipStream_t stream) 
     // and also when it is not but the column sums are wanted: dX and the column
     // sums then share the second pass over X and dY (two passes, not three)
     const int chunks = plan.split > 1 ? plan.split : 1;
+    if (a.dx != nullptr && want_cols && plan.few_waves > 0) {
+      float* sums = a.part_dg;
+      hipLaunchKernelGGL((norm_bwd_split_sums_kernel<T, WT, kStreamBlock, RMS>),
+                         dim3((unsigned)plan.few_chunks, (unsigned)a.M), dim3(kStreamBlock), 0, stream,
+                         (const T*)a.dy, (const T*)a.x, a.mean, a.rstd, (const WT*)a.gamma, sums, a.N,
+                         plan.few_chunk_packs);
+      const int64_t pieces = (a.N + 64 * E - 1) / (64 * E);
+      const int64_t per = kFewRowsWaves / plan.few_waves;
+      const int64_t bytes = a.M * (int64_t)a.N * (int64_t)sizeof(T);
+      auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((pieces + per - 1) / per)), dim3(kFewRowsWaves * 64), 0, stream,
+                           (const T*)a.dy, (const T*)a.x, dres, a.mean, a.rstd, (const WT*)a.gamma,
+                           (const float*)sums, plan.few_chunks, (T*)a.dx, (WT*)a.dgamma, (WT*)a.dbeta, (int)a.M,
+                           a.N, plan.few_waves);
+      };
+      if (plan.fast || (regions_disjoint(a.dx, bytes, a.dy, bytes) && regions_disjoint(a.dx, bytes, a.x, bytes) &&
+                        regions_disjoint(a.dx, bytes, dres, bytes)))
+        go(norm_bwd_few_rows_kernel<T, WT, RMS, ADD, true>);
+      else
+        go(norm_bwd_few_rows_kernel<T, WT, RMS, ADD, false>);
+      return (int)hipGetLastError();
+    }
     if (a.dx != nullptr && a.split_ws != nullptr && (chunks > 1 || want_cols) && a.M <= 65535) {
       const dim3 grid((unsigned)chunks, (unsigned)a.M);
       hipLaunchKernelGGL((norm_bwd_split_sums_kernel<T, WT, kStreamBlock, RMS>), grid,

@@ -61,6 +61,10 @@ struct Plan {
   // 0 or 1 = one workgroup per row.
   int split = 0;
   int64_t chunk_packs = 0;
+  // norm backward of few rows beyond the registers (norm_bwd_few_rows_kernel): wavefronts that share a piece of
+  // columns; 0: not planned; and the chunks its rows are cut into for their sums
+  int few_waves = 0, few_chunks = 0;
+  int64_t few_chunk_packs = 0;
   // softmax backward of rows beyond the registers of two tensors: grad alone fits
   // them (the log_softmax backward then keeps grad resident and streams y)
   bool grad_resident = false;
@@ -72,6 +76,7 @@ struct Plan {
   // compiled for, packs a workgroup, workgroups launched; team == 0: not planned
   int team = 0, team_v = 0;
   int64_t team_chunk_packs = 0, team_grid = 0;
+  bool team_small = false;  // fewer than kTeamMinTeams rows, all at once (the plan query reports the launches without)
   // norm backward of such rows held R = team_v rows at a time by teams of workgroups
   // (norm_bwd_team_kernel): the same fields, one stride of packs a workgroup, and the
   // partial rows of column sums that launch leaves (one a team; partial_rows is what
@@ -164,6 +169,10 @@ constexpr int kStreamBlock = 1024;
 // four of them (32768 16-bit elements); a row is cut into at most 1024 chunks.
 constexpr int kSplitMinStrides = 4;
 constexpr int kSplitMaxChunks = 1024;
+// norm_bwd_few_rows_kernel: rows at most, bytes of a tensor at most, wavefronts a workgroup
+constexpr int kFewRowsMax = 128;
+constexpr int64_t kFewRowsBytes = int64_t(32) << 20;
+constexpr int kFewRowsWaves = 8;
 
 // Preferred packs per lane: what the G ladder aims for.
 // Measured on MI355X: 16 elements a lane (two 16-bit packs, four fp32 packs)
@@ -1117,6 +1126,30 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
       !(oc == OC_NORM_BWD && p.fast && norm_bwd_exact_index(esize, packs, M, layer_norm, wide_weights, false) >= 0))
     p.waves = norm_waves_layout(oc == OC_NORM_BWD, esize, M, N, p.fast, layer_norm, wide_weights, p.partial_rows,
                                 num_cus);
+  // Backward of few rows beyond the registers, dX and column sums: two launches, no partial rows
+  // (norm_bwd_few_rows_kernel).  Wavefronts that share a piece of 64 packs of columns, a part of the rows each:
+  // as many as leave every compute unit one workgroup (us, 1 / 2 / 4 / 8 of them: bf16 LayerNorm [28, 70144] 28.0 /
+  // 18.8 / 13.5 / 10.4, [16, 200000] 20.6 / 15.1 / 12.1 / 14.7, [48, 385536] 50.8 / 40.1 / 44.3 / 44.9).  Against the
+  // four launches, or teams of workgroups and a second stage: [28, 70144] 27.9 -> 10.4, [3, 87936] 12.5 -> 7.4, [8,
+  // 292096] 25.5 -> 11.9, [64, 60000] 28.5 -> 16.9, [57, 156800] 34.2 -> 27.4.  The other sides of the lines: [251,
+  // 51584] 37.1 / 46.0, [100, 400000] 67 / 82, and rows that alone give every compute unit two workgroups, which
+  // the column-sum kernels serve without partial rows as well ([3, 1451648] 16.6 / 21.4, [7, 1413504] 29.3 / 32.3).
+  // An RMSNorm of whole packs keeps its teams, which have half the sums to exchange and to add, from half as many
+  // rows and bytes on ([24, 194976] 23.6 -> 14.7, but [75, 162328] 28.3 / 33.8, [108, 38472] 20.6 / 24.2, [19, 659856]
+  // 27.5 / 30.8).  200 random calls that take it: 0.58 of the time, two slower (1.03).
+  const int64_t few_part = layer_norm || !p.fast ? 1 : 2;
+  if (oc == OC_NORM_BWD && !p.resident && want_cols && want_dx && p.partial_rows > 1 && M * few_part <= kFewRowsMax &&
+      M * packs * 16 * few_part <= kFewRowsBytes && ov.G == 0 && ov.V == 0 && ov.bpc == 0 && ov.block == 0) {
+    const int64_t pieces = (packs + 63) / 64;
+    p.few_waves = kFewRowsWaves;
+    while (p.few_waves > 1 && pieces * p.few_waves > kFewRowsWaves * (int64_t)num_cus) p.few_waves /= 2;
+    // (chunks of whole strides, about four a compute unit; their sums fit the memory of the partial rows, which
+    // this call has none of: at most a 16th of one)
+    const int64_t most = (4 * (int64_t)num_cus + M - 1) / M;
+    const int64_t cp = ((packs + most - 1) / most + kStreamBlock - 1) / kStreamBlock * kStreamBlock;
+    p.few_chunk_packs = cp;
+    p.few_chunks = (int)((packs + cp - 1) / cp);
+  }
   // Rows beyond the registers, and too few of them to give every compute unit a
   // workgroup (the regime of the reference's split-row kernels, Norm.h:632-812):
   // cut each row into chunks so that about four workgroups per compute unit
@@ -1167,17 +1200,25 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
     // Fewer than 8 teams run their load, wait and store phases nearly in step, and
     // the wait (about 8 us a round) is not hidden by other teams: bf16 [128, 9834496]
     // (3 teams of 85, 43 rounds) took 1740 us against 1500 us for the two-pass kernel
-    // whose second pass comes out of the memory-side cache, [2, 1310720] 13.2 against
-    // 11.6 us; 8 teams ([8, 4194304], one round) 35.1 against 40.5 us, 64 teams
-    // ([512, 401408], 8 rounds) 177 against 196 us.
+    // whose second pass comes out of the memory-side cache; 8 teams ([8, 4194304], one
+    // round) 35.1 against 40.5 us, 64 teams ([512, 401408], 8 rounds) 177 against 196 us.
+    // Fewer than 8 rows, all at once: teams of at most an eighth of the machine, whose exchange is a single
+    // round trip ([2, 1310720] 10.7 us in three launches, 12.0 on teams of 256 workgroups, 9.4 on 64; [7, 1413504]
+    // 24.1, 13.4; [3, 87936] 10.3, 6.9; and one launch, where three bound such a call: [4, 506752] with its
+    // backward 26.6 -> 20.0 us).  More than eight packs a lane for one or two rows leave too much of the machine
+    // idle: [1, 4000000] 12.7, 16.8, but [5, 3000000] 25.6, 24.7.
     // (GroupNorm slabs have no split-row kernels to fall back on: with fewer slabs than 8
     // teams, all at once, the alternative is one workgroup a slab)
-    if (teams >= kTeamMinTeams || ((oc == OC_GROUP_FWD || few_rows) && teams >= 1 && teams == M)) {
+    const int64_t strides = (packs + kTeamBlock - 1) / kTeamBlock, eighth = cus / kTeamMinTeams;
+    const bool at_once = teams >= 1 && teams == M;
+    const bool small_teams = oc == OC_NORM_FWD && !p.resident && at_once && M < kTeamMinTeams &&
+                             strides <= eighth * (M < 3 ? kTeamMaxV / 2 : kTeamMaxV);
+    if (teams >= kTeamMinTeams || ((oc == OC_GROUP_FWD || few_rows) && at_once) || small_teams) {
       // a chunk is a whole number of workgroup strides, exactly the packs a lane the
       // kernel is compiled for: every workgroup but a row's last runs straight-line code
-      const int64_t strides = (packs + kTeamBlock - 1) / kTeamBlock;
       auto packs_a_lane = [&](int64_t n) {
-        const int64_t most = cus / n < strides ? cus / n : strides;
+        int64_t most = cus / n < strides ? cus / n : strides;
+        if (small_teams && most > eighth) most = eighth;
         return (strides + most - 1) / most;
       };
       // Two or three rounds, the last of them not full: as many teams as give every round the same rows, each
@@ -1209,6 +1250,7 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
       p.team_v = (int)v;
       p.team_chunk_packs = v * kTeamBlock;
       p.team_grid = teams * team;
+      p.team_small = small_teams;
     }
   }
   // Forward rows too long for at least eight such teams (beyond 256 / 8 * 16 * 512 packs),
@@ -1241,7 +1283,7 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
   // packs a workgroup, dY and X read once (norm_bwd_team_kernel).
   // (override G = -1 with block = 1: the team launch whatever the rounds, for tests)
   const bool team_bwd_forced = ov.G == -1 && ov.V == 0 && ov.block == 1 && ov.bpc == 0;
-  if (oc == OC_NORM_BWD && !p.resident && p.fast && !fused_add && want_dx &&
+  if (oc == OC_NORM_BWD && !p.resident && p.fast && !fused_add && want_dx && p.few_waves == 0 &&
       ((ov.G == 0 && ov.V == 0 && ov.bpc == 0 && ov.block == 0) || team_bwd_forced)) {
     const int64_t cus = num_cus * kTeamBwdPerCu < kTeamMaxWorkgroups ? num_cus * kTeamBwdPerCu : kTeamMaxWorkgroups;
     const int64_t chunk = (int64_t)kTeamBwdPacks * kTeamBlock;
