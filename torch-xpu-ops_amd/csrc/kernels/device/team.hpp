@@ -1,9 +1,10 @@
 // Device side of the exchange between the workgroups of a team (norm_fwd_team_kernel,
 // softmax_fwd_team_kernel): a row too long for one workgroup is held in the registers of
 // several, which pass two numbers each through library-owned device memory.  Below it: the
-// same exchange in two halves for K float64 values (norm_fwd_rows_team_kernel, which puts
-// a round of other work between publishing and gathering) and a lighter one of
-// self-validating words for float32 values (norm_bwd_team_kernel).
+// same exchange in two halves of self-validating words, for K float64 values
+// (norm_fwd_rows_team_kernel, which puts a round of other work between publishing and
+// gathering; norm_fwd_team_kernel WORDS) and for float32 values (norm_bwd_team_kernel, the
+// teams of softmax and of GroupNorm's backward).
 //
 // What crosses workgroups.  An entry is 128 bytes (neighbours' polls go to other memory
 // channels).  The two-number exchange (team_publish_and_gather) uses {tag, s1, s2}: the tag
@@ -219,11 +220,12 @@ __device__ __forceinline__ bool team_gather_tagged(TeamSlot* slot, const TeamEnt
 // The same with the team's numbers left one by one in part[j][0..K) (LDS): the kernel adds them
 // up by a rule of its own.  (The lanes of a wavefront see one another's LDS stores in program
 // order.)
-template <int K>
-__device__ __forceinline__ bool team_gather_each(TeamSlot* slot, const TeamEntry* mates, int team,
-                                                 unsigned int call_id, unsigned int round,
-                                                 unsigned long long wait_ticks, float (*part)[K]) {
-  constexpr int B = kTeamGatherBatch;
+template <int K, int B>
+__device__ __forceinline__ bool team_gather_each_by(TeamSlot* slot, const TeamEntry* mates,
+                                                    int team, unsigned int call_id,
+                                                    unsigned int round,
+                                                    unsigned long long wait_ticks,
+                                                    float (*part)[K]) {
   const int lane = (int)threadIdx.x;
   const unsigned int expect = team_word_tag(call_id, round);
   const unsigned long long t0 = wall_clock64();
@@ -270,6 +272,21 @@ __device__ __forceinline__ bool team_gather_each(TeamSlot* slot, const TeamEntry
     __hip_atomic_store(&slot->gave_up, call_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return complete;
 }
+// (As many entries a lane and a poll as the team has, up to four: a small team's poll asks
+// for no entry twice, a team of 65 to 128 needs no second round trip.  GroupNorm backward of
+// bf16 [2, 256, 256, 256], teams of 32 by words 42.2 -> 39.2 us; of [1, 512, 464, 464], teams
+// of 106: 153 us by tags, 156 by one entry at a time, 148 by two.)
+template <int K>
+__device__ __forceinline__ bool team_gather_each(TeamSlot* slot, const TeamEntry* mates, int team,
+                                                 unsigned int call_id, unsigned int round,
+                                                 unsigned long long wait_ticks, float (*part)[K]) {
+  if (team <= 64)
+    return team_gather_each_by<K, 1>(slot, mates, team, call_id, round, wait_ticks, part);
+  if (team <= 128)
+    return team_gather_each_by<K, 2>(slot, mates, team, call_id, round, wait_ticks, part);
+  return team_gather_each_by<K, kTeamGatherBatch>(slot, mates, team, call_id, round, wait_ticks,
+                                                  part);
+}
 
 // The same two halves for K float64 values a workgroup (K <= 6), each cut into two words
 // {32 bits, tag} of pad[] as in team_publish_and_gather, summed over the team in the fixed
@@ -290,13 +307,12 @@ __device__ __forceinline__ void team_publish_f64(TeamEntry* mine, unsigned int c
   }
 }
 
-template <int K>
+template <int K, int B = kTeamGatherBatch>
 __device__ __forceinline__ bool team_gather_sums_f64(TeamSlot* slot, const TeamEntry* mates,
                                                      int team, unsigned int call_id,
                                                      unsigned int round,
                                                      unsigned long long wait_ticks,
                                                      double (&v)[K]) {
-  constexpr int B = kTeamGatherBatch;
   const int lane = (int)threadIdx.x;
   const unsigned int expect = team_word_tag(call_id, round);
   const unsigned long long t0 = wall_clock64();

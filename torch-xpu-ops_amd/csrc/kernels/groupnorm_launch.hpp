@@ -94,7 +94,7 @@ int launch_group_norm_fwd(const Plan& plan, const GroupNormFwdArgs& a, hipStream
     gs.packs_per_channel = a.HxW / elems_per_pack<T>::value;
     auto go = [&](auto v) {
       constexpr int V = decltype(v)::value;
-      hipLaunchKernelGGL((norm_fwd_team_kernel<T, WT, V, false, true, WT>),
+      hipLaunchKernelGGL((norm_fwd_team_kernel<T, WT, V, false, true, true, WT>),
                          dim3((unsigned)plan.team_grid), dim3(kTeamBlock), 0, stream,
                          (const T*)a.x, (const WT*)a.gamma, (const WT*)a.beta, (T*)a.y,
                          (WT*)a.mean, (WT*)a.rstd, a.rows, a.L, a.eps, plan.team,

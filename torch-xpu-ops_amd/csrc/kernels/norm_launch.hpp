@@ -171,12 +171,18 @@ int launch_norm_fwd(const Plan& plan, const NormFwdArgs& a, hipStream_t stream) 
   } else if (norm_fwd_team_serves<T, TY, ADD>(plan, a)) {
     // one pass with the row in the registers of a team of workgroups
     TeamSlot* slot = (TeamSlot*)a.team_slot;
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)plan.team_grid), dim3(kTeamBlock), 0, stream,
+                         (const T*)a.x, (const WT*)a.gamma, (const WT*)a.beta, (T*)a.y, a.mean,
+                         a.rstd, a.M, a.N, a.eps, plan.team, plan.team_chunk_packs, slot,
+                         a.team_id, a.team_wait_ticks, TeamGroupShape{});
+    };
     auto go = [&](auto v) {
       constexpr int V = decltype(v)::value;
-      hipLaunchKernelGGL((norm_fwd_team_kernel<T, WT, V, RMS>), dim3((unsigned)plan.team_grid),
-                         dim3(kTeamBlock), 0, stream, (const T*)a.x, (const WT*)a.gamma,
-                         (const WT*)a.beta, (T*)a.y, a.mean, a.rstd, a.M, a.N, a.eps, plan.team,
-                         plan.team_chunk_packs, slot, a.team_id, a.team_wait_ticks);
+      if (a.M * plan.team <= plan.team_grid)  // every row in the first round
+        launch(norm_fwd_team_kernel<T, WT, V, RMS, true>);
+      else
+        launch(norm_fwd_team_kernel<T, WT, V, RMS, false>);
     };
     static_assert(kTeamMaxV == 16, "one case per pack count below");
     switch (plan.team_v) {

@@ -480,7 +480,10 @@ softmax_fwd_stream_kernel(const TI* __restrict__ x, TO* __restrict__ y, MaskRef 
 // units idle.  A workgroup whose wait runs out takes the whole row's maximum and sum
 // itself (a second pass over X, which no workgroup writes: Y must not overlap X), loads
 // its chunk again and goes on; every wave reaches the end of the kernel whatever the
-// other workgroups do.
+// other workgroups do.  What bounds few rows is the way from the last chunk's sum to the
+// first store, so the pair crosses as self-validating words (one round trip; a tag beside
+// the numbers, three): bf16 [16, 262144] 8.5 -> 7.4 us, [2, 1048576] 11.3 -> 8.8, [128,
+// 140000] 16.1 -> 15.2; backward 8.1 -> 7.0, 10.7 -> 7.4, 23.6 -> 22.0.
 template <class TI, class TO, int V>
 __global__ void __launch_bounds__(kTeamBlock, kTeamPerCu * kTeamBlock / 256)
 softmax_fwd_team_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t M, int N, int flags,
@@ -490,7 +493,7 @@ softmax_fwd_team_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t M,
   constexpr int BLOCK = kTeamBlock;
   constexpr bool PRECISE = sizeof(TO) == 4;
   __shared__ float red[reduce_lds_floats<BLOCK, BLOCK, 1>::value];
-  __shared__ double tpart[kTeamMaxWorkgroups][2];
+  __shared__ float tpart[kTeamMaxWorkgroups][2];
   __shared__ float stat[4];  // the row's maximum, 1 / sum or log(sum), -, whether the team failed
   int phase = 0;
   const bool is_log = (flags & kSoftmaxLog) != 0;
@@ -513,10 +516,10 @@ softmax_fwd_team_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t M,
     typedef __attribute__((address_space(1))) Elem* GlobalPtr;
     return (Elem*)reinterpret_cast<GlobalPtr>(reinterpret_cast<uintptr_t>(p) + off);
   };
+  bool lost = false;  // (first wavefront) the workgroup has stopped waiting for its team
   unsigned int round = 0;
   for (int64_t row = tm; row < M; row += teams, ++round) {
     TeamEntry* entries = slot->entry[round & 1u];
-    if (threadIdx.x == 0) team_store(&entries[blockIdx.x].tag, 0ull);
     const TI* xr = x + row * (int64_t)N;
     const TI* xb = xr + pbase * E;
     Pack<TI, E> xp[V];
@@ -559,18 +562,22 @@ softmax_fwd_team_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t M,
     group_allreduce<BLOCK, BLOCK, 1, SumOp>(sm, red, phase);
     if (threadIdx.x < 64) {  // the first wavefront publishes, waits and merges
       const int lane = (int)threadIdx.x;
-      const bool complete = team_publish_and_gather(slot, entries, tm, team, call_id, round,
-                                                    wait_ticks, (double)m_c, (double)sm[0], tpart);
+      if (lane == 0)
+        team_publish_tagged<2>(&entries[blockIdx.x], call_id, round, {m_c, sm[0]}, lost);
+      const bool complete =
+          !lost && team_gather_each<2>(slot, entries + tm * team, team, call_id, round,
+                                       wait_ticks, tpart);
+      lost = !complete;
       // (the lanes of a wavefront see one another's LDS stores in program order)
       if (complete) {
         float mm = -INFINITY;
-        for (int j = lane; j < team; j += 64) mm = fmaxf(mm, (float)tpart[j][0]);
+        for (int j = lane; j < team; j += 64) mm = fmaxf(mm, tpart[j][0]);
         mm = wave_group_allreduce<64, MaxOp>(mm);
         // a chunk with nothing finite adds 0; a row with nothing finite gives NaN, as
         // exp(-inf - -inf) does in the three-pass form
         float ss = 0.0f;
         for (int j = lane; j < team; j += 64) {
-          const float mj = (float)tpart[j][0], sj = (float)tpart[j][1];
+          const float mj = tpart[j][0], sj = tpart[j][1];
           ss += sj == 0.0f ? (mm == -INFINITY ? NAN : 0.0f) : sj * row_exp<PRECISE>(mj - mm);
         }
         ss = wave_group_allreduce<64, SumOp>(ss);
@@ -1085,7 +1092,7 @@ softmax_bwd_team_kernel(const TG* __restrict__ grad, const TG* __restrict__ y, T
   constexpr int BLOCK = kTeamBlock;
   constexpr bool PRECISE = sizeof(TO) == 4 && sizeof(TG) == 4;
   __shared__ float red[reduce_lds_floats<BLOCK, BLOCK, 1>::value];
-  __shared__ double tpart[kTeamMaxWorkgroups][2];
+  __shared__ float tpart[kTeamMaxWorkgroups][1];
   __shared__ float stat[4];  // the row's sum, -, -, whether the team failed
   int phase = 0;
   const bool is_log = (flags & kSoftmaxLog) != 0;
@@ -1106,10 +1113,10 @@ softmax_bwd_team_kernel(const TG* __restrict__ grad, const TG* __restrict__ y, T
     typedef __attribute__((address_space(1))) Elem* GlobalPtr;
     return (Elem*)reinterpret_cast<GlobalPtr>(reinterpret_cast<uintptr_t>(p) + off);
   };
+  bool lost = false;  // (first wavefront) the workgroup has stopped waiting for its team
   unsigned int round = 0;
   for (int64_t row = tm; row < M; row += teams, ++round) {
     TeamEntry* entries = slot->entry[round & 1u];
-    if (threadIdx.x == 0) team_store(&entries[blockIdx.x].tag, 0ull);
     const TG* gr = grad + row * (int64_t)N;
     const TG* yr = y + row * (int64_t)N;
     const TG* gb = gr + pbase * E;
@@ -1163,12 +1170,19 @@ softmax_bwd_team_kernel(const TG* __restrict__ grad, const TG* __restrict__ y, T
     group_allreduce<BLOCK, BLOCK, 1, SumOp>(sum, red, phase);
     if (threadIdx.x < 64) {  // the first wavefront publishes, waits and adds up
       const int lane = (int)threadIdx.x;
-      const bool complete = team_publish_and_gather(slot, entries, tm, team, call_id, round,
-                                                    wait_ticks, (double)sum[0], 0.0, tpart);
+      if (lane == 0) team_publish_tagged<1>(&entries[blockIdx.x], call_id, round, sum, lost);
+      bool complete = !lost;
+      if constexpr (V >= 8)  // (no registers left for more than an entry at a time)
+        complete = complete && team_gather_each_by<1, 1>(slot, entries + tm * team, team, call_id,
+                                                         round, wait_ticks, tpart);
+      else
+        complete = complete && team_gather_each<1>(slot, entries + tm * team, team, call_id,
+                                                   round, wait_ticks, tpart);
+      lost = !complete;
       // (the lanes of a wavefront see one another's LDS stores in program order)
       if (complete) {
         float ss = 0.0f;
-        for (int j = lane; j < team; j += 64) ss += (float)tpart[j][0];
+        for (int j = lane; j < team; j += 64) ss += tpart[j][0];
         ss = wave_group_allreduce<64, SumOp>(ss);
         if (lane == 0) {
           stat[0] = ss;
