@@ -389,6 +389,9 @@ int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_si
  * lane (float32 LayerNorm: 10), and the masked softmax calls beyond 32 elements a
  * lane on 1024 lanes (rows of more than 32768 elements; a forced layout beyond
  * that is ROWNORM_ERR_OVERRIDE for a masked call).
+ * Softmax calls on longer ragged rows without a mask are held by one workgroup all the same (up to 20 packs a lane;
+ * the backward: 8, log_softmax 20, with Y aligned like grad), few of them by teams; neither is reported here, where
+ * such rows appear as the multi-pass layout that serves them otherwise.
  * Fewer than eight forward rows of whole packs beyond one workgroup's registers are held by teams of at most an
  * eighth of the machine where the conditions of mi355x_rownorm_set_team_wait_us allow it; reported is the layout
  * they have otherwise.

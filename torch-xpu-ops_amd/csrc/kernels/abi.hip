@@ -461,10 +461,10 @@ int softmax_fwd(const void* x, const void* mask, void* y, int64_t rows, int64_t 
   SoftmaxFwdArgs a{x,    y, (const uint8_t*)mask, (uint32_t)mr.div, (uint32_t)mr.mod, mr.stride,
                    rows, (int)N, flags};
   hipStream_t s = (hipStream_t)stream;
-  // few very long rows: the team forward (whole packs on 16-byte aligned tensors, no mask,
-  // Y apart from X -- a workgroup whose team does not come together reads the whole row
-  // again -- and no stream capture)
-  if (plan.team > 0 && !mask && ((((uintptr_t)x) | ((uintptr_t)y)) & 15u) == 0) {
+  // few very long rows: the team forward (rows of whole packs on 16-byte aligned tensors or rows of
+  // no whole number of packs, no mask, Y apart from X -- a workgroup whose team does not come
+  // together reads the whole row again -- and no stream capture)
+  if (plan.team > 0 && !mask && (!plan.fast || ((((uintptr_t)x) | ((uintptr_t)y)) & 15u) == 0)) {
     const char* xb = (const char*)x;
     const char* yb = (const char*)y;
     const size_t xbytes = (size_t)rows * (size_t)N * (size_t)esize_of(id);
@@ -501,7 +501,7 @@ int softmax_bwd(const void* grad, const void* y, const void* mask, void* gi, int
   // few very long rows: the team backward, under the rules of the forward (gi apart from
   // grad and y)
   if (plan.team > 0 && !mask &&
-      ((((uintptr_t)grad) | ((uintptr_t)y) | ((uintptr_t)gi)) & 15u) == 0) {
+      (!plan.fast || ((((uintptr_t)grad) | ((uintptr_t)y) | ((uintptr_t)gi)) & 15u) == 0)) {
     const char* ob = (const char*)gi;
     const size_t ibytes = (size_t)rows * (size_t)N * (size_t)esize_of(gd);
     const size_t obytes = (size_t)rows * (size_t)N * (size_t)esize_of(od);
@@ -993,8 +993,9 @@ int mi355x_rownorm_plan_at(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_
   out->packs_per_lane = plan.V;
   out->block_threads = plan.block;
   out->rows_per_block = plan.rpb;
-  // (a forward row held by a team of workgroups: the team and its grid)
-  const bool team = plan.team > 0 && !plan.team_small;
+  // (a row held by a team of workgroups: the team and its grid; softmax: of whole packs)
+  const bool softmax = op == ROWNORM_OP_SOFTMAX_FWD || op == ROWNORM_OP_SOFTMAX_BWD;
+  const bool team = plan.team > 0 && !plan.team_small && !(softmax && !plan.fast);
   out->reserved = team ? plan.team : (plan.split > 1 ? plan.split : 0);
   out->grid_blocks = team ? plan.team_grid : plan.grid;
   out->partial_rows = (int64_t)bwd_partial_rows(plan);

@@ -68,6 +68,9 @@ struct Plan {
   // softmax backward of rows beyond the registers of two tensors: grad alone fits
   // them (the log_softmax backward then keeps grad resident and streams y)
   bool grad_resident = false;
+  // softmax rows of no whole number of packs that one workgroup of tail_g lanes (1024, forward also 512) holds in
+  // tail_v whole packs a lane, tail_packs at most in all (0: not such a row)
+  int tail_v = 0, tail_g = 0, tail_packs = 0, tail_cus = 0;
   // a layout was asked for by override: kernels chosen by other means than the
   // layout (softmax of short ragged rows through LDS) stand back
   bool forced = false;
@@ -159,8 +162,29 @@ constexpr int kMaxV = 16;
 // The 16-bit softmax forward alone goes to 20 packs a lane (163840-element rows:
 // the 151936 / 152064-entry vocabularies).
 constexpr int kSoftmaxFwdMaxV16 = 20;
+// Packs of each of its two tensors a lane of the one-workgroup softmax backward holds at most.
+constexpr int kSoftmaxBwdHoldMaxV = 8;
 // Packs of grad a lane of the grad-resident log_softmax backward holds at most.
 constexpr int kGradResidentMaxV = 20;
+// Softmax rows of no whole number of packs beyond the resident layouts: 3 packs a lane at least, on one workgroup of
+// 1024 lanes (TAIL in softmax_kernels.hpp).  Against the multi-pass kernels, which read X, or grad and y, twice, bf16
+// us: [4096, 128255] log_softmax 453 -> 396, backward 621 -> 587; [4096, 50257] 161 -> 148, 238 -> 232; [515, 50220] softmax
+// 26.7 -> 25.4, 40.3 -> 34.5; [2000, 17001] 32.2 -> 26.8, 46.0 -> 37.7.  (The same on packs at the row's own alignment: a 16-byte
+// access two bytes off costs twice, [4096, 128255] 479 and 677.)
+constexpr int kSoftmaxTailMinV = 3;
+// The forward on 512 lanes where more and smaller workgroups a compute unit overlap better: the shortest of these rows
+// and calls of few rows (bf16 softmax, 1024 / 512 lanes: [4096, 17001] 54.1 / 50.0 us, [2000, 24570] 39.0 / 37.0, [1000,
+// 20005] 18.5 / 14.5, [512, 41003] 16.2 / 15.0, but [4096, 28003] 80.4 / 84.9, [2000, 41003] 61.9 / 62.9).
+constexpr int kSoftmaxTailHalfMaxV = 16;
+constexpr bool softmax_tail_half_lanes(int64_t packs, int64_t M, int num_cus) {
+  return packs <= 2560 || (packs <= 4096 && M <= 8 * (int64_t)num_cus) ||
+         (packs <= kMaxG / 2 * kSoftmaxTailHalfMaxV - 1024 && M <= 2 * (int64_t)num_cus);
+}
+// The log_softmax backward holds grad alone from here on (both tensors: [2000, 49001] 112 us, grad alone 106, the
+// multi-pass kernel 106; [1000, 65001] 81.4, 72.7, 74.8).
+constexpr int kSoftmaxTailGradMinV = 4;
+// Bytes up to which a second pass over the inputs comes out of the 256 MB cache behind the L2s.
+constexpr int64_t kSoftmaxCachedBytes = (int64_t)320 << 20;
 constexpr int max_v_of(OpClass oc, int esize) {
   return oc == OC_SOFTMAX_FWD && esize == 2 ? kSoftmaxFwdMaxV16 : kMaxV;
 }
@@ -1312,24 +1336,31 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
       }
     }
   }
-  // Softmax forward / backward of few, very long rows of whole packs: one workgroup a row
+  // Softmax forward / backward of few, very long rows: one workgroup a row
   // would leave most compute units idle, so each row is held by a team of workgroups
   // (softmax_fwd_team_kernel / softmax_bwd_team_kernel): as few workgroups a row as hold it
   // with 16 (backward: 8 of each tensor) packs a lane, then as many teams as there are rows
   // and room, and a row spread over all the workgroups its team can have.  More rows than
   // teams run in rounds; even then, and with few teams whose waits nothing hides, one
   // workgroup a row is several times slower (fp32 [2, 16777216]: 4800 us).
-  if (softmax && p.fast && !masked && ov.G == 0 && ov.V == 0 && ov.bpc == 0 && ov.block == 0 &&
-      2 * M <= num_cus && packs >= kSoftmaxTeamMinPacks) {
+  // Rows of no whole number of packs, where one workgroup a row has rows enough to hide its way through
+  // memory, go to teams only from there on (us, one workgroup a row / teams, bf16: forward [32, 36002] 7.2 / 6.8,
+  // [64, 32769] 7.5 / 7.8, [64, 60004] 9.4 / 8.1, [128, 45001] 9.1 / 9.5, [128, 110001] 14.6 / 15.1, [16, 110001] 13.0 /
+  // 7.4; backward [32, 32769] 6.5 / 6.5, [100, 45001] 8.7 / 10.2, [100, 60004] 12.4 / 8.6, [128, 80001] 20.0 / 16.2).
+  // Before both they went through softmax_*_stream_kernel: 7.9, 7.5, 11.5, 9.9, 19.2, 17.7; 7.4, 8.4, 10.4, 19.9.
+  const int64_t row_packs = (N + E - 1) / E;
+  const bool team_rows = p.fast || (oc == OC_SOFTMAX_FWD ? 48 : 24) * (M - 24) <= row_packs - kSoftmaxTeamMinPacks;
+  if (softmax && team_rows && !force_general && !masked && ov.G == 0 && ov.V == 0 && ov.bpc == 0 && ov.block == 0 &&
+      2 * M <= num_cus && row_packs >= kSoftmaxTeamMinPacks) {
     const int64_t cus = num_cus * kTeamPerCu < kTeamMaxWorkgroups ? num_cus * kTeamPerCu : kTeamMaxWorkgroups;
     const int max_v = oc == OC_SOFTMAX_FWD ? kTeamMaxV : kSoftmaxBwdTeamMaxV;
     const int64_t per_wg = (int64_t)kTeamBlock * max_v;
-    const int64_t team_min = (packs + per_wg - 1) / per_wg;
+    const int64_t team_min = (row_packs + per_wg - 1) / per_wg;
     int64_t teams = team_min <= cus ? cus / team_min : 0;
     if (teams > M) teams = M;
     if (teams >= 1) {
       int64_t team_max = cus / teams;
-      const int64_t strides = (packs + kTeamBlock - 1) / kTeamBlock;
+      const int64_t strides = (row_packs + kTeamBlock - 1) / kTeamBlock;
       if (team_max > strides) team_max = strides;
       const int64_t v = (strides + team_max - 1) / team_max;
       const int64_t team = (strides + v - 1) / v;
@@ -1339,6 +1370,18 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
         p.team_chunk_packs = v * kTeamBlock;
         p.team_grid = teams * team;
       }
+    }
+  }
+  if (softmax && !p.resident && !p.fast && !masked && !p.forced && ov.G == 0) {
+    const int64_t held = (N + 2 * (E - 1)) / E;  // packs of the window, whatever its head
+    const bool on_half = oc == OC_SOFTMAX_FWD && softmax_tail_half_lanes(held, M, num_cus);
+    const int64_t v = (held + (on_half ? kMaxG / 2 : kMaxG) - 1) / (on_half ? kMaxG / 2 : kMaxG);
+    const int most = oc == OC_SOFTMAX_FWD ? max_v_of(oc, esize) : kGradResidentMaxV;
+    if (v >= kSoftmaxTailMinV && v <= most) {
+      p.tail_v = (int)v;
+      p.tail_packs = (int)held;
+      p.tail_cus = num_cus;
+      p.tail_g = on_half ? kMaxG / 2 : kMaxG;
     }
   }
   if (oc == OC_SOFTMAX_BWD && !p.resident && p.fast && ov.G == 0 &&

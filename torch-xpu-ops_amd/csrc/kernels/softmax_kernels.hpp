@@ -79,6 +79,34 @@ __device__ __forceinline__ Pack<T, E> stream_load(const T* row, int e0, int n, b
 // Packs a thread of the multi-pass kernels requests before using the first.
 constexpr int kStreamUnroll = 2;
 
+// TAIL kernels hold a row of no whole number of packs in V packs a lane of one workgroup of G lanes:
+// the 16-byte aligned window that holds the row, whose packs number (V - 1) * G or more whatever the
+// row's head.  So only a lane's first and last two packs can hold elements outside the row (edge_pack),
+// only the last can lie outside altogether, and everything else is the whole-pack kernels' straight-line code.
+template <int V>
+constexpr bool edge_pack(int c) {
+  return c == 0 || c >= V - 2;
+}
+// Pack c of this lane: a base that all lanes share and 32 bits of the lane's own (64-bit addresses a lane and
+// pack cost a register or two a pack; from 10 packs a lane on the forward, one workgroup a compute unit either way, is
+// 1 to 10 % faster with them).  `packs` in the window.
+template <int G, int V, class T>
+__device__ __forceinline__ T* tail_at(T* win, int c, int lane, int packs, int E) {
+  const int first = c < V - 1 ? c * G : (packs - 1 < c * G ? packs - 1 : c * G);
+  const int mine = c < V - 1 || lane < packs - first ? lane : packs - 1 - first;
+  using Byte = std::conditional_t<std::is_const<T>::value, const char, char>;
+  return reinterpret_cast<T*>(reinterpret_cast<Byte*>(win + first * E) + (uint32_t)mine * (uint32_t)(E * sizeof(T)));
+}
+template <class T, int E>
+__device__ __forceinline__ void trim_edge_pack(Pack<T, E>& p, int e0, int n, float fill, int lo) {
+  if (e0 < lo || e0 + E > n) {
+    asm volatile("" : "+v"(e0));  // (the index arithmetic stays inside the branch)
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+      if (e0 + i < lo || e0 + i >= n) p.v[i] = (T)fill;
+  }
+}
+
 // Rows of more than this many elements a lane are kept in storage format.
 constexpr int kSoftmaxWideElems = 16;
 
@@ -127,14 +155,17 @@ constexpr int softmax_fwd_min_blocks() {
   return (G == 1024 && FAST && !MASKED && V >= 5 && V <= kSoftmaxFreshOffsetsMaxV) ? 8 : 1;
 }
 
-template <class TI, class TO, int G, int V, int BLOCK, bool FAST, bool MASKED>
+// TAIL: see edge_pack().  HBM-bound like the whole-pack rows, once the row is read once; what it
+// measured stands at kSoftmaxTailMinV.
+template <class TI, class TO, int G, int V, int BLOCK, bool FAST, bool MASKED, bool TAIL = false>
 __global__ void __launch_bounds__(BLOCK, (softmax_fwd_min_blocks<TI, G, V, FAST, MASKED>()))
 softmax_fwd_resident_kernel(const TI* __restrict__ x, TO* __restrict__ y, MaskRef mask, int64_t M,
                             int N, int flags) {
   constexpr int E = elems_per_pack<TI>::value;
   constexpr int RPB = BLOCK / G;
+  static_assert(!TAIL || (FAST && !MASKED && G == BLOCK && V * E > kSoftmaxWideElems), "one row a workgroup");
   constexpr bool PRECISE = sizeof(TO) == 4;
-  constexpr bool WINDOW = !FAST && softmax_row_window<TI>();
+  constexpr bool WINDOW = TAIL || (!FAST && softmax_row_window<TI>());
   __shared__ float red[reduce_lds_floats<G, BLOCK, 1>::value];
   int phase = 0;
   const int slot = threadIdx.x / G;
@@ -164,11 +195,34 @@ softmax_fwd_resident_kernel(const TI* __restrict__ x, TO* __restrict__ y, MaskRe
     TO* yr = y + row * (int64_t)N - h;
     Pack<TI, E> xp[V];
 #pragma unroll
-    for (int c = 0; c < V; ++c)
-      xp[c] = row_load<TI, E, true, FAST>(xr, (c * G + lane) * E, nw, ok, -INFINITY, h, WINDOW);
+    for (int c = 0; c < V; ++c) {
+      const int e0 = (c * G + lane) * E;
+      if constexpr (TAIL)
+        xp[c] = Pack<TI, E>::load_stream(V < 10 ? tail_at<G, V>(xr, c, lane, (nw + E - 1) / E, E)
+                                                       : xr + (c < V - 1 || e0 < nw ? e0 : 0));
+      else
+        xp[c] = row_load<TI, E, true, FAST>(xr, e0, nw, ok, -INFINITY, h, WINDOW);
+    }
 #pragma unroll
-    for (int c = 0; c < V; ++c)
-      row_trim<TI, E, FAST>(xp[c], (c * G + lane) * E, nw, -INFINITY, h, WINDOW);
+    for (int c = 0; c < V; ++c) {
+      const int e0 = (c * G + lane) * E;
+      if constexpr (TAIL) {
+        if (edge_pack<V>(c)) trim_edge_pack<TI, E>(xp[c], e0, nw, -INFINITY, h);
+      } else {
+        row_trim<TI, E, FAST>(xp[c], e0, nw, -INFINITY, h, WINDOW);
+      }
+    }
+    auto put = [&](int c, int ls, const Pack<TO, E>& o) {
+      const int e0 = (c * G + ls) * E;
+      if constexpr (TAIL) {
+        if (edge_pack<V>(c))
+          store_row_pack<TO, E, true>(yr, e0, nw, true, o, h);
+        else
+          o.store_stream(V < 10 ? tail_at<G, V>(yr, c, ls, (nw + E - 1) / E, E) : yr + e0);
+      } else {
+        row_store<TO, E, true, FAST>(yr, e0, nw, ok, o, h);
+      }
+    };
     if constexpr (V * E > kSoftmaxWideElems) {
       // Long rows (a vocabulary-sized row is 16 packs a lane): the row stays in
       // storage format and each of the three passes widens it again; softmax
@@ -247,7 +301,7 @@ softmax_fwd_resident_kernel(const TI* __restrict__ x, TO* __restrict__ y, MaskRe
           Pack<TO, E> o;
 #pragma unroll
           for (int i = 0; i < E; ++i) o.set(i, (xp[c].get(i) - m) - k);
-          row_store<TO, E, true, FAST>(yr, (c * G + ls) * E, nw, ok, o, h);
+          put(c, ls, o);
         }
       } else if (is_safe) {
         ROWNORM_UNIFORM_ARM("safe softmax: zeros for a row without a finite element");
@@ -261,7 +315,7 @@ softmax_fwd_resident_kernel(const TI* __restrict__ x, TO* __restrict__ y, MaskRe
 #pragma unroll
           for (int i = 0; i < E; ++i)
             o.set(i, zero_row ? 0.0f : row_exp<PRECISE>(xp[c].get(i) - m) * k);
-          row_store<TO, E, true, FAST>(yr, (c * G + ls) * E, nw, ok, o, h);
+          put(c, ls, o);
         }
       } else {
         ROWNORM_UNIFORM_ARM("softmax: exp(x - max) / sum");
@@ -273,7 +327,7 @@ softmax_fwd_resident_kernel(const TI* __restrict__ x, TO* __restrict__ y, MaskRe
           Pack<TO, E> o;
 #pragma unroll
           for (int i = 0; i < E; ++i) o.set(i, row_exp<PRECISE>(xp[c].get(i) - m) * k);
-          row_store<TO, E, true, FAST>(yr, (c * G + ls) * E, nw, ok, o, h);
+          put(c, ls, o);
         }
       }
       continue;
@@ -465,8 +519,7 @@ softmax_fwd_stream_kernel(const TI* __restrict__ x, TO* __restrict__ y, MaskRef 
 }
 
 // ---------------------------------------------------------------------------
-// Forward for few, very long rows of whole packs (fewer rows than half the compute units;
-// 16-byte aligned X and Y, no mask): a row is held in the registers of a team of
+// Forward for few, very long rows (fewer rows than half the compute units; no mask): a row is held in the registers of a team of
 // workgroups, as in the norm forward for rows beyond the registers (norm_fwd_team_kernel).
 // The grid is at most two workgroups of 512 threads a compute unit, all resident at once;
 // workgroup b belongs to team b / team and keeps chunk b % team of the team's current
@@ -480,7 +533,9 @@ softmax_fwd_stream_kernel(const TI* __restrict__ x, TO* __restrict__ y, MaskRef 
 // units idle.  A workgroup whose wait runs out takes the whole row's maximum and sum
 // itself (a second pass over X, which no workgroup writes: Y must not overlap X), loads
 // its chunk again and goes on; every wave reaches the end of the kernel whatever the
-// other workgroups do.  What bounds few rows is the way from the last chunk's sum to the
+// other workgroups do.  In a row of no whole number of packs the last chunk starts a few elements
+// early (`before`) and ends with the row: every access is a whole pack, the chunk's sum leaves out
+// the elements that the chunk before holds as well, and both store the same values there.  What bounds few rows is the way from the last chunk's sum to the
 // first store, so the pair crosses as self-validating words (one round trip; a tag beside
 // the numbers, three): bf16 [16, 262144] 8.5 -> 7.4 us, [2, 1048576] 11.3 -> 8.8, [128,
 // 140000] 16.1 -> 15.2; backward 8.1 -> 7.0, 10.7 -> 7.4, 23.6 -> 22.0.
@@ -501,12 +556,14 @@ softmax_fwd_team_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t M,
   const int tm = (int)blockIdx.x / team;
   const int c = (int)blockIdx.x - tm * team;
   const int teams = (int)gridDim.x / team;
-  const int npacks = N / E;
+  const int npacks = (N + E - 1) / E;
   const int64_t p0 = (int64_t)c * chunk_packs;
   const int64_t p1 = p0 + chunk_packs < npacks ? p0 + chunk_packs : npacks;
   const int nloc = p1 > p0 ? (int)(p1 - p0) : 0;  // packs of this chunk
   const bool full = nloc == V * BLOCK;  // (uniform) all chunks but a row's last
-  const int64_t pbase = nloc > 0 ? p0 : 0;
+  // (a ragged row's last chunk starts `before` elements early, so that it ends with the row)
+  const int before = nloc > 0 && p1 == npacks ? npacks * E - N : 0;
+  const int64_t base = nloc > 0 ? p0 * E - before : 0;
   const uint32_t loff = (uint32_t)(threadIdx.x * 16);
   const uint32_t ooff = (uint32_t)(threadIdx.x * E * sizeof(TO));
   // (the sum is formed as a pointer into global memory: a pointer made from an integer
@@ -521,7 +578,7 @@ softmax_fwd_team_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t M,
   for (int64_t row = tm; row < M; row += teams, ++round) {
     TeamEntry* entries = slot->entry[round & 1u];
     const TI* xr = x + row * (int64_t)N;
-    const TI* xb = xr + pbase * E;
+    const TI* xb = xr + base;
     Pack<TI, E> xp[V];
     auto load_chunk = [&]() {
       if (full) {
@@ -552,10 +609,15 @@ softmax_fwd_team_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t M,
     // (nothing finite in the chunk: against 0, -inf elements add 0 and NaN still poisons)
     const float ref = m_c == -INFINITY ? 0.0f : m_c;
     float acc = 0.0f;
+    // (the maximum may know the elements before the chunk: they are the row's)
+    const int d = threadIdx.x == 0 ? before : 0;
 #pragma unroll
     for (int k = 0; k < V; ++k)
 #pragma unroll
-      for (int i = 0; i < E; ++i) acc += row_exp<PRECISE>(xp[k].get(i) - ref);
+      for (int i = 0; i < E; ++i) {
+        const float e = row_exp<PRECISE>(xp[k].get(i) - ref);
+        acc += k == 0 && i < d ? 0.0f : e;
+      }
 #pragma unroll
     for (int k = 0; k < V; ++k) keep_packed(xp[k]);
     float sm[1] = {acc};
@@ -601,8 +663,7 @@ softmax_fwd_team_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t M,
 #pragma unroll
         for (int u = 0; u < kStreamUnroll; ++u) {
           const int pk = pk0 + u * BLOCK;
-          pv[u] = Pack<TI, E>::splat(-INFINITY);
-          if (pk < npacks) pv[u] = Pack<TI, E>::load(xr + (int64_t)pk * E);
+          pv[u] = load_row_pack<TI, E, false>(xr, pk * E, N, pk < npacks, -INFINITY);
         }
 #pragma unroll
         for (int u = 0; u < kStreamUnroll; ++u) {
@@ -632,7 +693,7 @@ softmax_fwd_team_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t M,
     }
     const float m = stat[0], kk = stat[1];
     const bool zero_row = is_safe && m == -INFINITY;
-    TO* yb = y + row * (int64_t)N + pbase * E;
+    TO* yb = y + row * (int64_t)N + base;
 #pragma unroll
     for (int k = 0; k < V; ++k) {
       if (full || k * BLOCK + (int)threadIdx.x < nloc) {
@@ -659,14 +720,15 @@ softmax_fwd_team_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t M,
 
 // Backward.  TG: dtype of grad and of y (the saved forward output); TO: dtype
 // of the input gradient.
-template <class TG, class TO, int G, int V, int BLOCK, bool FAST, bool MASKED>
+// TAIL: as in the forward; y must be aligned like grad (the launcher's rule).
+template <class TG, class TO, int G, int V, int BLOCK, bool FAST, bool MASKED, bool TAIL = false>
 __global__ void __launch_bounds__(BLOCK)
 softmax_bwd_resident_kernel(const TG* __restrict__ grad, const TG* __restrict__ y,
                             TO* __restrict__ gi, MaskRef mask, int64_t M, int N, int flags) {
   constexpr int E = elems_per_pack<TG>::value;
   constexpr int RPB = BLOCK / G;
   constexpr bool PRECISE = sizeof(TO) == 4 && sizeof(TG) == 4;
-  constexpr bool WINDOW = !FAST && softmax_row_window<TG>();
+  constexpr bool WINDOW = TAIL || (!FAST && softmax_row_window<TG>());
   __shared__ float red[reduce_lds_floats<G, BLOCK, 1>::value];
   int phase = 0;
   const int slot = threadIdx.x / G;
@@ -677,7 +739,8 @@ softmax_bwd_resident_kernel(const TG* __restrict__ grad, const TG* __restrict__ 
   // 16-bit rows of more than 4 packs a lane on 1024 lanes: both tensors stay in storage
   // format across the reduction and are widened again for the output (as fp32 copies
   // they would take 16 registers a pack)
-  constexpr bool kPacked = FAST && !MASKED && G == 1024 && V > 4 && sizeof(TG) == 2;
+  static_assert(!TAIL || (FAST && !MASKED && G == BLOCK), "one row a workgroup");
+  constexpr bool kPacked = TAIL || (FAST && !MASKED && G == 1024 && V > 4 && sizeof(TG) == 2);
   const int64_t nrb = (M + RPB - 1) / RPB;
   for (int64_t rb = blockIdx.x; rb < nrb; rb += gridDim.x) {
     // ragged rows: opaque once a row and again before the stores (see the forward;
@@ -696,12 +759,24 @@ softmax_bwd_resident_kernel(const TG* __restrict__ grad, const TG* __restrict__ 
 #pragma unroll
     for (int c = 0; c < V; ++c) {
       const int e0 = (c * G + lane) * E;
+      if constexpr (TAIL) {
+        pg[c] = Pack<TG, E>::load_stream(tail_at<G, V>(gr, c, lane, (nw + E - 1) / E, E));
+        py[c] = Pack<TG, E>::load_stream(tail_at<G, V>(yr, c, lane, (nw + E - 1) / E, E));
+        continue;
+      }
       pg[c] = row_load<TG, E, true, FAST>(gr, e0, nw, ok, 0.0f, h, WINDOW);
       py[c] = row_load<TG, E, true, FAST>(yr, e0, nw, ok, 0.0f, h, y_whole);
     }
 #pragma unroll
     for (int c = 0; c < V; ++c) {
       const int e0 = (c * G + lane) * E;
+      if constexpr (TAIL) {
+        if (edge_pack<V>(c)) {
+          trim_edge_pack<TG, E>(pg[c], e0, nw, 0.0f, h);
+          trim_edge_pack<TG, E>(py[c], e0, nw, 0.0f, h);
+        }
+        continue;
+      }
       row_trim<TG, E, FAST, true>(pg[c], e0, nw, 0.0f, h, WINDOW);
       row_trim<TG, E, FAST, true>(py[c], e0, nw, 0.0f, h, y_whole);
     }
@@ -710,15 +785,26 @@ softmax_bwd_resident_kernel(const TG* __restrict__ grad, const TG* __restrict__ 
       if (is_log) {
         ROWNORM_UNIFORM_ARM("log_softmax backward: sum of grad");
 #pragma unroll
-        for (int c = 0; c < V; ++c)
+        for (int c = 0; c < V; ++c) {
 #pragma unroll
           for (int i = 0; i < E; ++i) sum[0] += pg[c].get(i);
+          if constexpr (TAIL) __builtin_amdgcn_sched_barrier(0);  // (one pack widened at a time)
+        }
       } else {
         ROWNORM_UNIFORM_ARM("softmax backward: sum of y * grad");
 #pragma unroll
-        for (int c = 0; c < V; ++c)
+        for (int c = 0; c < V; ++c) {
 #pragma unroll
           for (int i = 0; i < E; ++i) sum[0] = fmaf(py[c].get(i), pg[c].get(i), sum[0]);
+          if constexpr (TAIL) __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      if constexpr (TAIL) {
+#pragma unroll
+        for (int c = 0; c < V; ++c) {
+          keep_packed(pg[c]);
+          keep_packed(py[c]);
+        }
       }
       group_allreduce<G, BLOCK, 1, SumOp>(sum, red, phase);
       float s = sum[0];
@@ -733,7 +819,16 @@ softmax_bwd_resident_kernel(const TG* __restrict__ grad, const TG* __restrict__ 
           const float gv = pg[c].get(i), yv = py[c].get(i);
           o.set(i, is_log ? gv - row_exp<PRECISE>(yv) * s : yv * (gv - s));
         }
-        row_store<TO, E, true, FAST>(outr, (c * G + ls) * E, nw, ok, o, h);
+        const int e0 = (c * G + ls) * E;
+        if constexpr (TAIL) {
+          if (edge_pack<V>(c))
+            store_row_pack<TO, E, true>(outr, e0, nw, true, o, h);
+          else
+            o.store_stream(tail_at<G, V>(outr, c, ls, (nw + E - 1) / E, E));
+          __builtin_amdgcn_sched_barrier(0);
+        } else {
+          row_store<TO, E, true, FAST>(outr, e0, nw, ok, o, h);
+        }
       }
       continue;
     }
@@ -925,9 +1020,11 @@ softmax_bwd_flat_kernel(const T* __restrict__ grad, const T* __restrict__ y, T* 
 // number of packs and V = ceil(packs / BLOCK) exactly, so only a lane's last pack
 // can lie beyond the row end (it is requested from the row's first pack and never
 // used) and the others sit at constant strides from the lane's first.
+//
+// TAIL: rows of no whole number of packs, as in softmax_bwd_resident_kernel.
 constexpr int kGradResidentUnroll = 4;
 
-template <class TG, class TO, int V, int BLOCK>
+template <class TG, class TO, int V, int BLOCK, bool TAIL = false>
 __global__ void __launch_bounds__(BLOCK)
 log_softmax_bwd_grad_resident_kernel(const TG* __restrict__ grad, const TG* __restrict__ y,
                                      TO* __restrict__ gi, int64_t M, int N) {
@@ -937,11 +1034,13 @@ log_softmax_bwd_grad_resident_kernel(const TG* __restrict__ grad, const TG* __re
   __shared__ float red[reduce_lds_floats<BLOCK, BLOCK, 1>::value];
   int phase = 0;
   const int lane = threadIdx.x;
-  const bool last_in = ((V - 1) * BLOCK + lane) * E < N;  // this lane's last pack lies in the row
   for (int64_t row = blockIdx.x; row < M; row += gridDim.x) {
-    const TG* gr = grad + row * (int64_t)N + lane * E;
-    const TG* yr = y + row * (int64_t)N + lane * E;
-    TO* outr = gi + row * (int64_t)N + lane * E;
+    const int h = TAIL ? window_head<TG, E>(grad + row * (int64_t)N) : 0;
+    const int nw = N + h;
+    const bool last_in = ((V - 1) * BLOCK + lane) * E < nw;  // this lane's last pack lies in the row
+    const TG* gr = grad + row * (int64_t)N - h + lane * E;
+    const TG* yr = y + row * (int64_t)N - h + lane * E;
+    TO* outr = gi + row * (int64_t)N - h + lane * E;
     // element offset of pack c from the lane's first pack
     auto off = [&](int c) { return (c < V - 1 || last_in) ? c * BLOCK * E : 0; };
     Pack<TG, E> pg[V], py[U], pn[U];
@@ -955,6 +1054,11 @@ log_softmax_bwd_grad_resident_kernel(const TG* __restrict__ grad, const TG* __re
     request_y(0, pn);  // on its way while grad is summed
     float sum[1] = {0.0f};
     if (!last_in) pg[V - 1] = Pack<TG, E>::zero();
+    if constexpr (TAIL) {
+#pragma unroll
+      for (int c = 0; c < V; ++c)
+        if (edge_pack<V>(c)) trim_edge_pack<TG, E>(pg[c], (c * BLOCK + lane) * E, nw, 0.0f, h);
+    }
 #pragma unroll
     for (int c = 0; c < V; ++c)
 #pragma unroll
@@ -974,7 +1078,10 @@ log_softmax_bwd_grad_resident_kernel(const TG* __restrict__ grad, const TG* __re
 #pragma unroll
           for (int i = 0; i < E; ++i)
             o.set(i, pg[c0 + u].get(i) - row_exp<PRECISE>(py[u].get(i)) * s);
-          if (c0 + u < V - 1 || last_in) o.store_stream(outr + (c0 + u) * BLOCK * E);
+          if (TAIL && edge_pack<V>(c0 + u))
+            store_row_pack<TO, E, true>(outr - lane * E, ((c0 + u) * BLOCK + lane) * E, nw, true, o, h);
+          else if (c0 + u < V - 1 || last_in)
+            o.store_stream(outr + (c0 + u) * BLOCK * E);
         }
       }
     }
@@ -1099,12 +1206,14 @@ softmax_bwd_team_kernel(const TG* __restrict__ grad, const TG* __restrict__ y, T
   const int tm = (int)blockIdx.x / team;
   const int c = (int)blockIdx.x - tm * team;
   const int teams = (int)gridDim.x / team;
-  const int npacks = N / E;
+  const int npacks = (N + E - 1) / E;
   const int64_t p0 = (int64_t)c * chunk_packs;
   const int64_t p1 = p0 + chunk_packs < npacks ? p0 + chunk_packs : npacks;
   const int nloc = p1 > p0 ? (int)(p1 - p0) : 0;  // packs of this chunk
   const bool full = nloc == V * BLOCK;  // (uniform) all chunks but a row's last
-  const int64_t pbase = nloc > 0 ? p0 : 0;
+  // (a ragged row's last chunk starts `before` elements early, so that it ends with the row)
+  const int before = nloc > 0 && p1 == npacks ? npacks * E - N : 0;
+  const int64_t base = nloc > 0 ? p0 * E - before : 0;
   const uint32_t loff = (uint32_t)(threadIdx.x * 16);
   const uint32_t ooff = (uint32_t)(threadIdx.x * E * sizeof(TO));
   // (a pointer into global memory, as in the forward)
@@ -1119,8 +1228,8 @@ softmax_bwd_team_kernel(const TG* __restrict__ grad, const TG* __restrict__ y, T
     TeamEntry* entries = slot->entry[round & 1u];
     const TG* gr = grad + row * (int64_t)N;
     const TG* yr = y + row * (int64_t)N;
-    const TG* gb = gr + pbase * E;
-    const TG* yb = yr + pbase * E;
+    const TG* gb = gr + base;
+    const TG* yb = yr + base;
     Pack<TG, E> gp[V], yp[V];
     auto load_chunk = [&]() {
       if (full) {
@@ -1144,12 +1253,13 @@ softmax_bwd_team_kernel(const TG* __restrict__ grad, const TG* __restrict__ y, T
     };
     load_chunk();
     float sum[1] = {0.0f};
+    const int d = threadIdx.x == 0 ? before : 0;
     if (is_log) {
       ROWNORM_UNIFORM_ARM("log_softmax backward: sum of grad");
 #pragma unroll
       for (int k = 0; k < V; ++k) {
 #pragma unroll
-        for (int i = 0; i < E; ++i) sum[0] += gp[k].get(i);
+        for (int i = 0; i < E; ++i) sum[0] += k == 0 && i < d ? 0.0f : gp[k].get(i);
         __builtin_amdgcn_sched_barrier(0);  // (one pack widened at a time: registers)
       }
     } else {
@@ -1157,7 +1267,10 @@ softmax_bwd_team_kernel(const TG* __restrict__ grad, const TG* __restrict__ y, T
 #pragma unroll
       for (int k = 0; k < V; ++k) {
 #pragma unroll
-        for (int i = 0; i < E; ++i) sum[0] = fmaf(yp[k].get(i), gp[k].get(i), sum[0]);
+        for (int i = 0; i < E; ++i) {
+          const float with = fmaf(yp[k].get(i), gp[k].get(i), sum[0]);
+          sum[0] = k == 0 && i < d ? sum[0] : with;
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -1201,12 +1314,8 @@ softmax_bwd_team_kernel(const TG* __restrict__ grad, const TG* __restrict__ y, T
 #pragma unroll
         for (int u = 0; u < kStreamUnroll; ++u) {
           const int pk = pk0 + u * BLOCK;
-          pg[u] = Pack<TG, E>::zero();
-          py[u] = Pack<TG, E>::zero();
-          if (pk < npacks) {
-            pg[u] = Pack<TG, E>::load(gr + (int64_t)pk * E);
-            if (!is_log) py[u] = Pack<TG, E>::load(yr + (int64_t)pk * E);
-          }
+          pg[u] = load_row_pack<TG, E, false>(gr, pk * E, N, pk < npacks, 0.0f);
+          py[u] = load_row_pack<TG, E, false>(yr, pk * E, N, pk < npacks && !is_log, 0.0f);
         }
 #pragma unroll
         for (int u = 0; u < kStreamUnroll; ++u)
@@ -1220,7 +1329,7 @@ softmax_bwd_team_kernel(const TG* __restrict__ grad, const TG* __restrict__ y, T
       load_chunk();
     }
     const float s = stat[0];
-    TO* ob = gi + row * (int64_t)N + pbase * E;
+    TO* ob = gi + row * (int64_t)N + base;
 #pragma unroll
     for (int k = 0; k < V; ++k) {
       if (full || k * BLOCK + (int)threadIdx.x < nloc) {

@@ -98,6 +98,89 @@ bool launch_softmax_bwd_flat(FlatLayout f, const SoftmaxBwdArgs& a, hipStream_t 
   return false;
 }
 
+// Rows of no whole number of packs beyond the resident layouts, held by one workgroup of 1024 lanes
+// all the same (TAIL in the kernels).  False: not this case.
+#define ROWNORM_TAIL_CASES(CASE)                                                                 \
+  CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(9) CASE(10) CASE(11) CASE(12) CASE(13)    \
+  CASE(14) CASE(15) CASE(16) CASE(17) CASE(18) CASE(19) CASE(20)
+template <class T>
+constexpr bool softmax_tail_built(int g, int v, int most) {
+  return v <= (g == kMaxG ? most : kSoftmaxTailHalfMaxV) && v * elems_per_pack<T>::value > kSoftmaxWideElems;
+}
+
+template <class TI, class TO, int G, int V>
+bool launch_softmax_fwd_tail_v(const Plan& plan, const SoftmaxFwdArgs& a, hipStream_t stream) {
+  if constexpr (softmax_tail_built<TI>(G, V, max_v_of(OC_SOFTMAX_FWD, sizeof(TI))) && V != 17 && V != 19) {
+    hipLaunchKernelGGL((softmax_fwd_resident_kernel<TI, TO, G, V, G, true, false, true>),
+                       dim3((unsigned)plan.grid), dim3(G), 0, stream, (const TI*)a.x, (TO*)a.y,
+                       MaskRef{}, a.M, a.N, a.flags);
+    return true;
+  }
+  return false;
+}
+
+template <class TI, class TO>
+bool launch_softmax_fwd_tail(const Plan& plan, const SoftmaxFwdArgs& a, hipStream_t stream) {
+  // log_softmax of 6 or 7 packs a lane out of the cache: the two passes, with their two workgroups a compute unit at
+  // different places of a row, measured faster ([2000, 49001] 65.8 us against 73.5, [2000, 57001] 80.6 against 85.7, but
+  // [1000, 57001] 43.7 against 43.1 and [4096, 49001] 154 against 146)
+  if ((a.flags & kSoftmaxLog) && plan.tail_g == kMaxG && (plan.tail_v == 6 || plan.tail_v == 7) &&
+      a.M > 4 * (int64_t)plan.tail_cus && a.M * (int64_t)a.N * (int64_t)sizeof(TI) <= kSoftmaxCachedBytes)
+    return false;
+  // (17 and 19 packs a lane measured slower than the two passes as well, 16, 18 and 20 faster: [1603, 133540] 182 us
+  // against 187, [1603, 152001] 214 against 231; [1603, 131001] 182 against 166, [1603, 140001] 199 against 185)
+  if (plan.tail_v == 17 || plan.tail_v == 19) return false;
+  switch (plan.tail_v) {
+#define ROWNORM_TAIL_FWD(v)                                                                  \
+  case v:                                                                                    \
+    return plan.tail_g == kMaxG ? launch_softmax_fwd_tail_v<TI, TO, kMaxG, v>(plan, a, stream)     \
+                                : launch_softmax_fwd_tail_v<TI, TO, kMaxG / 2, v>(plan, a, stream);
+    ROWNORM_TAIL_CASES(ROWNORM_TAIL_FWD)
+#undef ROWNORM_TAIL_FWD
+  }
+  return false;
+}
+
+template <class TG, class TO, int V>
+bool launch_softmax_bwd_tail_v(const Plan& plan, const SoftmaxBwdArgs& a, hipStream_t stream) {
+  constexpr bool BUILT = softmax_tail_built<TG>(kMaxG, V, kGradResidentMaxV);
+  if constexpr (BUILT && V >= kSoftmaxTailGradMinV) {
+    if (a.flags & kSoftmaxLog) {
+      hipLaunchKernelGGL((log_softmax_bwd_grad_resident_kernel<TG, TO, V, kStreamBlock, true>),
+                         dim3((unsigned)plan.grid), dim3(kStreamBlock), 0, stream,
+                         (const TG*)a.grad, (const TG*)a.y, (TO*)a.gi, a.M, a.N);
+      return true;
+    }
+  }
+  if constexpr (BUILT && V <= kSoftmaxBwdHoldMaxV) {
+    hipLaunchKernelGGL((softmax_bwd_resident_kernel<TG, TO, kMaxG, V, kMaxG, true, false, true>),
+                       dim3((unsigned)plan.grid), dim3(kMaxG), 0, stream, (const TG*)a.grad,
+                       (const TG*)a.y, (TO*)a.gi, MaskRef{}, a.M, a.N, a.flags);
+    return true;
+  }
+  return false;
+}
+
+template <class TG, class TO>
+bool launch_softmax_bwd_tail(const Plan& plan, const SoftmaxBwdArgs& a, hipStream_t stream) {
+  if ((((uintptr_t)a.grad ^ (uintptr_t)a.y) & 15u) != 0) return false;  // (y in grad's window)
+  // softmax rows that leave much of 4 or 5 packs a lane empty, out of the cache, likewise: both tensors in registers
+  // are one workgroup a compute unit ([1000, 28003] 31.6 us against 33.3, [2000, 35001] 76.3 against 79.2, but [2000, 32750]
+  // 88.0 against 73.3, [4096, 28003] 145 against 129)
+  const bool few = a.M <= 2 * (int64_t)plan.tail_cus;
+  if (!(a.flags & kSoftmaxLog) &&
+      ((plan.tail_v == 4 && plan.tail_packs <= 3840) || (plan.tail_v == 5 && plan.tail_packs <= 4608 && !few)) &&
+      2 * a.M * (int64_t)a.N * (int64_t)sizeof(TG) <= kSoftmaxCachedBytes)
+    return false;
+  switch (plan.tail_v) {
+#define ROWNORM_TAIL_BWD(v)                                                                  \
+  case v: return launch_softmax_bwd_tail_v<TG, TO, v>(plan, a, stream);
+    ROWNORM_TAIL_CASES(ROWNORM_TAIL_BWD)
+#undef ROWNORM_TAIL_BWD
+  }
+  return false;
+}
+
 template <class TI, class TO, bool MASKED>
 int launch_softmax_fwd_m(const Plan& plan, const SoftmaxFwdArgs& a, hipStream_t stream) {
   if constexpr (!MASKED && std::is_same<TI, TO>::value) {
@@ -133,6 +216,8 @@ int launch_softmax_fwd_m(const Plan& plan, const SoftmaxFwdArgs& a, hipStream_t 
         plan.fast ? launch_variant<SoftmaxFwdLauncher<TI, TO, true, MASKED>::template At>(ctx)
                   : launch_variant<SoftmaxFwdLauncher<TI, TO, false, MASKED>::template At>(ctx);
     if (!launched) return (int)hipErrorInvalidConfiguration;
+  } else if (!MASKED && launch_softmax_fwd_tail<TI, TO>(plan, a, stream)) {
+    // (rows of no whole number of packs, read once)
   } else {
     hipLaunchKernelGGL((softmax_fwd_stream_kernel<TI, TO, kStreamBlock, MASKED>),
                        dim3((unsigned)plan.grid), dim3(kStreamBlock), 0, stream, (const TI*)a.x,
@@ -244,7 +329,9 @@ int launch_softmax_bwd_m(const Plan& plan, const SoftmaxBwdArgs& a, hipStream_t 
                   : launch_variant<SoftmaxBwdLauncher<TG, TO, false, MASKED>::template At>(ctx);
     if (!launched) return (int)hipErrorInvalidConfiguration;
   } else if (!MASKED && launch_log_softmax_bwd_grad_resident<TG, TO>(plan, a, stream)) {
-    // (log_softmax rows of up to 16 packs a lane: grad resident, y streamed)
+    // (log_softmax rows of up to 20 packs a lane: grad resident, y streamed)
+  } else if (!MASKED && launch_softmax_bwd_tail<TG, TO>(plan, a, stream)) {
+    // (rows of no whole number of packs, read once)
   } else {
     hipLaunchKernelGGL((softmax_bwd_stream_kernel<TG, TO, kStreamBlock, MASKED>),
                        dim3((unsigned)plan.grid), dim3(kStreamBlock), 0, stream,
