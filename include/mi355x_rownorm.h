@@ -391,7 +391,8 @@ int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_si
  * that is ROWNORM_ERR_OVERRIDE for a masked call).
  * Softmax calls on longer ragged rows without a mask are held by one workgroup all the same (up to 20 packs a lane;
  * the backward: 8, log_softmax 20, with Y aligned like grad), few of them by teams; neither is reported here, where
- * such rows appear as the multi-pass layout that serves them otherwise.
+ * such rows appear as the multi-pass layout that serves them otherwise.  Rows of whole packs reported with a team run
+ * on one workgroup each where the calls have many rows for their length and that is faster.
  * Fewer than eight forward rows of whole packs beyond one workgroup's registers are held by teams of at most an
  * eighth of the machine where the conditions of mi355x_rownorm_set_team_wait_us allow it; reported is the layout
  * they have otherwise.

@@ -464,7 +464,7 @@ int softmax_fwd(const void* x, const void* mask, void* y, int64_t rows, int64_t 
   // few very long rows: the team forward (rows of whole packs on 16-byte aligned tensors or rows of
   // no whole number of packs, no mask, Y apart from X -- a workgroup whose team does not come
   // together reads the whole row again -- and no stream capture)
-  if (plan.team > 0 && !mask && (!plan.fast || ((((uintptr_t)x) | ((uintptr_t)y)) & 15u) == 0)) {
+  if (plan.team > 0 && !plan.team_idle && !mask && (!plan.fast || ((((uintptr_t)x) | ((uintptr_t)y)) & 15u) == 0)) {
     const char* xb = (const char*)x;
     const char* yb = (const char*)y;
     const size_t xbytes = (size_t)rows * (size_t)N * (size_t)esize_of(id);
@@ -500,7 +500,7 @@ int softmax_bwd(const void* grad, const void* y, const void* mask, void* gi, int
   hipStream_t s = (hipStream_t)stream;
   // few very long rows: the team backward, under the rules of the forward (gi apart from
   // grad and y)
-  if (plan.team > 0 && !mask &&
+  if (plan.team > 0 && !plan.team_idle && !mask &&
       (!plan.fast || ((((uintptr_t)grad) | ((uintptr_t)y) | ((uintptr_t)gi)) & 15u) == 0)) {
     const char* ob = (const char*)gi;
     const size_t ibytes = (size_t)rows * (size_t)N * (size_t)esize_of(gd);

@@ -79,7 +79,9 @@ struct Plan {
   // compiled for, packs a workgroup, workgroups launched; team == 0: not planned
   int team = 0, team_v = 0;
   int64_t team_chunk_packs = 0, team_grid = 0;
-  bool team_small = false;  // fewer than kTeamMinTeams rows, all at once (the plan query reports the launches without)
+  bool team_small = false;
+  // a softmax row whose team (reported all the same) is not used: one workgroup a row is faster
+  bool team_idle = false;  // fewer than kTeamMinTeams rows, all at once (the plan query reports the launches without)
   // norm backward of such rows held R = team_v rows at a time by teams of workgroups
   // (norm_bwd_team_kernel): the same fields, one stride of packs a workgroup, and the
   // partial rows of column sums that launch leaves (one a team; partial_rows is what
@@ -1369,6 +1371,15 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
         p.team_v = (int)v;
         p.team_chunk_packs = v * kTeamBlock;
         p.team_grid = teams * team;
+        // Rows of whole packs that one workgroup a row serves faster, the exchange being longer than its way through
+        // the row: the more rows, the longer they may be (us, team / one workgroup, bf16 softmax: forward [16, 36032] 5.5 /
+        // 6.2, [48, 36032] 6.7 / 6.5, [64, 40000] 7.6 / 6.9, [64, 50048] 7.6 / 8.3, [128, 36032] 8.8 / 6.9, [128, 60032] 9.9 / 9.6,
+        // float32 [100, 25024] 8.5 / 9.8; backward [16, 32768] 5.0 / 3.6, [16, 45056] 5.1 / 5.5, [64, 40000] 7.0 / 5.9, [128,
+        // 32768] 7.7 / 4.7, [64, 50048] 7.2 / 7.7).
+        p.team_idle = p.fast && p.resident &&
+                      (oc == OC_SOFTMAX_FWD ? 48 * (M - 24) > row_packs - kSoftmaxTeamMinPacks &&
+                                                  (esize == 2 || row_packs <= 5120)
+                                            : row_packs <= kSoftmaxTeamMinPacks || (row_packs <= 5120 && M > 24));
       }
     }
   }
