@@ -428,8 +428,8 @@ int mi355x_rownorm_waves_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dtype
  * while another thread changes the override uses the old or the new variant,
  * never a mix.  Production callers never use it: with no override set (the
  * state a process starts in) every entry point is re-entrant, and the only
- * mutable global state any of them touches is the call counter and the
- * bookkeeping slots of the team launches described at
+ * mutable global state any of them touches is the call counter, the
+ * bookkeeping slots and the order of the team launches described at
  * mi355x_rownorm_set_team_wait_us.  A call whose shape the forced variant cannot hold
  * fails with ROWNORM_ERR_OVERRIDE instead of silently choosing another, and so
  * does a field outside 0..65535. */
@@ -451,7 +451,10 @@ int mi355x_rownorm_set_override(rownorm_op op, int lanes_per_row, int packs_per_
  * stream, in library-owned device memory (48 MiB a GPU); results do not depend on the slot.
  * A stream takes a slot with its first such call and keeps it; streams beyond the 64 slots
  * (8 of the strided softmax) take the multi-launch kernels, which exchange nothing, and so do these rows on a stream
- * under capture. */
+ * under capture.  The process has one such launch at a time running on a GPU: a call on another stream than
+ * the last one's is put behind that one by an event on the device (the host does not wait).  If the
+ * last one's stream is under capture by then, and no event stands behind that launch yet, the call takes
+ * the kernels that exchange nothing. */
 int mi355x_rownorm_set_team_wait_us(unsigned int microseconds);
 
 /* Measurement aid, no counterpart in the reference: a plain streaming kernel over

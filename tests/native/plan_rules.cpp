@@ -3,7 +3,24 @@
 #include "../../torch-xpu-ops_amd/csrc/kernels/plan.hpp"
 #include "../../torch-xpu-ops_amd/csrc/kernels/team_slots.hpp"
 
+#include <set>
+#include <thread>
+#include <vector>
+
 using namespace rownorm;
+
+// Streams and an event as the team launches' order sees them: the launches known to be over when a stream's next work
+// starts.
+struct FakeStreams {
+  using Stream = int;
+  std::vector<std::set<int>> over;
+  std::vector<char> captured;
+  std::set<int> event;
+  int records = 0, waits = 0, recorded_into_capture = 0;
+  bool capturing(Stream s) { return captured[s]; }
+  void record(Stream s) { ++records, recorded_into_capture += captured[s], event = over[s]; }
+  void wait(Stream s) { ++waits, over[s].insert(event.begin(), event.end()); }
+};
 
 extern "C" {
 
@@ -54,6 +71,52 @@ void rule_norm_team(int64_t M, int64_t N, int esize, int wide, int64_t out[3]) {
   Plan p;
   make_plan(OC_NORM_FWD, M, N, esize, 256, Override{}, false, &p, false, true, wide != 0);
   out[0] = p.team, out[1] = p.team_r ? 0 : p.team_v, out[2] = p.team ? p.team_grid / p.team : 0;
+}
+
+// n team launches in turn, number i on stream[i] (per_thread[i]: by a per-thread handle) while the streams of the bits
+// captured[i] are under capture.  ran[i]: 0 went without teams, 1 ran behind every team launch before it, 2 did not.
+// counts: events recorded, waits, events recorded on a stream under capture.
+void rule_team_order(int n, const int* stream, const int* captured, const int* per_thread, int streams, int* ran,
+                     int counts[3]) {
+  FakeStreams f;
+  f.over.resize(streams);
+  TeamOrder<FakeStreams> order;
+  std::set<int> before;
+  for (int i = 0; i < n; ++i) {
+    const int s = stream[i];
+    f.captured.assign(streams, 0);
+    for (int k = 0; k < streams; ++k) f.captured[k] = captured[i] >> k & 1;
+    ran[i] = 0;
+    if (!order.enter(f, (uintptr_t)s + 1, s, per_thread[i] != 0)) continue;
+    ran[i] = f.over[s] == before ? 1 : 2;
+    f.over[s].insert(i);
+    before.insert(i);
+    order.leave(f);
+  }
+  counts[0] = f.records, counts[1] = f.waits, counts[2] = f.recorded_into_capture;
+}
+
+// `threads` threads with a stream each, n launches a thread: the launches that were not behind all others before them
+int rule_team_order_threads(int threads, int n) {
+  FakeStreams f;
+  f.over.resize(threads);
+  f.captured.assign(threads, 0);
+  TeamOrder<FakeStreams> order;
+  std::set<int> before;
+  int unordered = 0;
+  std::vector<std::thread> ts;
+  for (int t = 0; t < threads; ++t)
+    ts.emplace_back([&, t] {
+      for (int i = 0; i < n; ++i) {
+        if (!order.enter(f, (uintptr_t)t + 1, t, false)) continue;
+        unordered += f.over[t] != before;  // (between enter and leave: one thread at a time)
+        f.over[t].insert(t * n + i);
+        before.insert(t * n + i);
+        order.leave(f);
+      }
+    });
+  for (auto& t : ts) t.join();
+  return unordered + (int)(before.size() != (size_t)threads * n);
 }
 
 // one table of slots for streams, as the library keeps one per device

@@ -1,8 +1,8 @@
-"""Team launches on several streams at once: every stream has exchange memory of its own and no team
-is larger than an eighth of the machine, so calls that share the machine finish without waiting for
-one another's end, with the results they have alone; a stream beyond the slots takes the launches that
-exchange nothing.  (The reference's kernels share nothing between calls: SpatialSoftmaxForward,
-src/ATen/native/xpu/sycl/SoftMaxKernels.cpp:725-950, LayerNormKernels.cpp:360-470.)"""
+"""Team launches on several streams at once: every stream has exchange memory of its own, and one such
+launch at a time runs on the device, so nobody's wait runs out and the results are those that the calls
+have alone; a stream beyond the slots takes the launches that exchange nothing.  (The reference's kernels
+share nothing between calls: SpatialSoftmaxForward, src/ATen/native/xpu/sycl/SoftMaxKernels.cpp:725-950,
+LayerNormKernels.cpp:360-470.)"""
 import time
 
 import pytest
@@ -81,8 +81,8 @@ def _large_calls(cabi, gpu, seed):
 
 
 def test_workgroups_that_need_a_whole_compute_unit_on_three_streams(cabi, gpu, streams):
-    """A large team shares the machine with other streams' teams and with kernels whose workgroups take any compute
-    unit that has room: nobody's wait runs out."""
+    """A large team takes turns with other streams' teams and shares the machine with kernels whose workgroups take any
+    compute unit that has room: nobody's wait runs out."""
     calls = [_large_calls(cabi, gpu, 2700 + i) for i in range(3)]
     alone = [[f() for f in fs] for fs in calls]
     for i, s in enumerate(streams):  # (the streams' slots, the allocator's blocks)

@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 @pytest.fixture(scope="module")
 def rules(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("rules") / "libplan_rules.so")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wno-unknown-pragmas", "-shared", "-fPIC",
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wno-unknown-pragmas", "-shared", "-fPIC", "-pthread",
                     os.path.join(HERE, "native", "plan_rules.cpp"), "-o", out], check=True)
     return ctypes.CDLL(out)
 
@@ -198,3 +198,37 @@ def test_strided_softmax_tile_or_teams(rules):
     assert width(0, 1, 8192, 8192, 2) == width(1, 1, 8192, 8192, 2) == 16
     assert width(0, 1, 8192, 136, 2) == 8 and width(1, 1, 30000, 136, 2) == 8
     assert _strided(rules, 0, 8, 8192, 16, 4)["team"] == 16
+
+
+def _team_order(rules, stream, captured=None, per_thread=None):
+    n, streams = len(stream), max(stream) + 1
+    ints = lambda v: (ctypes.c_int * n)(*(v or [0] * n))  # noqa: E731
+    ran, counts = ints(None), (ctypes.c_int * 3)()
+    rules.rule_team_order(n, ints(stream), ints(captured), ints(per_thread), streams, ran, counts)
+    return list(ran), list(counts)
+
+
+def test_one_team_launch_at_a_time(rules):
+    """Launches whose workgroups wait for one another never run beside one another, whatever the streams' turns; a
+    program on one stream records no event; nothing is recorded on a stream under capture."""
+    ran, counts = _team_order(rules, [0] * 1000)
+    assert ran == [1] * 1000 and counts == [0, 0, 0]
+    ran, counts = _team_order(rules, [0, 0, 1, 0])  # the first turn: the event goes behind the earlier stream's work
+    assert ran == [1] * 4 and counts == [3, 2, 0]
+    rng = random.Random(7)
+    for streams, stay in ((2, 1), (3, 1), (5, 4), (3, 40), (2, 300)):
+        order = [s for _ in range(12 if stay > 40 else 40) for s in [rng.randrange(streams)] * rng.randint(1, stay)]
+        ran, counts = _team_order(rules, order)
+        assert ran == [1] * len(order) and counts[2] == 0
+        ran, counts = _team_order(rules, order, per_thread=[1] * len(order))
+        assert ran == [1] * len(order)
+        under = [rng.randrange(1 << streams) & ~(1 << s) for s in order]  # (a stream's own capture is seen before)
+        ran, counts = _team_order(rules, order, captured=under)
+        assert 2 not in ran and counts[2] == 0
+    # quiet again: a launch on the same stream records nothing, one elsewhere still finds its order
+    ran, counts = _team_order(rules, [0, 1] + [1] * 600)
+    assert ran == [1] * 602 and counts == [1 + 256, 1, 0]
+    assert _team_order(rules, [0, 1] + [1] * 600 + [0]) == ([1] * 603, [1 + 256 + 2, 2, 0])
+    # the earlier stream under capture before its event exists: without teams, until it is out
+    assert _team_order(rules, [0, 1, 1, 1], captured=[0, 1, 0, 0])[0] == [1, 0, 1, 1]
+    assert rules.rule_team_order_threads(8, 60) == 0

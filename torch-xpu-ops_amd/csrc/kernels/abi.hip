@@ -194,18 +194,41 @@ uintptr_t stream_key(hipStream_t stream) {
   return (uintptr_t)stream;
 }
 
-// The slot and id of a new call on the current device out of the N slots of `slot_bytes` at
-// `symbol`, or null when the team kernel is not to be used: the address is not known, the stream is
-// being captured (a replay would run with the id of the capture), or other streams have all slots.
-template <int N>
-void* team_memory_for_call(TeamMemory<N>& memory, const void* symbol, size_t slot_bytes,
-                           hipStream_t stream, unsigned int* id) {
+// Whether a stream is under capture, or does not say.
+bool stream_capturing(hipStream_t stream) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &st) != hipSuccess) {
     (void)hipGetLastError();
-    return nullptr;
+    return true;
   }
-  if (st != hipStreamCaptureStatusNone) return nullptr;
+  return st != hipStreamCaptureStatusNone;
+}
+
+// The order of a device's team launches (TeamOrder), with the event behind the last of them.
+struct TeamEvents {
+  using Stream = hipStream_t;
+  hipEvent_t event = nullptr;
+  bool capturing(Stream s) { return stream_capturing(s); }
+  void record(Stream s) {
+    if (event == nullptr && hipEventCreateWithFlags(&event, hipEventDisableTiming) != hipSuccess) event = nullptr;
+    if (event == nullptr || hipEventRecord(event, s) != hipSuccess) (void)hipGetLastError();
+  }
+  void wait(Stream s) {
+    if (event != nullptr && hipStreamWaitEvent(s, event, 0) != hipSuccess) (void)hipGetLastError();
+  }
+};
+TeamOrder<TeamEvents> g_team_order[kMaxDevices];
+TeamEvents g_team_events[kMaxDevices];
+
+// The slot and id of a new call on the current device out of the N slots of `slot_bytes` at
+// `symbol`, or null when the team kernel is not to be used: the address is not known, the stream is
+// being captured (a replay would run with the id of the capture), or other streams have all slots.
+// With a slot the launch has its place behind the team launches of other streams: *device must leave
+// g_team_order behind it.
+template <int N>
+void* team_memory_for_call(TeamMemory<N>& memory, const void* symbol, size_t slot_bytes,
+                           hipStream_t stream, unsigned int* id, int* device) {
+  if (stream_capturing(stream)) return nullptr;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
   void* p = memory.address[dev].load(std::memory_order_acquire);
@@ -218,19 +241,34 @@ void* team_memory_for_call(TeamMemory<N>& memory, const void* symbol, size_t slo
   }
   const int slot = memory.slots[dev].of(stream_key(stream));
   if (slot < 0) return nullptr;
+  if (!g_team_order[dev].enter(g_team_events[dev], stream_key(stream), stream, stream == hipStreamPerThread))
+    return nullptr;
+  *device = dev;
   unsigned int n = g_team_calls.fetch_add(1, std::memory_order_relaxed) + 1;
   if (n == 0) n = g_team_calls.fetch_add(1, std::memory_order_relaxed) + 1;  // 0 tags nothing
   *id = n;
   return (char*)p + (size_t)slot * slot_bytes;
 }
 
-void* team_slot_for_call(hipStream_t stream, unsigned int* id) {
-  return team_memory_for_call(g_team_slots, HIP_SYMBOL(team_slots), sizeof(TeamSlot), stream, id);
-}
-void* team_columns_for_call(hipStream_t stream, unsigned int* id) {
-  return team_memory_for_call(g_team_columns, HIP_SYMBOL(team_columns), sizeof(TeamColumns),
-                              stream, id);
-}
+// A call's exchange memory, and its place in the order until the launch is out (the end of the scope).
+class TeamCall {
+ public:
+  TeamCall() = default;
+  TeamCall(const TeamCall&) = delete;
+  TeamCall& operator=(const TeamCall&) = delete;
+  ~TeamCall() {
+    if (dev_ >= 0) g_team_order[dev_].leave(g_team_events[dev_]);
+  }
+  void* slot(hipStream_t stream, unsigned int* id) {
+    return team_memory_for_call(g_team_slots, HIP_SYMBOL(team_slots), sizeof(TeamSlot), stream, id, &dev_);
+  }
+  void* columns(hipStream_t stream, unsigned int* id) {
+    return team_memory_for_call(g_team_columns, HIP_SYMBOL(team_columns), sizeof(TeamColumns), stream, id, &dev_);
+  }
+
+ private:
+  int dev_ = -1;
+};
 
 int esize_of(int dt) {
   switch (dt) {
@@ -287,13 +325,14 @@ int norm_fwd(const void* x, const void* res, const void* gamma, const void* beta
     a.h = h;
   }
   hipStream_t s = (hipStream_t)stream;
+  TeamCall team;
   // (not in place: a workgroup of the team kernel whose team does not come together
   // reads the whole row of X, which must then still be X)
   const uintptr_t xb = (uintptr_t)x, yb = (uintptr_t)y;
   const uintptr_t nbytes = (uintptr_t)M * (uintptr_t)N * (uintptr_t)esize_of(xd);
   const bool y_on_x = xb < yb + nbytes && yb < xb + nbytes;
   if (plan.team > 0 && !add && yd == xd && !y_on_x) {
-    a.team_slot = team_slot_for_call(s, &a.team_id);
+    a.team_slot = team.slot(s, &a.team_id);
     a.team_wait_ticks = g_team_wait_ticks.load(std::memory_order_relaxed);
   }
   if (xd == ROWNORM_F32) {
@@ -394,6 +433,7 @@ int norm_bwd(const void* dy, const void* x, const float* mean, const float* rstd
       workspace_bytes >= need + split_bytes(plan, M, want_cols))
     a.split_ws = (float*)((char*)workspace + need);
   hipStream_t s = (hipStream_t)stream;
+  TeamCall team;
   // rows beyond the registers: the team backward (whole packs on 16-byte aligned tensors, dX
   // apart from dY and X -- a workgroup whose team does not come together reads whole rows of
   // both while others write theirs)
@@ -403,7 +443,7 @@ int norm_bwd(const void* dy, const void* x, const float* mean, const float* rstd
     const size_t nbytes = (size_t)M * (size_t)N * (size_t)esize_of(xd);
     const char *db = (const char*)dx, *gb = (const char*)dy, *xb = (const char*)x;
     if (!(db < gb + nbytes && gb < db + nbytes) && !(db < xb + nbytes && xb < db + nbytes)) {
-      a.team_slot = team_slot_for_call(s, &a.team_id);
+      a.team_slot = team.slot(s, &a.team_id);
       a.team_wait_ticks = g_team_wait_ticks.load(std::memory_order_relaxed);
     }
   }
@@ -461,6 +501,7 @@ int softmax_fwd(const void* x, const void* mask, void* y, int64_t rows, int64_t 
   SoftmaxFwdArgs a{x,    y, (const uint8_t*)mask, (uint32_t)mr.div, (uint32_t)mr.mod, mr.stride,
                    rows, (int)N, flags};
   hipStream_t s = (hipStream_t)stream;
+  TeamCall team;
   // few very long rows: the team forward (rows of whole packs on 16-byte aligned tensors or rows of
   // no whole number of packs, no mask, Y apart from X -- a workgroup whose team does not come
   // together reads the whole row again -- and no stream capture)
@@ -470,7 +511,7 @@ int softmax_fwd(const void* x, const void* mask, void* y, int64_t rows, int64_t 
     const size_t xbytes = (size_t)rows * (size_t)N * (size_t)esize_of(id);
     const size_t ybytes = (size_t)rows * (size_t)N * (size_t)esize_of(od);
     if (!(xb < yb + ybytes && yb < xb + xbytes)) {
-      a.team_slot = team_slot_for_call(s, &a.team_id);
+      a.team_slot = team.slot(s, &a.team_id);
       a.team_wait_ticks = g_team_wait_ticks.load(std::memory_order_relaxed);
     }
   }
@@ -498,6 +539,7 @@ int softmax_bwd(const void* grad, const void* y, const void* mask, void* gi, int
   SoftmaxBwdArgs a{grad, y, gi, (const uint8_t*)mask, (uint32_t)mr.div, (uint32_t)mr.mod,
                    mr.stride, rows, (int)N, flags};
   hipStream_t s = (hipStream_t)stream;
+  TeamCall team;
   // few very long rows: the team backward, under the rules of the forward (gi apart from
   // grad and y)
   if (plan.team > 0 && !plan.team_idle && !mask &&
@@ -510,7 +552,7 @@ int softmax_bwd(const void* grad, const void* y, const void* mask, void* gi, int
       return !(ib < ob + obytes && ob < ib + ibytes);
     };
     if (apart(grad) && apart(y)) {
-      a.team_slot = team_slot_for_call(s, &a.team_id);
+      a.team_slot = team.slot(s, &a.team_id);
       a.team_wait_ticks = g_team_wait_ticks.load(std::memory_order_relaxed);
     }
   }
@@ -755,12 +797,13 @@ int mi355x_group_norm_fwd(const void* x, const void* gamma, const void* beta, vo
   GroupNormFwdArgs a{x,      gamma,      beta,     y,          mean,        rstd,
                      d.rows, (int)d.L, (int)HxW, (int)d.D, (int)groups, eps};
   hipStream_t s = (hipStream_t)stream;
+  TeamCall team;
   // slabs beyond the registers: the team forward, under the rules of the norm forward
   // (not on top of X, not on a stream under capture)
   const uintptr_t xb = (uintptr_t)x, yb = (uintptr_t)y;
   const uintptr_t nbytes = (uintptr_t)d.rows * (uintptr_t)d.L * (uintptr_t)esize_of(xd);
   if (plan.team > 0 && !(xb < yb + nbytes && yb < xb + nbytes)) {
-    a.team_slot = team_slot_for_call(s, &a.team_id);
+    a.team_slot = team.slot(s, &a.team_id);
     a.team_wait_ticks = g_team_wait_ticks.load(std::memory_order_relaxed);
   }
   if (xd == ROWNORM_F32) return launch_group_norm_fwd<float, float>(plan, a, s);
@@ -815,6 +858,7 @@ int mi355x_group_norm_bwd(const void* dy, const void* x, const void* mean, const
   GroupNormBwdArgs a{dy,      x,       mean,   rstd,     gamma,    dx,       dgamma,     dbeta,
                      part_dg, part_db, d.rows, (int)d.L, (int)HxW, (int)d.D, (int)groups};
   hipStream_t s = (hipStream_t)stream;
+  TeamCall team;
   // slabs beyond the registers whose channels are whole packs, 16-byte aligned tensors, dX
   // apart from dY and X (a workgroup whose team does not come together reads the whole slab
   // of both while others write theirs): teams of workgroups, dY and X read once.
@@ -831,7 +875,7 @@ int mi355x_group_norm_bwd(const void* dy, const void* x, const void* mean, const
       a.team_v = t.v;
       a.team_ahead = t.ahead;
       a.team_grid = t.grid;
-      a.team_slot = team_slot_for_call(s, &a.team_id);
+      a.team_slot = team.slot(s, &a.team_id);
       a.team_wait_ticks = g_team_wait_ticks.load(std::memory_order_relaxed);
     }
   }
@@ -887,11 +931,12 @@ int mi355x_softmax_strided_fwd(const void* x, void* y, int64_t outer, int64_t di
     return e;
   SoftmaxStridedFwdArgs a{x, y, outer, (int)dim_size, (int)inner, flags};
   hipStream_t s = (hipStream_t)stream;
+  TeamCall team;
   // (a workgroup whose team does not come together reads the whole strip again; a team of one
   // has nobody to wait for)
   const int64_t n = outer * dim_size * inner;
   if (plan.team_size() > 1 && regions_disjoint(y, n * esize_of(od), x, n * esize_of(id))) {
-    a.team_slot = team_columns_for_call(s, &a.team_id);
+    a.team_slot = team.columns(s, &a.team_id);
     a.team_wait_ticks = g_team_wait_ticks.load(std::memory_order_relaxed);
   }
   if (id == ROWNORM_F32) return launch_softmax_strided_fwd<float, float>(plan, a, s);
@@ -919,10 +964,11 @@ int mi355x_softmax_strided_bwd(const void* grad, const void* y, void* gi, int64_
     return e;
   SoftmaxStridedBwdArgs a{grad, y, gi, outer, (int)dim_size, (int)inner, flags};
   hipStream_t s = (hipStream_t)stream;
+  TeamCall team;
   const int64_t n = outer * dim_size * inner;
   if (plan.team_size() > 1 && regions_disjoint(gi, n * esize_of(od), grad, n * esize_of(gd)) &&
       regions_disjoint(gi, n * esize_of(od), y, n * esize_of(gd))) {
-    a.team_slot = team_columns_for_call(s, &a.team_id);
+    a.team_slot = team.columns(s, &a.team_id);
     a.team_wait_ticks = g_team_wait_ticks.load(std::memory_order_relaxed);
   }
   if (gd == ROWNORM_BF16) return launch_softmax_strided_bwd<bf16, bf16>(plan, a, s);

@@ -27,9 +27,11 @@
 // stops waiting when its team is complete, when any workgroup of the call has given
 // up before (a hint word in the slot), or after `wait_ticks` of the constant-rate
 // clock (the workgroups can only fail to be resident together while other kernels
-// hold compute units for that long).  What a workgroup does without its team is the
-// kernel's business; it keeps publishing its own numbers for the workgroups that do
-// wait.
+// hold compute units for that long; team launches of one process run one at a time,
+// TeamOrder in team_slots.hpp).  What a workgroup does without its team is the
+// kernel's business.  With the two-number exchange it keeps publishing its own numbers
+// for the workgroups that do wait; with self-validating words it publishes that it is
+// lost, and its team follows it (team_word_tag).
 #pragma once
 
 #include <stdint.h>

@@ -1556,15 +1556,10 @@ inline StridedTeam strided_team_of(bool backward, int64_t outer, int64_t D, int6
                                    int num_cus, bool large = false) {
   const int64_t per_cu = large ? 1 : kTeamPerCu, at_most = kTeamMaxWorkgroups / kTeamPerCu * per_cu;
   const int64_t wgs = num_cus * per_cu < at_most ? num_cus * per_cu : at_most;
-  // A team is an eighth of the machine at most.  Workgroups start in order, so a launch that shares
-  // the machine with others holds whole teams as soon as it holds that much of it, and those
-  // finish and make room: calls on several streams cannot keep one another's teams apart until
-  // the waits end.  (Larger teams gain nothing either, their exchange takes longer: bf16 [1, 8192,
-  // 136] forward on 64 workgroups 11.8 us, on 256 27.5.)
-  // A large workgroup enters an empty compute unit only, and other launches' workgroups may take any that has
-  // room; but what is not a team ends by itself, and what holds half of a compute unit for a team leaves the
-  // other half to that launch's next workgroups, so that the eight launches that can have a slot never hold
-  // the machine with incomplete teams alone (31 compute units a large launch at most, 63 halves a small one).
+  // A team is an eighth of the machine at most: larger ones gain nothing, their exchange takes longer (bf16 [1, 8192,
+  // 136] forward on 64 workgroups 11.8 us, on 256 27.5).  A large workgroup enters an empty compute unit only, and
+  // other launches' workgroups may take any that has room; but what is not a team ends by itself, and team launches of
+  // other streams run before or after (TeamOrder).
   // Beside two streams of calls that fill the machine 20 forward / backward calls of [1, 8192, 8192] took 8.7 /
   // 7.7 ms, on two workgroups a compute unit 8.8 / 9.2, and no wait ran out.
   const int64_t most_wgs = wgs / kTeamMinTeams > 0 ? wgs / kTeamMinTeams : 1;
