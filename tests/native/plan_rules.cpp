@@ -125,4 +125,15 @@ void* rule_slots_new() { return new StreamSlots<kTeamSlots>(); }
 void rule_slots_delete(void* t) { delete (StreamSlots<kTeamSlots>*)t; }
 int rule_slot_of(void* t, uintptr_t key) { return ((StreamSlots<kTeamSlots>*)t)->of(key); }
 
+// n calls, number at[i] in slot[i]: id[i], clear[i]
+void rule_team_ids(int n, const uint64_t* at, const int* slot, unsigned int* id, int* clear) {
+  TeamIds<kTeamSlots> ids;
+  for (int i = 0; i < n; ++i) {
+    bool c = false;
+    id[i] = ids.of(at[i], slot[i], &c);
+    clear[i] = c;
+  }
+}
+unsigned int rule_team_call_ids() { return kTeamCallIds; }
+
 }  // extern "C"

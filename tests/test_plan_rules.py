@@ -232,3 +232,26 @@ def test_one_team_launch_at_a_time(rules):
     # the earlier stream under capture before its event exists: without teams, until it is out
     assert _team_order(rules, [0, 1, 1, 1], captured=[0, 1, 0, 0])[0] == [1, 0, 1, 1]
     assert rules.rule_team_order_threads(8, 60) == 0
+
+
+def test_a_slot_never_meets_an_id_twice(rules):
+    """The tag of a word has room for 2^25 - 1 calls: a slot that a call before the ids came round has written to is
+    cleared before the next one reads it, whatever calls other slots have had in between."""
+    P = rules.rule_team_call_ids()
+    rng = random.Random(11)
+    slots, calls, n = 5, [], 0
+    for _ in range(4000):
+        n += rng.choice((1, 1, 1, 2, P // 3, P - 1, P, P + 1, 7 * P))
+        calls.append((n, rng.randrange(slots)))
+    calls = [(k, 0) for k in (0, P - 1, P, P + 1, 2 * P, 2 ** 32, 2 ** 32 + P)] + [(k + 2 ** 33, s) for k, s in calls]
+    k = len(calls)
+    ids, clear = (ctypes.c_uint * k)(), (ctypes.c_int * k)()
+    rules.rule_team_ids(k, (ctypes.c_uint64 * k)(*[c[0] for c in calls]), (ctypes.c_int * k)(*[c[1] for c in calls]),
+                        ids, clear)
+    seen = [set() for _ in range(slots)]
+    for i, (at, slot) in enumerate(calls):
+        if clear[i]:
+            seen[slot].clear()
+        assert 1 <= ids[i] <= P and ids[i] << 6 < 2 ** 31 and ids[i] not in seen[slot]
+        seen[slot].add(ids[i])
+    assert list(clear[:7]) == [0, 0, 1, 0, 1, 1, 1] and (ids[0], ids[1], ids[2]) == (1, P, 1)

@@ -167,8 +167,8 @@ int static_scratch(void** out) {
 }
 
 // Exchange memory of the team launches (the workgroups' partial sums), one slot a stream
-// (StreamSlots); per device, like `scratch`.  Zero at load and never cleared: every word a call
-// reads is tagged with the call's id.  16 MiB, and 32 MiB for the strided softmax, whose
+// (StreamSlots); per device, like `scratch`.  Zero at load: every word a call reads is tagged with the
+// call's id, so a slot is cleared only when the ids come round again (TeamIds).  16 MiB, and 32 MiB for the strided softmax, whose
 // workgroups pass numbers for every column.
 static __device__ __align__(256) __attribute__((used)) TeamSlot team_slots[kTeamSlots];
 static __device__ __align__(256) __attribute__((used)) TeamColumns team_columns[kTeamColumnSlots];
@@ -177,10 +177,11 @@ template <int N>
 struct TeamMemory {
   std::atomic<void*> address[kMaxDevices];
   StreamSlots<N> slots[kMaxDevices];
+  TeamIds<N> ids[kMaxDevices];
 };
 TeamMemory<kTeamSlots> g_team_slots;
 TeamMemory<kTeamColumnSlots> g_team_columns;
-std::atomic<unsigned int> g_team_calls{0};
+std::atomic<uint64_t> g_team_calls{0};
 // Bound of a workgroup's wait for its team, in ticks of the 100 MHz constant-rate
 // clock: one second unless mi355x_rownorm_set_team_wait_us() says otherwise.
 std::atomic<unsigned long long> g_team_wait_ticks{100000000ull};
@@ -192,6 +193,11 @@ uintptr_t stream_key(hipStream_t stream) {
   if (stream == nullptr || stream == hipStreamLegacy) return (uintptr_t)1;
   if (stream == hipStreamPerThread) return (uintptr_t)&own;
   return (uintptr_t)stream;
+}
+
+__global__ void team_clear_kernel(uint4* p, unsigned int n) {
+  for (unsigned int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    p[i] = uint4{0, 0, 0, 0};
 }
 
 // Whether a stream is under capture, or does not say.
@@ -244,10 +250,13 @@ void* team_memory_for_call(TeamMemory<N>& memory, const void* symbol, size_t slo
   if (!g_team_order[dev].enter(g_team_events[dev], stream_key(stream), stream, stream == hipStreamPerThread))
     return nullptr;
   *device = dev;
-  unsigned int n = g_team_calls.fetch_add(1, std::memory_order_relaxed) + 1;
-  if (n == 0) n = g_team_calls.fetch_add(1, std::memory_order_relaxed) + 1;  // 0 tags nothing
-  *id = n;
-  return (char*)p + (size_t)slot * slot_bytes;
+  // (the order holds other team calls on the device up until this one is out)
+  bool clear = false;
+  *id = memory.ids[dev].of(g_team_calls.fetch_add(1, std::memory_order_relaxed), slot, &clear);
+  p = (char*)p + (size_t)slot * slot_bytes;
+  if (clear)
+    hipLaunchKernelGGL(team_clear_kernel, dim3(256), dim3(256), 0, stream, (uint4*)p, (unsigned int)(slot_bytes / 16));
+  return p;
 }
 
 // A call's exchange memory, and its place in the order until the launch is out (the end of the scope).

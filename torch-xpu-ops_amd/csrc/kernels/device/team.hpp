@@ -9,7 +9,7 @@
 // What crosses workgroups.  An entry is 128 bytes (neighbours' polls go to other memory
 // channels).  The two-number exchange (team_publish_and_gather) uses {tag, s1, s2}: the tag
 // of a finished entry is (call id << 32) | (round + 1), ids being unique per call, so nothing
-// has to be cleared and an entry left by an earlier call or round never counts.  The writer
+// has to be cleared from call to call and an entry left by an earlier call or round never counts.  The writer
 // sets the tag to 0 when it starts on a row, later stores s1 and s2, waits for those stores
 // to be acknowledged and stores the tag; a reader accepts s1 and s2 only if it read the
 // expected tag before and after them.  The exchanges in two halves further down write
@@ -52,9 +52,10 @@ __device__ __forceinline__ void team_stores_done() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-// team_word_tag: the tag every word of the exchanges below carries -- ((call id mod 2^25 - 1)
-// + 1) << 6 | (round mod 64): never 0 (the memory starts as zeros), different for the rounds
-// that share a buffer, different from call to call; bit 31 is clear.
+// team_word_tag: the tag every word of the exchanges below carries -- call id << 6 | (round mod
+// 64): never 0 (the memory starts as zeros), different for the rounds that share a buffer,
+// different from call to call (ids are 25 bits wide; before they come round again a slot's
+// memory is cleared, TeamIds in team_slots.hpp); bit 31 is clear.
 //
 // A workgroup that has stopped waiting for its team (`lost`) never publishes a valid word
 // again: its words carry team_lost_tag -- the call's tag with bit 31 set, whatever the round
@@ -64,7 +65,7 @@ __device__ __forceinline__ void team_stores_done() {
 // slot's hint word spreads the news to the other teams of the call, which look at it now
 // and then.
 __device__ __forceinline__ unsigned int team_word_tag(unsigned int call_id, unsigned int round) {
-  return ((call_id % 0x1ffffffu) + 1u) << 6 | (round & 63u);
+  return call_id << 6 | (round & 63u);
 }
 __device__ __forceinline__ unsigned int team_lost_tag(unsigned int call_id) {
   return 0x80000000u | team_word_tag(call_id, 0);

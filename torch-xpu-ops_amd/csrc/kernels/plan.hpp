@@ -126,6 +126,8 @@ constexpr int kTeamBwdPerCu = 1;
 // norm_fwd_rows_team_kernel: packs of a row a lane, and the rounds from which it is taken
 constexpr int kTeamFwdLongPacks = 10;
 constexpr int kTeamFwdMinRounds = 16;
+// Ids that team calls draw in turn, from 1 on; as many as the tag of a word has room for (device/team.hpp).
+constexpr unsigned int kTeamCallIds = 0x1ffffff;
 // One stream's exchange memory (device/team.hpp, team_slots.hpp).
 struct TeamEntry {
   // the two-number exchange: (call id << 32) | (round + 1) once s1, s2 are in place, 0 while

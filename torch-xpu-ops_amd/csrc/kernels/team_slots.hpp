@@ -6,6 +6,8 @@
 #include <atomic>
 #include <mutex>
 
+#include "plan.hpp"
+
 namespace rownorm {
 
 // Calls on one stream run one after the other, so a slot that belongs to a stream never serves two
@@ -30,6 +32,25 @@ class StreamSlots {
 
  private:
   std::atomic<uintptr_t> key_[N] = {};
+};
+
+// Ids of team calls: kTeamCallIds of them in turn, then the same again.  A word that an earlier call left in a slot
+// carries that call's id, so a slot must not meet an id a second time before it is cleared: of() says when, with the
+// first call after the ids have come round.
+template <int N>
+class TeamIds {
+ public:
+  // The id of call number n (over all slots) in `slot`; *clear: the slot's memory must be zeroed first.  (One thread at a
+  // time for a slot.)
+  unsigned int of(uint64_t n, int slot, bool* clear) {
+    const uint64_t turn = n / kTeamCallIds;
+    *clear = turn_[slot] != turn;
+    turn_[slot] = turn;
+    return (unsigned int)(n % kTeamCallIds) + 1;
+  }
+
+ private:
+  uint64_t turn_[N] = {};
 };
 
 // One team launch at a time on a device.  The workgroups of a team wait for one another, so a launch must be able
