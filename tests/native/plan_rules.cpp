@@ -119,6 +119,14 @@ int rule_team_order_threads(int threads, int n) {
   return unordered + (int)(before.size() != (size_t)threads * n);
 }
 
+// workgroups of the team that holds a softmax row, 0: none does (widened: float32 output of 16-bit rows)
+int rule_softmax_team(int backward, int64_t M, int64_t N, int esize, int widened) {
+  Plan p;
+  make_plan(backward ? OC_SOFTMAX_BWD : OC_SOFTMAX_FWD, M, N, esize, 256, Override{}, false, &p, false, false, false, false,
+            false, false, true, widened != 0);
+  return p.team_idle ? 0 : p.team;
+}
+
 // one table of slots for streams, as the library keeps one per device
 int rule_team_slots() { return kTeamSlots; }
 void* rule_slots_new() { return new StreamSlots<kTeamSlots>(); }

@@ -255,3 +255,13 @@ def test_a_slot_never_meets_an_id_twice(rules):
         assert 1 <= ids[i] <= P and ids[i] << 6 < 2 ** 31 and ids[i] not in seen[slot]
         seen[slot].add(ids[i])
     assert list(clear[:7]) == [0, 0, 1, 0, 1, 1, 1] and (ids[0], ids[1], ids[2]) == (1, P, 1)
+
+
+def test_softmax_rows_with_a_wider_output_have_teams(rules):
+    """Few long float16 rows with a float32 output: teams for whole and ragged rows of any number, where one workgroup a
+    row measured up to half as slow again."""
+    f = lambda M, N, wide: rules.rule_softmax_team(0, ctypes.c_int64(M), ctypes.c_int64(N), 2, wide)  # noqa: E731
+    for M in (1, 30, 48, 64, 100, 128):
+        for N in (32768, 36032, 40963, 45008, 60032, 60035, 140000):
+            assert f(M, N, 1) >= 2, (M, N)
+    assert f(128, 32776, 0) == 0 and f(129, 60032, 1) == 0 and f(64, 32752, 1) == 0

@@ -850,7 +850,8 @@ inline WavesLayout norm_waves_layout(bool backward, int esize, int64_t M, int64_
 inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, const Override& ov,
                      bool want_cols, Plan* out, bool force_general = false,
                      bool layer_norm = false, bool wide_weights = false, bool off_line = false,
-                     bool fused_add = false, bool masked = false, bool want_dx = true) {
+                     bool fused_add = false, bool masked = false, bool want_dx = true,
+                     bool widened = false) {
   Plan p;
   const int E = 16 / esize;
   p.fast = (N % E) == 0 && !force_general;
@@ -1353,7 +1354,11 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
   // 7.4; backward [32, 32769] 6.5 / 6.5, [100, 45001] 8.7 / 10.2, [100, 60004] 12.4 / 8.6, [128, 80001] 20.0 / 16.2).
   // Before both they went through softmax_*_stream_kernel: 7.9, 7.5, 11.5, 9.9, 19.2, 17.7; 7.4, 8.4, 10.4, 19.9.
   const int64_t row_packs = (N + E - 1) / E;
-  const bool team_rows = p.fast || (oc == OC_SOFTMAX_FWD ? 48 : 24) * (M - 24) <= row_packs - kSoftmaxTeamMinPacks;
+  // (an output wider than the input, float16 -> float32, has teams for all of them: its stores are most of the call
+  // and one workgroup's worth of them at a time is slow; forward, one workgroup / teams: [48, 40960] 12.7 / 8.7, [100,
+  // 60032] 20.1 / 13.5, [64, 45008] 14.2 / 10.2, [100, 60035] 21.4 / 14.4; [128, 32776] 12.8 / 12.9)
+  const bool team_rows =
+      p.fast || widened || (oc == OC_SOFTMAX_FWD ? 48 : 24) * (M - 24) <= row_packs - kSoftmaxTeamMinPacks;
   if (softmax && team_rows && !force_general && !masked && ov.G == 0 && ov.V == 0 && ov.bpc == 0 && ov.block == 0 &&
       2 * M <= num_cus && row_packs >= kSoftmaxTeamMinPacks) {
     const int64_t cus = num_cus * kTeamPerCu < kTeamMaxWorkgroups ? num_cus * kTeamPerCu : kTeamMaxWorkgroups;
@@ -1378,7 +1383,7 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
         // 6.2, [48, 36032] 6.7 / 6.5, [64, 40000] 7.6 / 6.9, [64, 50048] 7.6 / 8.3, [128, 36032] 8.8 / 6.9, [128, 60032] 9.9 / 9.6,
         // float32 [100, 25024] 8.5 / 9.8; backward [16, 32768] 5.0 / 3.6, [16, 45056] 5.1 / 5.5, [64, 40000] 7.0 / 5.9, [128,
         // 32768] 7.7 / 4.7, [64, 50048] 7.2 / 7.7).
-        p.team_idle = p.fast && p.resident &&
+        p.team_idle = p.fast && p.resident && !widened &&
                       (oc == OC_SOFTMAX_FWD ? 48 * (M - 24) > row_packs - kSoftmaxTeamMinPacks &&
                                                   (esize == 2 || row_packs <= 5120)
                                             : row_packs <= kSoftmaxTeamMinPacks || (row_packs <= 5120 && M > 24));
