@@ -248,7 +248,10 @@ softmax_fwd_resident_kernel(const TI* __restrict__ x, TO* __restrict__ y, MaskRe
       float mx[1] = {-INFINITY};
       float sum[1] = {0.0f};
       float m;
-      if constexpr (!MASKED && FAST && V >= 8) {
+      // (TAIL float32 from 6 packs on: at 6 and 7 the other form keeps 69 and 77 registers of the 64 that two
+      // workgroups a compute unit leave, and spills: [1000, 24983] softmax 48.7 us, 39.3 in halves, 40.8 in two passes; [2000,
+      // 20887] 68.2, 63.4, 64.4)
+      if constexpr (!MASKED && FAST && V >= (TAIL && sizeof(TI) == 4 ? 6 : 8)) {
         // the lane's packs in two halves, each with its own maximum and sum of
         // exp(x - maximum): the first half is worked on while the second is still
         // arriving, and the exponentials no longer wait for the block maximum
