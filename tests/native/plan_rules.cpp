@@ -119,12 +119,20 @@ int rule_team_order_threads(int threads, int n) {
   return unordered + (int)(before.size() != (size_t)threads * n);
 }
 
-// workgroups of the team that holds a softmax row, 0: none does (widened: float32 output of 16-bit rows)
-int rule_softmax_team(int backward, int64_t M, int64_t N, int esize, int widened) {
+// What serves a softmax call (widened: float32 output of 16-bit rows): 1 rows in registers, 2 a team, 3 ragged rows held by
+// one workgroup, 0 the two passes; out: workgroups of the team, or lanes and packs a lane of the held form
+int rule_softmax_route(int backward, int is_log, int64_t M, int64_t N, int esize, int widened, int64_t out[2]) {
   Plan p;
-  make_plan(backward ? OC_SOFTMAX_BWD : OC_SOFTMAX_FWD, M, N, esize, 256, Override{}, false, &p, false, false, false, false,
-            false, false, true, widened != 0);
-  return p.team_idle ? 0 : p.team;
+  make_plan(backward ? OC_SOFTMAX_BWD : OC_SOFTMAX_FWD, M, N, esize, 256, Override{}, false, &p);
+  out[0] = out[1] = 0;
+  if (softmax_team_serves(p, backward != 0, is_log != 0, widened != 0, esize, M, N, 256)) {
+    out[0] = p.team;
+    return 2;
+  }
+  if (p.resident) return 1;
+  if (!softmax_tail_serves(p, backward != 0, is_log != 0, widened != 0, esize, M, N)) return 0;
+  out[0] = p.tail_g, out[1] = p.tail_v;
+  return 3;
 }
 
 // one table of slots for streams, as the library keeps one per device

@@ -257,11 +257,79 @@ def test_a_slot_never_meets_an_id_twice(rules):
     assert list(clear[:7]) == [0, 0, 1, 0, 1, 1, 1] and (ids[0], ids[1], ids[2]) == (1, P, 1)
 
 
+def _route(rules, backward, is_log, M, N, esize, widened=0):
+    out = (ctypes.c_int64 * 2)()
+    kind = rules.rule_softmax_route(backward, is_log, ctypes.c_int64(M), ctypes.c_int64(N), esize, widened, out)
+    return ("two passes", "registers", "team", "held")[kind], out[0], out[1]
+
+
 def test_softmax_rows_with_a_wider_output_have_teams(rules):
     """Few long float16 rows with a float32 output: teams for whole and ragged rows of any number, where one workgroup a
     row measured up to half as slow again."""
-    f = lambda M, N, wide: rules.rule_softmax_team(0, ctypes.c_int64(M), ctypes.c_int64(N), 2, wide)  # noqa: E731
+    f = lambda M, N, wide: _route(rules, 0, 0, M, N, 2, wide)[0]  # noqa: E731
     for M in (1, 30, 48, 64, 100, 128):
         for N in (32768, 36032, 40963, 45008, 60032, 60035, 140000):
-            assert f(M, N, 1) >= 2, (M, N)
-    assert f(128, 32776, 0) == 0 and f(129, 60032, 1) == 0 and f(64, 32752, 1) == 0
+            assert f(M, N, 1) == "team", (M, N)
+    assert f(128, 32776, 0) == "registers" and f(129, 60032, 1) == "registers" and f(64, 32752, 1) == "registers"
+
+
+def test_softmax_of_few_rows_by_teams_or_by_one_workgroup_each(rules):
+    """Both sides of every line as they measured: (backward, log, rows, elements, bytes an element) -> team or not."""
+    one = [(0, 0, 48, 32768, 2), (0, 0, 64, 36032, 2), (0, 0, 100, 40000, 2), (0, 0, 128, 50048, 2), (0, 1, 64, 40000, 2),
+           (0, 0, 8, 17024, 4), (0, 0, 64, 20480, 4), (0, 0, 128, 20480, 4),
+           (1, 0, 8, 32768, 2), (1, 0, 64, 36032, 2), (1, 1, 100, 36032, 2), (1, 0, 128, 50048, 2), (1, 1, 128, 55040, 2),
+           (1, 0, 8, 16384, 4), (1, 0, 64, 20480, 4), (1, 1, 128, 25024, 4),
+           # ragged: the slow side of the lines for whole rows was up to 1.4 times the two passes' time
+           (0, 0, 64, 45051, 2), (0, 0, 100, 61435, 2), (0, 0, 128, 102403, 2), (0, 1, 48, 61435, 2), (0, 1, 128, 94203, 2),
+           (0, 0, 128, 26619, 4), (0, 1, 30, 20475, 4),
+           (1, 0, 30, 36859, 2), (1, 0, 64, 58155, 2), (1, 0, 100, 53243, 2), (1, 0, 128, 53243, 2), (1, 0, 128, 64707, 2),
+           (1, 1, 48, 74539, 2), (1, 1, 64, 81091, 2), (1, 1, 128, 53243, 2), (1, 1, 128, 130243, 2),
+           (1, 0, 64, 28027, 4), (1, 1, 64, 24571, 4), (1, 1, 128, 28027, 4)]
+    team = [(0, 0, 8, 32768, 2), (0, 0, 48, 36032, 2), (0, 0, 64, 45056, 2), (0, 0, 100, 50048, 2), (0, 0, 100, 60032, 2),
+            (0, 0, 128, 65536, 2), (0, 0, 8, 22528, 4), (0, 0, 64, 22528, 4),
+            (1, 0, 8, 33792, 2), (1, 0, 30, 36032, 2), (1, 1, 48, 33792, 2), (1, 0, 64, 45056, 2), (1, 0, 128, 60032, 2),
+            (1, 1, 30, 20480, 4), (1, 0, 64, 22528, 4),
+            (0, 0, 8, 33579, 2), (0, 0, 64, 61435, 2), (0, 0, 100, 91000, 2), (0, 0, 128, 159739, 2), (0, 1, 64, 91003, 2),
+            (0, 0, 48, 20067, 4), (0, 1, 64, 32643, 4),
+            (1, 0, 8, 42000, 2), (1, 0, 30, 61435, 2), (1, 0, 128, 73475, 2), (1, 1, 8, 53243, 2), (1, 1, 64, 123691, 2),
+            (1, 0, 100, 40835, 4), (1, 1, 64, 40835, 4), (1, 1, 128, 45055, 4)]
+    for c in one:
+        assert _route(rules, *c)[0] in ("registers", "held"), c
+    for c in team:
+        assert _route(rules, *c)[0] == "team", c
+    for M in (1, 8, 48, 100, 128):  # without a held form there is nothing but teams or the two passes
+        assert _route(rules, 1, 0, M, 80003, 2)[0] == "team" and _route(rules, 0, 0, M, 200003, 2)[0] == "team"
+
+
+def test_which_ragged_softmax_rows_are_held(rules):
+    """Both sides of the lines of softmax_tail_serves(), and no pack count for which no kernel is built."""
+    held = [(0, 1, 3000, 53243, 2), (0, 1, 1000, 49963, 2), (0, 0, 2000, 53243, 2), (0, 1, 4096, 18431, 4), (0, 1, 2000, 26619, 4),
+            (0, 0, 200, 159739, 2), (0, 0, 1000, 159739, 2), (0, 0, 1000, 61847, 4), (0, 1, 2000, 37271, 4), (0, 0, 200, 37271, 4),
+            (1, 0, 2000, 32515, 2), (1, 0, 300, 29483, 2), (1, 0, 4096, 28003, 2), (1, 0, 2000, 16791, 4), (1, 1, 2000, 29483, 2),
+            (1, 1, 4096, 18839, 4), (1, 1, 1000, 16791, 4)]
+    passes = [(0, 1, 2000, 53243, 2), (0, 1, 1500, 61435, 2), (0, 1, 3000, 18431, 4), (0, 0, 300, 159739, 2),
+              (0, 0, 1000, 133540, 2), (0, 0, 4096, 152001, 2), (0, 0, 300, 61847, 4), (0, 0, 2000, 37271, 4), (0, 1, 700, 37271, 4),
+              (1, 0, 2000, 29483, 2), (1, 0, 2000, 31939, 2), (1, 1, 4096, 16791, 4), (0, 1, 700, 45463, 4),
+              (1, 0, 2000, 34003, 2), (1, 0, 2000, 66003, 2), (0, 0, 2000, 163843, 2)]
+    for c in held:
+        assert _route(rules, *c)[0] == "held", c
+    for c in passes:
+        assert _route(rules, *c)[0] == "two passes", c
+    wide = lambda M, N, log: _route(rules, 0, log, M, N, 2, 1)[0]  # noqa: E731
+    assert [wide(*a) for a in ((130, 53243, 0), (200, 36859, 0), (200, 53243, 0), (130, 53243, 1), (300, 53243, 0),
+                               (2000, 53243, 1))] == ["two passes"] * 2 + ["held"] * 4
+    for es in (2, 4):
+        E = 16 // es
+        for packs in range(2049 if es == 2 else 4097, 20600, 13):
+            for over in range(1, E, 3):
+                N = packs * E - E + over
+                for M in (129, 300, 513, 1100, 2050, 5000):
+                    kind, g, v = _route(rules, 0, 0, M, N, es)
+                    assert kind in ("held", "two passes")
+                    if kind == "held":
+                        window = (N + 2 * (E - 1)) // E
+                        assert (v - 1) * g < window <= v * g
+                        assert v in range(*((5, 15) if es == 2 else (9, 15))) if g == 512 else (
+                            g == 1024 and v in range(3 if es == 2 else 5, 21 if es == 2 else 17) and v not in (17, 19))
+                    kind, g, v = _route(rules, 1, 0, M, N, es)
+                    assert kind == "two passes" or (g == 1024 and (3 if es == 2 else 5) <= v <= 8)

@@ -505,7 +505,7 @@ int softmax_fwd(const void* x, const void* mask, void* y, int64_t rows, int64_t 
   const bool off_line = (((uintptr_t)x | (uintptr_t)y) & 127u) != 0;
   if (int e = make_plan(OC_SOFTMAX_FWD, rows, N, esize_of(id), current_num_cus(),
                         g_override[ROWNORM_OP_SOFTMAX_FWD], false, &plan, false, false, false,
-                        off_line, false, mask != nullptr, true, od != id))
+                        off_line, false, mask != nullptr))
     return e;
   SoftmaxFwdArgs a{x,    y, (const uint8_t*)mask, (uint32_t)mr.div, (uint32_t)mr.mod, mr.stride,
                    rows, (int)N, flags};
@@ -514,7 +514,9 @@ int softmax_fwd(const void* x, const void* mask, void* y, int64_t rows, int64_t 
   // few very long rows: the team forward (rows of whole packs on 16-byte aligned tensors or rows of
   // no whole number of packs, no mask, Y apart from X -- a workgroup whose team does not come
   // together reads the whole row again -- and no stream capture)
-  if (plan.team > 0 && !plan.team_idle && !mask && (!plan.fast || ((((uintptr_t)x) | ((uintptr_t)y)) & 15u) == 0)) {
+  if (!mask && (!plan.fast || ((((uintptr_t)x) | ((uintptr_t)y)) & 15u) == 0) &&
+      softmax_team_serves(plan, false, (flags & kSoftmaxLog) != 0, esize_of(od) > esize_of(id), esize_of(id), rows, N,
+                          current_num_cus())) {
     const char* xb = (const char*)x;
     const char* yb = (const char*)y;
     const size_t xbytes = (size_t)rows * (size_t)N * (size_t)esize_of(id);
@@ -551,8 +553,9 @@ int softmax_bwd(const void* grad, const void* y, const void* mask, void* gi, int
   TeamCall team;
   // few very long rows: the team backward, under the rules of the forward (gi apart from
   // grad and y)
-  if (plan.team > 0 && !plan.team_idle && !mask &&
-      (!plan.fast || ((((uintptr_t)grad) | ((uintptr_t)y) | ((uintptr_t)gi)) & 15u) == 0)) {
+  if (!mask && (!plan.fast || ((((uintptr_t)grad) | ((uintptr_t)y) | ((uintptr_t)gi)) & 15u) == 0) &&
+      softmax_team_serves(plan, true, (flags & kSoftmaxLog) != 0, false, esize_of(gd), rows, N, current_num_cus(),
+                          softmax_tail_aligned(grad, y))) {
     const char* ob = (const char*)gi;
     const size_t ibytes = (size_t)rows * (size_t)N * (size_t)esize_of(gd);
     const size_t obytes = (size_t)rows * (size_t)N * (size_t)esize_of(od);

@@ -68,8 +68,8 @@ struct Plan {
   // softmax backward of rows beyond the registers of two tensors: grad alone fits
   // them (the log_softmax backward then keeps grad resident and streams y)
   bool grad_resident = false;
-  // softmax rows of no whole number of packs that one workgroup of tail_g lanes (1024, forward also 512) holds in
-  // tail_v whole packs a lane, tail_packs at most in all (0: not such a row)
+  // softmax rows of no whole number of packs that one workgroup of tail_g lanes (1024, forward also 512) can hold in
+  // tail_v whole packs a lane, tail_packs at most in all (0: not such a row); softmax_tail_serves() says whether it does
   int tail_v = 0, tail_g = 0, tail_packs = 0, tail_cus = 0;
   // a layout was asked for by override: kernels chosen by other means than the
   // layout (softmax of short ragged rows through LDS) stand back
@@ -77,11 +77,10 @@ struct Plan {
   // norm forward of rows beyond one workgroup's registers held by a team of
   // workgroups (norm_fwd_team_kernel): workgroups a row, packs a lane the kernel is
   // compiled for, packs a workgroup, workgroups launched; team == 0: not planned
+  // (softmax: the team that could hold a row, whether it does is softmax_team_serves()'s)
   int team = 0, team_v = 0;
   int64_t team_chunk_packs = 0, team_grid = 0;
-  bool team_small = false;
-  // a softmax row whose team (reported all the same) is not used: one workgroup a row is faster
-  bool team_idle = false;  // fewer than kTeamMinTeams rows, all at once (the plan query reports the launches without)
+  bool team_small = false;  // fewer than kTeamMinTeams rows, all at once (the plan query reports the launches without)
   // norm backward of such rows held R = team_v rows at a time by teams of workgroups
   // (norm_bwd_team_kernel): the same fields, one stride of packs a workgroup, and the
   // partial rows of column sums that launch leaves (one a team; partial_rows is what
@@ -172,9 +171,9 @@ constexpr int kSoftmaxBwdHoldMaxV = 8;
 constexpr int kGradResidentMaxV = 20;
 // Softmax rows of no whole number of packs beyond the resident layouts: 3 packs a lane at least, on one workgroup of
 // 1024 lanes (TAIL in softmax_kernels.hpp).  Against the multi-pass kernels, which read X, or grad and y, twice, bf16
-// us: [4096, 128255] log_softmax 453 -> 396, backward 621 -> 587; [4096, 50257] 161 -> 148, 238 -> 232; [515, 50220] softmax
-// 26.7 -> 25.4, 40.3 -> 34.5; [2000, 17001] 32.2 -> 26.8, 46.0 -> 37.7.  (The same on packs at the row's own alignment: a 16-byte
-// access two bytes off costs twice, [4096, 128255] 479 and 677.)
+// us: [4096, 128255] log_softmax 453 -> 396, backward 621 -> 587; [4096, 50257] 161 -> 148, 238 -> 225; [515, 50220]
+// softmax 26.7 -> 25.4, 40.3 -> 34.5; [2000, 17001] 32.2 -> 26.8, 46.0 -> 37.7.  (The same on packs at the row's own
+// alignment: a 16-byte access two bytes off costs twice, [4096, 128255] 479 and 677.)
 constexpr int kSoftmaxTailMinV = 3;
 // The forward on 512 lanes where more and smaller workgroups a compute unit overlap better: the shortest of these rows
 // and calls of few rows (bf16 softmax, 1024 / 512 lanes: [4096, 17001] 54.1 / 50.0 us, [2000, 24570] 39.0 / 37.0, [1000,
@@ -185,10 +184,11 @@ constexpr bool softmax_tail_half_lanes(int64_t packs, int64_t M, int num_cus) {
          (packs <= kMaxG / 2 * kSoftmaxTailHalfMaxV - 1024 && M <= 2 * (int64_t)num_cus);
 }
 // The log_softmax backward holds grad alone from here on (both tensors: [2000, 49001] 112 us, grad alone 106, the
-// multi-pass kernel 106; [1000, 65001] 81.4, 72.7, 74.8).
+// multi-pass kernel 106; [1000, 65001] 81.4, 72.7, 74.8; float32 of 5 to 8 packs 0.97 to 1.05 of grad alone's time).
 constexpr int kSoftmaxTailGradMinV = 4;
-// Bytes up to which a second pass over the inputs comes out of the 256 MB cache behind the L2s.
-constexpr int64_t kSoftmaxCachedBytes = (int64_t)320 << 20;
+// Bytes of input up to which the two passes gain from the 256 MB cache behind the L2s (a crossover as measured: most
+// of a little more than the cache's size still comes out of it).
+constexpr int64_t kSoftmaxCachedBytes = (int64_t)288 << 20;
 constexpr int max_v_of(OpClass oc, int esize) {
   return oc == OC_SOFTMAX_FWD && esize == 2 ? kSoftmaxFwdMaxV16 : kMaxV;
 }
@@ -850,8 +850,7 @@ inline WavesLayout norm_waves_layout(bool backward, int esize, int64_t M, int64_
 inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, const Override& ov,
                      bool want_cols, Plan* out, bool force_general = false,
                      bool layer_norm = false, bool wide_weights = false, bool off_line = false,
-                     bool fused_add = false, bool masked = false, bool want_dx = true,
-                     bool widened = false) {
+                     bool fused_add = false, bool masked = false, bool want_dx = true) {
   Plan p;
   const int E = 16 / esize;
   p.fast = (N % E) == 0 && !force_general;
@@ -1348,18 +1347,10 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
   // and room, and a row spread over all the workgroups its team can have.  More rows than
   // teams run in rounds; even then, and with few teams whose waits nothing hides, one
   // workgroup a row is several times slower (fp32 [2, 16777216]: 4800 us).
-  // Rows of no whole number of packs, where one workgroup a row has rows enough to hide its way through
-  // memory, go to teams only from there on (us, one workgroup a row / teams, bf16: forward [32, 36002] 7.2 / 6.8,
-  // [64, 32769] 7.5 / 7.8, [64, 60004] 9.4 / 8.1, [128, 45001] 9.1 / 9.5, [128, 110001] 14.6 / 15.1, [16, 110001] 13.0 /
-  // 7.4; backward [32, 32769] 6.5 / 6.5, [100, 45001] 8.7 / 10.2, [100, 60004] 12.4 / 8.6, [128, 80001] 20.0 / 16.2).
-  // Before both they went through softmax_*_stream_kernel: 7.9, 7.5, 11.5, 9.9, 19.2, 17.7; 7.4, 8.4, 10.4, 19.9.
+  // (Before teams and held rows the ragged ones went through softmax_*_stream_kernel, bf16 us: forward [32, 36002] 7.9,
+  // [64, 60004] 11.5, [16, 110001] 17.7 -> 7.4; backward [32, 32769] 7.4, [100, 60004] 10.4, [128, 80001] 19.9 -> 16.2.)
   const int64_t row_packs = (N + E - 1) / E;
-  // (an output wider than the input, float16 -> float32, has teams for all of them: its stores are most of the call
-  // and one workgroup's worth of them at a time is slow; forward, one workgroup / teams: [48, 40960] 12.7 / 8.7, [100,
-  // 60032] 20.1 / 13.5, [64, 45008] 14.2 / 10.2, [100, 60035] 21.4 / 14.4; [128, 32776] 12.8 / 12.9)
-  const bool team_rows =
-      p.fast || widened || (oc == OC_SOFTMAX_FWD ? 48 : 24) * (M - 24) <= row_packs - kSoftmaxTeamMinPacks;
-  if (softmax && team_rows && !force_general && !masked && ov.G == 0 && ov.V == 0 && ov.bpc == 0 && ov.block == 0 &&
+  if (softmax && !force_general && !masked && ov.G == 0 && ov.V == 0 && ov.bpc == 0 && ov.block == 0 &&
       2 * M <= num_cus && row_packs >= kSoftmaxTeamMinPacks) {
     const int64_t cus = num_cus * kTeamPerCu < kTeamMaxWorkgroups ? num_cus * kTeamPerCu : kTeamMaxWorkgroups;
     const int max_v = oc == OC_SOFTMAX_FWD ? kTeamMaxV : kSoftmaxBwdTeamMaxV;
@@ -1378,15 +1369,6 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
         p.team_v = (int)v;
         p.team_chunk_packs = v * kTeamBlock;
         p.team_grid = teams * team;
-        // Rows of whole packs that one workgroup a row serves faster, the exchange being longer than its way through
-        // the row: the more rows, the longer they may be (us, team / one workgroup, bf16 softmax: forward [16, 36032] 5.5 /
-        // 6.2, [48, 36032] 6.7 / 6.5, [64, 40000] 7.6 / 6.9, [64, 50048] 7.6 / 8.3, [128, 36032] 8.8 / 6.9, [128, 60032] 9.9 / 9.6,
-        // float32 [100, 25024] 8.5 / 9.8; backward [16, 32768] 5.0 / 3.6, [16, 45056] 5.1 / 5.5, [64, 40000] 7.0 / 5.9, [128,
-        // 32768] 7.7 / 4.7, [64, 50048] 7.2 / 7.7).
-        p.team_idle = p.fast && p.resident && !widened &&
-                      (oc == OC_SOFTMAX_FWD ? 48 * (M - 24) > row_packs - kSoftmaxTeamMinPacks &&
-                                                  (esize == 2 || row_packs <= 5120)
-                                            : row_packs <= kSoftmaxTeamMinPacks || (row_packs <= 5120 && M > 24));
       }
     }
   }
@@ -1407,6 +1389,100 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
     p.grad_resident = true;
   *out = p;
   return 0;
+}
+
+// Calls of few softmax rows of kSoftmaxTeamMinPacks packs or more: whether one workgroup a row (`whole`: whole packs,
+// in registers; otherwise held, see softmax_tail_serves()) is faster than teams, whose exchange is longer than its way
+// through a short row and shorter than through a long one.  The more rows, the longer they may be: teams get smaller
+// and their loads are no longer the only ones under way.  Teams of four and less (more rows than 2 / 5 of the compute
+// units) gain last.  Measured on the same buffers:
+//   whole packs, us, one workgroup / team, bf16 forward [30, 32768] 5.7 / 5.5, [48, 32768] 5.8 / 6.4, [48, 36032] 7.2 /
+//     6.6, [64, 40000] 7.5 / 7.6, [64, 45056] 8.2 / 7.6, [100, 50048] 9.4 / 8.6, [128, 50048] 9.5 / 9.6, [128, 65536]
+//     10.0 / 9.8; float32 forward [64, 20480] 6.5 / 7.3, [64, 22528] 8.1 / 7.4; bf16 backward [8, 32768] 3.5 / 4.8,
+//     [48, 33792] 6.4 / 6.1, [64, 36032] 6.7 / 7.0, [64, 45056] 7.6 / 7.1, [128, 50048] 8.9 / 9.6, [128, 60032] 11.0 /
+//     9.9
+//   ragged, time over that of the two passes which served such rows before, one workgroup / team, bf16 at 64 rows:
+//     forward of 5 packs a lane of 1024 0.88 / 0.96, of 8 0.81 / 0.73; backward 5 0.78 / 1.01, 8 0.78 / 0.87;
+//     log_softmax backward 10 0.70 / 0.91, 16 0.67 / 0.59.  At 128 rows: forward 10 0.76 / 0.89, 18 0.68 / 0.68;
+//     backward 6 0.92 / 1.24, 8 0.79 / 1.03; log_softmax backward 7 0.73 / 1.10, 16 0.77 / 0.88
+inline bool softmax_one_workgroup(bool backward, bool is_log, bool whole, int esize, int64_t M, int64_t packs,
+                                  int num_cus) {
+  const int64_t m = M * 256 / num_cus;
+  const bool small_teams = 5 * M > 2 * (int64_t)num_cus;
+  const int64_t from = kSoftmaxTeamMinPacks;
+  auto least = [](int64_t a, int64_t b) { return a < b ? a : b; };
+  if (whole) {
+    if (!backward && esize == 4) return packs <= 5120;
+    if (packs <= from) return backward || m >= 40;
+    return packs <= (small_teams ? 7168 : m >= 60 ? 5120 : 0);
+  }
+  if (!backward) {
+    if (esize == 4) return packs <= from + (is_log ? least(90 * m - 300, 3072) : 32 * (m - 32));
+    return packs <= (small_teams ? 17 * kMaxG : from + (is_log ? 90 * m : 50 * (m - 8)));
+  }
+  if (!is_log) return esize == 4 || packs <= from + 100 * m;
+  if (esize == 4) return packs <= from + least(256 * m, 3072);
+  return small_teams || packs <= least(from + 160 * m, 12000);
+}
+
+// Whether a softmax row of no whole number of packs is held by one workgroup (p.tail_v) rather than read twice.
+// widened: a float32 output of 16-bit rows.  The two passes, two workgroups a compute unit at different places of their
+// rows, keep (us, two passes / held; measured over 200 to 8192 rows, three fills of every pack count):
+inline bool softmax_tail_serves(const Plan& p, bool backward, bool is_log, bool widened, int esize, int64_t M,
+                                int64_t N) {
+  const int v = p.tail_v;
+  const int64_t cus = p.tail_cus, bytes = M * N * esize;
+  if (v == 0) return false;
+  if (backward) {
+    if (!is_log && v > kSoftmaxBwdHoldMaxV) return false;
+    // 16-bit rows that leave much of 4 or 5 packs a lane empty while a second pass comes out of the cache: both tensors
+    // in registers are one workgroup a compute unit ([2000, 29483] 62.1 / 66.9, [2000, 31939] 66.7 / 70.2, but [2000,
+    // 32515] 80.3 / 70.7, [300, 29483] 12.7 / 11.9; float32 gains there too: [2000, 16791] 88.4 / 69.6)
+    if (!is_log && esize == 2 && M > 2 * cus && 2 * bytes <= kSoftmaxCachedBytes &&
+        ((v == 4 && p.tail_packs <= 4032) || (v == 5 && p.tail_packs <= 4704)))
+      return false;
+    // float32 rows whose last lane round is nearly empty, many of them, grad alone held: [4096, 16791] 139 / 149,
+    // [3000, 20887] 130 / 135, with a float16 gradient 102 / 111; but [4096, 18839] 0.96 of the time
+    if (is_log && esize == 4 && v <= 7 && M > 7 * cus && p.tail_packs <= (v - 1) * kMaxG + 320) return false;
+    return true;
+  }
+  if (v == 17 || v == 19) return false;  // (not built: 0.91 to 1.12 of the two passes, worst at 300 rows)
+  if (widened)
+    // few rows, whose stores go out at the kernel's end ([130, 53243] 19.3 / 20.6, [200, 36859] 15.8 / 17.2, but [200,
+    // 53243] 25.7 / 22.7, [300, 36859] 33.7 / 27.7; log_softmax gains everywhere)
+    return is_log || !((4 * M <= 3 * cus && p.tail_packs > 4096) ||
+                       (M <= cus && p.tail_packs > 3500 && p.tail_packs <= 4800));
+  // log_softmax, whose second pass is short, out of the cache: 16-bit [2000, 48323] 65.5 / 70.2, [2000, 54875] 73.6 /
+  // 80.5 (at 1500 rows 1.0 to 1.06 of the time), float32 [3000, 18431] 71.1 / 76.7; but out of it [3000, 53243] 123 /
+  // 115, float32 [4096, 18431] 113 / 103
+  if (is_log && p.tail_g == kMaxG && M > 4 * cus &&
+      (esize == 2 ? v >= 6 && v <= 10 && bytes <= kSoftmaxCachedBytes : v <= 6 && bytes <= kSoftmaxCachedBytes * 7 / 8))
+    return false;
+  // 1024 lanes, one workgroup a compute unit.  A few rows more than compute units are a second round: 16-bit of 20
+  // packs a lane [300, 159739] 57.9 / 58.4, log_softmax 51.7 / 55.5, float32 of 10 to 16 [300, 65123] 45.3 / 48.3 (at
+  // 400 rows 0.94 to 1.03 of the time, at 200 0.8)
+  if (p.tail_g == kMaxG && M > cus && 2 * M <= 3 * cus && (esize == 2 ? v == 20 : v >= 10)) return false;
+  // float32 of 10 to 12 packs, the least that fill it: [1000, 37271] 66.0 / 69.2, [2000, 37271] 129 / 135, log_softmax
+  // [700, 45463] 55.4 / 58.2, but [2000, 38911] 131 / 127, of 11 packs [2000, 43007] 150 / 147
+  if (p.tail_g == kMaxG && esize == 4 && M > cus &&
+      ((v == 10 && !is_log) || (v <= 12 && v >= 10 && M <= 3 * cus)))
+    return false;
+  return true;
+}
+
+// (the held backward reads y through grad's window)
+inline bool softmax_tail_aligned(const void* grad, const void* y) {
+  return (((uintptr_t)grad ^ (uintptr_t)y) & 15u) == 0;
+}
+
+// Whether a softmax call without a mask, with its output apart from its inputs, goes to teams of workgroups (p.team).
+// held: nothing but softmax_tail_serves() is in the way of the held form.
+inline bool softmax_team_serves(const Plan& p, bool backward, bool is_log, bool widened, int esize, int64_t M,
+                                int64_t N, int num_cus, bool held = true) {
+  if (p.team == 0 || widened) return p.team > 0;
+  const bool one = p.resident || (held && softmax_tail_serves(p, backward, is_log, widened, esize, M, N));
+  const int64_t E = 16 / esize;
+  return !(one && softmax_one_workgroup(backward, is_log, p.fast, esize, M, (N + E - 1) / E, num_cus));
 }
 
 // GroupNorm backward of slabs beyond the registers held by teams of workgroups, one workgroup or

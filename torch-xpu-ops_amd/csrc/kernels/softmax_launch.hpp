@@ -98,19 +98,17 @@ bool launch_softmax_bwd_flat(FlatLayout f, const SoftmaxBwdArgs& a, hipStream_t 
   return false;
 }
 
-// Rows of no whole number of packs beyond the resident layouts, held by one workgroup of 1024 lanes
-// all the same (TAIL in the kernels).  False: not this case.
+// Rows of no whole number of packs beyond the resident layouts, held by one workgroup of 1024 or 512 lanes
+// all the same (TAIL in the kernels; softmax_tail_serves()).  False: not this case.
 #define ROWNORM_TAIL_CASES(CASE)                                                                 \
   CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(9) CASE(10) CASE(11) CASE(12) CASE(13)    \
   CASE(14) CASE(15) CASE(16) CASE(17) CASE(18) CASE(19) CASE(20)
-template <class T>
-constexpr bool softmax_tail_built(int g, int v, int most) {
-  return v <= (g == kMaxG ? most : kSoftmaxTailHalfMaxV) && v * elems_per_pack<T>::value > kSoftmaxWideElems;
-}
 
 template <class TI, class TO, int G, int V>
 bool launch_softmax_fwd_tail_v(const Plan& plan, const SoftmaxFwdArgs& a, hipStream_t stream) {
-  if constexpr (softmax_tail_built<TI>(G, V, max_v_of(OC_SOFTMAX_FWD, sizeof(TI))) && V != 17 && V != 19) {
+  constexpr bool BUILT = V <= (G == kMaxG ? max_v_of(OC_SOFTMAX_FWD, sizeof(TI)) : kSoftmaxTailHalfMaxV) && V != 17 &&
+                         V != 19 && V * elems_per_pack<TI>::value > kSoftmaxWideElems;
+  if constexpr (BUILT) {
     hipLaunchKernelGGL((softmax_fwd_resident_kernel<TI, TO, G, V, G, true, false, true>),
                        dim3((unsigned)plan.grid), dim3(G), 0, stream, (const TI*)a.x, (TO*)a.y,
                        MaskRef{}, a.M, a.N, a.flags);
@@ -121,15 +119,8 @@ bool launch_softmax_fwd_tail_v(const Plan& plan, const SoftmaxFwdArgs& a, hipStr
 
 template <class TI, class TO>
 bool launch_softmax_fwd_tail(const Plan& plan, const SoftmaxFwdArgs& a, hipStream_t stream) {
-  // log_softmax of 6 or 7 packs a lane out of the cache: the two passes, with their two workgroups a compute unit at
-  // different places of a row, measured faster ([2000, 49001] 65.8 us against 73.5, [2000, 57001] 80.6 against 85.7, but
-  // [1000, 57001] 43.7 against 43.1 and [4096, 49001] 154 against 146)
-  if ((a.flags & kSoftmaxLog) && plan.tail_g == kMaxG && (plan.tail_v == 6 || plan.tail_v == 7) &&
-      a.M > 4 * (int64_t)plan.tail_cus && a.M * (int64_t)a.N * (int64_t)sizeof(TI) <= kSoftmaxCachedBytes)
+  if (!softmax_tail_serves(plan, false, (a.flags & kSoftmaxLog) != 0, sizeof(TO) > sizeof(TI), sizeof(TI), a.M, a.N))
     return false;
-  // (17 and 19 packs a lane measured slower than the two passes as well, 16, 18 and 20 faster: [1603, 133540] 182 us
-  // against 187, [1603, 152001] 214 against 231; [1603, 131001] 182 against 166, [1603, 140001] 199 against 185)
-  if (plan.tail_v == 17 || plan.tail_v == 19) return false;
   switch (plan.tail_v) {
 #define ROWNORM_TAIL_FWD(v)                                                                  \
   case v:                                                                                    \
@@ -143,7 +134,7 @@ bool launch_softmax_fwd_tail(const Plan& plan, const SoftmaxFwdArgs& a, hipStrea
 
 template <class TG, class TO, int V>
 bool launch_softmax_bwd_tail_v(const Plan& plan, const SoftmaxBwdArgs& a, hipStream_t stream) {
-  constexpr bool BUILT = softmax_tail_built<TG>(kMaxG, V, kGradResidentMaxV);
+  constexpr bool BUILT = V <= kGradResidentMaxV && V * elems_per_pack<TG>::value > kSoftmaxWideElems;
   if constexpr (BUILT && V >= kSoftmaxTailGradMinV) {
     if (a.flags & kSoftmaxLog) {
       hipLaunchKernelGGL((log_softmax_bwd_grad_resident_kernel<TG, TO, V, kStreamBlock, true>),
@@ -163,15 +154,8 @@ bool launch_softmax_bwd_tail_v(const Plan& plan, const SoftmaxBwdArgs& a, hipStr
 
 template <class TG, class TO>
 bool launch_softmax_bwd_tail(const Plan& plan, const SoftmaxBwdArgs& a, hipStream_t stream) {
-  if ((((uintptr_t)a.grad ^ (uintptr_t)a.y) & 15u) != 0) return false;  // (y in grad's window)
-  // softmax rows that leave much of 4 or 5 packs a lane empty, out of the cache, likewise: both tensors in registers
-  // are one workgroup a compute unit ([1000, 28003] 31.6 us against 33.3, [2000, 35001] 76.3 against 79.2, but [2000, 32750]
-  // 88.0 against 73.3, [4096, 28003] 145 against 129)
-  const bool few = a.M <= 2 * (int64_t)plan.tail_cus;
-  if (!(a.flags & kSoftmaxLog) &&
-      ((plan.tail_v == 4 && plan.tail_packs <= 3840) || (plan.tail_v == 5 && plan.tail_packs <= 4608 && !few)) &&
-      2 * a.M * (int64_t)a.N * (int64_t)sizeof(TG) <= kSoftmaxCachedBytes)
-    return false;
+  if (!softmax_tail_aligned(a.grad, a.y)) return false;
+  if (!softmax_tail_serves(plan, true, (a.flags & kSoftmaxLog) != 0, false, sizeof(TG), a.M, a.N)) return false;
   switch (plan.tail_v) {
 #define ROWNORM_TAIL_BWD(v)                                                                  \
   case v: return launch_softmax_bwd_tail_v<TG, TO, v>(plan, a, stream);
