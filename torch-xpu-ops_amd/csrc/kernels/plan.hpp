@@ -177,11 +177,13 @@ constexpr int kGradResidentMaxV = 20;
 constexpr int kSoftmaxTailMinV = 3;
 // The forward on 512 lanes where more and smaller workgroups a compute unit overlap better: the shortest of these rows
 // and calls of few rows (bf16 softmax, 1024 / 512 lanes: [4096, 17001] 54.1 / 50.0 us, [2000, 24570] 39.0 / 37.0, [1000,
-// 20005] 18.5 / 14.5, [512, 41003] 16.2 / 15.0, but [4096, 28003] 80.4 / 84.9, [2000, 41003] 61.9 / 62.9).
-constexpr int kSoftmaxTailHalfMaxV = 16;
+// 20005] 18.5 / 14.5, [512, 41003] 16.2 / 15.0, but [4096, 28003] 80.4 / 84.9, [2000, 41003] 61.9 / 62.9).  Rows of the
+// resident layouts end at 16384 elements, so a lane holds 5 packs at least (float32: 9).
+constexpr int kSoftmaxTailHalfMaxV = 14;
+constexpr int softmax_tail_half_min_v(int esize) { return esize == 2 ? 5 : 9; }
 constexpr bool softmax_tail_half_lanes(int64_t packs, int64_t M, int num_cus) {
   return packs <= 2560 || (packs <= 4096 && M <= 8 * (int64_t)num_cus) ||
-         (packs <= kMaxG / 2 * kSoftmaxTailHalfMaxV - 1024 && M <= 2 * (int64_t)num_cus);
+         (packs <= kMaxG / 2 * kSoftmaxTailHalfMaxV && M <= 2 * (int64_t)num_cus);
 }
 // The log_softmax backward holds grad alone from here on (both tensors: [2000, 49001] 112 us, grad alone 106, the
 // multi-pass kernel 106; [1000, 65001] 81.4, 72.7, 74.8; float32 of 5 to 8 packs 0.97 to 1.05 of grad alone's time).

@@ -106,8 +106,10 @@ bool launch_softmax_bwd_flat(FlatLayout f, const SoftmaxBwdArgs& a, hipStream_t 
 
 template <class TI, class TO, int G, int V>
 bool launch_softmax_fwd_tail_v(const Plan& plan, const SoftmaxFwdArgs& a, hipStream_t stream) {
-  constexpr bool BUILT = V <= (G == kMaxG ? max_v_of(OC_SOFTMAX_FWD, sizeof(TI)) : kSoftmaxTailHalfMaxV) && V != 17 &&
-                         V != 19 && V * elems_per_pack<TI>::value > kSoftmaxWideElems;
+  constexpr int ES = sizeof(TI);
+  constexpr bool BUILT = G == kMaxG ? V <= max_v_of(OC_SOFTMAX_FWD, ES) && V != 17 && V != 19 &&
+                                          V * elems_per_pack<TI>::value > kSoftmaxWideElems
+                                    : V >= softmax_tail_half_min_v(ES) && V <= kSoftmaxTailHalfMaxV;
   if constexpr (BUILT) {
     hipLaunchKernelGGL((softmax_fwd_resident_kernel<TI, TO, G, V, G, true, false, true>),
                        dim3((unsigned)plan.grid), dim3(G), 0, stream, (const TI*)a.x, (TO*)a.y,
