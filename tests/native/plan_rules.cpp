@@ -135,6 +135,14 @@ int rule_softmax_route(int backward, int is_log, int64_t M, int64_t N, int esize
   return 3;
 }
 
+// the backward of long norm rows: wavefronts that share a piece of columns (0: not the two launches without partial
+// rows), workgroups of the team that holds four rows at a time (0: none)
+void rule_norm_few_rows(int64_t M, int64_t N, int esize, int layer_norm, int wide, int64_t out[2]) {
+  Plan p;
+  make_plan(OC_NORM_BWD, M, N, esize, 256, Override{}, true, &p, false, layer_norm != 0, wide != 0);
+  out[0] = p.few_waves, out[1] = p.team;
+}
+
 // one table of slots for streams, as the library keeps one per device
 int rule_team_slots() { return kTeamSlots; }
 void* rule_slots_new() { return new StreamSlots<kTeamSlots>(); }

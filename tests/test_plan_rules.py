@@ -333,3 +333,26 @@ def test_which_ragged_softmax_rows_are_held(rules):
                             g == 1024 and v in range(3 if es == 2 else 5, 21 if es == 2 else 17) and v not in (17, 19))
                     kind, g, v = _route(rules, 1, 0, M, N, es)
                     assert kind == "two passes" or (g == 1024 and (3 if es == 2 else 5) <= v <= 8)
+
+
+def test_backward_of_few_long_norm_rows(rules):
+    """Both sides of the lines between the two launches without partial rows and the teams of whole-pack rows as they
+    measured: (rows, elements, bytes an element, LayerNorm, float32 weights of 16-bit rows)."""
+
+    def f(*c):
+        out = (ctypes.c_int64 * 2)()
+        rules.rule_norm_few_rows(*map(ctypes.c_int64, c[:2]), *c[2:], out)
+        return list(out)
+
+    few = [(40, 80000, 4, 1, 0), (24, 160000, 4, 1, 0), (16, 224000, 4, 1, 0), (64, 160000, 2, 1, 1), (48, 224000, 2, 1, 1),
+           (64, 160000, 2, 1, 0), (40, 224000, 2, 1, 0), (128, 66400, 2, 1, 0), (24, 320000, 4, 1, 0), (16, 520000, 4, 1, 0),
+           (80, 79997, 4, 1, 0), (100, 79997, 4, 1, 0), (24, 640000, 2, 1, 1), (64, 79997, 4, 0, 0), (16, 320000, 2, 0, 0)]
+    team = [(128, 40000, 4, 1, 0), (100, 56000, 4, 1, 0), (80, 80000, 4, 1, 0), (48, 112000, 4, 1, 0), (32, 160000, 4, 1, 0),
+            (48, 160000, 4, 1, 0), (24, 224000, 4, 1, 0), (80, 160000, 2, 1, 1), (64, 224000, 2, 1, 1), (40, 320000, 2, 1, 1),
+            (32, 448000, 2, 1, 1), (48, 320000, 2, 1, 0), (32, 160000, 4, 0, 0), (100, 112000, 2, 0, 0)]
+    for c in few:
+        assert f(*c)[0] in (1, 2, 4, 8) and f(*c)[1] == 0, (c, f(*c))
+    for c in team:
+        assert f(*c)[0] == 0 and f(*c)[1] >= 2, (c, f(*c))
+    assert [f(2, N, 2, 1, 0)[0] for N in (66400, 163840, 300000, 600000)] == [8, 4, 2, 1] and f(129, 66401, 2, 1, 0)[0] == 0
+    assert f(1, 66400, 2, 1, 0) == [0, 0] and f(2, 3000000, 2, 1, 0) == [0, 0]

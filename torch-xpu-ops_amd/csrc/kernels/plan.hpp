@@ -840,6 +840,35 @@ inline WavesLayout norm_waves_layout(bool backward, int esize, int64_t M, int64_
   return l;
 }
 
+// Teams of a norm backward whose rows of `packs` packs are beyond one workgroup's registers (norm_bwd_team_kernel):
+// workgroups a team, teams (0: none), whether they make enough rounds to be worth it.  whole: what the kernel takes
+// (whole packs, no residual gradient).
+struct NormBwdTeam {
+  int64_t team = 0, teams = 0;
+  bool rounds_ok = false;
+};
+inline NormBwdTeam norm_bwd_team(int64_t M, int64_t packs, bool whole, bool layer_norm, int num_cus) {
+  const int64_t cus = num_cus * kTeamBwdPerCu < kTeamMaxWorkgroups ? num_cus * kTeamBwdPerCu : kTeamMaxWorkgroups;
+  const int64_t chunk = (int64_t)kTeamBwdPacks * kTeamBlock;
+  const int64_t groups = (M + kTeamBwdRows - 1) / kTeamBwdRows;
+  NormBwdTeam t;
+  t.team = (packs + chunk - 1) / chunk;
+  if (!whole || t.team < 2 || t.team > cus) return t;
+  t.teams = cus / t.team < groups ? cus / t.team : groups;
+  // Worth it from the second round on (a call costs about 25 us beside 9.5-10 us a round,
+  // where the two passes of the other kernels cost about 14.6 us for a round's rows); a
+  // LayerNorm on large teams (more than 64 workgroups a row) from the fourth.  Measured,
+  // bf16, LayerNorm / RMSNorm, team against two passes in us: [512, 401408] (26 rounds)
+  // 258 / 243 against 359 / 350; [4096, 65536] (64) 330 / 308 against 478 / 468; [100,
+  // 401408] (5) 66 / 59 against 80 / 75; [1024, 40960] (5) 82 / 72 against 81 / 75; [512,
+  // 65536] (4) 62 / 52 against 68 / 63; [32, 401408] (2) 34 / 29 against 41 / 37; [64,
+  // 262144] (2) 41 / 32 against 41 / 38; [16, 1048576] (2, 128 workgroups a row) 41 / 31
+  // against 35 / 34; [8192, 24584] (a row's last workgroup holds a single pack) 327
+  // against 380.
+  t.rounds_ok = layer_norm && t.team > 64 ? groups >= 4 * t.teams : groups > t.teams;
+  return t;
+}
+
 // Returns 0, or -5 (ROWNORM_ERR_OVERRIDE) when a forced variant cannot hold the row.
 // force_general: take the general (ragged-row) kernels even when N % E == 0.
 // layer_norm: the norm op is LayerNorm (statistics of two sums, beta), not RMSNorm.
@@ -1164,12 +1193,19 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
   // 292096] 25.5 -> 11.9, [64, 60000] 28.5 -> 16.9, [57, 156800] 34.2 -> 27.4.  The other sides of the lines: [251,
   // 51584] 37.1 / 46.0, [100, 400000] 67 / 82, and rows that alone give every compute unit two workgroups, which
   // the column-sum kernels serve without partial rows as well ([3, 1451648] 16.6 / 21.4, [7, 1413504] 29.3 / 32.3).
-  // An RMSNorm of whole packs keeps its teams, which have half the sums to exchange and to add, from half as many
-  // rows and bytes on ([24, 194976] 23.6 -> 14.7, but [75, 162328] 28.3 / 33.8, [108, 38472] 20.6 / 24.2, [19, 659856]
-  // 27.5 / 30.8).  200 random calls that take it: 0.58 of the time, two slower (1.03).
+  // An RMSNorm of whole packs keeps its teams, which have half the sums to exchange and to add, from half as many rows
+  // and bytes on ([24, 194976] 23.6 -> 14.7, but [75, 162328] 28.3 / 33.8, [108, 38472] 20.6 / 24.2, [19, 659856] 27.5
+  // / 30.8), a LayerNorm that has teams from 16 (float32), 21 (float32 weights) and 24 MB a tensor on, where dY and X
+  // no longer come out of the L2s, 32 MB together, when they are read again: time over that of the teams, float32 [40,
+  // 112000] 17 MB 0.91, [48, 112000] 20 MB 1.06, [48, 160000] 29 MB 1.37; bf16 with float32 weights [64, 160000] 20 MB
+  // 0.92, [80, 160000] 24 MB 1.11; bf16 [80, 160000] 24 MB 1.02, [48, 320000] 29 MB 1.07; rows without teams, float32
+  // [24, 320000] 29 MB 0.95, [80, 79997] 24 MB 0.78.
   const int64_t few_part = layer_norm || !p.fast ? 1 : 2;
+  const int64_t few_bytes = layer_norm && norm_bwd_team(M, packs, p.fast && !fused_add, true, num_cus).rounds_ok
+                                ? (int64_t)(esize == 4 ? 16 : wide_weights ? 21 : 24) << 20
+                                : kFewRowsBytes;
   if (oc == OC_NORM_BWD && !p.resident && want_cols && want_dx && p.partial_rows > 1 && M * few_part <= kFewRowsMax &&
-      M * packs * 16 * few_part <= kFewRowsBytes && ov.G == 0 && ov.V == 0 && ov.bpc == 0 && ov.block == 0) {
+      M * packs * 16 * few_part <= few_bytes && ov.G == 0 && ov.V == 0 && ov.bpc == 0 && ov.block == 0) {
     const int64_t pieces = (packs + 63) / 64;
     p.few_waves = kFewRowsWaves;
     while (p.few_waves > 1 && pieces * p.few_waves > kFewRowsWaves * (int64_t)num_cus) p.few_waves /= 2;
@@ -1315,31 +1351,13 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
   const bool team_bwd_forced = ov.G == -1 && ov.V == 0 && ov.block == 1 && ov.bpc == 0;
   if (oc == OC_NORM_BWD && !p.resident && p.fast && !fused_add && want_dx && p.few_waves == 0 &&
       ((ov.G == 0 && ov.V == 0 && ov.bpc == 0 && ov.block == 0) || team_bwd_forced)) {
-    const int64_t cus = num_cus * kTeamBwdPerCu < kTeamMaxWorkgroups ? num_cus * kTeamBwdPerCu : kTeamMaxWorkgroups;
-    const int64_t chunk = (int64_t)kTeamBwdPacks * kTeamBlock;
-    const int64_t team = (packs + chunk - 1) / chunk;
-    const int64_t ngroups = (M + kTeamBwdRows - 1) / kTeamBwdRows;
-    if (team >= 2 && team <= cus) {
-      int64_t teams = cus / team;
-      if (teams > ngroups) teams = ngroups;
-      // Worth it from the second round on (a call costs about 25 us beside 9.5-10 us a round,
-      // where the two passes of the other kernels cost about 14.6 us for a round's rows); a
-      // LayerNorm on large teams (more than 64 workgroups a row) from the fourth.  Measured,
-      // bf16, LayerNorm / RMSNorm, team against two passes in us: [512, 401408] (26 rounds)
-      // 258 / 243 against 359 / 350; [4096, 65536] (64) 330 / 308 against 478 / 468; [100,
-      // 401408] (5) 66 / 59 against 80 / 75; [1024, 40960] (5) 82 / 72 against 81 / 75; [512,
-      // 65536] (4) 62 / 52 against 68 / 63; [32, 401408] (2) 34 / 29 against 41 / 37; [64,
-      // 262144] (2) 41 / 32 against 41 / 38; [16, 1048576] (2, 128 workgroups a row) 41 / 31
-      // against 35 / 34; [8192, 24584] (a row's last workgroup holds a single pack) 327
-      // against 380.
-      const bool rounds_ok = layer_norm && team > 64 ? ngroups >= 4 * teams : ngroups > teams;
-      if (teams >= 1 && (rounds_ok || team_bwd_forced)) {
-        p.team = (int)team;
-        p.team_v = kTeamBwdPacks;
-        p.team_chunk_packs = chunk;
-        p.team_grid = teams * team;
-        p.team_partial_rows = want_cols ? teams : 0;
-      }
+    const NormBwdTeam t = norm_bwd_team(M, packs, p.fast, layer_norm, num_cus);
+    if (t.teams >= 1 && (t.rounds_ok || team_bwd_forced)) {
+      p.team = (int)t.team;
+      p.team_v = kTeamBwdPacks;
+      p.team_chunk_packs = (int64_t)kTeamBwdPacks * kTeamBlock;
+      p.team_grid = t.teams * t.team;
+      p.team_partial_rows = want_cols ? t.teams : 0;
     }
   }
   // Softmax forward / backward of few, very long rows: one workgroup a row
