@@ -228,8 +228,9 @@ int mi355x_rms_norm_bwd_static(const void* dy, const void* x, const float* rstd,
  * for the inner_size == 1 case (SoftMaxKernels.cpp:1663-1720).  out_dtype is
  * in_dtype, or ROWNORM_F32 with a ROWNORM_F16 input (half_to_float,
  * SoftMaxKernels.cpp:2131-2135).  Few, very long rows (fewer rows than half the
- * compute units, 4096 16-byte packs a row or more, 16-byte aligned x and y that do
- * not overlap) are each held by a team of workgroups, under the rules described at
+ * compute units, 4096 16-byte packs a row or more, x and y that do not overlap, 16-byte
+ * aligned if the row is a whole number of packs) are each held by a team of workgroups
+ * where that is faster (mi355x_softmax_plan says where), under the rules described at
  * mi355x_rownorm_set_team_wait_us; mi355x_softmax_bwd likewise (gi apart from grad
  * and y). */
 int mi355x_softmax_fwd(const void* x, void* y, int64_t rows, int64_t N, rownorm_dtype in_dtype,
@@ -359,15 +360,15 @@ int mi355x_softmax_strided_plan(int backward, int64_t outer, int64_t dim_size, i
  * block_threads threads, packs_per_lane rows on each of the rows_per_block threads along
  * dim_size; grid_blocks / reserved teams walk the strips.  `reserved` == 0: no teams, the rest is what
  * mi355x_softmax_strided_plan reports.  Teams serve inner sizes of a pack or more, any alignment, where
- * they measured faster; reported are inner sizes of whole packs, and an inner size between two of those has
- * the teams of the larger one.  Teams of more than one workgroup pass the columns' partial results through
+ * they measured faster.  Teams of more than one workgroup pass the columns' partial results through
  * the stream's bookkeeping slot, under the rules of mi355x_rownorm_set_team_wait_us (eight streams
  * can hold a slot of this kind): a workgroup may wait for the others of its team for up to
  * that bound, and reads the whole strip itself if it runs out.  They need an output that overlaps no
  * input; such a call in place, on a stream under capture, or on a stream beyond the eight takes
  * mi355x_softmax_strided_plan's layout.  A team of one waits for nobody and has none of these
- * conditions, but where inner is not a whole number of packs the output must overlap no input.  Reported is the call whose output has the input's type: a float16 forward with a float32
- * output keeps to teams of which a compute unit holds two (packs_per_lane <= 16). */
+ * conditions, but where inner is not a whole number of packs the output must overlap no input.
+ * Reported is the call whose output has the input's type: a float16 forward with a float32 output
+ * keeps to teams of which a compute unit holds two (packs_per_lane <= 16). */
 int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_size, int64_t inner,
                                      rownorm_dtype dtype, rownorm_plan* out);
 
@@ -389,13 +390,12 @@ int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_si
  * lane (float32 LayerNorm: 10), and the masked softmax calls beyond 32 elements a
  * lane on 1024 lanes (rows of more than 32768 elements; a forced layout beyond
  * that is ROWNORM_ERR_OVERRIDE for a masked call).
- * Softmax calls on longer ragged rows without a mask are held by one workgroup all the same (up to 20 packs a lane;
- * the backward: 8, log_softmax 20, with Y aligned like grad), few of them by teams; neither is reported here, where
- * such rows appear as the multi-pass layout that serves them otherwise.  Rows of whole packs reported with a team run
- * on one workgroup each where the calls have many rows for their length and that is faster.
- * Fewer than eight forward rows of whole packs beyond one workgroup's registers are held by teams of at most an
- * eighth of the machine where the conditions of mi355x_rownorm_set_team_wait_us allow it; reported is the layout
- * they have otherwise.
+ * Of the softmax ops it is the layout of softmax with an output of the input's type
+ * (mi355x_softmax_plan, which also knows log_softmax and float16 <-> float32).  Rows held by
+ * teams of workgroups (reserved workgroups a row, grid_blocks of them) are reported where an
+ * ordinary call takes them: under the conditions of mi355x_rownorm_set_team_wait_us, with
+ * tensors on 16-byte boundaries; a call that does not meet those takes other launches.
+ * Norm backward calls that mi355x_rownorm_few_rows_plan reports run on two launches instead.
  * Norm calls that mi355x_rownorm_waves_plan reports a layout for run on that one instead; the one
  * reported here then serves the same call with a residual add or gradient, an output cast, or a forced field. */
 int mi355x_rownorm_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_dtype,
@@ -418,6 +418,24 @@ int mi355x_rownorm_plan_at(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_
  * norm; equal calls give equal bits. */
 int mi355x_rownorm_waves_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_dtype,
                               rownorm_dtype w_dtype, rownorm_plan* out);
+
+/* The layout of an unmasked softmax / log_softmax call (backward != 0: grad and y in in_dtype, the gradient in
+ * out_dtype) whose tensors start on a 128-byte line and whose output overlaps no input, on a stream that is not under
+ * capture.  `reserved` > 0: a row is held by a team of that many workgroups of block_threads threads, packs_per_lane
+ * packs a lane; such a call in place, captured, off a 16-byte boundary (whole packs) or on a stream without a slot
+ * runs without teams.  Otherwise `resident` != 0: a row is held by lanes_per_row lanes, rows of no whole number of packs
+ * beyond 16384 elements in whole packs of the 16-byte aligned window around the row (the backward: with y aligned like
+ * grad; the log_softmax backward from 4 packs a lane on holds grad alone); resident == 0: two passes over the inputs.
+ * The LDS-staged kernels of short rows are described at mi355x_rownorm_plan. */
+int mi355x_softmax_plan(int backward, int is_log, int64_t rows, int64_t N, rownorm_dtype in_dtype,
+                        rownorm_dtype out_dtype, rownorm_plan* out);
+
+/* The layout of a LayerNorm / RMSNorm backward of few rows beyond one workgroup's registers, dX and column sums
+ * wanted, in two launches without partial rows: `reserved` wavefronts share 64 packs of columns (lanes_per_row lanes, a
+ * pack each) and walk all rows_per_block = M rows under them, grid_blocks workgroups of block_threads threads.
+ * `reserved` == 0: not this call, the rest is what mi355x_rownorm_plan reports. */
+int mi355x_rownorm_few_rows_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_dtype,
+                                 rownorm_dtype w_dtype, rownorm_plan* out);
 
 /* Test and tuning hook: force lanes_per_row / packs_per_lane / threads per
  * workgroup / workgroups per compute unit for one op (0 keeps the automatic

@@ -52,6 +52,8 @@ DECL(mi355x_group_norm_plan);
 DECL(mi355x_rownorm_plan);
 DECL(mi355x_rownorm_plan_at);
 DECL(mi355x_rownorm_waves_plan);
+DECL(mi355x_rownorm_few_rows_plan);
+DECL(mi355x_softmax_plan);
 DECL(mi355x_rownorm_set_override);
 
 static int failures = 0;

@@ -138,11 +138,11 @@ def test_plan_invariants(cabi, op, dt):
             p = cabi.plan(op, M, N, dt, dt)
             assert p["grid_blocks"] >= 1
             if op in (cabi.OP_SOFTMAX_FWD, cabi.OP_SOFTMAX_BWD) and p["row_chunks"] > 0:
-                # few, very long softmax rows of whole packs: a team of `row_chunks` workgroups
+                # few, very long softmax rows: a team of `row_chunks` workgroups
                 # of 512 threads holds a row (16 packs a lane at most, the backward 8 of each
                 # tensor), no more teams than rows
                 team = p["row_chunks"]
-                assert N % E == 0 and N // E >= 4096 and 2 * M <= 256, (M, N, p)
+                assert N // E >= 4096 and 2 * M <= 256 and p["block_threads"] == 512, (M, N, p)
                 assert team >= 2 and p["grid_blocks"] % team == 0 and p["grid_blocks"] <= 512
                 assert 1 <= p["grid_blocks"] // team <= M
                 assert team * 512 * (16 if op == cabi.OP_SOFTMAX_FWD else 8) * E >= N
@@ -169,12 +169,13 @@ def test_plan_invariants(cabi, op, dt):
                 assert M >= 16 * teams and 5 * (N // E) >= 4 * team * 5120
             elif (op in (cabi.OP_LAYER_NORM_FWD, cabi.OP_RMS_NORM_FWD) and N % E == 0 and
                   p["grid_blocks"] > M):
-                # rows of whole packs beyond one workgroup's registers, 8 teams or more: a team
-                # of `row_chunks` workgroups holds a row, at most one workgroup a compute unit,
-                # no more teams than rows, every workgroup with at most 16 packs a lane
+                # rows of whole packs beyond one workgroup's registers, 8 teams or more, or fewer
+                # rows all at once: a team of `row_chunks` workgroups holds a row, no more teams
+                # than rows, every workgroup with at most 16 packs a lane
                 team = p["row_chunks"]
                 assert p["rows_per_block"] == 1 and team >= 1 and p["grid_blocks"] % team == 0
-                assert p["grid_blocks"] <= 512 and 8 <= p["grid_blocks"] // team <= M
+                assert p["grid_blocks"] <= 512 and min(8, M) <= p["grid_blocks"] // team <= M
+                assert M >= 8 or team <= 64
                 assert team * 512 * 16 * E >= N
             elif (op in (cabi.OP_LAYER_NORM_BWD, cabi.OP_RMS_NORM_BWD) and N % E == 0 and
                   p["row_chunks"] >= 2 and p["block_threads"] == 512 and p["packs_per_lane"] == 2):
@@ -452,7 +453,7 @@ def test_strided_softmax_team_plans(cabi):
                     seen.add("none")
                     continue
                 seen.add("one" if t["team"] == 1 else "several")
-                assert inner % E == 0 and t["resident"] == 1 and t["block_threads"] == 512
+                assert inner >= E and t["resident"] == 1 and t["block_threads"] == 512
                 assert t["lanes_per_row"] * t["rows_per_block"] == 512
                 assert t["team"] * t["rows_per_block"] * t["packs_per_lane"] >= D
                 assert t["grid_blocks"] % t["team"] == 0 and t["grid_blocks"] <= 512
@@ -464,6 +465,36 @@ def test_strided_softmax_team_plans(cabi):
     p = cabi.Plan()
     assert cabi.lib().mi355x_softmax_strided_team_plan(0, 1, -1, 8, cabi.F32, p) == -2
     assert cabi.lib().mi355x_softmax_strided_team_plan(0, 1, 8, 8, 7, p) < 0
+
+
+def test_softmax_and_few_rows_plans(cabi):
+    """The queries report the launch that an ordinary call runs on: teams, rows in registers, ragged rows held by one
+    workgroup, grad alone, two passes."""
+    f = cabi.softmax_plan
+    for M, N, dt in ((4, 32771, cabi.BF16), (64, 45056, cabi.BF16), (8, 22528, cabi.F32), (200, 32768, cabi.BF16),
+                     (128, 32768, cabi.BF16), (2000, 32515, cabi.BF16), (2000, 66003, cabi.F32), (16384, 4096, cabi.BF16)):
+        for bwd, op in ((0, cabi.OP_SOFTMAX_FWD), (1, cabi.OP_SOFTMAX_BWD)):
+            p, q = f(bwd, 0, M, N, dt), cabi.plan(op, M, N, dt, dt)
+            assert p.pop("team") == q.pop("row_chunks") and p == q
+    shape = lambda p: (p["team"], p["resident"], p["lanes_per_row"], p["packs_per_lane"])  # noqa: E731
+    for c, want in (((0, 0, 128, 32768), (0, 1, 1024, 4)), ((0, 0, 4096, 50257), (0, 1, 1024, 7)),
+                    ((0, 1, 4096, 17001), (0, 1, 512, 5)), ((1, 0, 4096, 17001), (0, 1, 1024, 3)),
+                    ((1, 1, 4096, 128255), (0, 1, 1024, 16)), ((1, 1, 4096, 128256), (0, 1, 1024, 16)),
+                    ((0, 0, 4096, 163840), (0, 1, 1024, 20))):
+        assert shape(f(*c, cabi.BF16)) == want, c
+    assert f(0, 0, 4, 32771, cabi.BF16)["team"] == 9
+    assert f(1, 0, 4096, 128256, cabi.BF16)["resident"] == 0 and f(0, 0, 4096, 133540, cabi.BF16)["resident"] == 0
+    assert f(0, 0, 100, 60032, cabi.F16, cabi.F32)["team"] > 1 and f(0, 0, 100, 40000, cabi.F16)["team"] == 0
+    few = cabi.few_rows_plan(cabi.OP_LAYER_NORM_BWD, 28, 70144, cabi.BF16, cabi.BF16)
+    assert (few["waves"], few["block_threads"], few["rows_per_block"], few["grid_blocks"]) == (8, 512, 28, 137)
+    assert cabi.few_rows_plan(cabi.OP_RMS_NORM_BWD, 75, 162328, cabi.BF16, cabi.BF16)["waves"] == 0
+    assert cabi.few_rows_plan(cabi.OP_LAYER_NORM_FWD, 28, 70144, cabi.BF16, cabi.BF16)["waves"] == 0
+    p, L = cabi.Plan(), cabi.lib()
+    assert L.mi355x_softmax_plan(0, 0, -1, 8, cabi.F32, cabi.F32, p) == -2
+    assert L.mi355x_softmax_plan(0, 0, 8, 8, cabi.F32, cabi.F16, p) < 0
+    assert L.mi355x_softmax_plan(1, 0, 8, 8, 7, 7, p) < 0 and L.mi355x_softmax_plan(0, 0, 8, 8, 0, 0, None) < 0
+    assert L.mi355x_softmax_plan(1, 0, 8, 8, cabi.F32, cabi.F16, p) == 0
+    assert L.mi355x_rownorm_few_rows_plan(99, 8, 8, cabi.F32, cabi.F32, p) < 0
 
 
 def test_group_norm_validation_and_plans(cabi):

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 # (outer, D, columns beyond whole packs, whole packs): one pack and an element; a strip's last pack alone in a strip
 # of its own; the one-workgroup tile at its largest D and beyond; teams of one, of several, of whole compute units.
-# Beside each: the workgroups of a team in the 16-bit forward and backward.
+# Beside each: the workgroups of a team in the forward and backward.
 SHAPES = {(3, 5, 1, 1): (0, 0), (2, 40, 3, 4): (0, 0), (2, 256, 1, 16): (0, 0), (1, 300, 1, 1): (0, 0),
           (2, 600, 2, 16): (19, 19), (2, 2300, 3, 32): (18, 18), (600, 300, 1, 8): (1, 2), (1000, 300, 1, 7): (1, 1),
           (1, 8200, 3, 512): (13, 43)}
@@ -26,9 +26,8 @@ SHAPES = {(3, 5, 1, 1): (0, 0), (2, 40, 3, 4): (0, 0), (2, 256, 1, 16): (0, 0), 
 def test_rows_of_no_whole_packs(cabi, oracle, gpu, dtype, shape):
     outer, D, over, packs = shape
     inner = packs * (4 if dtype == torch.float32 else 8) + over
-    if dtype != torch.float32:  # (the teams of the next inner size of whole packs)
-        assert tuple(cabi.strided_team_plan(b, outer, D, (packs + 1) * 8, cabi.BF16)["team"]
-                     for b in (0, 1)) == SHAPES[shape]
+    teams = tuple(cabi.strided_team_plan(b, outer, D, inner, cabi.dtype_code(dtype))["team"] for b in (0, 1))
+    assert teams == SHAPES[shape]
     print("case strided softmax, ragged", dtype, (outer, D, inner), flush=True)
     g = gen(3100 + D)
     x = (3.0 * torch.randn(outer, D, inner, generator=g)).to(dtype)

@@ -1,5 +1,5 @@
-"""softmax / log_softmax forward and backward of few, very long rows (fewer rows than half the
-compute units, 32768 16-bit or 16384 float32 elements and more, whole 16-byte packs):
+"""softmax / log_softmax forward and backward of few, very long rows of whole 16-byte packs (fewer rows than half the
+compute units, more than 32768 16-bit or 16384 float32 elements; ragged ones: test_gpu_softmax_long_ragged.py):
 softmax_fwd_team_kernel / softmax_bwd_team_kernel, where a team of workgroups holds a row in
 registers and exchanges (maximum, sum) pairs -- the backward: sums -- through library-owned device
 memory with a bounded wait.  It serves the rows the reference gives one
@@ -18,10 +18,17 @@ from helpers import assert_close, gen, rowsum_slack, to_np32
 pytestmark = pytest.mark.gpu
 
 DTYPES = [torch.float32, torch.float16, torch.bfloat16]
-# (rows, packs a row): one team of 8; five teams whose last chunk is ragged; 40 teams of 9 with
+# (rows, packs a row): one team of 11; five teams whose last chunk is ragged; 40 teams of 12 with
 # one pack in the last chunk; 100 teams of 5 with four packs a lane; two rounds of 56 teams of 9
 # with 16 packs a lane
-SHAPES = [(1, 4096), (5, 5000), (40, 4097), (100, 9000), (100, 70000)]
+SHAPES = [(1, 5632), (5, 6000), (40, 5633), (100, 9000), (100, 70000)]
+
+
+def _team(cabi, backward, M, N, in_dtype, out_dtype=None):
+    """The plan of a call that a team holds, softmax and log_softmax alike."""
+    plans = [cabi.softmax_plan(backward, is_log, M, N, in_dtype, out_dtype) for is_log in (0, 1)]
+    assert plans[0] == plans[1] and plans[0]["team"] >= 2, plans
+    return plans[0]
 
 
 def _with_wait(cabi, us, fn):
@@ -47,10 +54,9 @@ def test_team_softmax_against_oracle_fallback_and_row_kernels(cabi, oracle, gpu,
     for i, (M, packs) in enumerate(SHAPES):
         N = packs * E
         print("case softmax team rows", dtype, (M, N), flush=True)
-        p = cabi.plan(cabi.OP_SOFTMAX_FWD, M, N, code, code)
-        assert p["row_chunks"] >= 2 and p["grid_blocks"] <= 512, p
-        assert p["grid_blocks"] % p["row_chunks"] == 0, p
-        teams = p["grid_blocks"] // p["row_chunks"]
+        p = _team(cabi, 0, M, N, code)
+        assert p["grid_blocks"] <= 512 and p["grid_blocks"] % p["team"] == 0, p
+        teams = p["grid_blocks"] // p["team"]
         assert teams == M or 8 <= teams < M, p
         g = gen(2100 + i)
         x = (3.0 * torch.randn(M, N, generator=g)).to(dtype)
@@ -95,8 +101,7 @@ def test_team_softmax_float16_rows_to_float32(cabi, oracle, gpu):
     M, N = 6, 50000 * 8
     x = (2.0 * torch.randn(M, N, generator=gen(2150))).half()
     xg = x.to(gpu)
-    p = cabi.plan(cabi.OP_SOFTMAX_FWD, M, N, cabi.F16, cabi.F16)
-    assert p["row_chunks"] >= 2, p
+    _team(cabi, 0, M, N, cabi.F16, cabi.F32)
     for is_log in (False, True):
         y = cabi.softmax_fwd(xg, is_log, out_dtype=torch.float32)
         assert y.dtype == torch.float32
@@ -106,11 +111,22 @@ def test_team_softmax_float16_rows_to_float32(cabi, oracle, gpu):
 
 
 def test_shapes_the_team_does_not_take(cabi, oracle, gpu):
-    """Ragged rows, rows off a 16-byte boundary, more rows than half the compute units and rows
-    under 4096 packs keep the one-workgroup-a-row kernels (the plan says which)."""
-    for (M, N) in ((4, 8 * 4096 + 3), (200, 8 * 4096), (4, 8 * 4000)):
+    """Rows off a 16-byte boundary, more rows than half the compute units, rows under 4096 packs and rows that one
+    workgroup is through with before a team has exchanged keep the one-workgroup-a-row kernels (the plan says which);
+    ragged rows have teams of their own."""
+    for (M, N) in ((200, 8 * 4096), (4, 8 * 4000), (128, 8 * 4096), (128, 8 * 5000 + 3)):
         p = cabi.plan(cabi.OP_SOFTMAX_FWD, M, N, cabi.BF16, cabi.BF16)
         assert p["row_chunks"] == 0 and p["grid_blocks"] <= M, p
+        assert cabi.softmax_plan(0, 0, M, N, cabi.BF16)["team"] == 0
+    assert cabi.plan(cabi.OP_SOFTMAX_FWD, 4, 8 * 4096 + 3, cabi.BF16, cabi.BF16)["row_chunks"] == 9
+    x = (2 * torch.randn(128, 8 * 4096, generator=gen(2161))).bfloat16().to(gpu)
+    y = cabi.softmax_fwd(x)
+    assert_close(y, oracle.softmax_fwd(to_np32(x), False), torch.bfloat16, "128 rows, one workgroup each")
+    grad = torch.randn(128, 8 * 4096, generator=gen(2162)).bfloat16().to(gpu)
+    assert cabi.softmax_plan(1, 0, 128, 8 * 4096, cabi.BF16)["team"] == 0
+    yy = y.cpu().float()
+    assert_close(cabi.softmax_bwd(grad, y), oracle.softmax_bwd(to_np32(grad), to_np32(y), False), torch.bfloat16,
+                 "128 rows, one workgroup each, backward", slack=rowsum_slack(grad.cpu().float() * yy, yy))
     M, N = 4, 8 * 4096
     x = torch.randn(M, N + 8, generator=gen(2160)).bfloat16().to(gpu)
     xo = x.reshape(-1)[1:1 + M * N].view(M, N)  # 2-byte aligned rows
@@ -125,9 +141,8 @@ def test_team_softmax_backward_against_oracle_fallback_and_row_kernels(cabi, ora
     for i, (M, packs) in enumerate(SHAPES):
         N = packs * E
         print("case softmax team rows backward", dtype, (M, N), flush=True)
-        p = cabi.plan(cabi.OP_SOFTMAX_BWD, M, N, code, code)
-        assert p["row_chunks"] >= 2 and p["grid_blocks"] <= 512, p
-        assert p["grid_blocks"] % p["row_chunks"] == 0, p
+        p = _team(cabi, 1, M, N, code)
+        assert p["grid_blocks"] <= 512 and p["grid_blocks"] % p["team"] == 0, p
         g = gen(2200 + i)
         x = (3.0 * torch.randn(M, N, generator=g)).to(dtype)
         x[0, :5] = float("-inf")
@@ -163,8 +178,7 @@ def test_team_softmax_backward_float32_to_float16(cabi, oracle, gpu):
     x = (2.0 * torch.randn(M, N, generator=g))
     grad = torch.randn(M, N, generator=g)
     y = torch.softmax(x, -1)
-    p = cabi.plan(cabi.OP_SOFTMAX_BWD, M, N, cabi.F32, cabi.F32)
-    assert p["row_chunks"] >= 2, p
+    _team(cabi, 1, M, N, cabi.F32, cabi.F16)
     gi = cabi.softmax_bwd(grad.to(gpu), y.to(gpu), False, gi_dtype=torch.float16)
     assert gi.dtype == torch.float16
     assert_close(gi, oracle.softmax_bwd(to_np32(grad), to_np32(y), False), torch.float16, "float to half")

@@ -113,11 +113,13 @@ def test_team_forward_against_oracle_fallback_and_split_kernels(cabi, oracle, gp
 
 
 def test_fewer_than_eight_teams_keep_the_multi_launch_kernels(cabi, oracle, gpu):
-    """Rows that would make fewer than 8 teams (their phases run in step and nothing hides the
-    wait) keep the split-row / two-pass kernels; the result is the same to the tolerance."""
-    for (M, N) in ((3, 16385 * 8), (2, 1310720)):
+    """More rows than fewer than 8 teams hold at once (their phases run in step and nothing hides the wait), one or
+    two rows of more than eight packs a lane on the teams of 64 that fewer than eight rows have
+    (test_gpu_norm_few_rows.py), and ragged rows keep the split-row / two-pass kernels; the result is the same to the
+    tolerance."""
+    for (M, N) in ((9, 4218880), (2, 2400000), (3, 16385 * 8 + 1)):
         p = cabi.plan(cabi.OP_LAYER_NORM_FWD, M, N, cabi.BF16, cabi.BF16)
-        assert p["resident"] == 0 and p["grid_blocks"] <= M, p
+        assert p["resident"] == 0 and p["grid_blocks"] <= M and p["row_chunks"] > 1, p
         x, gamma, beta = _mk(M, N, torch.bfloat16, torch.bfloat16, 1640)
         y, mean, rstd = cabi.layer_norm_fwd(x.to(gpu), gamma.to(gpu), beta.to(gpu), 1e-5)
         oy, om, orr = oracle.layer_norm_fwd(to_np32(x), (N,), to_np32(gamma), to_np32(beta), 1e-5)

@@ -7,13 +7,27 @@ lane's last pack, misaligned
 tensors and -inf / NaN entries, against the CPU oracle at the family's tolerances (float32
 rtol = atol = 1e-5; 16-bit atol 1e-2, rtol 1.6e-2) and against the multi-pass kernel forced on
 the same inputs.  The 16-bit forward holds rows of 17..20 packs a lane (the 151936 / 152064-entry
-vocabularies) in registers as well: checked against the oracle and the multi-pass kernel."""
+vocabularies) in registers as well: checked against the oracle and the multi-pass kernel.  Calls of so few rows go to
+teams of workgroups (test_gpu_softmax_team_rows.py), so the kernels named here are asked for with a grid bound, which
+keeps teams out, and the plan says that they run."""
+import contextlib
+
 import pytest
 import torch
 
 from helpers import assert_close, gen, offset_view, rowsum_slack, to_np32
 
 pytestmark = pytest.mark.gpu
+
+
+@contextlib.contextmanager
+def _without_teams(cabi, op):
+    """(a bound of two workgroups a compute unit, which binds nothing here)"""
+    try:
+        cabi.set_override(op, 0, 0, 0, 2)
+        yield
+    finally:
+        cabi.clear_overrides()
 
 
 def _case(cabi, oracle, gpu, M, N, dtype, off, seed, gi_dtype=None):
@@ -24,11 +38,16 @@ def _case(cabi, oracle, gpu, M, N, dtype, off, seed, gi_dtype=None):
     y = torch.log_softmax(x, -1).to(dtype)
     put = (lambda t: offset_view(t.to(gpu), off)) if off else (lambda t: t.to(gpu))
     yg, gg = put(y), put(grad)
-    p = cabi.plan(cabi.OP_SOFTMAX_BWD, M, N, cabi.dtype_code(dtype), cabi.dtype_code(dtype))
-    # 16-bit rows up to 65536 elements hold both tensors in registers (storage format); beyond
-    # that, and for float32 rows beyond 32768, grad alone stays resident
-    assert p["resident"] == (1 if dtype != torch.float32 and N <= 65536 else 0), p
-    gi = cabi.softmax_bwd(gg, yg, True, gi_dtype=gi_dtype)
+    E = 4 if dtype == torch.float32 else 8
+    with _without_teams(cabi, cabi.OP_SOFTMAX_BWD):
+        p = cabi.softmax_plan(1, 1, M, N, cabi.dtype_code(dtype), cabi.dtype_code(gi_dtype or dtype))
+        assert p["team"] == 0, p
+        assert (p["resident"], p["lanes_per_row"], p["packs_per_lane"]) == (1, 1024, -(-N // (1024 * E))), p
+        # 16-bit rows up to 65536 elements hold both tensors in registers (storage format); beyond
+        # that, and for float32 rows beyond 32768, grad alone stays resident
+        two = cabi.softmax_plan(1, 0, M, N, cabi.dtype_code(dtype))["resident"]
+        assert two == (1 if dtype != torch.float32 and N <= 65536 else 0)
+        gi = cabi.softmax_bwd(gg, yg, True, gi_dtype=gi_dtype)
     try:
         cabi.set_override(cabi.OP_SOFTMAX_BWD, -1, 1)     # the multi-pass kernel
         ref = cabi.softmax_bwd(gg, yg, True, gi_dtype=gi_dtype)
@@ -70,20 +89,23 @@ def test_float32_grad_to_float16_gradient(cabi, oracle, gpu):
 
 
 def test_nan_poisons_its_row_only(cabi, gpu):
-    M, N = 3, 50304
-    y = torch.log_softmax(torch.randn(M, N, generator=gen(990)), -1).bfloat16()
-    grad = torch.randn(M, N, generator=gen(991)).bfloat16()
-    grad[1, 777] = float("nan")
-    gi = cabi.softmax_bwd(grad.to(gpu), y.to(gpu), True)
-    assert bool(torch.isnan(gi[1]).all())
-    assert bool(torch.isfinite(gi[0]).all()) and bool(torch.isfinite(gi[2]).all())
+    for M, N in ((3, 50304), (3, 80000)):  # both tensors held; grad alone
+        y = torch.log_softmax(torch.randn(M, N, generator=gen(990)), -1).bfloat16()
+        grad = torch.randn(M, N, generator=gen(991)).bfloat16()
+        grad[1, 777] = float("nan")
+        with _without_teams(cabi, cabi.OP_SOFTMAX_BWD):
+            gi = cabi.softmax_bwd(grad.to(gpu), y.to(gpu), True)
+        assert bool(torch.isnan(gi[1]).all())
+        assert bool(torch.isfinite(gi[0]).all()) and bool(torch.isfinite(gi[2]).all())
 
 
 def test_softmax_and_ragged_rows_keep_the_multi_pass_kernel(cabi, oracle, gpu):
-    """The kernel serves log_softmax on whole packs only; softmax and ragged rows of that length
+    """grad alone is no help to softmax, and a ragged row beyond 20 packs a lane is held by nothing: both
     still go through the multi-pass kernel and agree with the oracle."""
-    M = 2
-    for N, is_log in ((50304, False), (50257, True)):
+    M = 129
+    for N, is_log in ((66000, False), (66003, False), (164003, True)):
+        p = cabi.softmax_plan(1, is_log, M, N, cabi.BF16)
+        assert p["team"] == 0 and p["resident"] == 0, p
         g = gen(995)
         x = torch.randn(M, N, generator=g)
         grad = torch.randn(M, N, generator=g).bfloat16()
@@ -101,13 +123,15 @@ def test_forward_rows_of_17_to_20_packs_a_lane(cabi, oracle, gpu, dtype, is_log)
                                 (20, 163840))):
         M = 3
         print("case vocabulary forward", dtype, is_log, (M, N), flush=True)
-        p = cabi.plan(cabi.OP_SOFTMAX_FWD, M, N, code, code)
-        assert (p["resident"], p["lanes_per_row"], p["packs_per_lane"]) == (1, 1024, V), p
         x = (3.0 * torch.randn(M, N, generator=gen(1500 + i))).to(dtype)
         x[0, N // 2:] = float("-inf")
         x[1, -1] = 30.0  # the maximum in the last pack of the row
         xg = x.to(gpu)
-        y = cabi.softmax_fwd(xg, is_log)
+        with _without_teams(cabi, cabi.OP_SOFTMAX_FWD):
+            p = cabi.softmax_plan(0, is_log, M, N, code)
+            assert (p["team"], p["resident"], p["lanes_per_row"], p["packs_per_lane"]) == (0, 1, 1024, V), p
+            y = cabi.softmax_fwd(xg, is_log)
+            assert torch.equal(cabi.softmax_fwd(xg, is_log).view(torch.uint8), y.view(torch.uint8))
         oy = oracle.softmax_fwd(to_np32(x), is_log)
         assert_close(y, oy, dtype, "forward [%d, %d] %s" % (M, N, dtype))
         try:
@@ -116,15 +140,17 @@ def test_forward_rows_of_17_to_20_packs_a_lane(cabi, oracle, gpu, dtype, is_log)
         finally:
             cabi.clear_overrides()
         assert_close(y, to_np32(ref), dtype, "register-resident vs multi-pass forward %d" % N)
-        assert torch.equal(cabi.softmax_fwd(xg, is_log).view(torch.uint8), y.view(torch.uint8))
     # float32 output from float16 input (half_to_float, SoftMax.cpp:49-55) on the same kernels
     if dtype == torch.float16:
         x = (3.0 * torch.randn(2, 151936, generator=gen(1510))).to(dtype)
-        y32 = cabi.softmax_fwd(x.to(gpu), is_log, out_dtype=torch.float32)
+        with _without_teams(cabi, cabi.OP_SOFTMAX_FWD):
+            assert cabi.softmax_plan(0, is_log, 2, 151936, cabi.F16, cabi.F32)["packs_per_lane"] == 19
+            y32 = cabi.softmax_fwd(x.to(gpu), is_log, out_dtype=torch.float32)
         assert_close(y32, oracle.softmax_fwd(to_np32(x), is_log), torch.float32,
                      "half_to_float 151936")
     # one row more than the registers hold: the multi-pass kernel
-    assert cabi.plan(cabi.OP_SOFTMAX_FWD, 3, 163848, code, code)["resident"] == 0
+    with _without_teams(cabi, cabi.OP_SOFTMAX_FWD):
+        assert cabi.softmax_plan(0, is_log, 3, 163848, code)["resident"] == 0
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
@@ -136,15 +162,17 @@ def test_backward_rows_of_5_to_8_packs_a_lane_in_storage_format(cabi, oracle, gp
                                 (8, 65528), (8, 65536))):
         M = 3
         print("case packed softmax backward", dtype, is_log, (M, N), flush=True)
-        p = cabi.plan(cabi.OP_SOFTMAX_BWD, M, N, code, code)
-        assert (p["resident"], p["lanes_per_row"], p["packs_per_lane"]) == (1, 1024, V), p
         g = gen(1600 + i)
         x = 2.0 * torch.randn(M, N, generator=g)
         x[0, N // 3] = float("-inf")
         y = (torch.log_softmax(x, -1) if is_log else torch.softmax(x, -1)).to(dtype)
         grad = torch.randn(M, N, generator=g).to(dtype)
         yg, gg = y.to(gpu), grad.to(gpu)
-        gi = cabi.softmax_bwd(gg, yg, is_log)
+        with _without_teams(cabi, cabi.OP_SOFTMAX_BWD):
+            p = cabi.softmax_plan(1, is_log, M, N, code)
+            assert (p["team"], p["resident"], p["lanes_per_row"], p["packs_per_lane"]) == (0, 1, 1024, V), p
+            gi = cabi.softmax_bwd(gg, yg, is_log)
+            assert torch.equal(cabi.softmax_bwd(gg, yg, is_log).view(torch.uint8), gi.view(torch.uint8))
         ogi = oracle.softmax_bwd(to_np32(grad), to_np32(y), is_log)
         what = "[%d, %d] %s" % (M, N, dtype)
         assert_close(gi, ogi, dtype, "backward " + what)
@@ -154,7 +182,6 @@ def test_backward_rows_of_5_to_8_packs_a_lane_in_storage_format(cabi, oracle, gp
         finally:
             cabi.clear_overrides()
         assert_close(gi, to_np32(ref), dtype, "register-resident vs multi-pass backward " + what)
-        assert torch.equal(cabi.softmax_bwd(gg, yg, is_log).view(torch.uint8), gi.view(torch.uint8))
 
 
 def test_masked_backward_beyond_4_packs_a_lane_keeps_the_multi_pass_kernel(cabi, oracle, gpu):

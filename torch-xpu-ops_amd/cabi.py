@@ -29,6 +29,7 @@ EXPORTED_SYMBOLS = (
     "mi355x_softmax_strided_plan", "mi355x_softmax_strided_team_plan", "mi355x_group_norm_fwd",
     "mi355x_group_norm_bwd_workspace_bytes", "mi355x_group_norm_bwd", "mi355x_group_norm_plan",
     "mi355x_rownorm_plan", "mi355x_rownorm_plan_at", "mi355x_rownorm_waves_plan", "mi355x_rownorm_set_override",
+    "mi355x_softmax_plan", "mi355x_rownorm_few_rows_plan",
     "mi355x_rownorm_stream_probe", "mi355x_rownorm_set_team_wait_us",
 )
 
@@ -110,6 +111,10 @@ def lib():
                                              ctypes.POINTER(Plan)]
         L.mi355x_rownorm_waves_plan.argtypes = [_int, _i64, _i64, _int, _int, ctypes.POINTER(Plan)]
         L.mi355x_rownorm_waves_plan.restype = _int
+        L.mi355x_rownorm_few_rows_plan.argtypes = [_int, _i64, _i64, _int, _int, ctypes.POINTER(Plan)]
+        L.mi355x_rownorm_few_rows_plan.restype = _int
+        L.mi355x_softmax_plan.argtypes = [_int, _int, _i64, _i64, _int, _int, ctypes.POINTER(Plan)]
+        L.mi355x_softmax_plan.restype = _int
         L.mi355x_rownorm_set_override.argtypes = [_int, _int, _int, _int, _int]
         L.mi355x_rownorm_stream_probe.argtypes = [_vp, _vp, _vp, ctypes.c_size_t, _int, _vp]
         L.mi355x_rownorm_stream_probe.restype = _int
@@ -162,6 +167,26 @@ def waves_plan(op, M, N, x_dtype=F32, w_dtype=F32):
     """The layout of a norm call on whole wavefronts; "waves" 0: not this call, the rest is plan()'s."""
     p = Plan()
     _check(lib().mi355x_rownorm_waves_plan(op, M, N, x_dtype, w_dtype, ctypes.byref(p)), "waves_plan")
+    d = p.as_dict()
+    d["waves"] = p.reserved
+    return d
+
+
+def softmax_plan(backward, is_log, M, N, in_dtype=F32, out_dtype=None):
+    """The layout an unmasked softmax / log_softmax call runs on; "team" workgroups a row (0: no team)."""
+    p = Plan()
+    _check(lib().mi355x_softmax_plan(int(backward), int(is_log), M, N, in_dtype,
+                                     in_dtype if out_dtype is None else out_dtype, ctypes.byref(p)), "softmax_plan")
+    d = p.as_dict()
+    d["team"] = p.reserved
+    return d
+
+
+def few_rows_plan(op, M, N, x_dtype=F32, w_dtype=F32):
+    """The backward of few long norm rows without partial rows; "waves" that share a piece of columns, 0: not this
+    call, the rest is plan()'s."""
+    p = Plan()
+    _check(lib().mi355x_rownorm_few_rows_plan(op, M, N, x_dtype, w_dtype, ctypes.byref(p)), "few_rows_plan")
     d = p.as_dict()
     d["waves"] = p.reserved
     return d

@@ -574,6 +574,35 @@ int softmax_bwd(const void* grad, const void* y, const void* mask, void* gi, int
                            : launch_softmax_bwd<float, float>(plan, a, s);
 }
 
+// What an unmasked softmax call of this plan runs on.
+void softmax_layout(const Plan& plan, bool backward, bool is_log, bool widened, int esize, int64_t M, int64_t N,
+                    rownorm_plan* out) {
+  const bool team = softmax_team_serves(plan, backward, is_log, widened, esize, M, N, current_num_cus());
+  const bool grad = backward && is_log && !plan.resident;
+  const int64_t packs = N / (16 / esize);
+  out->resident = plan.resident ? 1 : 0;
+  out->lanes_per_row = plan.G;
+  out->packs_per_lane = plan.V;
+  out->block_threads = plan.block;
+  out->rows_per_block = plan.rpb;
+  out->reserved = team ? plan.team : 0;
+  out->grid_blocks = team ? plan.team_grid : plan.grid;
+  out->partial_rows = 0;
+  if (team) {
+    out->lanes_per_row = out->block_threads = kTeamBlock;
+    out->packs_per_lane = plan.team_v;
+    out->rows_per_block = 1;
+  } else if (!plan.resident && softmax_tail_serves(plan, backward, is_log, widened, esize, M, N)) {
+    out->resident = 1;
+    out->lanes_per_row = out->block_threads = plan.tail_g;
+    out->packs_per_lane = plan.tail_v;
+  } else if (grad && plan.grad_resident) {
+    out->resident = 1;
+    out->lanes_per_row = out->block_threads = kStreamBlock;
+    out->packs_per_lane = (int)((packs + kStreamBlock - 1) / kStreamBlock);
+  }
+}
+
 // Shape of a GroupNorm call as the kernels see it; returns 0 or an error code.
 struct GroupDims {
   int64_t rows = 0;  // N * groups
@@ -1020,7 +1049,7 @@ int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_si
     return e;
   const bool large = plan.large_team > 0;
   const int tx_log2 = large ? plan.large_tx_log2 : plan.team_tx_log2;
-  out->reserved = plan.fast ? plan.team_size() : 0;  // (rows of whole packs: see the header)
+  out->reserved = plan.team_size();
   if (out->reserved == 0) return 0;
   out->resident = 1;
   out->lanes_per_row = 1 << tx_log2;
@@ -1028,6 +1057,22 @@ int mi355x_softmax_strided_team_plan(int backward, int64_t outer, int64_t dim_si
   out->block_threads = kTeamBlock;
   out->rows_per_block = kTeamBlock >> tx_log2;
   out->grid_blocks = large ? plan.large_grid : plan.team_grid;
+  return 0;
+}
+
+int mi355x_softmax_plan(int backward, int is_log, int64_t rows, int64_t N, rownorm_dtype in_dtype,
+                        rownorm_dtype out_dtype, rownorm_plan* out) {
+  const int id = (int)in_dtype, od = (int)out_dtype;
+  if (!out) return ROWNORM_ERR_NULL;
+  if (esize_of(id) == 0 || esize_of(od) == 0) return ROWNORM_ERR_DTYPE;
+  const bool other = backward ? id == ROWNORM_F32 && od == ROWNORM_F16 : id == ROWNORM_F16 && od == ROWNORM_F32;
+  if (od != id && !other) return ROWNORM_ERR_DTYPE;
+  if (int e = shape_check(rows, N)) return e;
+  Plan plan;
+  if (int e = make_plan(backward ? OC_SOFTMAX_BWD : OC_SOFTMAX_FWD, rows, N, esize_of(id), current_num_cus(),
+                        g_override[backward ? ROWNORM_OP_SOFTMAX_BWD : ROWNORM_OP_SOFTMAX_FWD], false, &plan))
+    return e;
+  softmax_layout(plan, backward != 0, is_log != 0, esize_of(od) > esize_of(id), esize_of(id), rows, N, out);
   return 0;
 }
 
@@ -1046,16 +1091,18 @@ int mi355x_rownorm_plan_at(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_
                         oc == OC_NORM_BWD, &plan, false, layer_norm,
                         esize_of((int)w_dtype) > esize_of((int)x_dtype), off))
     return e;
+  if (oc == OC_SOFTMAX_FWD || oc == OC_SOFTMAX_BWD) {
+    softmax_layout(plan, oc == OC_SOFTMAX_BWD, false, false, esize_of((int)x_dtype), M, N, out);
+    return 0;
+  }
   out->resident = plan.resident ? 1 : 0;
   out->lanes_per_row = plan.G;
   out->packs_per_lane = plan.V;
   out->block_threads = plan.block;
   out->rows_per_block = plan.rpb;
-  // (a row held by a team of workgroups: the team and its grid; softmax: of whole packs)
-  const bool softmax = op == ROWNORM_OP_SOFTMAX_FWD || op == ROWNORM_OP_SOFTMAX_BWD;
-  const bool team = plan.team > 0 && !plan.team_small && !(softmax && !plan.fast);
-  out->reserved = team ? plan.team : (plan.split > 1 ? plan.split : 0);
-  out->grid_blocks = team ? plan.team_grid : plan.grid;
+  // (a row held by a team of workgroups: the team and its grid)
+  out->reserved = plan.team > 0 ? plan.team : (plan.split > 1 ? plan.split : 0);
+  out->grid_blocks = plan.team > 0 ? plan.team_grid : plan.grid;
   out->partial_rows = (int64_t)bwd_partial_rows(plan);
   // (groups of rows held by teams: the workgroup, the packs of a row a lane holds, the rows)
   if (plan.team > 0 && (op == ROWNORM_OP_LAYER_NORM_BWD || op == ROWNORM_OP_RMS_NORM_BWD)) {
@@ -1099,6 +1146,28 @@ int mi355x_rownorm_waves_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dtype
   out->rows_per_block = l.slots;
   out->grid_blocks = l.grid;
   out->partial_rows = oc == OC_NORM_BWD ? l.grid : 0;
+  return 0;
+}
+
+int mi355x_rownorm_few_rows_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_dtype,
+                                 rownorm_dtype w_dtype, rownorm_plan* out) {
+  if (int e = mi355x_rownorm_plan(op, M, N, x_dtype, w_dtype, out)) return e;
+  out->reserved = 0;
+  if (class_of((int)op) != OC_NORM_BWD) return 0;
+  const int esize = esize_of((int)x_dtype), E = 16 / esize;
+  Plan plan;
+  if (int e = make_plan(OC_NORM_BWD, M, N, esize, current_num_cus(), g_override[(int)op], true, &plan, false,
+                        op == ROWNORM_OP_LAYER_NORM_BWD, esize_of((int)w_dtype) > esize))
+    return e;
+  if (plan.few_waves == 0) return 0;
+  const int64_t pieces = (N + 64 * E - 1) / (64 * E), a_block = kFewRowsWaves / plan.few_waves;
+  out->reserved = plan.few_waves;
+  out->lanes_per_row = 64;
+  out->packs_per_lane = 1;
+  out->block_threads = kFewRowsWaves * 64;
+  out->rows_per_block = (int32_t)M;
+  out->grid_blocks = (pieces + a_block - 1) / a_block;
+  out->partial_rows = 0;
   return 0;
 }
 

@@ -80,7 +80,6 @@ struct Plan {
   // (softmax: the team that could hold a row, whether it does is softmax_team_serves()'s)
   int team = 0, team_v = 0;
   int64_t team_chunk_packs = 0, team_grid = 0;
-  bool team_small = false;  // fewer than kTeamMinTeams rows, all at once (the plan query reports the launches without)
   // norm backward of such rows held R = team_v rows at a time by teams of workgroups
   // (norm_bwd_team_kernel): the same fields, one stride of packs a workgroup, and the
   // partial rows of column sums that launch leaves (one a team; partial_rows is what
@@ -1316,7 +1315,6 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
       p.team_v = (int)v;
       p.team_chunk_packs = v * kTeamBlock;
       p.team_grid = teams * team;
-      p.team_small = small_teams;
     }
   }
   // Forward rows too long for at least eight such teams (beyond 256 / 8 * 16 * 512 packs),
