@@ -12,10 +12,10 @@ from helpers import assert_close, colsum_slack, gen, offset_view, to_np32
 pytestmark = pytest.mark.gpu
 
 DTYPES = [torch.float32, torch.float16, torch.bfloat16]
-# rows, elements beyond whole packs, whole packs: fewer rows than a wavefront takes at once; wavefronts that share a
-# piece of columns (8, 4, 2, 1 of them), with rows missing; the most rows; the last piece one pack or one element
-SHAPES = [(2, 0, 8200), (3, 1, 6000), (7, 0, 40001), (9, 0, 12800), (33, 3, 8193), (64, 0, 5121), (128, 1, 4160),
-          (5, 0, 131071)]
+# (rows, elements beyond whole packs, whole packs): the wavefronts that share a piece of columns.  Fewer rows than a
+# wavefront takes at once, rows missing in its last turn, the most rows; the last piece one pack or one element
+SHAPES = {(2, 0, 8200): 8, (3, 1, 6000): 8, (9, 0, 12800): 8, (33, 3, 8193): 8, (64, 0, 5121): 8, (128, 1, 4160): 8,
+          (11, 0, 20001): 4, (10, 1, 20000): 4, (7, 0, 40001): 2, (3, 3, 40000): 2, (3, 0, 70001): 1, (5, 1, 100000): 1}
 
 
 def _inputs(M, N, dtype, seed):
@@ -26,13 +26,14 @@ def _inputs(M, N, dtype, seed):
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
-@pytest.mark.parametrize("shape", SHAPES, ids=str)
+@pytest.mark.parametrize("shape", list(SHAPES), ids=str)
 def test_backward_against_oracle(cabi, oracle, gpu, dtype, shape):
     M, over, packs = shape
     N = packs * (4 if dtype == torch.float32 else 8) + over
     print("case few rows", dtype, (M, N), flush=True)
     code = cabi.dtype_code(dtype)
-    assert cabi.plan(cabi.OP_LAYER_NORM_BWD, M, N, code, code)["resident"] == 0
+    for op in (cabi.OP_LAYER_NORM_BWD, cabi.OP_RMS_NORM_BWD):
+        assert cabi.few_rows_plan(op, M, N, code, code)["waves"] == SHAPES[shape]
     x, dy, gamma, beta = _inputs(M, N, dtype, 4100 + M)
     xg, dyg, gg = x.to(gpu), dy.to(gpu), gamma.to(gpu)
     _, mean, rstd = cabi.layer_norm_fwd(xg, gg, None, 1e-5)
@@ -76,6 +77,8 @@ def test_forward_by_small_teams(cabi, oracle, gpu, dtype, M, packs):
     """Fewer than eight rows: teams of at most 64 workgroups, and what a workgroup does without its team."""
     N = packs * (4 if dtype == torch.float32 else 8)
     print("case few rows forward", dtype, (M, N), flush=True)
+    p = cabi.plan(cabi.OP_LAYER_NORM_FWD, M, N, cabi.dtype_code(dtype), cabi.dtype_code(dtype))
+    assert p["resident"] == 0 and 2 <= p["row_chunks"] <= 64 and p["grid_blocks"] == M * p["row_chunks"], p
     x, _, gamma, beta = _inputs(M, N, dtype, 4200 + M)
     xg, gg, bg = x.to(gpu), gamma.to(gpu), beta.to(gpu)
     oy, om, orr = oracle.layer_norm_fwd(to_np32(x), (N,), to_np32(gamma), to_np32(beta), 1e-5)

@@ -1,10 +1,11 @@
-"""softmax / log_softmax of long rows that are no whole number of packs: one workgroup of 1024 lanes holds the row in 3
-to 20 whole packs a lane (TAIL of softmax_fwd_resident_kernel, softmax_bwd_resident_kernel and
+"""softmax / log_softmax of long rows that are no whole number of packs: one workgroup of 1024 or 512 lanes holds the
+row in 3 to 20 whole packs a lane (TAIL of softmax_fwd_resident_kernel, softmax_bwd_resident_kernel and
 log_softmax_bwd_grad_resident_kernel), few rows are held by teams of workgroups whose last chunk starts early
 (softmax_fwd_team_kernel, softmax_bwd_team_kernel).  The regime of the reference's vocabulary-sized rows
 (src/ATen/native/xpu/sycl/SoftMaxKernels.cpp:546-684, 991-1150).  Against float64: the last pack one element to one
 short of whole, the last one of a lane round or the only one in it, off a 16-byte boundary, in place, rows without a
-finite element and with infinities and NaN where neighbouring packs meet, and every wait given up."""
+finite element and with infinities and NaN where neighbouring packs meet, and every wait given up.  The plan says of
+every case which lanes, packs or team it runs on."""
 import math
 
 import pytest
@@ -35,7 +36,8 @@ def _forward(cabi, x, is_log, what, y=None):
     y = cabi.softmax_fwd(x, is_log, y=y)
     # exp's and log's own error against float64: 4 units of float32 over arguments up to 2^7
     own = 2.0 ** -15 if not is_log else 2.0 ** -20
-    _near(y, ref, UNIT[y.dtype] * ref.abs() + (own + _sum(x.shape[-1])) * (torch.ones_like(ref) if is_log else ref) + TINY[y.dtype], what)
+    slack = (own + _sum(x.shape[-1])) * (torch.ones_like(ref) if is_log else ref)
+    _near(y, ref, UNIT[y.dtype] * ref.abs() + slack + TINY[y.dtype], what)
     return y
 
 
@@ -74,22 +76,96 @@ def _all(cabi, gpu, M, N, dtype, seed):
         _backward(cabi, grad, over_y, is_log, "gi over y " + what, gi=over_y)
 
 
-# packs beyond whole lane rounds of 1024, and the elements of the last pack
+def _row(lanes, v, last, E):
+    """The longest ragged row whose window has one pack in the last lane round, or (last) all of them."""
+    window = lanes * v if last else lanes * (v - 1) + 1
+    return next(n for n in range(window * E - E + 1, 0, -1) if n % E and (n + 2 * (E - 1)) // E == window)
+
+
+def _held(cabi, backward, is_log, M, N, dtype, lanes, v):
+    p = cabi.softmax_plan(backward, is_log, M, N, cabi.dtype_code(dtype))
+    assert (p["team"], p["resident"], p["lanes_per_row"], p["packs_per_lane"]) == (0, 1, lanes, v), (M, N, p)
+
+
+# (lanes, packs a lane, a number of rows for which the forward runs on these)
+HELD16 = [(512, v, 129) for v in range(5, 15)] + [(1024, 3, 2100), (1024, 4, 2100)] + [(1024, v, 520) for v in (5, 6, 7)] + \
+    [(1024, v, 129) for v in (8, 9, 10, 11, 12, 13, 14, 15, 16, 18, 20)]
+HELD32 = [(512, v, 129) for v in range(9, 15)] + [(1024, v, 520) for v in (5, 6, 7)] + [(1024, v, 129) for v in range(8, 17)]
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=str)
-def test_every_pack_count(cabi, gpu, dtype):
+def test_every_pack_count_forward(cabi, gpu, dtype):
     E = 4 if dtype == torch.float32 else 8
-    for v in range(3 if E == 8 else 5, 22):
-        packs = (1024 * v, 1024 * (v - 1) + 1, 1024 * (v - 1) + 517)[v % 3]
-        _all(cabi, gpu, 130 if v in (4, 9) else 129, (packs - 1) * E + 1 + v % (E - 1), dtype, 7000 + v)
+    for lanes, v, M in HELD32 if E == 4 else HELD16:
+        for last in (False, True):
+            if (lanes, v, last) == (1024, 3, False):
+                continue  # (rows of up to 2560 packs run on 512 lanes)
+            N = _row(lanes, v, last, E)
+            x, _ = _rows(M, N, dtype, 7000 + v)
+            x = x.to(gpu)
+            for is_log in (False, True):
+                what = "[%d, %d] %s log %d, %d packs on %d lanes" % (M, N, dtype, is_log, v, lanes)
+                print("case", what, flush=True)
+                _held(cabi, 0, is_log, M, N, dtype, lanes, v)
+                y = _forward(cabi, x, is_log, what)
+                assert torch.equal(y, cabi.softmax_fwd(x, is_log)), "run to run " + what
+                _forward(cabi, offset_view(x, 3), is_log, "off a boundary " + what)
+                over = x.clone()
+                _forward(cabi, over, is_log, "in place " + what, y=over)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=str)
+def test_every_pack_count_backward(cabi, gpu, dtype):
+    E, M = 4 if dtype == torch.float32 else 8, 129
+    for v in range(5 if E == 4 else 3, 21):
+        for last in (False, True):
+            N = _row(1024, v, last, E)
+            x, grad = (t.to(gpu) for t in _rows(M, N, dtype, 7050 + v))
+            for is_log in (False, True):
+                if v > 8 and not is_log:
+                    continue
+                what = "[%d, %d] %s log %d backward, %d packs" % (M, N, dtype, is_log, v)
+                print("case", what, flush=True)
+                _held(cabi, 1, is_log, M, N, dtype, 1024, v)
+                y = cabi.softmax_fwd(x, is_log)
+                gi = _backward(cabi, grad, y, is_log, what)
+                assert torch.equal(gi, cabi.softmax_bwd(grad, y, is_log)), "run to run " + what
+                _backward(cabi, offset_view(grad, 3), offset_view(y, 3), is_log, "off a boundary " + what)
+                _backward(cabi, offset_view(grad, 1), offset_view(y, 2), is_log, "windows apart " + what)
+                over_g, over_y = grad.clone(), y.clone()
+                _backward(cabi, over_g, y, is_log, "gi over grad " + what, gi=over_g)
+                _backward(cabi, grad, over_y, is_log, "gi over y " + what, gi=over_y)
+
+
+def test_float32_output_of_every_pack_count(cabi, gpu):
+    """float16 -> float32: the held forward stores 32 bytes a lane and pack."""
+    for lanes, v, M in HELD16:
+        M = max(M, 200)  # (fewer rows: two passes, see the plan)
+        N = _row(lanes, v, v == 3 or v % 2 == 0, 8)
+        x, _ = _rows(M, N, torch.float16, 7300 + v)
+        x = x.to(gpu)
+        for is_log in (False, True):
+            p = cabi.softmax_plan(0, is_log, M, N, cabi.F16, cabi.F32)
+            if not is_log and p["resident"] == 0:
+                continue
+            assert (p["team"], p["lanes_per_row"], p["packs_per_lane"]) == (0, lanes, v), p
+            y = cabi.softmax_fwd(x, is_log, out_dtype=torch.float32)
+            ref = torch.log_softmax(x.double(), -1) if is_log else torch.softmax(x.double(), -1)
+            tol = 2.0 ** -20 * (ref.abs() + 1) + _sum(N) if is_log else (2.0 ** -18 + _sum(N)) * ref
+            _near(y, ref, tol, "half to float %s log %d" % ((M, N), is_log))
 
 
 @pytest.mark.parametrize("M", [1, 3, 64, 128])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=str)
 def test_teams(cabi, gpu, dtype, M):
     E = 4 if dtype == torch.float32 else 8
-    # (packs: the fewest; the last chunk one pack; the last chunk whole; two rounds of a full machine)
-    for packs in (4096, 4097, 9 * 512 + 1, 16 * 512 * (1 if M > 8 else 64) + 300):
+    # (packs: some of the fewest; the last chunk one pack; the last chunk whole; more than one workgroup holds, in the
+    # backward two rounds of a full machine at 128 rows)
+    for packs in {1: (4224, 4609, 5120), 3: (4224, 4609, 5120), 64: (7168, 12801, 14336),
+                  128: (21505, 24577, 24576)}[M] + (16 * 512 * (8 if M > 8 else 64) + 300,):
         N = (packs - 1) * E + 1 + packs % (E - 1)
+        on = [(b, l) for b in (0, 1) for l in (0, 1) if cabi.softmax_plan(b, l, M, N, cabi.dtype_code(dtype))["team"] > 1]
+        assert (0, 0) in on and (packs < 8192 or len(on) == 4), (M, N, on)
         _all(cabi, gpu, M, N, dtype, 7100 + packs)
         x, grad = (t.to(gpu) for t in _rows(M, N, dtype, 7200 + packs))
         try:

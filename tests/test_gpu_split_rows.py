@@ -8,7 +8,7 @@ import ctypes
 import pytest
 import torch
 
-from helpers import assert_close, gen, offset_view, to_np32
+from helpers import assert_close, colsum_slack, gen, offset_view, to_np32
 
 pytestmark = pytest.mark.gpu
 
@@ -110,12 +110,14 @@ def test_constant_rows_give_beta_bit_for_bit(cabi, gpu):
 
 
 def test_fallbacks_keep_a_row_on_one_workgroup(cabi, oracle, gpu):
-    """Without mean / rstd outputs, with Y on top of X, or with a workspace that only holds the
-    column sums, the call still succeeds: the row is not split."""
+    """Without mean / rstd outputs or with Y on top of X the call still succeeds: the row is not split.  With a
+    workspace that only holds the column sums, few rows keep their row sums there (two launches without partial
+    rows), and each of more rows stays on one workgroup."""
     L = cabi.lib()
     P = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else None
     stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     M, N = 2, 150000
+    assert cabi.few_rows_plan(cabi.OP_LAYER_NORM_BWD, M, N, cabi.F32, cabi.F32)["waves"] > 0
     x, dy, gamma, beta = _mk(M, N, torch.float32, 84)
     xg, dyg, gg, bg = (t.to(gpu) for t in (x, dy, gamma, beta))
     oy, om, orr = oracle.layer_norm_fwd(to_np32(x), (N,), to_np32(gamma), to_np32(beta), 1e-5)
@@ -156,6 +158,26 @@ def test_fallbacks_keep_a_row_on_one_workgroup(cabi, oracle, gpu):
     assert L.mi355x_layer_norm_bwd(P(dyg), P(xg), P(mean_g), P(rstd_g), P(gg), P(dx2), None, None,
                                    None, 0, M, N, F32, F32, stream) == 0
     assert_close(dx2, odx, torch.float32, "dx, no workspace")
+    # the short workspace again, rows beyond those two launches: with the full one they are split
+    M, N = 129, 66001
+    p = cabi.few_rows_plan(cabi.OP_LAYER_NORM_BWD, M, N, F32, F32)
+    q = cabi.plan(cabi.OP_LAYER_NORM_BWD, M, N, F32, F32)
+    assert p["waves"] == 0 and q["resident"] == 0 and q["row_chunks"] > 1 and q["partial_rows"] > 1, (p, q)
+    x, dy, gamma, beta = _mk(M, N, torch.float32, 85)
+    xg, dyg, gg = (t.to(gpu) for t in (x, dy, gamma))
+    _, mean, rstd = cabi.layer_norm_fwd(xg, gg, None, 1e-5)
+    odx, odg, odb = oracle.layer_norm_bwd(to_np32(dy), to_np32(x), (N,), to_np32(mean), to_np32(rstd), to_np32(gamma))
+    full = L.mi355x_layer_norm_bwd_workspace_bytes(M, N, F32, F32, 1, 1)
+    cols = 2 * q["partial_rows"] * N * 4
+    assert 0 < cols < full
+    ws = torch.empty(cols, dtype=torch.uint8, device=gpu)
+    dx, dg, db = torch.empty_like(xg), torch.empty_like(gg), torch.empty_like(gg)
+    assert L.mi355x_layer_norm_bwd(P(dyg), P(xg), P(mean), P(rstd), P(gg), P(dx), P(dg), P(db), P(ws), cols, M, N, F32,
+                                   F32, stream) == 0
+    xhat = (x.double() - mean.cpu().double()[:, None]) * rstd.cpu().double()[:, None]
+    assert_close(dx, odx, torch.float32, "dx, short workspace, 129 rows")
+    assert_close(dg, odg, torch.float32, "dgamma, short workspace, 129 rows", slack=colsum_slack(dy.double() * xhat))
+    assert_close(db, odb, torch.float32, "dbeta, short workspace, 129 rows", slack=colsum_slack(dy))
 
 
 @pytest.mark.parametrize("wdtype", [torch.bfloat16, torch.float32], ids=str)
