@@ -433,7 +433,8 @@ int mi355x_softmax_plan(int backward, int is_log, int64_t rows, int64_t N, rowno
 /* The layout of a LayerNorm / RMSNorm backward of few rows beyond one workgroup's registers, dX and column sums
  * wanted, in two launches without partial rows: `reserved` wavefronts share 64 packs of columns (lanes_per_row lanes, a
  * pack each) and walk all rows_per_block = M rows under them, grid_blocks workgroups of block_threads threads.
- * `reserved` == 0: not this call, the rest is what mi355x_rownorm_plan reports. */
+ * `reserved` == 0: not this call, the rest is what mi355x_rownorm_plan reports (LayerNorm rows of up to 32 MB there held
+ * by teams run in the two launches where the call cannot have teams). */
 int mi355x_rownorm_few_rows_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dtype x_dtype,
                                  rownorm_dtype w_dtype, rownorm_plan* out);
 

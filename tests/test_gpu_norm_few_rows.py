@@ -71,6 +71,42 @@ def test_backward_against_oracle(cabi, oracle, gpu, dtype, shape):
     assert_close(rdg, ordg, dtype, "rms dgamma %s" % ((M, N),), slack=None if slack[1] is None else colsum_slack(terms))
 
 
+@pytest.mark.parametrize("M,N,dtype", [(48, 112000, torch.float32), (48, 320000, torch.bfloat16)], ids=str)
+def test_rows_of_teams_where_no_team_can_run(cabi, oracle, gpu, M, N, dtype):
+    """Rows beyond the line of the teams, dX over an input or captured: the two launches again, whose bits the call
+    with a residual gradient of zeros shows (it never has teams; -0 equals 0)."""
+    print("case few rows, no team", dtype, (M, N), flush=True)
+    code = cabi.dtype_code(dtype)
+    assert cabi.few_rows_plan(cabi.OP_LAYER_NORM_BWD, M, N, code, code)["waves"] == 0
+    assert cabi.plan(cabi.OP_LAYER_NORM_BWD, M, N, code, code)["row_chunks"] > 1
+    x, dy, gamma, _ = _inputs(M, N, dtype, 4300 + M)
+    xg, dyg, gg = x.to(gpu), dy.to(gpu), gamma.to(gpu)
+    _, mean, rstd = cabi.layer_norm_fwd(xg, gg, None, 1e-5)
+    two = cabi.add_layer_norm_bwd(dyg, torch.zeros_like(xg), xg, mean, rstd, gg)
+    o = oracle.layer_norm_bwd(to_np32(dy), to_np32(x), (N,), to_np32(mean), to_np32(rstd), to_np32(gamma))
+    xhat = (x.double() - mean.cpu().double().reshape(M, 1)) * rstd.cpu().double().reshape(M, 1)
+    slack = (None, colsum_slack(dy.double() * xhat), colsum_slack(dy)) if dtype == torch.float32 else (None,) * 3
+    for name, a, b, s in zip(("dx", "dgamma", "dbeta"), two, o, slack):
+        assert_close(a, b, dtype, name, slack=s)
+    for which in (0, 1):
+        pair = [dyg.clone(), xg.clone()]
+        got = cabi.layer_norm_bwd(*pair, mean, rstd, gg, dx=pair[which])
+        assert all(torch.equal(a, b) for a, b in zip(got, two)), "dx over %s" % ("dy", "x")[which]
+    torch.cuda.synchronize()
+    out = torch.empty_like(xg), torch.empty_like(gg), torch.empty_like(gg)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        cabi.layer_norm_bwd(dyg, xg, mean, rstd, gg, dx=out[0], dgamma=out[1], dbeta=out[2])
+    for k in range(3):
+        for t in out:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, two)), "replay %d" % k
+        for name, a, b, s in zip(("dx", "dgamma", "dbeta"), cabi.layer_norm_bwd(dyg, xg, mean, rstd, gg), o, slack):
+            assert_close(a, b, dtype, name + " by teams", slack=s)
+
+
 @pytest.mark.parametrize("dtype", DTYPES, ids=str)
 @pytest.mark.parametrize("M,packs", [(1, 32769), (2, 40000), (3, 300001), (7, 20000), (7, 70000)], ids=str)
 def test_forward_by_small_teams(cabi, oracle, gpu, dtype, M, packs):

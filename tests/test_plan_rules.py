@@ -352,7 +352,8 @@ def test_backward_of_few_long_norm_rows(rules):
             (32, 448000, 2, 1, 1), (48, 320000, 2, 1, 0), (32, 160000, 4, 0, 0), (100, 112000, 2, 0, 0)]
     for c in few:
         assert f(*c)[0] in (1, 2, 4, 8) and f(*c)[1] == 0, (c, f(*c))
+    # (a LayerNorm call that cannot have its teams keeps the two launches, up to 32 MB)
     for c in team:
-        assert f(*c)[0] == 0 and f(*c)[1] >= 2, (c, f(*c))
+        assert f(*c)[1] >= 2 and (f(*c)[0] > 0) == bool(c[3] and c[0] * c[1] * c[2] <= 32 << 20), (c, f(*c))
     assert [f(2, N, 2, 1, 0)[0] for N in (66400, 163840, 300000, 600000)] == [8, 4, 2, 1] and f(129, 66401, 2, 1, 0)[0] == 0
     assert f(1, 66400, 2, 1, 0) == [0, 0] and f(2, 3000000, 2, 1, 0) == [0, 0]

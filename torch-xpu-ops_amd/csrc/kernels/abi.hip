@@ -168,8 +168,8 @@ int static_scratch(void** out) {
 
 // Exchange memory of the team launches (the workgroups' partial sums), one slot a stream
 // (StreamSlots); per device, like `scratch`.  Zero at load: every word a call reads is tagged with the
-// call's id, so a slot is cleared only when the ids come round again (TeamIds).  16 MiB, and 32 MiB for the strided softmax, whose
-// workgroups pass numbers for every column.
+// call's id, so a slot is cleared only when the ids come round again (TeamIds).  16 MiB, and 32 MiB for
+// the strided softmax, whose workgroups pass numbers for every column.
 static __device__ __align__(256) __attribute__((used)) TeamSlot team_slots[kTeamSlots];
 static __device__ __align__(256) __attribute__((used)) TeamColumns team_columns[kTeamColumnSlots];
 
@@ -1159,7 +1159,7 @@ int mi355x_rownorm_few_rows_plan(rownorm_op op, int64_t M, int64_t N, rownorm_dt
   if (int e = make_plan(OC_NORM_BWD, M, N, esize, current_num_cus(), g_override[(int)op], true, &plan, false,
                         op == ROWNORM_OP_LAYER_NORM_BWD, esize_of((int)w_dtype) > esize))
     return e;
-  if (plan.few_waves == 0) return 0;
+  if (plan.few_waves == 0 || plan.team > 0) return 0;
   const int64_t pieces = (N + 64 * E - 1) / (64 * E), a_block = kFewRowsWaves / plan.few_waves;
   out->reserved = plan.few_waves;
   out->lanes_per_row = 64;

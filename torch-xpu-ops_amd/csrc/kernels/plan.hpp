@@ -62,7 +62,8 @@ struct Plan {
   int split = 0;
   int64_t chunk_packs = 0;
   // norm backward of few rows beyond the registers (norm_bwd_few_rows_kernel): wavefronts that share a piece of
-  // columns; 0: not planned; and the chunks its rows are cut into for their sums
+  // columns; 0: not planned; and the chunks its rows are cut into for their sums.  With a team (`team`) beside it:
+  // where the call cannot have that
   int few_waves = 0, few_chunks = 0;
   int64_t few_chunk_packs = 0;
   // softmax backward of rows beyond the registers of two tensors: grad alone fits
@@ -1198,13 +1199,13 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
   // no longer come out of the L2s, 32 MB together, when they are read again: time over that of the teams, float32 [40,
   // 112000] 17 MB 0.91, [48, 112000] 20 MB 1.06, [48, 160000] 29 MB 1.37; bf16 with float32 weights [64, 160000] 20 MB
   // 0.92, [80, 160000] 24 MB 1.11; bf16 [80, 160000] 24 MB 1.02, [48, 320000] 29 MB 1.07; rows without teams, float32
-  // [24, 320000] 29 MB 0.95, [80, 79997] 24 MB 0.78.
+  // [24, 320000] 29 MB 0.95, [80, 79997] 24 MB 0.78.  Such a LayerNorm call that teams cannot take (captured, dX over an
+  // input, no slot) keeps the two launches, the plan has both (dX over dY, four launches / these: float32 [48, 112000]
+  // 32.7 / 26.3, [48, 160000] 38.4 / 34.1, bf16 [48, 320000] 40.2 / 37.0, [100, 150000] 42.0 / 43.2).
   const int64_t few_part = layer_norm || !p.fast ? 1 : 2;
-  const int64_t few_bytes = layer_norm && norm_bwd_team(M, packs, p.fast && !fused_add, true, num_cus).rounds_ok
-                                ? (int64_t)(esize == 4 ? 16 : wide_weights ? 21 : 24) << 20
-                                : kFewRowsBytes;
+  const int64_t few_team_bytes = layer_norm ? (int64_t)(esize == 4 ? 16 : wide_weights ? 21 : 24) << 20 : kFewRowsBytes;
   if (oc == OC_NORM_BWD && !p.resident && want_cols && want_dx && p.partial_rows > 1 && M * few_part <= kFewRowsMax &&
-      M * packs * 16 * few_part <= few_bytes && ov.G == 0 && ov.V == 0 && ov.bpc == 0 && ov.block == 0) {
+      M * packs * 16 * few_part <= kFewRowsBytes && ov.G == 0 && ov.V == 0 && ov.bpc == 0 && ov.block == 0) {
     const int64_t pieces = (packs + 63) / 64;
     p.few_waves = kFewRowsWaves;
     while (p.few_waves > 1 && pieces * p.few_waves > kFewRowsWaves * (int64_t)num_cus) p.few_waves /= 2;
@@ -1347,7 +1348,8 @@ inline int make_plan(OpClass oc, int64_t M, int64_t N, int esize, int num_cus, c
   // packs a workgroup, dY and X read once (norm_bwd_team_kernel).
   // (override G = -1 with block = 1: the team launch whatever the rounds, for tests)
   const bool team_bwd_forced = ov.G == -1 && ov.V == 0 && ov.block == 1 && ov.bpc == 0;
-  if (oc == OC_NORM_BWD && !p.resident && p.fast && !fused_add && want_dx && p.few_waves == 0 &&
+  if (oc == OC_NORM_BWD && !p.resident && p.fast && !fused_add && want_dx &&
+      (p.few_waves == 0 || M * packs * 16 > few_team_bytes) &&
       ((ov.G == 0 && ov.V == 0 && ov.bpc == 0 && ov.block == 0) || team_bwd_forced)) {
     const NormBwdTeam t = norm_bwd_team(M, packs, p.fast, layer_norm, num_cus);
     if (t.teams >= 1 && (t.rounds_ok || team_bwd_forced)) {
