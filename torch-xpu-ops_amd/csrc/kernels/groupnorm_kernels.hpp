@@ -1016,8 +1016,9 @@ __device__ __forceinline__ int64_t gn_team_row(uint32_t j, int tm, int teams, in
 // X read once: a team of workgroups holds a (sample, group) slab, `wpc` workgroups a channel,
 // V packs of dY and of X a lane.  A workgroup publishes its piece's sums of dy * (x - mean)
 // * rstd and of dy (as words: [1, 128, 512, 512] 43.4 -> 40.4 us, [1, 128, 144, 144] 9.3 -> 8.8
-// against a tag and two numbers); every workgroup adds the team's numbers channel by channel in a fixed order, forms s1 = sum_c gamma_c * db_c and s2 = sum_c gamma_c * dg_c
-// (the reference's ComputeBackwardFusedParamsFunctor, GroupNormKernels.cpp:1088-1165) and
+// against a tag and two numbers); every workgroup adds the team's numbers channel by channel
+// in a fixed order, forms s1 = sum_c gamma_c * db_c and s2 = sum_c gamma_c * dg_c (the
+// reference's ComputeBackwardFusedParamsFunctor, GroupNormKernels.cpp:1088-1165) and
 // writes dX for what it holds; the first workgroup of a channel has the channel's sums
 // and leaves them in the [N, C] partial buffers for the second stage.  SUMS: a team takes whole groups,
 // all samples of one after the other, so that this workgroup meets every number of its channel: it adds them

@@ -985,8 +985,8 @@ struct TeamGroupShape {
 // For slabs, and for rows that are all done in one round, where nothing hides the
 // exchange: bf16 LayerNorm [8, 292096] 8.8 -> 8.1 us, [48, 385536] 15.9 -> 14.6 us,
 // GroupNorm [1, 256, 96, 96] 8.1 -> 7.5 us, [2, 128, 264, 264] 14.4 -> 13.5 us.  Rows in
-// several rounds keep the tag: bound by HBM, they measured 1 to 4 % slower by words
-// ([322, 144512] 45.8 -> 46.3 us, [29, 1699456] 45.0 -> 48.3 us), the polls of waiting
+// several rounds keep the tag: bound by HBM, they measured 1 to 7 % slower by words
+// ([322, 144512] 45.8 -> 47.3 us, [29, 1699456] 45.0 -> 48.3 us), the polls of waiting
 // teams being in the way of the others' loads.
 template <class T, class WT, int V, bool RMS, bool WORDS, bool GROUP = false, class ST = float>
 __global__ void __launch_bounds__(kTeamBlock, kTeamPerCu * kTeamBlock / 256)
@@ -1277,9 +1277,10 @@ norm_fwd_team_kernel(const T* __restrict__ x, const WT* __restrict__ gamma,
 // a team lives in set j % 3; in round j a workgroup requests group j + 2, sums group j + 1
 // (requested a round ago) and publishes its 2 R float64 sums, gathers group j (published a
 // round earlier) and writes its Y: neither the loads nor the exchange are waited for with
-// nothing else to do.  One workgroup a compute unit.  The statistics are those of norm_fwd_team_kernel (float64 sums about the median of
-// the row's first three elements; mean = hi + lo).  A workgroup whose wait runs out sums its
-// R rows itself (Y must not overlap X) and loads its packs again.
+// nothing else to do.  One workgroup a compute unit.  The statistics are those of
+// norm_fwd_team_kernel (float64 sums about the median of the row's first three elements;
+// mean = hi + lo).  A workgroup whose wait runs out sums its R rows itself (Y must not overlap
+// X) and loads its packs again.
 template <class T, class WT, bool RMS, int R, int V>
 __global__ void __launch_bounds__(kTeamBlock, kTeamBlock / 256)
 norm_fwd_rows_team_kernel(const T* __restrict__ x, const WT* __restrict__ gamma,

@@ -249,8 +249,8 @@ softmax_fwd_resident_kernel(const TI* __restrict__ x, TO* __restrict__ y, MaskRe
       float sum[1] = {0.0f};
       float m;
       // (TAIL float32 from 6 packs on: at 6 and 7 the other form keeps 69 and 77 registers of the 64 that two
-      // workgroups a compute unit leave, and spills: [1000, 24983] softmax 48.7 us, 39.3 in halves, 40.8 in two passes; [2000,
-      // 20887] 68.2, 63.4, 64.4)
+      // workgroups a compute unit leave, and spills: [1000, 24983] softmax 48.7 us, 39.3 in halves, 40.8 in two
+      // passes; [2000, 20887] 68.2, 63.4, 64.4)
       if constexpr (!MASKED && FAST && V >= (TAIL && sizeof(TI) == 4 ? 6 : 8)) {
         // the lane's packs in two halves, each with its own maximum and sum of
         // exp(x - maximum): the first half is worked on while the second is still
@@ -529,8 +529,9 @@ softmax_fwd_stream_kernel(const TI* __restrict__ x, TO* __restrict__ y, MaskRef 
 }
 
 // ---------------------------------------------------------------------------
-// Forward for few, very long rows (fewer rows than half the compute units; no mask): a row is held in the registers of a team of
-// workgroups, as in the norm forward for rows beyond the registers (norm_fwd_team_kernel).
+// Forward for few, very long rows (fewer rows than half the compute units; no mask): a row is
+// held in the registers of a team of workgroups, as in the norm forward for rows beyond the
+// registers (norm_fwd_team_kernel).
 // The grid is at most two workgroups of 512 threads a compute unit, all resident at once;
 // workgroup b belongs to team b / team and keeps chunk b % team of the team's current
 // row, V packs a lane.  It finds its chunk's maximum m_c and s_c = sum exp(x - m_c),
@@ -545,10 +546,12 @@ softmax_fwd_stream_kernel(const TI* __restrict__ x, TO* __restrict__ y, MaskRef 
 // its chunk again and goes on; every wave reaches the end of the kernel whatever the
 // other workgroups do.  In a row of no whole number of packs the last chunk starts a few elements
 // early (`before`) and ends with the row: every access is a whole pack, the chunk's sum leaves out
-// the elements that the chunk before holds as well, and both store the same values there.  What bounds few rows is the way from the last chunk's sum to the
-// first store, so the pair crosses as self-validating words (one round trip; a tag beside
-// the numbers, three): bf16 [16, 262144] 8.5 -> 7.4 us, [2, 1048576] 11.3 -> 8.8, [128,
-// 140000] 16.1 -> 15.2; backward 8.1 -> 7.0, 10.7 -> 7.4, 23.6 -> 22.0.
+// the elements that the chunk before holds as well, and both store the same values there.
+// What bounds few rows is the way from the last chunk's sum to the first store, so the pair
+// crosses as self-validating words (one round trip; a tag beside the numbers, three): bf16
+// [16, 262144] 8.5 -> 7.4 us, [2, 1048576] 11.3 -> 8.8, [128, 140000] 16.1 -> 15.2; backward
+// 8.1 -> 7.0, 10.7 -> 7.4, 23.6 -> 22.0.  (Rows in several rounds gain less, and a few lose:
+// [100, 1048576] 91.7 -> 95.4, float32 [100, 524288] 90.0 -> 95.4.)
 template <class TI, class TO, int V>
 __global__ void __launch_bounds__(kTeamBlock, kTeamPerCu * kTeamBlock / 256)
 softmax_fwd_team_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t M, int N, int flags,

@@ -40,8 +40,8 @@ class StreamSlots {
 template <int N>
 class TeamIds {
  public:
-  // The id of call number n (over all slots) in `slot`; *clear: the slot's memory must be zeroed first.  (One thread at a
-  // time for a slot.)
+  // The id of call number n (over all slots) in `slot`; *clear: the slot's memory must be zeroed first.  (One
+  // thread at a time for a slot.)
   unsigned int of(uint64_t n, int slot, bool* clear) {
     const uint64_t turn = n / kTeamCallIds;
     *clear = turn_[slot] != turn;
